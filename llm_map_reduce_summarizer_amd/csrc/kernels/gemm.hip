@@ -40,6 +40,11 @@
 //   * the MFMA computes the transposed tile (A = W fragment, B = X fragment) so each lane ends with 4
 //     consecutive output columns of one row: 8-byte bf16 stores, and the fused SwiGLU epilogue of the
 //     [8 gate | 8 up]-interleaved gate_up weight is a lane-xor-32 exchange.
+//   * split tail: tiles behind the last whole round of 256 (all of them where M and N are small) would leave most CUs
+//     idle for a full K loop, so each is cut into S slices of K.  A slice writes its fp32 accumulators to scratch in
+//     register order (lane-contiguous 16-B stores) and gemm_tail_kernel adds them in slice order and runs the
+//     epilogue: a second launch and no ticket, so results do not depend on arrival and concurrent streams share
+//     nothing.  Which S: ops/hip.py gemm_splits.
 //   * M32 variant: the same ring, phases and quadrants on 32x32 MFMA tiles (v_mfma_f32_32x32x16_bf16 /
 //     v_mfma_scale_f32_32x32x64_f8f6f4); a lane then holds 4 register groups of 4 consecutive columns,
 //     and the SwiGLU gate / up halves of a 16-column group sit in adjacent groups of the same lane.
@@ -52,7 +57,7 @@ constexpr int HALF = 16384;
 constexpr int TILE = 4 * HALF;
 constexpr int LOOK = 6;
 
-enum { GEPI_BF16 = 0, GEPI_SWIGLU = 1, GEPI_GELU = 2 };
+enum { GEPI_BF16 = 0, GEPI_SWIGLU = 1, GEPI_GELU = 2, GEPI_F32 = 3 };
 
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 
@@ -66,6 +71,9 @@ struct GemmArgs {
     int M, N, kb;           // kb = K-tiles (128 bytes of every row each)
     int kbw;                // W's K-tiles: kb, or kb / 2 for two-term X (X tiles kt >= kbw re-read W tile kt - kbw)
     int tiles_m, tiles_n, group_m;
+    int whole;    // raster positions below it run whole, the others in ``splits`` slices of K each
+    int splits;
+    float* part;  // [tiles - whole][splits][TILE_F] fp32 accumulators of the slices
     GluArgs glu;  // GEPI_SWIGLU
 #ifdef MRSUM_CLOCK_STAMPS
     unsigned long long* stamps;  // diagnostic build only (tools/gemm_clock.py): [grid][2] shader / 100 MHz ticks
@@ -100,10 +108,16 @@ __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, char* dst, int v
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)dst, 16, voff, soff, 0, 0);
 }
 
-// bijective XCD remap (blocks b, b+8, ... share an XCD) then a grouped raster of group_m tile rows
-__device__ __forceinline__ void tile_of(int bid, int nwg, int tiles_m, int tiles_n, int group_m, int& tm, int& tn) {
+constexpr int TILE_F = 256 * 256;  // accumulators of one tile
+
+// bijective XCD remap: blocks b, b+8, ... (one XCD's) get consecutive positions
+__device__ __forceinline__ int xcd_position(int bid, int nwg) {
     const int xcd = bid & 7, local = bid >> 3, q = nwg >> 3, r = nwg & 7;
-    const int p = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + local;
+    return (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + local;
+}
+
+// grouped raster of group_m tile rows
+__device__ __forceinline__ void tile_of(int p, int tiles_m, int tiles_n, int group_m, int& tm, int& tn) {
     const int gsz = group_m * tiles_n;
     const int g = p / gsz, first = g * group_m;
     const int gm = min(tiles_m - first, group_m);
@@ -128,7 +142,19 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmArgs a) {
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = w >> 2, wc = w & 3;
     int tm, tn;
-    tile_of(blockIdx.x, gridDim.x, a.tiles_m, a.tiles_n, a.group_m, tm, tn);
+    // whole tiles first; then the slices, one K range after the other, so that an XCD's slices read the same panels
+    int pos, slice = -1, kt0 = 0, kt1 = a.kb;
+    if ((int)blockIdx.x < a.whole) {
+        pos = xcd_position(blockIdx.x, a.whole);
+    } else {
+        const int rest = a.tiles_m * a.tiles_n - a.whole;
+        const int p = xcd_position(blockIdx.x - a.whole, gridDim.x - a.whole);
+        slice = p / rest;
+        pos = a.whole + p - slice * rest;
+        kt0 = a.kb * slice / a.splits;
+        kt1 = a.kb * (slice + 1) / a.splits;
+    }
+    tile_of(pos, a.tiles_m, a.tiles_n, a.group_m, tm, tn);
     const int m0 = tm * 256, n0 = tn * 256;
     const int xrows = min(a.M - m0, 256), wrows = min(a.N - n0, 256);
     const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
@@ -143,10 +169,11 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmArgs a) {
     const int vx0 = srow * a.ldx_b + ch0, vx1 = (srow + 8) * a.ldx_b + ch1;
     const int vw0 = srow * a.ldw_b + ch0, vw1 = (srow + 8) * a.ldw_b + ch1;
     const int xh = 128 * a.ldx_b, wh = 128 * a.ldw_b;
-    const int nk = a.kb, htot = 4 * nk;
+    const int nk = kt1 - kt0, htot = 4 * nk;
 
     auto stage = [&](int part, int kt) {
         char* dst = lds + ((4 * kt + part) % NS) * HALF + w * 2048;
+        kt += kt0;
         const int soff = kt * 128;
         if (part == 0 || part == 3) {
             const int o = part == 3 ? xh : 0;
@@ -266,7 +293,7 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmArgs a) {
     };
     auto slot = [&](int kt, int part) -> const char* { return lds + ((4 * kt + part) % NS) * HALF; };
     auto ktile = [&](int kt, auto tail) {
-        const int xsc = FP8 && kt >= a.kbw ? 123 : 127;  // E8M0 2^-4 on the lo half of two-term X
+        const int xsc = FP8 && kt0 + kt >= a.kbw ? 123 : 127;  // E8M0 2^-4 on the lo half of two-term X
         // phase 0: quadrant (0, 0) -- X0, W0
         read_x(slot(kt, 0));
         read_w(slot(kt, 1), wf0);
@@ -298,6 +325,22 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmArgs a) {
     for (; kt < nk; ++kt) ktile(kt, std::true_type{});
     if (wr == 0) bar();
 
+    if constexpr (!M32) {
+        if (slice >= 0) {
+            // accumulator vector v of this lane at [v][thread]; 16-row blocks past M are skipped
+            f32x4* out = reinterpret_cast<f32x4*>(a.part + ((size_t)(pos - a.whole) * a.splits + slice) * TILE_F) + tid;
+#pragma unroll
+            for (int qm = 0; qm < 2; ++qm)
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    if (128 * qm + 64 * wr + 16 * b >= xrows) continue;
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) out[((qm * 4 + b) * 4 + v) * 512] = acc[qm][b][v >> 1][v & 1];
+                }
+            return;
+        }
+    }
+
     // epilogue: lane holds C[m][n .. n+3] of every 16 x 16 block, m = .. + (lane & 15), n = .. + 4 (lane >> 4).
     // LEPI: every wave writes its bf16 results into a [256 rows][RB bytes] LDS image of the whole tile
     // (16-B unit u of row r at u ^ (r & 7): 2-way ds_write_b64, conflict-free ds_read_b128), then each
@@ -322,6 +365,11 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmArgs a) {
         if constexpr (EPI == GEPI_GELU) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) v[j] = gelu_tanh<bf16>(v[j]);
+        }
+        if constexpr (EPI == GEPI_F32) {
+            if (m0 + rl < a.M && n0 + gcol < a.N)
+                *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.c) + (size_t)(m0 + rl) * a.ldc + n0 + (cbyte >> 1)) = v;
+            return;
         }
         const uint2 pk = make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
         if constexpr (LEPI) {
@@ -422,6 +470,56 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmArgs a) {
 #endif
 }
 
+// Adds the slices of the split tiles and runs the epilogue.  One workgroup per (tile, 2 x 16 rows): the four vectors
+// that every lane of gemm_kernel holds for one of its eight row blocks.
+template <bool FP8, int EPI>
+__global__ __launch_bounds__(512) void gemm_tail_kernel(const GemmArgs a) {
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, wr = w >> 2, wc = w & 3, g4 = lane >> 4;
+    const int t = blockIdx.x >> 3, rb = blockIdx.x & 7;
+    int tm, tn;
+    tile_of(a.whole + t, a.tiles_m, a.tiles_n, a.group_m, tm, tn);
+    const int n0 = tn * 256, r0 = tm * 256 + 128 * (rb >> 2) + 64 * wr + 16 * (rb & 3);
+    if (r0 >= a.M) return;
+    const f32x4* in = reinterpret_cast<const f32x4*>(a.part + (size_t)t * a.splits * TILE_F) + rb * 4 * 512 + tid;
+    f32x4 v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = in[j * 512];
+    for (int s = 1; s < a.splits; ++s) {
+        in += TILE_F / 4;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] += in[j * 512];
+    }
+    const int m = r0 + (lane & 15);
+    float rs = 1.f;
+    if constexpr (FP8) rs = a.sx[min(m, a.M - 1)];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int cb = n0 + 128 * (j >> 1) + 32 * wc + 16 * (j & 1);  // 16-column block, wholly in or out of range
+        if constexpr (FP8) {
+            const float4 s4 = *reinterpret_cast<const float4*>(a.sw + min(cb + 4 * g4, a.N - 4));
+            v[j][0] *= rs * s4.x; v[j][1] *= rs * s4.y; v[j][2] *= rs * s4.z; v[j][3] *= rs * s4.w;
+        }
+        int col = cb + 4 * g4;
+        if constexpr (EPI == GEPI_SWIGLU) {  // the up columns sit in lane xor 32
+            f32x4 up;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) up[k] = __shfl_xor(v[j][k], 32, 64);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[j][k] = glu(v[j][k], up[k], a.glu);
+            col = (cb >> 1) + 4 * g4;
+        } else if constexpr (EPI == GEPI_GELU) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[j][k] = gelu_tanh<bf16>(v[j][k]);
+        }
+        if (m >= a.M || cb >= a.N || (EPI == GEPI_SWIGLU && lane >= 32)) continue;
+        if constexpr (EPI == GEPI_F32)
+            *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.c) + (size_t)m * a.ldc + col) = v[j];
+        else
+            *reinterpret_cast<uint2*>(reinterpret_cast<bf16*>(a.c) + (size_t)m * a.ldc + col) =
+                make_uint2(pack2(v[j][0], v[j][1]), pack2(v[j][2], v[j][3]));
+    }
+}
+
 #ifdef MRSUM_CLOCK_STAMPS
 static unsigned long long* g_stamps = nullptr;
 static int g_nstamps = 0;
@@ -436,18 +534,22 @@ MRSUM_API int mrsum_gemm_stamps(unsigned long long* host, int max_words) {
 #endif
 
 // x [M, K] (row stride ldx elements), w [N, K] (ldw), c [M, N] bf16 (ldc) -- or [M, N / 2] for
-// epi 1 (SwiGLU of the [8 gate | 8 up]-interleaved gate_up rows) -- or gelu(C) for epi 2 (bf16 only).  fp8: x, w are e4m3fn bytes,
+// epi 1 (SwiGLU of the [8 gate | 8 up]-interleaved gate_up rows) -- or gelu(C) for epi 2, or C in
+// fp32 for epi 3 (both bf16 operands only).  fp8: x, w are e4m3fn bytes,
 // sx [M] / sw [N] fp32 row scales; split: x is two-term [hi | lo] of 2K bytes per row over w's K.
+// whole / splits / part: tiles from raster position ``whole`` on run in ``splits`` slices of K through ``part``
+// [tiles - whole][splits][65536] fp32 (splits 1: none, part unused;
+// 16x16 MFMA tiles only).
 // Requirements (checked by the Python wrapper too): K % 64 (bf16) / K % 128 (fp8), N % 16, 16-byte
 // aligned rows.
 MRSUM_API int mrsum_gemm(const void* x, int ldx, const void* w, int ldw, void* c, int ldc, int M, int N, int K,
                          int fp8, int epi, const float* sx, const float* sw, int group_m, int split, float glu_limit,
-                         float glu_alpha, float glu_shift, hipStream_t s) {
+                         float glu_alpha, float glu_shift, int whole, int splits, float* part, hipStream_t s) {
     if (M <= 0 || N <= 0) return 0;
     const int es = fp8 ? 1 : 2;
     if ((K * es) % 128 || N % 16 || (ldx * es) % 16 || (ldw * es) % 16 || ldc % 4) return (int)hipErrorInvalidValue;
     if ((size_t)256 * ldx * es >= (1u << 31) || (size_t)256 * ldw * es >= (1u << 31)) return (int)hipErrorInvalidValue;
-    if (epi < GEPI_BF16 || epi > GEPI_GELU || (epi == GEPI_GELU && (fp8 || ((group_m >> 8) & 1))))
+    if (epi < GEPI_BF16 || epi > GEPI_F32 || (epi >= GEPI_GELU && (fp8 || ((group_m >> 8) & 1))))
         return (int)hipErrorInvalidValue;
     if (fp8 && (!sx || !sw)) return (int)hipErrorInvalidValue;
     GemmArgs a;
@@ -466,7 +568,14 @@ MRSUM_API int mrsum_gemm(const void* x, int ldx, const void* w, int ldw, void* c
     const bool m32 = (group_m >> 8) & 1;
     group_m &= 255;
     a.group_m = group_m > 0 ? group_m : 4;
-    const dim3 grid(a.tiles_m * a.tiles_n), block(512);
+    const int tiles = a.tiles_m * a.tiles_n;
+    if (splits > 1 && (whole < 0 || whole >= tiles || splits > a.kb || !part || m32))
+        return (int)hipErrorInvalidValue;
+    a.splits = splits > 1 ? splits : 1;
+    a.whole = splits > 1 ? whole : tiles;
+    a.part = part;
+    const int rest = tiles - a.whole;
+    const dim3 grid(a.whole + rest * a.splits), block(512);
 #ifdef MRSUM_CLOCK_STAMPS
     static unsigned long long* stamps = nullptr;
     static size_t nstamps = 0;
@@ -491,6 +600,7 @@ MRSUM_API int mrsum_gemm(const void* x, int ldx, const void* w, int ldw, void* c
     } else {                                                                       \
         if (lepi) gemm_kernel<F, E, 8, true, false><<<grid, block, 0, s>>>(a);     \
         else gemm_kernel<F, E, 8, false, false><<<grid, block, 0, s>>>(a);         \
+        if (rest) gemm_tail_kernel<F, E><<<rest * 8, block, 0, s>>>(a);            \
     }
     if (fp8) {
         if (epi == GEPI_SWIGLU) { GEMM_LAUNCH(true, GEPI_SWIGLU) } else { GEMM_LAUNCH(true, GEPI_BF16) }
@@ -500,6 +610,10 @@ MRSUM_API int mrsum_gemm(const void* x, int ldx, const void* w, int ldw, void* c
         } else if (epi == GEPI_GELU) {
             if (lepi) gemm_kernel<false, GEPI_GELU, 8, true, false><<<grid, block, 0, s>>>(a);
             else gemm_kernel<false, GEPI_GELU, 8, false, false><<<grid, block, 0, s>>>(a);
+            if (rest) gemm_tail_kernel<false, GEPI_GELU><<<rest * 8, block, 0, s>>>(a);
+        } else if (epi == GEPI_F32) {
+            gemm_kernel<false, GEPI_F32, 8, false, false><<<grid, block, 0, s>>>(a);
+            if (rest) gemm_tail_kernel<false, GEPI_F32><<<rest * 8, block, 0, s>>>(a);
         } else {
             GEMM_LAUNCH(false, GEPI_BF16)
         }

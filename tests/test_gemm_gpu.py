@@ -139,3 +139,40 @@ def test_gemm_graph_capture():
     g.replay()
     torch.cuda.synchronize()
     _check(out, x.float() @ w.float().t())
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 32, 2048), (130, 544, 2112), (257, 4096, 2112), (4097, 4096, 2048)])
+@pytest.mark.parametrize("epi", ["bf16", "swiglu", "gelu", "f32"])
+def test_gemm_split_tail(M, N, K, epi):
+    """Tiles behind the last whole round run in slices of K that a second launch adds: one tile of one row, a ragged
+    last slice, few tiles, and 16 sliced tiles behind a whole round; repeated calls are the same bits."""
+    assert hip.gemm_splits(M, N, K // 64)[1] > 1
+    x, w = _rand(M, K, seed=12, scale=0.5, offset=0.02), _rand(N, K, seed=13, scale=0.03, offset=0.001)
+    if epi == "swiglu":
+        w[-16:] *= 2
+    kw = {} if epi == "bf16" else {epi: True}
+    out = hip.gemm(x, w, **kw)
+    assert torch.equal(out, hip.gemm(x, w, **kw))
+    y = x.double() @ w.double().t()
+    if epi == "f32":
+        # each of the K products and sums rounds by at most 2^-24 of the sum of magnitudes
+        bound = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+        assert out.dtype == torch.float32 and bool(((out.double() - y).abs() <= bound).all())
+        return
+    if epi == "swiglu":
+        g = y.reshape(M, -1, 2, 8)
+        y = (torch.nn.functional.silu(g[:, :, 0]) * g[:, :, 1]).reshape(M, -1)
+    elif epi == "gelu":
+        y = torch.nn.functional.gelu(y, approximate="tanh")
+    # one bf16 rounding (2^-9 relative) behind fp32 sums; the activations' fp32 exponentials add far less
+    assert bool(((out.double() - y).abs() <= 2.0 ** -8 * y.abs() + 1e-4).all())
+
+
+@pytest.mark.parametrize("M", [128, 129, 256, 257])
+def test_stream_parts_beyond_tall_tiles(M):
+    """Split-K slab consumers get one fp32 slab of the tile GEMM above the stream kernel's tallest x tile."""
+    x, w = _rand(M, 1024, seed=14, scale=0.5), _rand(4096, 1024, seed=15, scale=0.03)
+    parts = hip.linear_parts(x, w, 2, nt=4, kernel="stream")
+    assert parts.dtype == torch.float32 and parts.shape == (2 if M <= 128 else 1, M, 4096)
+    bound = 1024 * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    assert bool(((parts.sum(0).double() - x.double() @ w.double().t()).abs() <= bound).all())
