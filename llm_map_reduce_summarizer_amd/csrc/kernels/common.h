@@ -212,6 +212,55 @@ __device__ __forceinline__ float gelu_tanh(float z) {
 }
 
 
+// Sums over aligned groups of 16 lanes without LDS traffic.
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E;             // quad_perm [1 0 3 2], [2 3 0 1]
+constexpr int DPP_HALF_MIRROR = 0x141, DPP_MIRROR = 0x140;  // lane i of 8 <- 7 - i, lane i of 16 <- 15 - i
+__device__ __forceinline__ float sum16(float v) {
+    v += dpp<DPP_MIRROR>(v);
+    v += dpp<DPP_HALF_MIRROR>(v);
+    v += dpp<DPP_XOR2>(v);
+    return v + dpp<DPP_XOR1>(v);
+}
+// R sums at once: lane l ends with the sum of v[(l & 15) * R / 16]; each exchange halves what is left to add
+template <int R>
+__device__ __forceinline__ float sum16_scatter(const float (&v)[R], int l) {
+    static_assert(R == 1 || R == 2 || R == 4, "rows");
+    if constexpr (R == 1) {
+        return sum16(v[0]);
+    } else {
+        const bool hi = l & 8;
+        float s;
+        if constexpr (R == 4) {
+            const float a = (hi ? v[2] : v[0]) + dpp<DPP_MIRROR>(hi ? v[0] : v[2]);
+            const float b = (hi ? v[3] : v[1]) + dpp<DPP_MIRROR>(hi ? v[1] : v[3]);
+            const bool h4 = l & 4;
+            s = (h4 ? b : a) + dpp<DPP_HALF_MIRROR>(h4 ? a : b);
+        } else {
+            s = (hi ? v[1] : v[0]) + dpp<DPP_MIRROR>(hi ? v[0] : v[1]);
+            s += dpp<DPP_HALF_MIRROR>(s);
+        }
+        s += dpp<DPP_XOR2>(s);
+        return s + dpp<DPP_XOR1>(s);
+    }
+}
+
+// four columns of a bf16 / fp32 row; ``whole``: 4-element aligned, else one by one up to ``n``
+template <typename T>
+__device__ __forceinline__ float4 row4(const T* p, bool whole, int n) {
+    if (n <= 0) return make_float4(0.f, 0.f, 0.f, 0.f);
+    if (whole) {
+        if constexpr (sizeof(T) == 4) return *reinterpret_cast<const float4*>(p);
+        const uint2 v = *reinterpret_cast<const uint2*>(p);
+        return make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
+                           __uint_as_float(v.y & 0xffff0000u));
+    }
+    return make_float4((float)p[0], n > 1 ? (float)p[1] : 0.f, n > 2 ? (float)p[2] : 0.f, n > 3 ? (float)p[3] : 0.f);
+}
+
 static inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
 // Columns [at, at + n) of a projection's slabs through gelu into rows out + t * ldo (n = 0: nothing): a job that kernels

@@ -341,17 +341,161 @@ static int launch_step(const void* xbc, const ScanArgs& a, const SegArgs& sg, in
     return (int)hipGetLastError();
 }
 
-// Segments [seg0, seg0 + nseg) token by token.  xbc [T][ldx] bf16 / fp32 (x32), u: dt columns at dt_at.
+// ------------------------------------------------------------------------------------------------ recurrence, portions
+constexpr int PORTION = 16;  // rows staged at a time
+
+// The same recurrence over longer segments.  A (segment, head) is one serial chain of rows: reading each row's operands
+// from memory inside the chain costs a memory latency a row (2.3 us).  Here blocks of 16 rows arrive in LDS ahead of
+// their use, with the step sizes and decays already computed, and what is left per row and lane is 12 NV R multiply-adds
+// on 4 NV R state values, 2 NV LDS reads and a DPP sum.  16 lanes hold a state row, R rows (value columns) per lane
+// group; a block has 16 R value columns of one head.
+template <bool PARTS, typename T, int NV, int R>
+__global__ __launch_bounds__(256) void ssm_portion_kernel(const T* __restrict__ xbc, ScanArgs a, SegArgs sg) {
+    constexpr int NF = 64 * NV, RB = 16 * R;
+    __shared__ __attribute__((aligned(16))) float s_bc[2][PORTION][2][NF];
+    __shared__ float s_x[2][PORTION][RB];
+    __shared__ float2 s_d[2][PORTION];  // step size, decay
+    const int seg = a.seg0 + blockIdx.z, head = blockIdx.y, tid = threadIdx.x;
+    const int r = tid >> 4, l = tid & 15, p0 = blockIdx.x * RB;
+    const int b = sg.cu[seg], e = sg.cu[seg + 1];
+    float* st = a.state + ((size_t)sg.slots[seg] * a.heads + head) * a.P * a.N4;
+    const bool cont = sg.pos0[seg] > 0;
+    const float an = a.a_neg[head], db = a.dt_bias[head], dsk = a.d_skip[head];
+    const int inner = a.heads * a.P, g = head / (a.heads / a.groups);
+    const int bcol = inner + g * a.N, cstep = a.groups * a.N;
+    const bool whole = a.N % 4 == 0 && a.ldx % 4 == 0 && inner % 4 == 0 && (uintptr_t)xbc % (4 * sizeof(T)) == 0;
+    float4 S[R][NV];
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const int p = p0 + r * R + i, n = 4 * (l + 16 * v);
+            S[i][v] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (cont && p < a.P && n < a.N4) S[i][v] = *reinterpret_cast<const float4*>(st + (size_t)p * a.N4 + n);
+        }
+    // lane group r fetches row r of the block: B and C, and R value columns a lane; its first lane the step size
+    float4 fb[2][NV];
+    float fx[R], fd = 0.f;
+    auto fetch = [&](int t0) {
+        const int t = t0 + r;
+        const bool in = t < e;
+        const T* row = xbc + (size_t)(in ? t : b) * a.ldx;
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int v = 0; v < NV; ++v) {
+                const int n = 4 * (l + 16 * v);
+                fb[k][v] = row4(row + bcol + k * cstep + n, whole, in ? a.N - n : 0);
+            }
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            const int p = p0 + l + 16 * i;
+            fx[i] = in && p < a.P ? (float)row[head * a.P + p] : 0.f;
+        }
+        if (l == 0 && in) fd = proj_at<PARTS>(a.u, t, a.dt_at + head);
+    };
+    auto put = [&](int buf, int t0) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int v = 0; v < NV; ++v) *reinterpret_cast<float4*>(&s_bc[buf][r][k][4 * (l + 16 * v)]) = fb[k][v];
+#pragma unroll
+        for (int i = 0; i < R; ++i) s_x[buf][r][l + 16 * i] = fx[i];
+        if (l == 0) {  // rows past the end leave the state as it is
+            const float dt = t0 + r < e ? softplus(fd + db) : 0.f;
+            s_d[buf][r] = make_float2(dt, expf(an * dt));
+        }
+    };
+    fetch(b);
+    put(0, b);
+    __syncthreads();
+    int buf = 0;
+    const int yi = l * R / 16, yp = p0 + r * R + yi;  // the value column whose sum this lane ends with
+    const bool writes = l % (16 / R) == 0 && yp < a.P;
+    for (int t0 = b; t0 < e; t0 += PORTION, buf ^= 1) {
+        const bool more = t0 + PORTION < e;
+        if (more) fetch(t0 + PORTION);
+#pragma unroll 4
+        for (int k = 0; k < PORTION; ++k) {
+            const float2 d = s_d[buf][k];
+            float4 B[NV], C[NV];
+#pragma unroll
+            for (int v = 0; v < NV; ++v) {
+                B[v] = *reinterpret_cast<const float4*>(&s_bc[buf][k][0][4 * (l + 16 * v)]);
+                C[v] = *reinterpret_cast<const float4*>(&s_bc[buf][k][1][4 * (l + 16 * v)]);
+            }
+            float y[R];
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                const float dx = d.x * s_x[buf][k][r * R + i];
+                y[i] = 0.f;
+#pragma unroll
+                for (int v = 0; v < NV; ++v) {
+                    float4& w = S[i][v];
+                    w.x = d.y * w.x + dx * B[v].x;
+                    w.y = d.y * w.y + dx * B[v].y;
+                    w.z = d.y * w.z + dx * B[v].z;
+                    w.w = d.y * w.w + dx * B[v].w;
+                    y[i] += w.x * C[v].x + w.y * C[v].y + w.z * C[v].z + w.w * C[v].w;
+                }
+            }
+            const float s = sum16_scatter<R>(y, l);
+            if (writes && t0 + k < e)
+                a.y[(size_t)(t0 + k) * inner + head * a.P + yp] = s + dsk * s_x[buf][k][r * R + yi];
+        }
+        if (more) put(buf ^ 1, t0 + PORTION);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const int p = p0 + r * R + i, n = 4 * (l + 16 * v);
+            if (p < a.P && n < a.N4) *reinterpret_cast<float4*>(st + (size_t)p * a.N4 + n) = S[i][v];
+        }
+}
+
+template <bool PARTS, typename T>
+static int launch_portion(const void* xbc, const ScanArgs& a, const SegArgs& sg, int nseg, hipStream_t s) {
+#define PK(V, R) ssm_portion_kernel<PARTS, T, V, R><<<dim3(ceil_div(a.P, 16 * R), a.heads, nseg), 256, 0, s>>>((const T*)xbc, a, sg)
+#define PK_R(V)                                                                     \
+    {                                                                               \
+        if (r == 1) PK(V, 1);                                                       \
+        else if (r == 2) PK(V, 2);                                                  \
+        else PK(V, 4);                                                              \
+    }
+    // One row per lane group has the shortest row time, more rows share the LDS reads: one while two blocks a CU hold
+    // them all.  fp32, state 128, 64-wide heads, us at 1 / 2 / 4 rows: 128 heads, one segment of 900 rows (512 blocks)
+    // 246 / 285 / 371 (read from memory inside the chain: 2180); 64 heads, four of 1200 (1024) 476 / 425 / 492; 128 heads,
+    // four of 1200 (2048) 920 / 634 / 563.
+    const long long one = (long long)ceil_div(a.P, 16) * a.heads * nseg;  // blocks at one row per lane group
+    const int r = one <= 512 ? 1 : one <= 1024 ? 2 : 4;
+    if (a.N4 <= 64) PK_R(1)
+    else if (a.N4 <= 128) PK_R(2)
+    else if (a.N4 <= 256) PK_R(4)
+    else return (int)hipErrorInvalidValue;
+#undef PK_R
+#undef PK
+    return (int)hipGetLastError();
+}
+
+// Segments [seg0, seg0 + nseg) token by token (portions: in the form for longer segments, N <= 256).  xbc [T][ldx] bf16 /
+// fp32 (x32), u: dt columns at dt_at.
 MRSUM_API int mrsum_ssm_step(const void* xbc, int ldx, int x32, const void* u, int S, int ld, int T, int dt_at,
                              const float* dt_bias, const float* a_neg, const float* d_skip, float* state,
                              const int* cu, const int* slots, const int* pos0, int seg0, int nseg, float* y, int heads,
-                             int P, int N, int groups, hipStream_t s) {
+                             int P, int N, int groups, int portions, hipStream_t s) {
     if (T <= 0 || nseg <= 0) return 0;
-    if (heads % groups || heads > 65535 || nseg > 65535 || dt_at + heads > ld || ldx < heads * P + 2 * groups * N || (x32 && S < 1))
+    if ((portions && !cu) || heads % groups || heads > 65535 || nseg > 65535 || dt_at + heads > ld || ldx < heads * P + 2 * groups * N || (x32 && S < 1))
         return (int)hipErrorInvalidValue;
     const ScanArgs a{ProjSrc{u, S, (size_t)T * ld, ld}, dt_at, dt_bias, a_neg, d_skip, state, y, ldx,
                      heads, P, N, (N + 3) / 4 * 4, groups, seg0};
     const SegArgs sg{cu, nullptr, slots, pos0};
+    if (portions) {
+        if (x32) return launch_portion<true, float>(xbc, a, sg, nseg, s);
+        if (S) return launch_portion<true, bf16>(xbc, a, sg, nseg, s);
+        return launch_portion<false, bf16>(xbc, a, sg, nseg, s);
+    }
     if (x32) return launch_step<true, float>(xbc, a, sg, nseg, s);
     if (S) return launch_step<true, bf16>(xbc, a, sg, nseg, s);
     return launch_step<false, bf16>(xbc, a, sg, nseg, s);

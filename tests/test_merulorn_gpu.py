@@ -167,6 +167,31 @@ def test_state_space_scan(heads, P, N, groups, dtype):
             b += n
 
 
+@pytest.mark.parametrize("copies,dtype,N", [(1, F32, 24), (2, F32, 24), (4, F32, 7), (1, BF, 260 - 12)])
+def test_state_space_portions_token_by_token(copies, dtype, N):
+    """Portions around the 16 rows that the stepped kernel stages at a time, few and many (segment, head) pairs (one, two
+    and four state rows per lane group), and the 16-bit head size that the chunked form does not take."""
+    from llm_map_reduce_summarizer_amd import ops
+    from llm_map_reduce_summarizer_amd.ops import hip
+    heads, P, groups = 64, 20 if dtype == F32 else 136, 2
+    lens = [1, 15, 16, 17, 33] * copies
+    assert not (dtype == BF and hip.ssm_chunk_ok(P, N))
+    T, Cp = sum(lens), heads * P + 2 * groups * N + (-(2 * groups * N)) % 8
+    lens.sort(key=lambda n: n != 1)
+    xbc, u = rnd(T, Cp, std=0.7).to(dtype), rnd(1, T, heads, seed=1)
+    vec = [rnd(heads, seed=2, std=1.5) - 2, -torch.exp(rnd(heads, seed=3)), rnd(heads, seed=4)]
+    slots, pos0 = list(range(1, len(lens) + 1)), [7 * (i % 2) for i in range(len(lens))]
+    state = rnd(len(lens) + 1, heads, P, N + (-N) % 4, seed=5, std=0.5)
+    state[..., N:] = 0
+    got_s, want_s = dev(state), state.clone()
+    segs = segments(lens, slots, pos0)
+    got = ops.ssm_scan(dev(xbc), dev(u), 0, *map(dev, vec), got_s, segs, heads, P, N, groups)
+    host = ops.Segments(segs.slots.cpu(), segs.pos0.cpu(), segs.cu.cpu(), segs.row_seg.cpu(), lens)
+    want = ops.ssm_scan(xbc, u, 0, *vec, want_s, host, heads, P, N, groups)
+    # both sides are fp32: a few roundings of 2^-24 a row, over up to 33 rows of a decaying state
+    assert rel(got, want) < 3e-6 and rel(got_s, want_s) < 3e-6
+
+
 def scan_with_state(x, B, C, dt, A_log, D, groups, S0):
     """The oracle's scan continued from S0 [heads, P, N]: the carried state as one more leading token is not possible,
     so its contribution decays beside the oracle's own output."""

@@ -294,6 +294,39 @@ def test_delta_rule(H, G, dim, vdim, dtype, monkeypatch):
             b = e
 
 
+@pytest.mark.parametrize("copies,dim,dtype", [(1, 24, F32), (3, 24, F32), (6, 7, F32), (1, 40, F32)])
+def test_delta_portions_token_by_token(copies, dim, dtype):
+    """Portions around the 16 rows that the stepped kernel stages at a time; one, two and four state rows per lane group."""
+    from llm_map_reduce_summarizer_amd import ops
+    from llm_map_reduce_summarizer_amd.engine import mixers
+    from llm_map_reduce_summarizer_amd.engine.config import DeltaSpec
+    H, G, vdim = 64, 32, 20
+    m = mixers.DeltaMixer(DeltaSpec(H, G, dim, vdim, 2), torch.device(DEV), dtype)
+    cols = [0]
+
+    def take(n):
+        at = cols[0]
+        cols[0] = -(-(at + n) // 8) * 8
+        return at
+    m.columns(take)
+    m.col = 8
+    lens = sorted([1, 15, 16, 17, 33] * copies, key=lambda n: n != 1)
+    T = sum(lens)
+    x, u = rnd(T, m.channels, std=0.8), rnd(1, T, cols[0], seed=1)
+    vec = [-torch.exp(rnd(H, seed=2)), rnd(H, seed=3) - 3, rnd(vdim, seed=4, std=0.2) + 1]
+    slots, pos0 = list(range(1, len(lens) + 1)), [7 * (i % 2) for i in range(len(lens))]
+    state = rnd(len(lens) + 1, H, vdim, dim + (-dim) % 4, seed=5, std=0.5)
+    state[..., dim:] = 0
+    got_s, want_s = dev(state), state.clone()
+    got, want = torch.zeros(T, m.col + m.width, device=DEV), torch.zeros(T, m.col + m.width)
+    segs = segments(lens, slots, pos0)
+    host = ops.Segments(segs.slots.cpu(), segs.pos0.cpu(), segs.cu.cpu(), segs.row_seg.cpu(), lens)
+    ops.delta_mix(dev(x), dev(u), m, *map(dev, vec), 1e-3, got_s, segs, got)
+    ops.delta_mix(x, u, m, *vec, 1e-3, want_s, host, want)
+    # both sides are fp32; corrections chain through at most 33 rows
+    assert rel(got, want) < 1e-5 and rel(got_s, want_s) < 1e-5
+
+
 # ------------------------------------------------------------------ whole models
 @pytest.mark.parametrize("name", sorted(M.CONFIGS))
 @pytest.mark.parametrize("dtype", DTYPES)
