@@ -3,7 +3,8 @@
 //     C[M, N] = X[M, K] . W[N, K]^T        K % 32 == 0
 //
 // 128 x 128 output tile per 256-thread workgroup, two workgroups per CU; wave (wr, wc) owns 64 x 64 outputs as 4 x 4
-// blocks.  K-tiles of 32 (128 bytes a row) arrive by LDS-DMA in two buffers, chunk c of row r at c ^ ((r >> 1) & 7)
+// blocks, or for M <= 64 (LOW) wave w 64 x 32, so that all four SIMDs have work
+// (64 x 28672 x 4096: 248 -> 145 us; a form of its own: a branch cost the others 9 %).  K-tiles of 32 (128 bytes a row) arrive by LDS-DMA in two buffers, chunk c of row r at c ^ ((r >> 1) & 7)
 // (conflict-free b128 fragment reads); a fragment's four floats feed four instructions, so a K-tile is 16 LDS reads for
 // 128 instructions of 32 cycles, and the matrix cores set the time (1.7 us a K-tile) once a CU has work.  16-row
 // blocks past M are skipped.  903 x 28672 x 4096: 2310 (64 x 64 tiles, loads between barriers) -> 1650 us, 129 TFLOP/s of
@@ -46,6 +47,7 @@ __device__ __forceinline__ void store_c(const Gemm32Args& a, int m, int n, const
 }
 }  // namespace
 
+template <bool LOW>
 __global__ __launch_bounds__(256, 2) void gemm32_kernel(const Gemm32Args a) {
     __shared__ __attribute__((aligned(1024))) char lds[4 * STAGE];  // [buffer][x | w]
     typedef __attribute__((address_space(3))) void* lds_ptr;
@@ -84,21 +86,23 @@ __global__ __launch_bounds__(256, 2) void gemm32_kernel(const Gemm32Args a) {
     int lo[2];
 #pragma unroll
     for (int r = 0; r < 2; ++r) lo[r] = (lane & 15) * 128 + (((4 * r + (lane >> 4)) ^ ((lane >> 1) & 7)) << 4);
-    f32x4 acc[4][4];  // [row block][column block]
+    constexpr int NC = LOW ? 2 : 4;
+    f32x4 acc[4][NC];  // [row block][column block]
 #pragma unroll
     for (int b = 0; b < 4; ++b)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc[b][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int nb = min(4, (xrows - 64 * wr + 15) >> 4);  // this wave's row blocks (<= 0: none)
+        for (int i = 0; i < NC; ++i) acc[b][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int rbase = LOW ? 0 : 64 * wr, cbase = LOW ? 32 * w : 64 * wc;  // this wave's outputs
+    const int nb = min(4, (xrows - rbase + 15) >> 4);                     // its row blocks (<= 0: none)
     auto compute = [&](int buf, auto all) {
-        const char* xs = lds + buf * 2 * STAGE + 64 * wr * 128;
-        const char* ws = lds + buf * 2 * STAGE + STAGE + 64 * wc * 128;
+        const char* xs = lds + buf * 2 * STAGE + rbase * 128;
+        const char* ws = lds + buf * 2 * STAGE + STAGE + cbase * 128;
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
-            f32x4 xf[4], wf[4];
+            f32x4 xf[4], wf[NC];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                wf[i] = *reinterpret_cast<const f32x4*>(ws + i * 2048 + lo[r]);
+                if (i < NC) wf[i] = *reinterpret_cast<const f32x4*>(ws + i * 2048 + lo[r]);
                 xf[i] = *reinterpret_cast<const f32x4*>(xs + i * 2048 + lo[r]);
             }
 #pragma unroll
@@ -107,7 +111,7 @@ __global__ __launch_bounds__(256, 2) void gemm32_kernel(const Gemm32Args a) {
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
+                    for (int i = 0; i < NC; ++i)
                         acc[b][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[i][j], xf[b][j], acc[b][i], 0, 0, 0);
             }
         }
@@ -136,34 +140,36 @@ __global__ __launch_bounds__(256, 2) void gemm32_kernel(const Gemm32Args a) {
         for (int b = 0; b < 4; ++b)
             if (b < nb)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) out[(b * 4 + i) * 256] = acc[b][i];
+                for (int i = 0; i < NC; ++i) out[(b * 4 + i) * 256] = acc[b][i];
         return;
     }
 #pragma unroll
     for (int b = 0; b < 4; ++b)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            store_c(a, m0 + 64 * wr + 16 * b + (lane & 15), n0 + 64 * wc + 16 * i + 4 * (lane >> 4), acc[b][i]);
+        for (int i = 0; i < NC; ++i)
+            store_c(a, m0 + rbase + 16 * b + (lane & 15), n0 + cbase + 16 * i + 4 * (lane >> 4), acc[b][i]);
 }
 
 // adds the slices of the split tiles; one workgroup per (tile, 2 x 16 rows)
+template <bool LOW>
 __global__ __launch_bounds__(256) void gemm32_tail_kernel(const Gemm32Args a) {
-    const int tid = threadIdx.x, lane = tid & 63, wr = tid >> 7, wc = (tid >> 6) & 1, t = blockIdx.x >> 2, b = blockIdx.x & 3;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, t = blockIdx.x >> 2, b = blockIdx.x & 3;
     int tm, tn;
     tile32(a, a.whole + t, tm, tn);
-    const int m = tm * T32 + 64 * wr + 16 * b;
+    constexpr int NC = LOW ? 2 : 4;
+    const int m = tm * T32 + (LOW ? 0 : 64 * (w >> 1)) + 16 * b, n = tn * T32 + (LOW ? 32 * w : 64 * (w & 1));
     if (m >= a.M) return;
     const f32x4* in = reinterpret_cast<const f32x4*>(a.part + (size_t)t * a.splits * (T32 * T32)) + b * 4 * 256 + tid;
-    f32x4 v[4];
+    f32x4 v[NC];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = in[i * 256];
+    for (int i = 0; i < NC; ++i) v[i] = in[i * 256];
     for (int s = 1; s < a.splits; ++s) {
         in += T32 * T32 / 4;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] += in[i * 256];
+        for (int i = 0; i < NC; ++i) v[i] += in[i * 256];
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) store_c(a, m + (lane & 15), tn * T32 + 64 * wc + 16 * i + 4 * (lane >> 4), v[i]);
+    for (int i = 0; i < NC; ++i) store_c(a, m + (lane & 15), n + 16 * i + 4 * (lane >> 4), v[i]);
 }
 
 // x [M][ldx], w [N][ldw], c [M][ldc]; tiles from raster position ``whole`` on in ``splits`` slices of K through ``part``
@@ -180,7 +186,12 @@ MRSUM_API int mrsum_gemm32(const float* x, int ldx, const float* w, int ldw, flo
     a.whole = splits > 1 ? whole : tiles;
     a.splits = splits > 1 ? splits : 1;
     const int rest = tiles - a.whole;
-    gemm32_kernel<<<a.whole + rest * a.splits, 256, 0, s>>>(a);
-    if (rest) gemm32_tail_kernel<<<rest * 4, 256, 0, s>>>(a);
+    if (M <= 64) {
+        gemm32_kernel<true><<<a.whole + rest * a.splits, 256, 0, s>>>(a);
+        if (rest) gemm32_tail_kernel<true><<<rest * 4, 256, 0, s>>>(a);
+    } else {
+        gemm32_kernel<false><<<a.whole + rest * a.splits, 256, 0, s>>>(a);
+        if (rest) gemm32_tail_kernel<false><<<rest * 4, 256, 0, s>>>(a);
+    }
     return (int)hipGetLastError();
 }
