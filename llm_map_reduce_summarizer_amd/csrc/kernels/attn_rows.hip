@@ -98,3 +98,224 @@ MRSUM_API int mrsum_attn_rows(const void* q, const void* kc, const void* vc, con
                                                 (bf16*)out, out_stride);
     return (int)hipGetLastError();
 }
+
+// ------------------------------------------------------------------------------------------------ prompt portions
+// The same attention for many rows of few sequences, on the fp32 matrix instruction.  The row kernel reads every key
+// from memory for every (row, head): 1088 us for 900 rows of 32 heads of 128 over 8 kv heads, 4380 over 576-wide latents.
+// Here (183 and 755 us, 36 TFLOP/s; the exponentials and their exchange are the rest) 64 (row, head) pairs -- RB consecutive rows of HB heads of one kv head -- share
+// key and value tiles of 32 in LDS (two buffers, the next tile on its way in registers), a wave for 16 pairs.
+//
+// Scores are computed transposed, S^T = K Q^T: lane (pair = lane & 15, g = lane >> 4) holds the scores of keys 4 g .. 4 g
+// + 3 of a 16-key block, which is how the second product O^T = V^T P^T takes its right operand, so weights stay in
+// registers, in fp32.  Every sequence that has rows in the block is a run of its own over the same accumulators.  Tile
+// rows are padded by 4 floats (conflict-free b128 key reads and value reads).
+// Forms (NQ, NV: 16-column steps of keys and values; SHARED: values are the keys' first columns): KT 32, but 16 where 36 + 32
+// steps leave no registers for a larger tile on its way.
+template <typename T, int NQ, int NV, bool SHARED, int KT>
+__global__ __launch_bounds__(256, NQ <= 8 ? 2 : 1) void attn_portion_kernel(
+    const T* __restrict__ q, const T* __restrict__ kc, const T* __restrict__ vc, const int* __restrict__ positions,
+    const int* __restrict__ seq_idx, const int* __restrict__ block_tables, int bt_stride, int rows, int H, int G, int dk,
+    int dv, int ldv, int pitch, float scale, const float* __restrict__ gate, T* __restrict__ out, int out_stride, int HB,
+    int RB) {
+    constexpr int LK = NQ * 16 + 4, LV = SHARED ? LK : NV * 16 + 4;
+    constexpr int TPR = 256 / KT, FK = (NQ * 4 + TPR - 1) / TPR, FV = SHARED ? 1 : (NV * 4 + TPR - 1) / TPR;
+    __shared__ __attribute__((aligned(16))) float s_k[2][KT][LK];
+    __shared__ __attribute__((aligned(16))) float s_v[SHARED ? 1 : 2][SHARED ? 1 : KT][LV];
+    __shared__ int s_bad[2];  // the tile holds a value that is not finite
+    const int tid = threadIdx.x, lane = tid & 63, j16 = lane & 15, g4 = lane >> 4;
+    const int gh = H / G, hblocks = (gh + HB - 1) / HB, g = blockIdx.y / hblocks, h0 = blockIdx.y % hblocks * HB;
+    const int t0 = blockIdx.x * RB, tend = min(rows, t0 + RB);
+    const int pair = 16 * (tid >> 6) + j16, trow = t0 + pair / HB, hh = h0 + pair % HB;
+    const bool valid = pair < RB * HB && trow < tend && hh < gh;
+    const int t = valid ? trow : t0, head = g * gh + (valid ? hh : h0), pos = positions[t];
+    float4 qf[NQ];
+#pragma unroll
+    for (int r = 0; r < NQ; ++r) {
+        const int c = 16 * r + 4 * g4;
+        qf[r] = valid && c < dk ? ld4(q + ((size_t)t * H + head) * dk + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    float m = -INFINITY, l = 0.f;
+    f32x4 o[NV];
+#pragma unroll
+    for (int c = 0; c < NV; ++c) o[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    // tile loads: TPR threads a row, four columns each at a time
+    const int lr = tid / TPR, lc = 4 * (tid % TPR);
+    float4 fk[FK], fv[FV];
+    for (int a = t0; a < tend;) {
+        const int seq = seq_idx[a];
+        int b = a + 1, last = positions[a];
+        while (b < tend && seq_idx[b] == seq) last = max(last, positions[b++]);
+        const bool mine = valid && t >= a && t < b;
+        const int* bt = block_tables + (size_t)seq * bt_stride;
+        auto fetch = [&](int k0) {
+            const int key = k0 + lr;
+            const bool in = key <= last;
+            const size_t slab = in ? ((size_t)bt[key / ROW_PAGE] * G + g) * ROW_PAGE + key % ROW_PAGE : 0;
+#pragma unroll
+            for (int i = 0; i < FK; ++i) {
+                const int c = lc + 4 * TPR * i;
+                fk[i] = in && c < dk ? ld4(kc + slab * dk + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+            if constexpr (!SHARED) {
+#pragma unroll
+                for (int i = 0; i < FV; ++i) {
+                    const int c = lc + 4 * TPR * i;
+                    fv[i] = in && c < dv ? ld4(vc + slab * ldv + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+                }
+            }
+        };
+        auto put = [&](int buf) {
+            bool bad = false;
+#pragma unroll
+            for (int i = 0; i < FK; ++i) {
+                if (lc + 4 * TPR * i < NQ * 16) *reinterpret_cast<float4*>(&s_k[buf][lr][lc + 4 * TPR * i]) = fk[i];
+                if (SHARED && lc + 4 * TPR * i < dv) bad |= !(fabsf(fk[i].x) + fabsf(fk[i].y) + fabsf(fk[i].z) + fabsf(fk[i].w) < INFINITY);
+            }
+            if constexpr (!SHARED) {
+#pragma unroll
+                for (int i = 0; i < FV; ++i) {
+                    if (lc + 4 * TPR * i < NV * 16) *reinterpret_cast<float4*>(&s_v[buf][lr][lc + 4 * TPR * i]) = fv[i];
+                    bad |= !(fabsf(fv[i].x) + fabsf(fv[i].y) + fabsf(fv[i].z) + fabsf(fv[i].w) < INFINITY);
+                }
+            }
+            if (bad) s_bad[buf] = 1;
+        };
+        if (tid < 2) s_bad[tid] = 0;
+        fetch(0);
+        __syncthreads();
+        put(0);
+        __syncthreads();
+        for (int k0 = 0, buf = 0; k0 <= last; k0 += KT, buf ^= 1) {
+            const bool more = k0 + KT <= last;
+            if (more) fetch(k0 + KT);
+            f32x4 s[KT / 16];
+#pragma unroll
+            for (int kb = 0; kb < KT / 16; ++kb) s[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int r = 0; r < NQ; ++r) {
+                if (16 * r >= dk) break;
+                float4 kf[KT / 16];
+#pragma unroll
+                for (int kb = 0; kb < KT / 16; ++kb)
+                    kf[kb] = *reinterpret_cast<const float4*>(&s_k[buf][16 * kb + j16][16 * r + 4 * g4]);
+#pragma unroll
+                for (int kb = 0; kb < KT / 16; ++kb) s[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[kb].x, qf[r].x, s[kb], 0, 0, 0);
+#pragma unroll
+                for (int kb = 0; kb < KT / 16; ++kb) s[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[kb].y, qf[r].y, s[kb], 0, 0, 0);
+#pragma unroll
+                for (int kb = 0; kb < KT / 16; ++kb) s[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[kb].z, qf[r].z, s[kb], 0, 0, 0);
+#pragma unroll
+                for (int kb = 0; kb < KT / 16; ++kb) s[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[kb].w, qf[r].w, s[kb], 0, 0, 0);
+            }
+            float mx = -INFINITY;
+#pragma unroll
+            for (int kb = 0; kb < KT / 16; ++kb)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    s[kb][i] = mine && k0 + 16 * kb + 4 * g4 + i <= pos ? s[kb][i] * scale : -INFINITY;
+                    mx = fmaxf(mx, s[kb][i]);
+                }
+            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            const float mn = fmaxf(m, mx), alpha = mn == m ? 1.f : expf(m - mn);
+            m = mn;
+            l *= alpha;
+            if (__any(alpha != 1.f)) {
+#pragma unroll
+                for (int c = 0; c < NV; ++c) o[c] *= alpha;
+            }
+#pragma unroll
+            for (int kb = 0; kb < KT / 16; ++kb)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float x = s[kb][i];
+                    s[kb][i] = mine && k0 + 16 * kb + 4 * g4 + i <= pos ? expf(x - mn) : 0.f;
+                    l += s[kb][i];
+                }
+            auto vrow = [&](int k) -> const float* { return SHARED ? s_k[buf][k] : s_v[SHARED ? 0 : buf][SHARED ? 0 : k]; };
+            if (!s_bad[buf]) {
+#pragma unroll
+                for (int kb = 0; kb < KT / 16; ++kb)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float* v = vrow(16 * kb + 4 * g4 + i) + j16;
+#pragma unroll
+                        for (int c = 0; c < NV; ++c) {
+                            if (16 * c >= dv) break;
+                            o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[16 * c], s[kb][i], o[c], 0, 0, 0);
+                        }
+                    }
+            } else {  // a later key's infinity times a weight of zero would be no number: only keys that count
+                for (int k = 0; k < KT; ++k) {
+                    float p = 0.f;
+#pragma unroll
+                    for (int kb = 0; kb < KT / 16; ++kb)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const float x = __shfl(s[kb][i], j16 + 16 * ((k >> 2) & 3), 64);
+                            if (k >> 4 == kb && (k & 3) == i) p = x;
+                        }
+                    if (mine && k0 + k <= pos)
+#pragma unroll
+                        for (int c = 0; c < NV; ++c)
+                            if (16 * c < dv)
+#pragma unroll
+                                for (int i = 0; i < 4; ++i) o[c][i] += p * vrow(k)[16 * c + 4 * g4 + i];
+                }
+            }
+            if (tid == 0) s_bad[buf ^ 1] = 0;
+            __syncthreads();
+            if (more) put(buf ^ 1);
+            __syncthreads();
+        }
+        a = b;
+    }
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    if (!valid) return;
+    const float f = (gate ? gate[(size_t)t * H + head] : 1.f) / l;
+    T* dst = out + (size_t)t * out_stride + (size_t)head * pitch;
+#pragma unroll
+    for (int c = 0; c < NV; ++c)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int d = 16 * c + 4 * g4 + i;
+            if (d < pitch) dst[d] = (T)(o[c][i] * f);
+        }
+}
+
+template <typename T>
+static int launch_portions(const void* q, const void* kc, const void* vc, const int* positions, const int* seq_idx,
+                           const int* block_tables, int bt_stride, int rows, int H, int G, int dk, int dv, int ldv, int pitch,
+                           float scale, const float* gate, void* out, int out_stride, hipStream_t s) {
+    const int gh = H / G, HB = std::min(gh, 32), RB = 64 / HB;
+    const dim3 grid(ceil_div(rows, RB), G * ceil_div(gh, HB));
+#define AP(NQ, NV, SH, KT)                                                                                               \
+    attn_portion_kernel<T, NQ, NV, SH, KT><<<grid, 256, 0, s>>>((const T*)q, (const T*)kc, (const T*)vc, positions, seq_idx,  \
+                                                            block_tables, bt_stride, rows, H, G, dk, dv, ldv, pitch,      \
+                                                            scale, gate, (T*)out, out_stride, HB, RB)
+    if (dk <= 64 && dv <= 64) AP(4, 4, false, 32);
+    else if (dk <= 128 && dv <= 128) AP(8, 8, false, 32);
+    else if (dk <= 256 && dv <= 256) AP(16, 16, false, 32);
+    else if (kc == vc && ldv == dk && dk <= 576 && dv <= 512) AP(36, 32, true, 16);
+    else return (int)hipErrorInvalidValue;
+#undef AP
+    return (int)hipGetLastError();
+}
+
+// Arguments as mrsum_attn_rows; widths multiples of 4, rows 16-byte (fp32) or 8-byte (bf16) aligned, and up to 256 wide, or
+// up to 576 / 512 where the values are the first columns of the keys.
+MRSUM_API int mrsum_attn_portions(const void* q, const void* kc, const void* vc, const int* positions, const int* seq_idx,
+                                  const int* block_tables, int bt_stride, int T, int H, int G, int dk, int dv, int ldv,
+                                  int pitch, float scale, const float* gate, void* out, int out_stride, int f32,
+                                  hipStream_t s) {
+    if (T <= 0) return 0;
+    if (G <= 0 || H % G || dk % 4 || dv % 4 || ldv % 4 || pitch > dv || ldv < dv || G * ceil_div(H / G, 32) > 65535)
+        return (int)hipErrorInvalidValue;
+    if (f32)
+        return launch_portions<float>(q, kc, vc, positions, seq_idx, block_tables, bt_stride, T, H, G, dk, dv, ldv, pitch,
+                                      scale, gate, out, out_stride, s);
+    return launch_portions<bf16>(q, kc, vc, positions, seq_idx, block_tables, bt_stride, T, H, G, dk, dv, ldv, pitch, scale,
+                                 gate, out, out_stride, s);
+}

@@ -339,6 +339,52 @@ def attention_of(u, w, al, H, G, dim, vdim, scale, coef, every, eps):
     return O.attention(cols, ww, "a.", c, eps)
 
 
+@pytest.mark.parametrize("H,G,dk,dv", [(8, 2, 48, 32), (6, 2, 128, 100), (5, 5, 64, 64), (4, 1, 200, 256), (70, 1, 16, 8),
+                                       (32, 1, 576, 512), (3, 1, 300, 20)])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_row_attention_portions(H, G, dk, dv, dtype, monkeypatch):
+    """Portions in tiles that rows and heads share: several sequences in a block, rows from the middle of a sequence, page
+    and tile borders, a later key that is infinite, values that are the keys' first columns; decoded rows in front."""
+    from llm_map_reduce_summarizer_amd import ops
+    from llm_map_reduce_summarizer_amd.ops import hip
+    monkeypatch.setattr(hip, "PORTION_PAIRS", 0)
+    latent, page, lens, pre = dk > 256, 64, [1, 1, 2, 31, 130, 66, 20], [70, 0, 5, 0, 33, 63, 200]
+    n, width = sum(lens), dk
+    kc = rnd(40, G, page, width, seed=1, dtype=dtype)
+    vc = kc if latent else rnd(40, G, page, dv, seed=2, dtype=dtype)
+    tables = torch.zeros(len(lens), 8, dtype=torch.int32)
+    at = 1
+    for i, (a, b) in enumerate(zip(pre, lens)):
+        need = -(-(a + b) // page)
+        tables[i, :need] = torch.arange(at, at + need)
+        at += need
+        kc[at - 1, :, (a + b - 1) % page + 1:] = float("inf")  # rows past the sequence
+        vc[at - 1, :, (a + b - 1) % page + 1:] = float("nan")
+    pos = torch.cat([torch.arange(a, a + b) for a, b in zip(pre, lens)]).int()
+    seq = torch.repeat_interleave(torch.arange(len(lens)), torch.tensor(lens)).int()
+    last = int(tables[4, (pre[4] + lens[4] - 1) // page]), (pre[4] + lens[4] - 1) % page
+    q = rnd(n, H * dk, seed=3, std=2.0, dtype=dtype)
+    if not latent:
+        vc[last[0], :, last[1]] = float("inf")  # the last token of a sequence: its own row alone sees it
+    args = (dk ** -0.5,)
+    i32 = [pos, seq, tables]
+    if latent:
+        want = ops.latent_rows(q, kc, *i32, H, dv, page, *args)
+        got = ops.latent_rows(dev(q), dev(kc), *map(dev, i32), H, dv, page, *args, singles=2)
+    else:
+        gate, vp = torch.sigmoid(rnd(n, H, seed=4)), dv
+        want, got = torch.zeros(n, H * vp, dtype=dtype), torch.zeros(n, H * vp, dtype=dtype, device=DEV)
+        ops.attn_rows(q, kc, vc, *i32, H, G, vp, page, *args, gate, want)
+        ops.attn_rows(dev(q), dev(kc), dev(vc), *map(dev, i32), H, G, vp, page, *args, dev(gate), got, singles=2)
+    got, odd = got.cpu().float(), sum(lens[:5]) - 1
+    keep = [t for t in range(n) if latent or t != odd]
+    assert bool(torch.isfinite(got[keep]).all())
+    # fp32 scores of up to 220 keys and dk products, exp: a few 2^-24 each; 16-bit results round by 2^-9
+    assert rel(got[keep], want[keep].float()) < (4e-3 if dtype == BF else 2e-6)
+    if not latent:
+        assert bool((got[odd] == float("inf")).all())
+
+
 @pytest.mark.parametrize("M,N,K,split", [(1, 130, 1024, True), (17, 1023, 2048, True), (129, 2062, 512, True),
                                          (500, 8200, 256, True), (1100, 4096, 128, False), (3, 40000, 64, False)])
 def test_gemm32_edges(M, N, K, split):
