@@ -25,6 +25,7 @@ import functools
 import logging
 import os
 import time
+from array import array
 from dataclasses import dataclass, field
 from types import SimpleNamespace
 from typing import Dict, List, Optional, Sequence, Tuple
@@ -45,6 +46,42 @@ MAX_WINDOW = 256  # decode steps between host syncs when no row can stop early (
 
 def _always() -> bool:
     return True
+
+
+def _token_ids(toks: Sequence[int], vocab: int) -> np.ndarray:
+    """The ids as int32, checked to be non-empty and in range."""
+    try:
+        if isinstance(toks, (bytes, bytearray)):  # array() would take them for memory
+            raise TypeError
+        a = np.frombuffer(array("q", toks), dtype=np.int64) if len(toks) else None  # 20 ns an id
+    except (TypeError, OverflowError):  # ids that are not plain integers
+        a = [int(t) for t in toks]
+        a = None if min(a) < 0 or max(a) >= vocab else np.asarray(a)
+    if a is None or int(a.min()) < 0 or int(a.max()) >= vocab:
+        raise ValueError("empty step entry or token id out of range")
+    return a.astype(np.int32)
+
+
+class _Upload:
+    """Host arrays of one pass, brought to the device in one copy: ``add`` hands out a number, ``send`` the tensors by
+    number (pieces start at multiples of 256 bytes).  A copy each cost 10 - 15 us of host time ahead of the first launch."""
+
+    def __init__(self):
+        self.parts: List[Tuple[int, np.ndarray]] = []
+        self.size = 0
+
+    def add(self, a, dtype=np.int32) -> int:
+        a = np.ascontiguousarray(a, dtype=dtype)
+        self.parts.append((self.size, a))
+        self.size += -(-a.nbytes // 256) * 256
+        return len(self.parts) - 1
+
+    def send(self, device) -> List[torch.Tensor]:
+        buf = np.empty(self.size, dtype=np.uint8)
+        for at, a in self.parts:
+            buf[at: at + a.nbytes] = a.reshape(-1).view(np.uint8)
+        t = torch.from_numpy(buf).to(device, non_blocking=True)
+        return [t[at: at + a.nbytes].view(torch.int64 if a.dtype == np.int64 else torch.int32) for at, a in self.parts]
 
 
 @dataclass
@@ -374,39 +411,46 @@ class LLMEngine:
             self._prefill_pass(part, spans, paged=True, final=(r == rounds - 1))
 
     def _pass_inputs(self, seqs: List[_Seq], spans, paged: bool, tables: Optional[torch.Tensor] = None,
-                     slots: Optional[List[int]] = None, sample: Optional[List[bool]] = None):
+                     slots: Optional[List[int]] = None, sample: Optional[List[bool]] = None,
+                     rows: Optional[List[int]] = None):
         """Device inputs of one packed forward over prompt slices ``spans`` [(start, end)] of ``seqs``
         (block-table rows ``slots`` of ``tables``: default the decode slots of the decode state;
-        ``sample``: which sequences' last rows feed the LM head, default all)."""
+        ``sample``: which sequences' last rows feed the LM head, default all; ``rows``: those rows themselves)."""
         st, dev = self.state, self.device
         tables = st.block_tables if tables is None else tables
         slots = [s.slot for s in seqs] if slots is None else slots
         # numpy assembly: torch.tensor() over Python lists of a 16k-token pass cost ~5 ms of host time
         lens = [e - b for b, e in spans]
+        pre = [b for b, _ in spans]
         cu = np.zeros(len(spans) + 1, dtype=np.int32)
         np.cumsum(lens, out=cu[1:])
-        ids = np.concatenate([np.asarray(s.prompt[b:e], dtype=np.int32) for s, (b, e) in zip(seqs, spans)])
-        pos = np.concatenate([np.arange(b, e, dtype=np.int32) for b, e in spans])
-        sidx = np.repeat(np.asarray(slots, dtype=np.int32), lens)
-        last = [int(cu[k + 1]) - 1 for k in range(len(spans)) if sample is None or sample[k]]
-        h = lambda x: torch.from_numpy(np.ascontiguousarray(x, dtype=np.int32)).to(dev, non_blocking=True)  # noqa: E731
-        items = self.model.pass_items(lens) if dev.type == "cuda" and not self.model.recurrent else None
-        pp = None
-        pre = [b for b, _ in spans]
-        if paged and not self.model.recurrent:
-            pp = ops.PagedPrefill(tables, h(slots), h(pre), list(slots), pre)
-        x = SimpleNamespace(ids=h(ids), positions=h(pos), seq_idx=h(sidx), cu_seqlens=h(cu),
-                            last_rows=torch.tensor(last, dtype=torch.long).to(dev, non_blocking=True),
-                            seqlens=lens, items=items, paged=pp, tables=tables)
-        if self.model.recurrent:
+        if rows is None:
+            rows = [int(cu[k + 1]) - 1 for k in range(len(spans)) if sample is None or sample[k]]
+        up = _Upload()
+        at = {"ids": up.add(np.concatenate([np.asarray(s.prompt[b:e], dtype=np.int32) for s, (b, e) in zip(seqs, spans)])),
+              "positions": up.add(np.concatenate([np.arange(b, e, dtype=np.int32) for b, e in spans])),
+              "seq_idx": up.add(np.repeat(np.asarray(slots, dtype=np.int32), lens)), "cu_seqlens": up.add(cu),
+              "last_rows": up.add(rows, np.int64)}
+        recurrent = self.model.recurrent
+        if recurrent:
             # leading single tokens run as decode rows, the other segments as prompt portions of the same pass
             nd = next((k for k, n in enumerate(lens) if n != 1), len(lens))
+            segs = [up.add([s.state_slot for s in seqs]), up.add(pre),
+                    up.add(np.repeat(np.arange(len(lens), dtype=np.int32), lens))]
+            at["cu_portions"] = up.add(cu[nd:] - nd)
+            part = [up.add(slots[nd:]), up.add(pre[nd:]), up.add(slots[:nd])]
+        elif paged:
+            part = [up.add(slots), up.add(pre)]
+        items = self.model.pass_items(lens) if dev.type == "cuda" and not recurrent else None
+        d = up.send(dev)
+        x = SimpleNamespace(seqlens=lens, items=items, paged=None, tables=tables, **{k: d[i] for k, i in at.items()})
+        if paged and not recurrent:
+            x.paged = ops.PagedPrefill(tables, d[part[0]], d[part[1]], list(slots), pre)
+        if recurrent:
             x.n_decode, x.portion_lens = nd, lens[nd:]
-            x.segs = ops.Segments(h([s.state_slot for s in seqs]), h(pre), x.cu_seqlens,
-                                  h(np.repeat(np.arange(len(lens), dtype=np.int32), lens)), lens)
-            x.cu_portions = h(cu[nd:] - nd)
-            x.paged = ops.PagedPrefill(tables, h(slots[nd:]), h(pre[nd:]), list(slots[nd:]), pre[nd:])
-            x.decode_tables = tables.index_select(0, torch.tensor(slots[:nd], dtype=torch.long).to(dev))
+            x.segs = ops.Segments(d[segs[0]], d[segs[1]], x.cu_seqlens, d[segs[2]], lens)
+            x.paged = ops.PagedPrefill(tables, d[part[0]], d[part[1]], list(slots[nd:]), pre[nd:])
+            x.decode_tables = tables.index_select(0, d[part[2]])
             x.workspace = (self._workspace(self._bucket(nd)) or {}) if nd else {}
             x.items = self.model.pass_items(lens[nd:]) if dev.type == "cuda" else None
             x.context = functools.lru_cache(None)(lambda: ops.PortionContext(lens[nd:], pre[nd:], slots[nd:], dev))
@@ -624,12 +668,46 @@ class LLMEngine:
         if len({e[0] for e in entries}) != len(entries):
             raise ValueError("a request appears twice in one step")
         order = sorted(range(len(entries)), key=lambda k: len(entries[k][1]) != 1)  # single tokens first
-        seqs, spans, wanted = [], [], []
+        seqs, spans, wanted, pages = [], [], [], []
+        try:
+            self._admit_step(entries, order, seqs, spans, wanted, pages)
+        finally:  # pages that were taken stand in the table, also where a later entry was refused
+            if pages:
+                up = _Upload()
+                where = up.add(np.concatenate([np.arange(a, a + len(p)) for a, p in pages]), np.int64)
+                which = up.add(np.concatenate([p for _, p in pages]))
+                d = up.send(self.device)
+                self.pf_tables.view(-1).index_copy_(0, d[where], d[which])
+        out: List[Optional[torch.Tensor]] = [None] * len(entries)
+        if entries:
+            if self.device.type == "cuda":
+                from ..ops.hip import ctx_class
+                self._ctx_cls = ctx_class(max(e for _, e in spans))
+            starts = np.cumsum([0] + [e - b for b, e in spans])
+            rows = [int(starts[j]) + w for j, ws in enumerate(wanted) for w in ws]
+            x = self._pass_inputs(seqs, spans, paged=True, tables=self.pf_tables, slots=[s.pf_slot for s in seqs],
+                                  rows=rows)
+            logits = self.model.forward_pass(x, self.kv, logits=bool(rows))
+            logits = logits.float() if rows else None
+            at = 0
+            for j, k in enumerate(order):
+                n = len(wanted[j])
+                out[k] = (logits[at: at + n] if n else
+                          torch.empty(0, self.cfg.vocab_size, dtype=torch.float32, device=self.device))
+                at += n
+            self._sync()
+        for rid in end:
+            s = self._stepped.pop(rid)
+            self.pf_tables[s.pf_slot].zero_()
+            self._release(s)
+        return out  # type: ignore[return-value]
+
+    def _admit_step(self, entries, order, seqs: List[_Seq], spans, wanted, pages) -> None:
+        """Admit the entries of a step in ``order``: their requests, spans and wanted rows, and the newly taken pages as
+        (first place in the flattened prefill table, page ids)."""
         for k in order:
             rid, toks, want = entries[k]
-            toks = [int(t) for t in toks]
-            if not toks or min(toks) < 0 or max(toks) >= self.cfg.vocab_size:
-                raise ValueError("empty step entry or token id out of range")
+            toks = _token_ids(toks, self.cfg.vocab_size)
             s = self._stepped.get(rid)
             if s is None:
                 used = {q.pf_slot for q in self._stepped.values()}
@@ -646,34 +724,11 @@ class LLMEngine:
             self._hold(s, need)
             self._stepped[rid] = s
             if need:
-                self.pf_tables[s.pf_slot, held: held + need] = torch.tensor(s.pages[held:], dtype=torch.int32).to(
-                    self.device)
-            s.prompt = s.prompt + toks
+                pages.append((s.pf_slot * self.max_pages + held, s.pages[held:]))
+            s.prompt = toks if b == 0 else np.concatenate((s.prompt, toks))  # (stepped requests keep their ids as an array)
             seqs.append(s)
             spans.append((b, len(s.prompt)))
             wanted.append([int(w) for w in want])
-        out: List[Optional[torch.Tensor]] = [None] * len(entries)
-        if entries:
-            if self.device.type == "cuda":
-                from ..ops.hip import ctx_class
-                self._ctx_cls = ctx_class(max(e for _, e in spans))
-            x = self._pass_inputs(seqs, spans, paged=True, tables=self.pf_tables, slots=[s.pf_slot for s in seqs])
-            starts = np.cumsum([0] + [e - b for b, e in spans])
-            rows = [int(starts[j]) + w for j, ws in enumerate(wanted) for w in ws]
-            x.last_rows = torch.tensor(rows, dtype=torch.long).to(self.device)
-            logits = self.model.forward_pass(x, self.kv, logits=bool(rows))
-            at = 0
-            for j, k in enumerate(order):
-                n = len(wanted[j])
-                out[k] = (logits[at: at + n].float() if n else
-                          torch.empty(0, self.cfg.vocab_size, dtype=torch.float32, device=self.device))
-                at += n
-            self._sync()
-        for rid in end:
-            s = self._stepped.pop(rid)
-            self.pf_tables[s.pf_slot].zero_()
-            self._release(s)
-        return out  # type: ignore[return-value]
 
     def _fit_ctx_class(self, seqs: Sequence[_Seq]) -> None:
         """Decode attention split plan (graphs are keyed by it) for the longest sequence in flight."""

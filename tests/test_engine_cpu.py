@@ -2,6 +2,7 @@
 
 import math
 
+import numpy as np
 import pytest
 import torch
 
@@ -422,3 +423,18 @@ def test_window_rule():
     assert e._window([40, 7], False) == 7  # pinned: until the first row runs out
     assert e._window([4000, 3000], False) == 256  # at most MAX_WINDOW
     assert e._window([40, 7], True) == 16  # a feeder / stream hook / interleaved prefill wants sync points
+
+
+@pytest.mark.parametrize("toks,want", [([5, 0, 99], [5, 0, 99]), ((7,), [7]), (range(3), [0, 1, 2]), ([2.0, True], [2, 1]),
+                                       (np.array([4, 9], dtype=np.uint8), [4, 9]), (torch.tensor([3, 98]), [3, 98]),
+                                       (b"\x01\x02", [1, 2]), (["6"], [6]), ([], None), ([100], None), ([-1], None),
+                                       ([1 << 70], None), ([1 << 40], None), ([-(1 << 70)], None)])
+def test_step_token_ids(toks, want):
+    """Everything int() takes is a token id; empty entries and ids outside the vocabulary are refused."""
+    from llm_map_reduce_summarizer_amd.engine.engine import _token_ids
+    if want is None:
+        with pytest.raises(ValueError):
+            _token_ids(toks, 100)
+    else:
+        got = _token_ids(toks, 100)
+        assert got.dtype == np.int32 and got.tolist() == want
