@@ -98,7 +98,8 @@ struct GluArgs {
 __device__ __forceinline__ float glu(float g, float u, const GluArgs& a) {
     g = fminf(g, a.limit);
     u = fminf(fmaxf(u, -a.limit), a.limit);
-    return g / (1.f + __expf(-a.alpha * g)) * (u + a.shift);
+    // hardware reciprocal: an IEEE division for 64 values a thread was 5 us of the GEMM's 108 us a tile
+    return g * __builtin_amdgcn_rcpf(1.f + __expf(-a.alpha * g)) * (u + a.shift);
 }
 
 // Attention output form: head h of row t goes to columns [h * pitch, (h + 1) * pitch) of the row, times
