@@ -74,6 +74,7 @@ struct GemmArgs {
     int whole;    // raster positions below it run whole, the others in ``splits`` slices of K each
     int splits;
     float* part;  // [tiles - whole][splits][TILE_F] fp32 accumulators of the slices
+    int slabs;    // GEPI_F32, every tile split: part is [splits][M][N] rows instead, for a consumer that adds the slabs
     GluArgs glu;  // GEPI_SWIGLU
 #ifdef MRSUM_CLOCK_STAMPS
     unsigned long long* stamps;  // diagnostic build only (tools/gemm_clock.py): [grid][2] shader / 100 MHz ticks
@@ -326,6 +327,22 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmArgs a) {
     if (wr == 0) bar();
 
     if constexpr (!M32) {
+        if (EPI == GEPI_F32 && a.slabs) {
+            float* out = a.part + ((size_t)slice * a.M + m0) * a.N + n0 + 32 * wc + 4 * (lane >> 4);
+#pragma unroll
+            for (int qm = 0; qm < 2; ++qm)
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    const int rl = 128 * qm + 64 * wr + 16 * b + (lane & 15);
+                    if (rl >= xrows) continue;
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        if (32 * wc + 128 * (v >> 1) + 16 * (v & 1) < wrows)
+                            *reinterpret_cast<f32x4*>(out + (size_t)rl * a.N + 128 * (v >> 1) + 16 * (v & 1)) =
+                                acc[qm][b][v >> 1][v & 1];
+                }
+            return;
+        }
         if (slice >= 0) {
             // accumulator vector v of this lane at [v][thread]; 16-row blocks past M are skipped
             f32x4* out = reinterpret_cast<f32x4*>(a.part + ((size_t)(pos - a.whole) * a.splits + slice) * TILE_F) + tid;
@@ -539,12 +556,13 @@ MRSUM_API int mrsum_gemm_stamps(unsigned long long* host, int max_words) {
 // sx [M] / sw [N] fp32 row scales; split: x is two-term [hi | lo] of 2K bytes per row over w's K.
 // whole / splits / part: tiles from raster position ``whole`` on run in ``splits`` slices of K through ``part``
 // [tiles - whole][splits][65536] fp32 (splits 1: none, part unused;
-// 16x16 MFMA tiles only).
+// 16x16 MFMA tiles only).  slabs (epi 3, whole 0): the slices stay apart, in part [splits][M][N]; c unused.
 // Requirements (checked by the Python wrapper too): K % 64 (bf16) / K % 128 (fp8), N % 16, 16-byte
 // aligned rows.
 MRSUM_API int mrsum_gemm(const void* x, int ldx, const void* w, int ldw, void* c, int ldc, int M, int N, int K,
                          int fp8, int epi, const float* sx, const float* sw, int group_m, int split, float glu_limit,
-                         float glu_alpha, float glu_shift, int whole, int splits, float* part, hipStream_t s) {
+                         float glu_alpha, float glu_shift, int whole, int splits, float* part, int slabs,
+                         hipStream_t s) {
     if (M <= 0 || N <= 0) return 0;
     const int es = fp8 ? 1 : 2;
     if ((K * es) % 128 || N % 16 || (ldx * es) % 16 || (ldw * es) % 16 || ldc % 4) return (int)hipErrorInvalidValue;
@@ -574,6 +592,8 @@ MRSUM_API int mrsum_gemm(const void* x, int ldx, const void* w, int ldw, void* c
     a.splits = splits > 1 ? splits : 1;
     a.whole = splits > 1 ? whole : tiles;
     a.part = part;
+    a.slabs = slabs;
+    if (slabs && (epi != GEPI_F32 || splits <= 1 || whole || N % 16)) return (int)hipErrorInvalidValue;
     const int rest = tiles - a.whole;
     const dim3 grid(a.whole + rest * a.splits), block(512);
 #ifdef MRSUM_CLOCK_STAMPS
@@ -613,7 +633,7 @@ MRSUM_API int mrsum_gemm(const void* x, int ldx, const void* w, int ldw, void* c
             if (rest) gemm_tail_kernel<false, GEPI_GELU><<<rest * 8, block, 0, s>>>(a);
         } else if (epi == GEPI_F32) {
             gemm_kernel<false, GEPI_F32, 8, false, false><<<grid, block, 0, s>>>(a);
-            if (rest) gemm_tail_kernel<false, GEPI_F32><<<rest * 8, block, 0, s>>>(a);
+            if (rest && !slabs) gemm_tail_kernel<false, GEPI_F32><<<rest * 8, block, 0, s>>>(a);
         } else {
             GEMM_LAUNCH(false, GEPI_BF16)
         }

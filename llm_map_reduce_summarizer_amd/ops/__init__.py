@@ -263,14 +263,18 @@ def add_norm32(residual, src, w, eps, dtype, width):
 
 
 def project(x, w, role):
-    """x @ w^T for a consumer that sums slabs: fp32 [S, T, N] split-K slabs at decode row counts (and always in fp32
-    mode), 16-bit rows [T, N] of the MFMA GEMM above them."""
+    """x @ w^T for a consumer that sums slabs: fp32 [S, T, N] split-K slabs at decode row counts, where the MFMA GEMM splits
+    a whole product ("o", "down"), and always in fp32 mode; else 16-bit rows [T, N] of the MFMA GEMM."""
     if not _use_hip(x):
         return reference.project(x, w)
     from . import hip
     if x.dtype == torch.float32:
         return hip.gemm32(x, w)[None]
     M, (N, K) = x.shape[0], w.shape
+    if role in ("o", "down") and M > hip.STREAM_TALL_M:
+        parts = hip.gemm_slabs(x, w)
+        if parts is not None:
+            return parts
     cfg = hip.project_config(N, K) if M <= hip.STREAM_MAX_M else None
     if cfg is not None:
         return hip.linear_parts(x, w, cfg[1], nt=cfg[0], kernel="stream")
@@ -684,6 +688,10 @@ def proj_add_rmsnorm(a, w, residual, ln, eps, role="o", all_reduce=None, quant=F
         from . import hip
         fused = _fused_ar(all_reduce, a.shape[0], residual.shape[1])
         one = 1 if (all_reduce and not fused) else None  # a plain all-reduce takes one slab
+        if not all_reduce and not quant and a.shape[0] > hip.STREAM_TALL_M:
+            parts = hip.gemm_slabs(a, w)
+            if parts is not None:
+                return hip.add_rmsnorm_parts(parts, residual, ln, eps)
         p = hip.plan(role, a.shape[0], w.shape[0], w.shape[1], splits=one)
         if p[0] != "gemm":
             parts = _plan_parts(hip, p, a, w, one)

@@ -176,3 +176,14 @@ def test_stream_parts_beyond_tall_tiles(M):
     assert parts.dtype == torch.float32 and parts.shape == (2 if M <= 128 else 1, M, 4096)
     bound = 1024 * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
     assert bool(((parts.sum(0).double() - x.double() @ w.double().t()).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 32, 2048), (130, 544, 2112), (257, 4096, 2112)])
+def test_gemm_slabs(M, N, K):
+    """A grid whose tiles all run in slices of K leaves the slices apart; other grids give none."""
+    x, w = _rand(M, K, seed=16, scale=0.5), _rand(N, K, seed=17, scale=0.03)
+    parts = hip.gemm_slabs(x, w)
+    assert parts.shape == (hip.gemm_splits(M, N, K // 64)[1], M, N) and parts.dtype == torch.float32
+    bound = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    assert bool(((parts.double().sum(0) - x.double() @ w.double().t()).abs() <= bound).all())
+    assert hip.gemm_slabs(x[:, :64], w[:, :64]) is None and hip.gemm_slabs(_rand(4097, K), _rand(4096, K)) is None
