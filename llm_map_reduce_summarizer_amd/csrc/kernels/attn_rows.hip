@@ -1,8 +1,9 @@
 // Row attention over the paged cache for any head width and value width, in bf16 or fp32 storage with fp32
-// arithmetic throughout: one wave per (row, query head).  Every lane scores one key of a 64-key page; the softmax is
-// online across pages; the value sum runs with the lanes over the value columns.  It serves fp32 models and heads
-// the MFMA kernels do not take (attn_prefill.hip / attn_decode.hip / latent_attn.hip), prompt portions and decoded
-// tokens alike; latent attention runs it with the cached rows as keys and their first columns as values.
+// arithmetic throughout: one wave, or a few, per (row, query head).  Every lane scores one key of a 64-key page; the
+// softmax is online across pages; the value sum runs with the lanes over the value columns.  It serves fp32 models and
+// heads the MFMA kernels do not take (attn_prefill.hip / attn_decode.hip / latent_attn.hip): decoded tokens and short
+// prompt portions here, long ones in the tiled kernel below; latent attention runs both with the cached rows as keys and
+// their first columns as values.
 #include "common.h"
 
 constexpr int ROW_PAGE = 64;
@@ -15,29 +16,36 @@ __device__ __forceinline__ float4 ld4(const bf16* p) {
                        __uint_as_float(v.y & 0xffff0000u));
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void attn_rows_kernel(const T* __restrict__ q, const T* __restrict__ kc,
-                                                        const T* __restrict__ vc, const int* __restrict__ positions,
-                                                        const int* __restrict__ seq_idx,
-                                                        const int* __restrict__ block_tables, int bt_stride, int H,
-                                                        int G, int dk, int dv, int ldv, int pitch, float scale,
-                                                        const float* __restrict__ gate, T* __restrict__ out,
-                                                        int out_stride) {
-    extern __shared__ float sm[];  // per wave: q [dk], p [64]
-    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int t = blockIdx.x, h = blockIdx.y * 4 + wv;
-    if (h >= H) return;
-    float* sq = sm + wv * (dk + ROW_PAGE);
-    float* sp = sq + dk;
-    const T* qr = q + ((size_t)t * H + h) * dk;
-    for (int d = lane; d < dk; d += 64) sq[d] = (float)qr[d];  // q and K are zero past the head's width
-    __builtin_amdgcn_wave_barrier();
-    const int pos = positions[t], g = h / (H / G);
+// W waves share one (row, head): wave i walks pages i, i + W, ...; their sums meet in LDS (W 4: one workgroup per head, W 8
+// and 16: likewise with more waves; W 1: four heads a workgroup).  A wave's walk is a chain of loads, so few (row, head)
+// pairs leave the chip idle: 3 rows of 32 fp32 heads of 128 over 2000 keys took 389 us on one wave each, 56 on 16.
+template <typename T, int W>
+__global__ __launch_bounds__(W > 4 ? 64 * W : 256) void attn_rows_kernel(
+    const T* __restrict__ q, const T* __restrict__ kc, const T* __restrict__ vc, const int* __restrict__ positions,
+    const int* __restrict__ seq_idx, const int* __restrict__ block_tables, int bt_stride, int H, int G, int dk, int dv,
+    int ldv, int pitch, float scale, const float* __restrict__ gate, T* __restrict__ out, int out_stride) {
+    constexpr int HPB = W > 4 ? 1 : 4 / W;  // heads of a workgroup
+    extern __shared__ float sm[];           // q [HPB][dk], p [waves][64]; W > 1: sums [waves][dv], (maximum, sum) [waves]
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, part = wv % W;
+    const int t = blockIdx.x, h = blockIdx.y * HPB + wv / W;
+    const bool live = h < H;
+    if (W == 1 && !live) return;
+    float* sq = sm + wv / W * dk;
+    float* sp = sm + HPB * dk + wv * ROW_PAGE;
+    const T* qr = q + ((size_t)t * H + (live ? h : 0)) * dk;
+    if (W == 1) {
+        for (int d = lane; d < dk; d += 64) sq[d] = (float)qr[d];  // q and K are zero past the head's width
+        __builtin_amdgcn_wave_barrier();
+    } else {
+        for (int d = 64 * part + lane; d < dk; d += 64 * W) sq[d] = (float)qr[d];
+        __syncthreads();
+    }
+    const int pos = live ? positions[t] : -1, g = (live ? h : 0) / (H / G);
     const int* bt = block_tables + (size_t)seq_idx[t] * bt_stride;
     float m = -INFINITY, l = 0.f, acc[ROW_MAXV];
 #pragma unroll
     for (int j = 0; j < ROW_MAXV; ++j) acc[j] = 0.f;
-    for (int k0 = 0; k0 <= pos; k0 += ROW_PAGE) {
+    for (int k0 = part * ROW_PAGE; k0 <= pos; k0 += W * ROW_PAGE) {
         const size_t slab = ((size_t)bt[k0 / ROW_PAGE] * G + g) * ROW_PAGE;
         float s = -INFINITY;
         if (k0 + lane <= pos) {
@@ -50,7 +58,9 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(const T* __restrict__ q,
             s *= scale;
         }
         const float mn = fmaxf(m, wave_max(s));
-        const float alpha = expf(m - mn), p = expf(s - mn);
+        // nothing but minus infinity so far: no weight (the difference of the two would be NaN)
+        const float alpha = W > 1 && mn == -INFINITY ? 1.f : expf(m - mn);
+        const float p = W > 1 && mn == -INFINITY ? (s == s ? 0.f : s) : expf(s - mn);
         m = mn;
         l = l * alpha + wave_sum(p);
         __builtin_amdgcn_wave_barrier();
@@ -67,6 +77,38 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(const T* __restrict__ q,
                 acc[j] = a;
             }
         }
+    }
+    if constexpr (W > 1) {
+        constexpr int WAVES = HPB * W;
+        float* so = sm + HPB * dk + WAVES * ROW_PAGE;
+        float* sml = so + WAVES * dv;
+#pragma unroll
+        for (int j = 0; j < ROW_MAXV; ++j)
+            if (lane + 64 * j < dv) so[wv * dv + lane + 64 * j] = acc[j];
+        if (lane == 0) {
+            sml[2 * wv] = m;
+            sml[2 * wv + 1] = l;
+        }
+        __syncthreads();
+        if (!live) return;
+        const int w0 = wv - part;
+        float top = -INFINITY, sum = 0.f, f[W];
+#pragma unroll
+        for (int i = 0; i < W; ++i) top = fmaxf(top, sml[2 * (w0 + i)]);
+#pragma unroll
+        for (int i = 0; i < W; ++i) {
+            f[i] = expf(sml[2 * (w0 + i)] - top);
+            sum += f[i] * sml[2 * (w0 + i) + 1];
+        }
+        const float scl = (gate ? gate[(size_t)t * H + h] : 1.f) / sum;
+        T* o = out + (size_t)t * out_stride + (size_t)h * pitch;
+        for (int d = 64 * part + lane; d < pitch; d += 64 * W) {
+            float v = 0.f;
+#pragma unroll
+            for (int i = 0; i < W; ++i) v += f[i] * so[(w0 + i) * dv + d];
+            o[d] = (T)(v * scl);
+        }
+        return;
     }
     const float f = (gate ? gate[(size_t)t * H + h] : 1.f) / l;
     T* o = out + (size_t)t * out_stride + (size_t)h * pitch;
@@ -85,18 +127,33 @@ MRSUM_API int mrsum_attn_rows(const void* q, const void* kc, const void* vc, con
                               hipStream_t s) {
     if (T <= 0) return 0;
     if (H % G || dk % 4 || pitch > dv || dv > 64 * ROW_MAXV || ldv < dv) return (int)hipErrorInvalidValue;
-    const dim3 grid(T, ceil_div(H, 4));
-    const size_t lds = 4 * (dk + ROW_PAGE) * sizeof(float);
-    if (lds > 64 * 1024) return (int)hipErrorInvalidValue;
-    if (f32)
-        attn_rows_kernel<<<grid, 256, lds, s>>>((const float*)q, (const float*)kc, (const float*)vc, positions, seq_idx,
-                                                block_tables, bt_stride, H, G, dk, dv, ldv, pitch, scale, gate,
-                                                (float*)out, out_stride);
-    else
-        attn_rows_kernel<<<grid, 256, lds, s>>>((const bf16*)q, (const bf16*)kc, (const bf16*)vc, positions, seq_idx,
-                                                block_tables, bt_stride, H, G, dk, dv, ldv, pitch, scale, gate,
-                                                (bf16*)out, out_stride);
-    return (int)hipGetLastError();
+    if (4 * (dk + ROW_PAGE) * sizeof(float) > 64 * 1024) return (int)hipErrorInvalidValue;
+    // Waves per (row, head), from 4 to 8192 pairs of four head shapes over 60 to 6000 keys.  One wave against 16 at 256 pairs:
+    // 388 and 52 us (fp32 heads of 128, 2000 keys), 1028 and 172 (latents); 8 against 16 at 512: 101 and 110; 4 against 8 at
+    // 1024: 238 and 243, one wave 555.  From 2048 the chip is full: 163 against one wave's 198 for the former at 600 keys,
+    // but 484 against 460 for latents, and more at 60 keys.
+    const size_t pairs = (size_t)T * H;
+    const int waves = pairs <= 256 ? 16 : pairs <= 512 ? 8 : pairs <= 1024 ? 4 : 1;
+#define ROWS(T_, W_)                                                                                                   \
+    {                                                                                                                  \
+        constexpr int HPB = W_ > 4 ? 1 : 4 / W_, WAVES = HPB * W_;                                                     \
+        const size_t lds = (HPB * dk + WAVES * (ROW_PAGE + (W_ > 1 ? dv + 2 : 0))) * sizeof(float);                    \
+        attn_rows_kernel<T_, W_><<<dim3(T, ceil_div(H, HPB)), 64 * WAVES, lds, s>>>(                                   \
+            (const T_*)q, (const T_*)kc, (const T_*)vc, positions, seq_idx, block_tables, bt_stride, H, G, dk, dv,     \
+            ldv, pitch, scale, gate, (T_*)out, out_stride);                                                            \
+        return (int)hipGetLastError();                                                                                 \
+    }
+#define FORMS(T_)                   \
+    if (waves == 16) ROWS(T_, 16)   \
+    if (waves == 8) ROWS(T_, 8)     \
+    if (waves == 4) ROWS(T_, 4)     \
+    ROWS(T_, 1)
+    if (f32) {
+        FORMS(float)
+    }
+    FORMS(bf16)
+#undef FORMS
+#undef ROWS
 }
 
 // ------------------------------------------------------------------------------------------------ prompt portions
