@@ -62,6 +62,9 @@ constexpr int KBLK = 128;
 // one KiB scratch for the dummy x pieces + 2 KiB for the consumer's row-norm partials [64][SS_PARTS]
 constexpr int LDS_XTRA = 3 * 1024;
 constexpr int LDS_BUDGET = 160 * 1024 - LDS_XTRA;
+// the same for an x tile of 16 mt rows: tall tiles take no deferred norm, and no dummy pieces where the waves share the x
+// pieces evenly -- 96 rows beside 64 W rows then have 4 slots in 160 KiB (N 4096, K 14336, 92 rows: 29.5 -> 28.2 us)
+constexpr int lds_extra(int mt, int wpb) { return mt <= 4 ? LDS_XTRA : 4 * mt % wpb ? 1024 : 0; }
 
 // deferred-RMSNorm operands (see the header); all null / zero for a plain GEMM
 struct NormArgs {
@@ -378,13 +381,14 @@ __global__ __launch_bounds__(64 * WPB, 1) void stream_gemm_kernel(const bf16* __
                                                                   const NormArgs e) {
     constexpr int R = 16 * WPB, BM = 16 * MT;
     constexpr int WBYTES = R * 256, SLOT = WBYTES + BM * 256;
-    constexpr int D = (LDS_BUDGET / SLOT) < 6 ? (LDS_BUDGET / SLOT) : 6;
-    static_assert(D >= 2, "ring too shallow");
     constexpr int XP = 2 * BM / 8;               // x pieces per slot (= 4 MT)
     constexpr int XI = (XP + WPB - 1) / WPB;     // x pieces per wave (padded)
     constexpr int NI = 4 + XI;                   // DMA instructions per wave per slot (W: R/4 pieces / WPB = 4)
-    __shared__ __attribute__((aligned(1024))) char lds[D * SLOT + LDS_XTRA];
-    float* const s_ss = reinterpret_cast<float*>(lds + D * SLOT + 1024);  // consumer row-norm partials
+    constexpr int XTRA = lds_extra(MT, WPB), FIT = (160 * 1024 - XTRA) / SLOT;
+    constexpr int D = FIT < 6 ? FIT : 6;
+    static_assert(D >= 2, "ring too shallow");
+    __shared__ __attribute__((aligned(1024))) char lds[D * SLOT + XTRA];
+    float* const s_ss = reinterpret_cast<float*>(lds + (MT > 4 ? 0 : D * SLOT + 1024));  // consumer row-norm partials
 
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int n0 = blockIdx.x * R;
@@ -472,7 +476,7 @@ static bool tp_push_ok(const void* ar, int epi, int M, int N) {
 // launch leaves them zero again).  ssq (any epilogue): deferred-RMSNorm input, [M, ssq_tiles] fp32 row
 // sums of squares of x (x = the un-normalised residual rows), ssq_tiles % 32 == 0; the product rows are
 // scaled by rsqrt(sum / K + eps).  N % (16 wpb) == 0, wpb in {4, 5, 6, 7, 8}, M <= 64 -- or 64 < M <= 128
-// (decode batches of 65-128 sequences: 96- / 128-row x tiles, one pass over the weights instead of one per
+// (decode batches of 65-128 sequences: 80- to 128-row x tiles, one pass over the weights instead of one per
 // 64-row chunk) for the bf16 / fp32-slab / SwiGLU epilogues without a deferred norm.
 // Decode weights are streamed with nontemporal loads (each weight row read once per step by one CU:
 // MI355X_MICROARCH.md "nt-weights"; profiles/r1_decode_nt_ab.jsonl).
@@ -489,8 +493,8 @@ MRSUM_API int mrsum_stream_gemm(const void* x, int ldx, const void* W, int N, in
     if (M > 64) {
         // tall tiles only at widths whose slot (16 wpb W rows + 16 MT x rows, 256 B each) leaves a ring of at
         // least 3 slots (one being filled, two published); ops/hip.py _TALL_WPB lists the same widths
-        const int slot = (16 * wpb + 16 * (M > 96 ? 8 : 6)) * 256;
-        if (LDS_BUDGET / slot < 3) return (int)hipErrorInvalidValue;
+        const int mt = (M + 15) / 16, slot = (16 * wpb + 16 * mt) * 256;
+        if ((160 * 1024 - lds_extra(mt, wpb)) / slot < 3) return (int)hipErrorInvalidValue;
     }
     const bool split_epi = epi == EPI_SWIGLU_SPLIT || epi == EPI_RESID_SPLIT;
     if (epi != EPI_F32_PARTIAL && !split_epi && splits != 1) return (int)hipErrorInvalidValue;
@@ -535,7 +539,9 @@ MRSUM_API int mrsum_stream_gemm(const void* x, int ldx, const void* W, int N, in
         case 2: BY_EPI(2); break;
         case 3: BY_EPI(3); break;
         case 4: BY_EPI(4); break;
-        case 5: case 6: BY_EPI_TALL(6); break;
+        case 5: BY_EPI_TALL(5); break;
+        case 6: BY_EPI_TALL(6); break;
+        case 7: BY_EPI_TALL(7); break;
         default: BY_EPI_TALL(8); break;
     }
 #undef BY_EPI_TALL

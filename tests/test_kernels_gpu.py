@@ -1114,6 +1114,22 @@ def test_stream_gemm_tall_tiles_match_row_chunks(M, monkeypatch):
             _close(outs[0].sum(0), x.float() @ w.float().t(), 1e-3, 1e-3)
 
 
+@pytest.mark.parametrize("M,wpb", [(65, 8), (80, 7), (80, 8), (81, 7), (96, 4), (97, 6), (112, 5), (113, 5)])
+def test_stream_gemm_tall_widths(M, wpb):
+    """Every tile height and the widths it newly takes, rings of 3 and 4 slots: equal to the 64-row chunks, bit for bit."""
+    K, n = 1024, 16 * wpb * 3
+    x, w = _rand(M, K, seed=82), _rand(n, K, scale=0.05, seed=83)
+    for epi, S in ((hip.EPI_F32_PARTIAL, 2), (hip.EPI_BF16, 1), (hip.EPI_SWIGLU, 1)):
+        cols = n // 2 if epi == hip.EPI_SWIGLU else n
+        shape, dt = ((S, M, n), torch.float32) if epi == hip.EPI_F32_PARTIAL else ((M, cols), torch.bfloat16)
+        one, two = (torch.full(shape, float("nan"), dtype=dt, device=DEV) for _ in range(2))
+        hip._stream_launch(x, w, one, epi, S, cols, wpb, None, None, None, None, None, M if S > 1 else 0)
+        for a, b in ((0, 64), (64, M)):
+            o = two[:, a:b] if S > 1 else two[a:b]
+            hip._stream_launch(x[a:b], w, o, epi, S, cols, wpb, None, None, None, None, None, M if S > 1 else 0)
+        assert torch.equal(one, two), epi
+
+
 @pytest.mark.parametrize("M", [65, 96, 128])
 def test_linear_tall_lm_head(M):
     """linear() of 65-128 rows of a stream shape (the decode LM head of the 24 h map's bucket 96) runs the
