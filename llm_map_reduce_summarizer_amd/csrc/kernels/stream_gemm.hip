@@ -1,4 +1,4 @@
-// Decode GEMM with an LDS-DMA weight ring: out[M, N] = x[M, K] . W[N, K]^T, M <= 64.
+// Decode GEMM with an LDS-DMA weight ring: out[M, N] = x[M, K] . W[N, K]^T, M <= 128.
 //
 // Why a second decode GEMM: the register-streaming kernels (skinny_gemm.hip) keep 8-16 KiB of W
 // in flight per workgroup and reach 4-5 TB/s; at M = 16-64 the x fragments they re-read and the
@@ -64,7 +64,14 @@ constexpr int LDS_XTRA = 3 * 1024;
 constexpr int LDS_BUDGET = 160 * 1024 - LDS_XTRA;
 // the same for an x tile of 16 mt rows: tall tiles take no deferred norm, and no dummy pieces where the waves share the x
 // pieces evenly -- 96 rows beside 64 W rows then have 4 slots in 160 KiB (N 4096, K 14336, 92 rows: 29.5 -> 28.2 us)
-constexpr int lds_extra(int mt, int wpb) { return mt <= 4 ? LDS_XTRA : 4 * mt % wpb ? 1024 : 0; }
+constexpr int lds_extra(int mt, int wpb, int halves) { return mt <= 4 ? LDS_XTRA : 2 * halves * mt % wpb ? 1024 : 0; }
+constexpr int ring_slots(int mt, int wpb, int halves) {
+    const int fit = (160 * 1024 - lds_extra(mt, wpb, halves)) / (2048 * halves * (wpb + mt));
+    return fit < 6 ? fit : 6;
+}
+// 64-wide halves of a k block in a slot: one where two leave a tall tile less than 3 slots (128 W rows beside 96 or more).  A
+// slot's x share falls with its W rows: N 128256, K 4096, 128 x rows: 299 us at 64 W rows, 254 at 128.
+constexpr int slot_halves(int mt, int wpb) { return mt > 4 && ring_slots(mt, wpb, 2) < 3 ? 1 : 2; }
 
 // deferred-RMSNorm operands (see the header); all null / zero for a plain GEMM
 struct NormArgs {
@@ -94,8 +101,9 @@ __device__ __forceinline__ void raw_barrier() {
     asm volatile("" ::: "memory");
 }
 
+template <int H = 2>
 __device__ __forceinline__ int img_off(int row, int chunk) {
-    return (((row >> 3) << 1) + (chunk >> 3)) * 1024 + ((row & 7) << 7) + ((((chunk & 7) ^ (row & 7))) << 4);
+    return ((row >> 3) * H + (chunk >> 3)) * 1024 + ((row & 7) << 7) + ((((chunk & 7) ^ (row & 7))) << 4);
 }
 
 template <int AUX = 0>
@@ -380,30 +388,30 @@ __global__ __launch_bounds__(64 * WPB, 1) void stream_gemm_kernel(const bf16* __
                                                                   float* __restrict__ parts, int* __restrict__ counters,
                                                                   const NormArgs e) {
     constexpr int R = 16 * WPB, BM = 16 * MT;
-    constexpr int WBYTES = R * 256, SLOT = WBYTES + BM * 256;
-    constexpr int XP = 2 * BM / 8;               // x pieces per slot (= 4 MT)
+    constexpr int H = slot_halves(MT, WPB), KB = 64 * H;  // 64-wide pieces of a row in a slot
+    constexpr int WBYTES = R * 128 * H, SLOT = WBYTES + BM * 128 * H;
+    constexpr int XP = H * BM / 8;               // x pieces per slot
     constexpr int XI = (XP + WPB - 1) / WPB;     // x pieces per wave (padded)
-    constexpr int NI = 4 + XI;                   // DMA instructions per wave per slot (W: R/4 pieces / WPB = 4)
-    constexpr int XTRA = lds_extra(MT, WPB), FIT = (160 * 1024 - XTRA) / SLOT;
-    constexpr int D = FIT < 6 ? FIT : 6;
-    static_assert(D >= 2, "ring too shallow");
+    constexpr int NI = 2 * H + XI;               // DMA instructions per wave per slot
+    constexpr int XTRA = lds_extra(MT, WPB, H), D = ring_slots(MT, WPB, H);
+    static_assert(D >= 3 || MT <= 4, "ring too shallow");
     __shared__ __attribute__((aligned(1024))) char lds[D * SLOT + XTRA];
     float* const s_ss = reinterpret_cast<float*>(lds + (MT > 4 ? 0 : D * SLOT + 1024));  // consumer row-norm partials
 
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int n0 = blockIdx.x * R;
     const int ks = blockIdx.y * kper;
-    const int nkb = kper / KBLK;
+    const int nkb = kper / KB;
 
     // per-lane source rows/chunks of this wave's pieces (fixed over k)
     const int prow = lane >> 3, pslot = lane & 7;
-    // W pieces q = 4w + p (p < 4): rows 8 (q >> 1) + prow, k half q & 1
-    const bf16* wsrc[4];
+    // W pieces q = 2 H w + p: rows 8 (q / H) + prow, k half q % H
+    const bf16* wsrc[2 * H];
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        const int q = 4 * w + p;
-        const int row = 8 * (q >> 1) + prow;
-        wsrc[p] = W + (size_t)(n0 + row) * K + ks + 8 * (8 * (q & 1) + (pslot ^ prow));
+    for (int p = 0; p < 2 * H; ++p) {
+        const int q = 2 * H * w + p;
+        const int row = 8 * (q / H) + prow;
+        wsrc[p] = W + (size_t)(n0 + row) * K + ks + 8 * (8 * (q % H) + (pslot ^ prow));
     }
     const bf16* xsrc[XI];
     int xdst[XI];
@@ -411,14 +419,14 @@ __global__ __launch_bounds__(64 * WPB, 1) void stream_gemm_kernel(const bf16* __
     for (int i = 0; i < XI; ++i) {
         const int q = w + WPB * i;  // x piece index; >= XP -> dummy
         const int qq = q < XP ? q : 0;
-        const int row = 8 * (qq >> 1) + prow;
-        xsrc[i] = x + (size_t)min(row, M - 1) * ldx + ks + 8 * (8 * (qq & 1) + (pslot ^ prow));
+        const int row = 8 * (qq / H) + prow;
+        xsrc[i] = x + (size_t)min(row, M - 1) * ldx + ks + 8 * (8 * (qq % H) + (pslot ^ prow));
         xdst[i] = q < XP ? WBYTES + q * 1024 : -1;
     }
 #define ISSUE(slot, kb)                                                                              \
     {                                                                                                \
         char* base = lds + (slot) * SLOT;                                                            \
-        _Pragma("unroll") for (int p = 0; p < 4; ++p) glds16<NTW ? 2 : 0>(wsrc[p] + (kb), base + (4 * w + p) * 1024); \
+        _Pragma("unroll") for (int p = 0; p < 2 * H; ++p) glds16<NTW ? 2 : 0>(wsrc[p] + (kb), base + (2 * H * w + p) * 1024); \
         _Pragma("unroll") for (int i = 0; i < XI; ++i)                                               \
             glds16(xsrc[i] + (kb), xdst[i] >= 0 ? base + xdst[i] : lds + D * SLOT);                  \
     }
@@ -429,22 +437,22 @@ __global__ __launch_bounds__(64 * WPB, 1) void stream_gemm_kernel(const bf16* __
 
     // prologue: D-1 slots in flight (clamped k blocks past the end are never read)
 #pragma unroll
-    for (int s = 0; s < D - 1; ++s) ISSUE(s, min(s, nkb - 1) * KBLK);
+    for (int s = 0; s < D - 1; ++s) ISSUE(s, min(s, nkb - 1) * KB);
 
     const int r = lane & 15, g = lane >> 4;
     for (int j = 0; j < nkb; ++j) {
         if (j + D - 2 < nkb) wait_vmcnt<NI * (D - 2)>();  // slots j+1 .. j+D-2 stay in flight
         else wait_vmcnt<0>();
         raw_barrier();
-        if (j + D - 1 < nkb) ISSUE((j + D - 1) % D, (j + D - 1) * KBLK);
+        if (j + D - 1 < nkb) ISSUE((j + D - 1) % D, (j + D - 1) * KB);
         const char* wl = lds + (j % D) * SLOT;
         const char* xl = wl + WBYTES;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const u32x4 av = *reinterpret_cast<const u32x4*>(wl + img_off(16 * w + r, 4 * i + g));
+        for (int i = 0; i < 2 * H; ++i) {
+            const u32x4 av = *reinterpret_cast<const u32x4*>(wl + img_off<H>(16 * w + r, 4 * i + g));
 #pragma unroll
             for (int m = 0; m < MT; ++m) {
-                const u32x4 bv = *reinterpret_cast<const u32x4*>(xl + img_off(16 * m + r, 4 * i + g));
+                const u32x4 bv = *reinterpret_cast<const u32x4*>(xl + img_off<H>(16 * m + r, 4 * i + g));
                 acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av),
                                                                  __builtin_bit_cast(bf16x8, bv), acc[m], 0, 0, 0);
             }
@@ -490,12 +498,6 @@ MRSUM_API int mrsum_stream_gemm(const void* x, int ldx, const void* W, int N, in
         return (int)hipErrorInvalidValue;
     if (M > 64 && (ssq || (epi != EPI_BF16 && epi != EPI_F32_PARTIAL && epi != EPI_SWIGLU)))
         return (int)hipErrorInvalidValue;  // tall tiles: no deferred norm, no split-K last-arriver epilogue
-    if (M > 64) {
-        // tall tiles only at widths whose slot (16 wpb W rows + 16 MT x rows, 256 B each) leaves a ring of at
-        // least 3 slots (one being filled, two published); ops/hip.py _TALL_WPB lists the same widths
-        const int mt = (M + 15) / 16, slot = (16 * wpb + 16 * mt) * 256;
-        if ((160 * 1024 - lds_extra(mt, wpb)) / slot < 3) return (int)hipErrorInvalidValue;
-    }
     const bool split_epi = epi == EPI_SWIGLU_SPLIT || epi == EPI_RESID_SPLIT;
     if (epi != EPI_F32_PARTIAL && !split_epi && splits != 1) return (int)hipErrorInvalidValue;
     if (split_epi && (!parts || !counters)) return (int)hipErrorInvalidValue;

@@ -1114,9 +1114,10 @@ def test_stream_gemm_tall_tiles_match_row_chunks(M, monkeypatch):
             _close(outs[0].sum(0), x.float() @ w.float().t(), 1e-3, 1e-3)
 
 
-@pytest.mark.parametrize("M,wpb", [(65, 8), (80, 7), (80, 8), (81, 7), (96, 4), (97, 6), (112, 5), (113, 5)])
+@pytest.mark.parametrize("M,wpb", [(65, 8), (80, 7), (81, 7), (96, 4), (96, 8), (97, 6), (112, 7), (113, 5),
+                                   (113, 6), (128, 7), (128, 8)])
 def test_stream_gemm_tall_widths(M, wpb):
-    """Every tile height and the widths it newly takes, rings of 3 and 4 slots: equal to the 64-row chunks, bit for bit."""
+    """Every tile height and the widths it newly takes, slots of 64 and 128 of k: equal to the 64-row chunks, bit for bit."""
     K, n = 1024, 16 * wpb * 3
     x, w = _rand(M, K, seed=82), _rand(n, K, scale=0.05, seed=83)
     for epi, S in ((hip.EPI_F32_PARTIAL, 2), (hip.EPI_BF16, 1), (hip.EPI_SWIGLU, 1)):
