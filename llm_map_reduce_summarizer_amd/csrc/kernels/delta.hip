@@ -1,5 +1,5 @@
 // Gated delta rule, token by token (decoded tokens; 32-bit models; head sizes the chunked form does not take), with the
-// gated head-wise output norm in the same launch.  Per head, S [dim][vdim]:
+// gated head-wise output norm in the same launch; prompt portions have a kernel of their own that stages the rows ahead.  Per head, S [dim][vdim]:
 //
 //     S <- g S;   u = beta (v - S^T k);   S <- S + k u^T;   o = S^T q
 //     out = o / rms(o) * w * silu(gate)

@@ -3,13 +3,13 @@
 //     C[M, N] = X[M, K] . W[N, K]^T        K % 32 == 0
 //
 // 128 x 128 output tile per 256-thread workgroup, two workgroups per CU; wave (wr, wc) owns 64 x 64 outputs as 4 x 4
-// blocks, or for M <= 64 (LOW) wave w 64 x 32, so that all four SIMDs have work
-// (64 x 28672 x 4096: 248 -> 145 us; a form of its own: a branch cost the others 9 %).  K-tiles of 32 (128 bytes a row) arrive by LDS-DMA in two buffers, chunk c of row r at c ^ ((r >> 1) & 7)
-// (conflict-free b128 fragment reads); a fragment's four floats feed four instructions, so a K-tile is 16 LDS reads for
-// 128 instructions of 32 cycles, and the matrix cores set the time (1.7 us a K-tile) once a CU has work.  16-row
-// blocks past M are skipped.  903 x 28672 x 4096: 2310 (64 x 64 tiles, loads between barriers) -> 1650 us, 129 TFLOP/s of
-// 157 and 146 counting the rows that pad the last tile.  Tiles that would leave CUs idle run in slices of K (ops/hip.py gemm32_splits), whose
-// fp32 sums a second launch adds in slice order.
+// blocks, or for M <= 64 (LOW) wave w 64 x 32, so that all four SIMDs have work (64 x 28672 x 4096: 248 -> 145 us; a form
+// of its own: a branch cost the others 9 %).  K-tiles of 32 (128 bytes a row) arrive by LDS-DMA in two buffers, chunk c of
+// row r at c ^ ((r >> 1) & 7) (conflict-free b128 fragment reads); a fragment's four floats feed four instructions, so a
+// K-tile is 16 LDS reads for 128 instructions of 32 cycles, and the matrix cores set the time (1.7 us a K-tile) once a CU
+// has work.  16-row blocks past M are skipped.  903 x 28672 x 4096: 2310 (64 x 64 tiles, loads between barriers) -> 1650
+// us, 129 TFLOP/s of 157 and 146 counting the rows that pad the last tile.  Tiles that would leave CUs idle run in slices
+// of K (ops/hip.py gemm32_splits), whose fp32 sums a second launch adds in slice order.
 #include "common.h"
 
 #include <type_traits>
