@@ -141,11 +141,12 @@ def test_gemm_graph_capture():
     _check(out, x.float() @ w.float().t())
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 32, 2048), (130, 544, 2112), (257, 4096, 2112), (4097, 4096, 2048)])
+@pytest.mark.parametrize("M,N,K", [(1, 32, 2048), (130, 544, 2112), (257, 4096, 2112), (4097, 4096, 2048),
+                                   (3300, 2560, 12288)])
 @pytest.mark.parametrize("epi", ["bf16", "swiglu", "gelu", "f32"])
 def test_gemm_split_tail(M, N, K, epi):
     """Tiles behind the last whole round run in slices of K that a second launch adds: one tile of one row, a ragged
-    last slice, few tiles, and 16 sliced tiles behind a whole round; repeated calls are the same bits."""
+    last slice, few tiles, 16 sliced tiles behind a whole round, and two rounds of thirds; repeated calls are the same bits."""
     assert hip.gemm_splits(M, N, K // 64)[1] > 1
     x, w = _rand(M, K, seed=12, scale=0.5, offset=0.02), _rand(N, K, seed=13, scale=0.03, offset=0.001)
     if epi == "swiglu":
@@ -178,7 +179,7 @@ def test_stream_parts_beyond_tall_tiles(M):
     assert bool(((parts.sum(0).double() - x.double() @ w.double().t()).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 32, 2048), (130, 544, 2112), (257, 4096, 2112)])
+@pytest.mark.parametrize("M,N,K", [(1, 32, 2048), (130, 544, 2112), (257, 4096, 2112), (3300, 2560, 12288)])
 def test_gemm_slabs(M, N, K):
     """A grid whose tiles all run in slices of K leaves the slices apart; other grids give none."""
     x, w = _rand(M, K, seed=16, scale=0.5), _rand(N, K, seed=17, scale=0.03)
