@@ -159,8 +159,9 @@ MRSUM_API int mrsum_attn_rows(const void* q, const void* kc, const void* vc, con
 // ------------------------------------------------------------------------------------------------ prompt portions
 // The same attention for many rows of few sequences, on the fp32 matrix instruction.  The row kernel reads every key
 // from memory for every (row, head): 1088 us for 900 rows of 32 heads of 128 over 8 kv heads, 4380 over 576-wide latents.
-// Here (183 and 755 us, 36 TFLOP/s; the exponentials and their exchange are the rest) 64 (row, head) pairs -- RB consecutive rows of HB heads of one kv head -- share
-// key and value tiles of 32 in LDS (two buffers, the next tile on its way in registers), a wave for 16 pairs.
+// Here (183 and 755 us, 36 TFLOP/s; the exponentials and their exchange are the rest) 64 (row, head) pairs -- RB
+// consecutive rows of HB heads of one kv head -- share key and value tiles of 32 in LDS (two buffers, the next tile on its
+// way in registers), a wave for 16 pairs.
 //
 // Scores are computed transposed, S^T = K Q^T: lane (pair = lane & 15, g = lane >> 4) holds the scores of keys 4 g .. 4 g
 // + 3 of a 16-key block, which is how the second product O^T = V^T P^T takes its right operand, so weights stay in
