@@ -100,13 +100,6 @@ __device__ __forceinline__ float glu(float g, float u, const GluArgs& a) {
     u = fminf(fmaxf(u, -a.limit), a.limit);
     return g / (1.f + __expf(-a.alpha * g)) * (u + a.shift);
 }
-// With the hardware reciprocal, for values that leave as 16-bit: in the tile GEMM, 64 values a thread, the division was 2 % of
-// the kernel (8192 x 28672 x 4096 1464 -> 1440 us).
-__device__ __forceinline__ float glu_rcp(float g, float u, const GluArgs& a) {
-    g = fminf(g, a.limit);
-    u = fminf(fmaxf(u, -a.limit), a.limit);
-    return g * __builtin_amdgcn_rcpf(1.f + __expf(-a.alpha * g)) * (u + a.shift);
-}
 
 // Attention output form: head h of row t goes to columns [h * pitch, (h + 1) * pitch) of the row, times
 // gate[t * gate_ld + h] when a gate is given.

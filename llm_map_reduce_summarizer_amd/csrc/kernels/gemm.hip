@@ -373,7 +373,7 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmArgs a) {
     auto silu_mul = [&](const f32x4& g, const f32x4& u) {
         f32x4 r;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) r[j] = glu_rcp(g[j], u[j], a.glu);
+        for (int j = 0; j < 4; ++j) r[j] = glu(g[j], u[j], a.glu);
         return r;
     };
     // 4 bf16 outputs of tile row rl at byte cbyte of the output tile row; gcol = first weight column of
@@ -522,7 +522,7 @@ __global__ __launch_bounds__(512) void gemm_tail_kernel(const GemmArgs a) {
 #pragma unroll
             for (int k = 0; k < 4; ++k) up[k] = __shfl_xor(v[j][k], 32, 64);
 #pragma unroll
-            for (int k = 0; k < 4; ++k) v[j][k] = glu_rcp(v[j][k], up[k], a.glu);
+            for (int k = 0; k < 4; ++k) v[j][k] = glu(v[j][k], up[k], a.glu);
             col = (cb >> 1) + 4 * g4;
         } else if constexpr (EPI == GEPI_GELU) {
 #pragma unroll

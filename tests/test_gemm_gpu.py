@@ -169,6 +169,20 @@ def test_gemm_split_tail(M, N, K, epi):
     assert bool(((out.double() - y).abs() <= 2.0 ** -8 * y.abs() + 1e-4).all())
 
 
+@pytest.mark.parametrize("K", [64, 2048])
+def test_gemm_swiglu_small_gates(K):
+    """sigmoid(gate) below the smallest normal number (gates under -87.3) times a large up value, one launch (K 64) and
+    slices of K (2048): the quotient gate / (1 + e^-gate) is a normal number and must not become 0."""
+    gate = torch.tensor([-86.0, -87.0, -88.0, -88.5], dtype=torch.float64)
+    x, w = torch.zeros(4, K, dtype=torch.bfloat16), torch.zeros(32, K, dtype=torch.bfloat16)
+    x[range(4), range(4)] = 1
+    w[:, :4] = torch.where(torch.arange(32)[:, None] % 16 < 8, gate, torch.tensor(2.0 ** 100, dtype=torch.float64))
+    out = hip.gemm(x.to(DEV), w.to(DEV), swiglu=True).cpu().double()
+    want = (gate / (1 + torch.exp(-gate)) * 2.0 ** 100)[:, None].expand(4, 16)
+    # one bf16 rounding (2^-9); the fp32 exponential of 88 is good to 88 * 2^-23
+    assert bool(((out - want).abs() <= 2.0 ** -8 * want.abs()).all())
+
+
 @pytest.mark.parametrize("M", [128, 129, 256, 257])
 def test_stream_parts_beyond_tall_tiles(M):
     """Split-K slab consumers get one fp32 slab of the tile GEMM above the stream kernel's tallest x tile."""
