@@ -402,9 +402,10 @@ __global__ __launch_bounds__(256) void ssm_portion_kernel(const T* __restrict__ 
             for (int v = 0; v < NV; ++v) *reinterpret_cast<float4*>(&s_bc[buf][r][k][4 * (l + 16 * v)]) = fb[k][v];
 #pragma unroll
         for (int i = 0; i < R; ++i) s_x[buf][r][l + 16 * i] = fx[i];
-        if (l == 0) {  // rows past the end leave the state as it is
-            const float dt = t0 + r < e ? softplus(fd + db) : 0.f;
-            s_d[buf][r] = make_float2(dt, expf(an * dt));
+        if (l == 0) {  // rows past the end leave the state as it is, also where the decay is total (0 * -inf is NaN)
+            const bool in = t0 + r < e;
+            const float dt = in ? softplus(fd + db) : 0.f;
+            s_d[buf][r] = make_float2(dt, in ? expf(an * dt) : 1.f);
         }
     };
     fetch(b);

@@ -192,6 +192,29 @@ def test_state_space_portions_token_by_token(copies, dtype, N):
     assert rel(got, want) < 3e-6 and rel(got_s, want_s) < 3e-6
 
 
+@pytest.mark.parametrize("dtype,P,N", [(F32, 20, 24), (F32, 64, 128), (BF, 136, 248)])
+def test_state_space_portions_total_decay(dtype, P, N):
+    """A_log so large that -exp(A_log) is minus infinity: every row forgets the state before it, and the rows that pad a
+    portion to the 16 that are staged at a time leave the last row's state alone."""
+    from llm_map_reduce_summarizer_amd import ops
+    heads, groups, lens = 3, 1, [1, 15, 16, 17]
+    T, C = sum(lens), heads * P + 2 * groups * N
+    xbc, u = rnd(T, C + (-C) % 8, std=0.7).to(dtype), rnd(1, T, 8, seed=1)
+    A_log = torch.tensor([0.5, 89.0, 100.0])
+    vec = [rnd(heads, seed=2), -torch.exp(A_log), rnd(heads, seed=4)]
+    slots, pos0 = [2, 1, 4, 3], [5, 0, 9, 7]
+    state = rnd(5, heads, P, N + (-N) % 4, seed=5, std=0.5)
+    state[..., N:] = 0
+    got_s, want_s = dev(state), state.clone()
+    segs = segments(lens, slots, pos0)
+    host = ops.Segments(segs.slots.cpu(), segs.pos0.cpu(), segs.cu.cpu(), segs.row_seg.cpu(), lens)
+    got = ops.ssm_scan(dev(xbc), dev(u), 0, *map(dev, vec), got_s, segs, heads, P, N, groups)
+    want = ops.ssm_scan(xbc, u, 0, *vec, want_s, host, heads, P, N, groups)
+    assert bool(torch.isfinite(want).all() and torch.isfinite(want_s).all())
+    # as above
+    assert rel(got, want) < 3e-6 and rel(got_s, want_s) < 3e-6
+
+
 def scan_with_state(x, B, C, dt, A_log, D, groups, S0):
     """The oracle's scan continued from S0 [heads, P, N]: the carried state as one more leading token is not possible,
     so its contribution decays beside the oracle's own output."""
