@@ -58,9 +58,9 @@ __global__ __launch_bounds__(W > 4 ? 64 * W : 256) void attn_rows_kernel(
             s *= scale;
         }
         const float mn = fmaxf(m, wave_max(s));
-        // nothing but minus infinity so far: no weight (the difference of the two would be NaN)
-        const float alpha = W > 1 && mn == -INFINITY ? 1.f : expf(m - mn);
-        const float p = W > 1 && mn == -INFINITY ? (s == s ? 0.f : s) : expf(s - mn);
+        // while all scores are minus infinity there is no weight yet (-inf - -inf would be NaN)
+        const float ref = mn == -INFINITY ? 0.f : mn;
+        const float alpha = expf(m - ref), p = expf(s - ref);
         m = mn;
         l = l * alpha + wave_sum(p);
         __builtin_amdgcn_wave_barrier();
@@ -277,6 +277,7 @@ __global__ __launch_bounds__(256, NQ <= 8 ? 2 : 1) void attn_portion_kernel(
             mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
             const float mn = fmaxf(m, mx), alpha = mn == m ? 1.f : expf(m - mn);
+            const float ref = mn == -INFINITY ? 0.f : mn;  // no weight yet, as in the row kernel
             m = mn;
             l *= alpha;
             if (__any(alpha != 1.f)) {
@@ -288,7 +289,7 @@ __global__ __launch_bounds__(256, NQ <= 8 ? 2 : 1) void attn_portion_kernel(
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const float x = s[kb][i];
-                    s[kb][i] = mine && k0 + 16 * kb + 4 * g4 + i <= pos ? expf(x - mn) : 0.f;
+                    s[kb][i] = mine && k0 + 16 * kb + 4 * g4 + i <= pos ? expf(x - ref) : 0.f;
                     l += s[kb][i];
                 }
             auto vrow = [&](int k) -> const float* { return SHARED ? s_k[buf][k] : s_v[SHARED ? 0 : buf][SHARED ? 0 : k]; };

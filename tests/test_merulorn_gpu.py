@@ -393,6 +393,43 @@ def test_row_attention_waves(H, G, dk, dv, dtype, n):
     assert rel(got.float(), want.float()) < (4e-3 if dtype == BF else 2e-6)
 
 
+@pytest.mark.parametrize("copies", [1, 43, 86, 171])  # decoded rows: 6, 258, 516 and 1026 pairs; portions: tiles
+@pytest.mark.parametrize("first", [20, 40, 100])
+@pytest.mark.parametrize("H,G,dk,dv", [(6, 2, 64, 64), (6, 3, 200, 256), (6, 1, 576, 512)])
+def test_row_attention_first_keys_without_weight(H, G, dk, dv, first, copies, monkeypatch):
+    """Scores of minus infinity at the head of a sequence, over less than a tile, more than a tile and more than a page: rows
+    that see a finite score give it the weight, rows that see none are no numbers, in every form of the kernels."""
+    from llm_map_reduce_summarizer_amd import ops
+    from llm_map_reduce_summarizer_amd.ops import hip
+    latent, page, args = dk > 256, 64, (64, dk ** -0.5)
+    kc = rnd(5, G, page, dk, seed=1)
+    kc[1, :, :first, -1] = float("-inf")
+    kc[2, :, :max(0, first - page), -1] = float("-inf")
+    vc = kc if latent else rnd(5, G, page, dv, seed=2)
+    pos = torch.cat([torch.tensor([first - 5, first, first + 60]).repeat(copies)[:copies],
+                     torch.arange(first - 10, first + 50)]).int()
+    n, singles = len(pos), copies
+    seq = torch.cat([torch.arange(copies), torch.full((60,), copies)]).int()
+    tables = torch.tensor([[1, 2, 3, 4]]).repeat(copies + 1, 1).int()
+    q = rnd(n, H * dk, seed=3)
+    q[:, dk - 1::dk].abs_().add_(1)
+    monkeypatch.setattr(hip, "PORTION_PAIRS", 0)
+    i32 = [pos, seq, tables]
+    if latent:
+        want = ops.latent_rows(q, kc, *i32, H, dv, *args)
+        got = ops.latent_rows(dev(q), dev(kc), *map(dev, i32), H, dv, *args, singles=singles)
+    else:
+        gate = torch.sigmoid(rnd(n, H, seed=5))
+        want, got = torch.zeros(n, H * dv), torch.zeros(n, H * dv, device=DEV)
+        ops.attn_rows(q, kc, vc, *i32, H, G, dv, *args, gate, want)
+        ops.attn_rows(dev(q), dev(kc), dev(vc), *map(dev, i32), H, G, dv, *args, dev(gate), got, singles=singles)
+    got, some = got.cpu(), pos >= first
+    assert bool(torch.isfinite(want[some]).all()) and bool(torch.isnan(want[~some]).all())
+    assert bool(torch.isnan(got[~some]).all())
+    # fp32 scores of dk products, exp, sums of up to 161 keys: a few 2^-24 each
+    assert rel(got[some], want[some]) < 2e-6
+
+
 @pytest.mark.parametrize("H,G,dk,dv", [(8, 2, 48, 32), (6, 2, 128, 100), (5, 5, 64, 64), (4, 1, 200, 256), (70, 1, 16, 8),
                                        (32, 1, 576, 512), (3, 1, 300, 20)])
 @pytest.mark.parametrize("dtype", DTYPES)
