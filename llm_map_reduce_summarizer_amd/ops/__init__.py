@@ -277,7 +277,7 @@ def project(x, w, role):
             return parts
     cfg = hip.project_config(N, K) if M <= hip.STREAM_MAX_M else None
     if cfg is not None:
-        return hip.linear_parts(x, w, cfg[1], nt=cfg[0], kernel="stream")
+        return hip.stream_slabs(x, w, cfg[1], cfg[0])
     p = hip.plan(role, M, N, K)
     return hip.gemm(x, w) if p[0] == "gemm" else _plan_parts(hip, p, x, w, None)
 
@@ -463,7 +463,7 @@ def _plan_parts(hip, p, x, w, splits):
     if p[0] == "stream":
         if isinstance(x, NormRows):
             return hip.linear_parts(x.h, w, p[2], nt=p[1], kernel="stream", norm=x.norm)
-        return hip.linear_parts(x, w, p[2], nt=p[1], kernel="stream")
+        return hip.stream_slabs(x, w, p[2], p[1])
     x = rows(x)
     if p[0] == "lds":
         return hip.linear_parts(x, w, splits or p[1], kernel="lds")

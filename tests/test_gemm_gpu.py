@@ -185,12 +185,13 @@ def test_gemm_swiglu_small_gates(K):
 
 @pytest.mark.parametrize("M", [128, 129, 256, 257])
 def test_stream_parts_beyond_tall_tiles(M):
-    """Split-K slab consumers get one fp32 slab of the tile GEMM above the stream kernel's tallest x tile."""
+    """linear_parts gives the slabs it is asked for at any row count; consumers that add however many there are get one
+    fp32 slab of the tile GEMM above the stream kernel's tallest x tile."""
     x, w = _rand(M, 1024, seed=14, scale=0.5), _rand(4096, 1024, seed=15, scale=0.03)
-    parts = hip.linear_parts(x, w, 2, nt=4, kernel="stream")
-    assert parts.dtype == torch.float32 and parts.shape == (2 if M <= 128 else 1, M, 4096)
     bound = 1024 * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
-    assert bool(((parts.sum(0).double() - x.double() @ w.double().t()).abs() <= bound).all())
+    for parts, n in ((hip.linear_parts(x, w, 2, nt=4, kernel="stream"), 2), (hip.stream_slabs(x, w, 2, 4), 2 if M <= 128 else 1)):
+        assert parts.dtype == torch.float32 and parts.shape == (n, M, 4096)
+        assert bool(((parts.sum(0).double() - x.double() @ w.double().t()).abs() <= bound).all())
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 32, 2048), (130, 544, 2112), (257, 4096, 2112), (3300, 2560, 12288)])
