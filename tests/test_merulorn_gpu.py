@@ -490,6 +490,27 @@ def test_gemm32_edges(M, N, K, split):
     assert got.shape == (M, N) and bool(((got - x.double() @ w.double().T).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("M", [5, 130])
+@pytest.mark.parametrize("off_x,off_w", [(1, 0), (0, 3), (2, 1)])
+def test_gemm32_unaligned_storage(M, off_x, off_w):
+    """Contiguous operands that begin anywhere in their storage."""
+    from llm_map_reduce_summarizer_amd.ops import hip
+    N, K = 200, 256
+    x, w = dev(rnd(M * K + 8, seed=1)), dev(rnd(N * K + 8, seed=2))
+    x, w = x[off_x: off_x + M * K].view(M, K), w[off_w: off_w + N * K].view(N, K)
+    assert torch.equal(hip.gemm32(x, w), hip.gemm32(x.clone(), w.clone()))
+
+
+def test_gemm32_deep():
+    """K beyond what 31-bit offsets over a tile's rows reach."""
+    from llm_map_reduce_summarizer_amd.ops import hip
+    K = hip.GEMM32_MAX_K + 96
+    x, w = rnd(2, K, seed=1), rnd(3, K, seed=2)
+    got, want = hip.gemm32(dev(x), dev(w)).double().cpu(), x.double() @ w.double().T
+    # K roundings, each at most 2^-24 of a sum of the size sqrt(K), add up to sqrt(K) of one: four times that
+    assert bool(((got - want).abs() <= 4 * K ** 0.5 * 2.0 ** -24 * K ** 0.5).all())
+
+
 def test_gemm32_shapes():
     from llm_map_reduce_summarizer_amd.ops import hip
     for Mr, N, K in ((1, 16, 32), (70, 130, 96), (64, 64, 128), (129, 77, 256)):
