@@ -294,14 +294,13 @@ def test_delta_rule(H, G, dim, vdim, dtype, monkeypatch):
             b = e
 
 
-@pytest.mark.parametrize("copies,dim,dtype", [(1, 24, F32), (3, 24, F32), (6, 7, F32), (1, 40, F32)])
-def test_delta_portions_token_by_token(copies, dim, dtype):
-    """Portions around the 16 rows that the stepped kernel stages at a time; one, two and four state rows per lane group."""
+def delta_portions(H, G, dim, vdim, dtype, lens, off=0):
+    """Both sides of one delta_mix over segments of ``lens`` rows; ``off``: first element of ``a`` and the norm weights in
+    their storage.  Returns (rows, states) errors."""
     from llm_map_reduce_summarizer_amd import ops
     from llm_map_reduce_summarizer_amd.engine import mixers
     from llm_map_reduce_summarizer_amd.engine.config import DeltaSpec
-    H, G, vdim = 64, 32, 20
-    m = mixers.DeltaMixer(DeltaSpec(H, G, dim, vdim, 2), torch.device(DEV), dtype)
+    m = mixers.DeltaMixer(DeltaSpec(H, G, dim, vdim, 2), torch.device("cpu"), dtype)
     cols = [0]
 
     def take(n):
@@ -310,7 +309,6 @@ def test_delta_portions_token_by_token(copies, dim, dtype):
         return at
     m.columns(take)
     m.col = 8
-    lens = sorted([1, 15, 16, 17, 33] * copies, key=lambda n: n != 1)
     T = sum(lens)
     x, u = rnd(T, m.channels, std=0.8), rnd(1, T, cols[0], seed=1)
     vec = [-torch.exp(rnd(H, seed=2)), rnd(H, seed=3) - 3, rnd(vdim, seed=4, std=0.2) + 1]
@@ -318,13 +316,28 @@ def test_delta_portions_token_by_token(copies, dim, dtype):
     state = rnd(len(lens) + 1, H, vdim, dim + (-dim) % 4, seed=5, std=0.5)
     state[..., dim:] = 0
     got_s, want_s = dev(state), state.clone()
-    got, want = torch.zeros(T, m.col + m.width, device=DEV), torch.zeros(T, m.col + m.width)
+    width = m.col + m.width
+    got, want = torch.zeros(T * width + off, device=DEV)[off:].view(T, width), torch.zeros(T, width)
+    norm = torch.zeros(vdim + off, device=DEV)[off:]
+    norm.copy_(vec[2])
     segs = segments(lens, slots, pos0)
     host = ops.Segments(segs.slots.cpu(), segs.pos0.cpu(), segs.cu.cpu(), segs.row_seg.cpu(), lens)
-    ops.delta_mix(dev(x), dev(u), m, *map(dev, vec), 1e-3, got_s, segs, got)
+    ops.delta_mix(dev(x), dev(u), m, dev(vec[0]), dev(vec[1]), norm, 1e-3, got_s, segs, got)
     ops.delta_mix(x, u, m, *vec, 1e-3, want_s, host, want)
+    return rel(got, want), rel(got_s, want_s)
+
+
+@pytest.mark.parametrize("copies,dim,rows", [(1, 24, 1), (2, 24, 2), (3, 24, 4), (6, 7, 4), (1, 40, 1), (2, 128, 2),
+                                             (6, 128, 4), (2, 200, 2)])
+def test_delta_portions_token_by_token(copies, dim, rows):
+    """Portions around the 16 rows that the stepped kernel stages at a time; ``rows`` state rows per lane group: one up to
+    512 workgroups at one row each, two up to 1024, then four."""
+    H, vdim = 64, 20
+    lens = sorted([1, 15, 16, 17, 33] * copies, key=lambda n: n != 1)
+    one = -(-vdim // 16) * H * sum(n > 1 for n in lens)
+    assert rows == (1 if one <= 512 else 2 if one <= 1024 else 4)
     # both sides are fp32; corrections chain through at most 33 rows
-    assert rel(got, want) < 1e-5 and rel(got_s, want_s) < 1e-5
+    assert max(delta_portions(H, 32, dim, vdim, F32, lens)) < 1e-5
 
 
 # ------------------------------------------------------------------ whole models
