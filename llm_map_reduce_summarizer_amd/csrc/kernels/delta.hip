@@ -345,14 +345,16 @@ static int launch_delta_portion(const void* x, const DeltaArgs& a, const SegArgs
     return (int)hipGetLastError();
 }
 
-// Segments [seg0, seg0 + nseg) of several rows each; y [T - y0][heads * P] fp32, N <= 256.  The rest as mrsum_delta_step.
+// Segments [seg0, seg0 + nseg) of several rows each; y [T - y0][heads * P] fp32.  The rest as mrsum_delta_step, which the
+// head sizes that it takes come from: a request's prompt is not taken where its decoded tokens would be refused.
 MRSUM_API int mrsum_delta_portion(const void* x, int ldx, int x32, int xk, int xv, const void* u, int S, int ld, int T,
                                   int b_at, int a_at, const float* dt_bias, const float* a_neg, float* state,
                                   const int* cu, const int* slots, const int* pos0, int seg0, int nseg, float* y, int y0,
                                   int heads, int kv_heads, int P, int N, hipStream_t s) {
     if (T <= 0 || nseg <= 0) return 0;
     if (!cu || heads <= 0 || heads > 65535 || kv_heads <= 0 || heads % kv_heads || nseg > 65535 || b_at + heads > ld ||
-        a_at + heads > ld || ldx < xv + heads * P || xk < kv_heads * N || xv < xk + kv_heads * N || (x32 && S < 1))
+        a_at + heads > ld || ldx < xv + heads * P || xk < kv_heads * N || xv < xk + kv_heads * N || (x32 && S < 1) ||
+        P > (N <= 32 ? 512 : N <= 128 ? 256 : 128))
         return (int)hipErrorInvalidValue;
     const DeltaArgs a{ProjSrc{u, S, (size_t)T * ld, ld}, b_at, a_at, 0, dt_bias, a_neg, nullptr, 0.f,
                       1.f / sqrtf((float)N), ldx, xk, xv, 0, 0, 0, heads, kv_heads, P, N, (N + 3) / 4 * 4};

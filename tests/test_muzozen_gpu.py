@@ -340,6 +340,18 @@ def test_delta_portions_token_by_token(copies, dim, rows):
     assert max(delta_portions(H, 32, dim, vdim, F32, lens)) < 1e-5
 
 
+@pytest.mark.parametrize("dim,vdim,ok", [(32, 512, True), (32, 513, False), (128, 256, True), (64, 257, False), (200, 128, True),
+                                         (256, 129, False)])
+@pytest.mark.parametrize("lens", [[1, 1], [2, 17]])
+def test_delta_head_limits(dim, vdim, ok, lens):
+    """Decoded tokens and prompt portions take the same head sizes."""
+    if ok:
+        assert max(delta_portions(2, 1, dim, vdim, F32, lens)) < 1e-5
+    else:
+        with pytest.raises(RuntimeError):
+            delta_portions(2, 1, dim, vdim, F32, lens)
+
+
 # ------------------------------------------------------------------ whole models
 @pytest.mark.parametrize("name", sorted(M.CONFIGS))
 @pytest.mark.parametrize("dtype", DTYPES)
