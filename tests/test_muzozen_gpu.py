@@ -340,6 +340,12 @@ def test_delta_portions_token_by_token(copies, dim, rows):
     assert max(delta_portions(H, 32, dim, vdim, F32, lens)) < 1e-5
 
 
+def test_delta_portions_unaligned():
+    """Output rows and norm weights that are not 16-byte aligned: the separate norm does not take them, so portions run with
+    the norm in the same launch."""
+    assert max(delta_portions(4, 2, 24, 20, F32, [1, 15, 33], off=1)) < 1e-5
+
+
 @pytest.mark.parametrize("dim,vdim,ok", [(32, 512, True), (32, 513, False), (128, 256, True), (64, 257, False), (200, 128, True),
                                          (256, 129, False)])
 @pytest.mark.parametrize("lens", [[1, 1], [2, 17]])
