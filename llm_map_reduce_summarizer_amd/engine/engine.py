@@ -447,7 +447,7 @@ class LLMEngine:
         if paged and not recurrent:
             x.paged = ops.PagedPrefill(tables, d[part[0]], d[part[1]], list(slots), pre)
         if recurrent:
-            x.n_decode, x.portion_lens = nd, lens[nd:]
+            x.n_decode, x.portion_lens, x.portions = nd, lens[nd:], tuple(zip(lens[nd:], pre[nd:]))
             x.segs = ops.Segments(d[segs[0]], d[segs[1]], x.cu_seqlens, d[segs[2]], lens)
             x.paged = ops.PagedPrefill(tables, d[part[0]], d[part[1]], list(slots[nd:]), pre[nd:])
             x.decode_tables = tables.index_select(0, d[part[2]])

@@ -259,6 +259,6 @@ class HybridModel:
         """One token for each of the first ``B`` rows of the decode state ``st``."""
         segs = ops.Segments(st.state_slots[:B], st.positions[:B])
         b = SimpleNamespace(ids=st.next_ids[:B], positions=st.positions[:B], seq_idx=st.seq_idx[:B],
-                            tables=st.block_tables[:B], decode_tables=st.block_tables[:B], n_decode=B,
+                            tables=st.block_tables[:B], decode_tables=st.block_tables[:B], n_decode=B, portions=(),
                             workspace=workspace or {}, segs=segs)
         return self.logits(self._forward(b, kv))

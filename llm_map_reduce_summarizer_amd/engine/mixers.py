@@ -131,7 +131,7 @@ class AttnMixer(Mixer):
                                b.tables, kc, vc, page, self.dtype)
         if not self.mfma:
             ops.attn_rows(q, kc, vc, b.positions, b.seq_idx, b.tables, sp.heads, sp.kv_heads, self.vp, page, sp.scale,
-                          gate, a, b.n_decode)
+                          gate, a, b.n_decode, b.portions)
             return
         nd = b.n_decode
         if nd:
@@ -285,7 +285,7 @@ class LatentMixer(Mixer):
             n = b.n_decode if self.mfma else 0
             if n < nd:
                 o = ops.latent_rows(qa[n:], cache, b.positions[n:nd], b.seq_idx[n:nd], b.tables, s.heads, self.rank8,
-                                    page, s.scale, b.n_decode - n)
+                                    page, s.scale, b.n_decode - n, b.portions)
                 ops.latent_out(o, self, w.w_uv, a[n:nd], self.col)
         if nd < T:
             ctx = b.context()

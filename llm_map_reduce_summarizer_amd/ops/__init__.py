@@ -298,10 +298,12 @@ def qkv_prep(u, al, bias, q_norm, k_norm, eps, out_scale, positions, seq_idx, bl
                              vcache, page, dtype)
 
 
-def attn_rows(q, kcache, vcache, positions, seq_idx, block_tables, hq, hkv, pitch, page, scale, gate, out, singles=None):
-    """``singles``: leading rows that are alone in their sequences (None: all may be); the others come as portions."""
+def attn_rows(q, kcache, vcache, positions, seq_idx, block_tables, hq, hkv, pitch, page, scale, gate, out, singles=None,
+              portions=None):
+    """``singles``: leading rows that are alone in their sequences (None: all may be); the others come as ``portions``,
+    (rows, first position) each (None: not known)."""
     return _impl(q).attn_rows(q, kcache, vcache, positions, seq_idx, block_tables, hq, hkv, pitch, page, scale, gate,
-                              out, singles)
+                              out, singles, portions)
 
 
 def conv_silu(u, at, kernel, bias, state, segs, dtype, gelu=None):
@@ -383,8 +385,8 @@ def latent_absorb(q, n, m, w_uk, cs, positions, dtype):
     return _impl(q).latent_absorb(q, n, m, w_uk, cs, positions, dtype)
 
 
-def latent_rows(q, cache, positions, seq_idx, block_tables, heads, rank, page, scale, singles=None):
-    return _impl(q).latent_rows(q, cache, positions, seq_idx, block_tables, heads, rank, page, scale, singles)
+def latent_rows(q, cache, positions, seq_idx, block_tables, heads, rank, page, scale, singles=None, portions=None):
+    return _impl(q).latent_rows(q, cache, positions, seq_idx, block_tables, heads, rank, page, scale, singles, portions)
 
 
 def latent_out(o, m, w_uv, a, col):

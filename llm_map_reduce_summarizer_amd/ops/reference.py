@@ -476,7 +476,7 @@ def qkv_prep(u, al, bias, q_norm, k_norm, eps: float, out_scale: float, position
 
 
 def attn_rows(q, kcache, vcache, positions, seq_idx, block_tables, hq: int, hkv: int, pitch: int, page: int,
-              scale: float, gate, out, singles=None) -> None:
+              scale: float, gate, out, singles=None, portions=None) -> None:
     """Every row attends to its sequence's cached keys [0, position]; head h of row t -> out[t, h * pitch :
     (h + 1) * pitch], times gate[t, h]."""
     dk, dv, g = kcache.shape[3], vcache.shape[3], hq // hkv
@@ -625,7 +625,7 @@ def latent_absorb(q, n: int, m, w_uk, cs, positions, dtype) -> torch.Tensor:
 
 
 def latent_rows(q, cache, positions, seq_idx, block_tables, heads: int, rank: int, page: int, scale: float,
-                singles=None):
+                singles=None, portions=None):
     """Attention of absorbed query rows over the cached rows: weighted sums of latents [T, H * rank]."""
     T, row = q.shape[0], cache.shape[3]
     out = torch.empty(T, heads, rank, dtype=q.dtype, device=q.device)

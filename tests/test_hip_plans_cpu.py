@@ -2,6 +2,7 @@
 covers every query row of every sequence exactly once at each GQA ratio, heaviest blocks first, and the
 decode-attention split plan keeps its measured choices (ops/hip.py)."""
 import pytest
+import torch
 
 from llm_map_reduce_summarizer_amd.ops import hip
 
@@ -116,3 +117,23 @@ def test_narrow_gate_up_split_rules():
     assert hip.plan("gate_up", 10, 7168, 4096) == ("stream_split", 7, 4)
     assert hip.plan("gate_up", 1, 3584, 4096)[0] == "skinny"
     assert hip.plan("gate_up", 1, 14336, 4096) == ("stream", 4, 1)
+
+
+@pytest.mark.parametrize("portions,hkv,tiles", [
+    # 32 heads of 128: row kernel and tiles, us (profiles/row_attention_portions.jsonl)
+    ([(2, 1998)] * 32, 32, False),  # 775, 9457: 32 contexts in one workgroup's chain
+    ([(2, 1998)] * 32, 8, False),   # 639, 2374
+    ([(8, 1992)] * 32, 8, True),    # 1509, 612
+    ([(16, 584)] * 8, 32, False),   # 237, 371
+    ([(32, 568)] * 8, 32, True),    # 427, 192
+    ([(900, 0)], 8, True),          # 1088, 183
+    ([(900, 0), (2, 30)], 8, True)])
+def test_row_attention_of_short_portions(portions, hkv, tiles, monkeypatch):
+    """Prompt portions go to the tiled kernel where it leads: not where a workgroup would walk many contexts."""
+    ran = []
+    monkeypatch.setattr(hip, "_fn", lambda name: lambda *a: ran.append((name, a[7])) or 0)
+    monkeypatch.setattr(hip, "_stream", lambda: 0)
+    rows, one = 3 + sum(n for n, _ in portions), torch.zeros(1, dtype=torch.int32)
+    t = torch.zeros(rows, 32 * 128)
+    hip._rows_attention(t, t, t.clone(), one, one, one[None], 32, hkv, 128, 128, 128, 128, 1.0, None, t, 3, portions, "")
+    assert ran == ([("mrsum_attn_rows", 3), ("mrsum_attn_portions", rows - 3)] if tiles else [("mrsum_attn_rows", rows)])
