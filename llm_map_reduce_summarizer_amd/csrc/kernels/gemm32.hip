@@ -172,14 +172,66 @@ __global__ __launch_bounds__(256) void gemm32_tail_kernel(const Gemm32Args a) {
     for (int i = 0; i < NC; ++i) store_c(a, m + (lane & 15), n + 16 * i + 4 * (lane >> 4), v[i]);
 }
 
+// Short K: 64 x 64 tiles, loads and products in turns, wave w rows [16 w, 16 w + 16).  A K-tile takes half the time that a
+// lone workgroup of the larger tiles takes, and four times as many workgroups share a small product (256 x 4096 x 256: 22 us
+// in 128 x 128 tiles, 12 here); from K 512 on the larger tiles' rate leads.  Which one: ops/hip.py gemm32_small.
+constexpr int TS = 64, LDS32 = 32 + 4;  // tile, padded row of a K-tile
+
+__global__ __launch_bounds__(256) void gemm32_small_kernel(const float* __restrict__ x, int ldx, const float* __restrict__ w,
+                                                           int ldw, float* __restrict__ c, int ldc, int M, int N, int K) {
+    __shared__ __attribute__((aligned(16))) float sx[TS * LDS32];
+    __shared__ __attribute__((aligned(16))) float sw[TS * LDS32];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int m0 = blockIdx.y * TS, n0 = blockIdx.x * TS;
+    const int lr = tid >> 3, lc = (tid & 7) * 4;  // staging: rows lr and lr + 32, 4 columns
+    f32x4 acc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int r16 = lane & 15, kq = lane >> 4;
+    for (int k0 = 0; k0 < K; k0 += 32) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int r = lr + 32 * i;
+            float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
+            if (m0 + r < M) a = *reinterpret_cast<const float4*>(x + (size_t)(m0 + r) * ldx + k0 + lc);
+            if (n0 + r < N) b = *reinterpret_cast<const float4*>(w + (size_t)(n0 + r) * ldw + k0 + lc);
+            *reinterpret_cast<float4*>(sx + r * LDS32 + lc) = a;
+            *reinterpret_cast<float4*>(sw + r * LDS32 + lc) = b;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < 32; k += 4) {
+            const float a = sx[(16 * wv + r16) * LDS32 + k + kq];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, sw[(16 * i + r16) * LDS32 + k + kq], acc[i], 0, 0, 0);
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int n = n0 + 16 * i + r16;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int m = m0 + 16 * wv + 4 * kq + j;
+            if (m < M && n < N) c[(size_t)m * ldc + n] = acc[i][j];
+        }
+    }
+}
+
 // x [M][ldx], w [N][ldw], c [M][ldc]; tiles from raster position ``whole`` on in ``splits`` slices of K through ``part``
-// [tiles - whole][splits][16384] (splits 1: none, part unused)
+// [tiles - whole][splits][16384] (splits 1: none, part unused); splits 0: 64 x 64 tiles
 MRSUM_API int mrsum_gemm32(const float* x, int ldx, const float* w, int ldw, float* c, int ldc, int M, int N, int K,
                            int whole, int splits, float* part, hipStream_t s) {
     if (M <= 0 || N <= 0) return 0;
     if (K % 32 || ldx % 4 || ldw % 4 || (uintptr_t)x % 16 || (uintptr_t)w % 16 || (size_t)T32 * ldx * 4 >= (1u << 31) ||
         (size_t)T32 * ldw * 4 >= (1u << 31))
         return (int)hipErrorInvalidValue;
+    if (splits == 0) {
+        if (ceil_div(M, TS) > 65535) return (int)hipErrorInvalidValue;
+        gemm32_small_kernel<<<dim3(ceil_div(N, TS), ceil_div(M, TS)), 256, 0, s>>>(x, ldx, w, ldw, c, ldc, M, N, K);
+        return (int)hipGetLastError();
+    }
     Gemm32Args a{x, w, c, ldx, ldw, ldc, M, N, K / 32, ceil_div(M, T32), ceil_div(N, T32), 0, 1, part};
     const int tiles = a.tiles_m * a.tiles_n;
     if (splits > 1 && (whole < 0 || whole >= tiles || splits > a.kb || !part)) return (int)hipErrorInvalidValue;

@@ -137,3 +137,18 @@ def test_row_attention_of_short_portions(portions, hkv, tiles, monkeypatch):
     t = torch.zeros(rows, 32 * 128)
     hip._rows_attention(t, t, t.clone(), one, one, one[None], 32, hkv, 128, 128, 128, 128, 1.0, None, t, 3, portions, "")
     assert ran == ([("mrsum_attn_rows", 3), ("mrsum_attn_portions", rows - 3)] if tiles else [("mrsum_attn_rows", rows)])
+
+
+@pytest.mark.parametrize("M,N,K,small", [
+    # us in 128 x 128 and 64 x 64 tiles (profiles/gemm32_short_k.jsonl)
+    (256, 4096, 256, True),    # 22, 12
+    (300, 2048, 192, True),    # 17, 10
+    (520, 8192, 192, True),    # 31, 23
+    (64, 4096, 256, True),     # 13, 11
+    (900, 16384, 128, True),   # 45, 43
+    (1500, 8192, 256, False),  # 56, 64
+    (300, 4096, 768, False),   # 33, 38
+    (8, 16384, 256, False),    # 8, 13
+    (903, 4096, 4096, False)])
+def test_fp32_gemm_of_short_k(M, N, K, small):
+    assert hip.gemm32_small(M, N, K // 32) == small

@@ -478,11 +478,24 @@ def test_row_attention_portions(H, G, dk, dv, dtype, monkeypatch):
 
 @pytest.mark.parametrize("M,N,K,split", [(1, 130, 1024, True), (17, 1023, 2048, True), (129, 2062, 512, True),
                                          (500, 8200, 256, True), (1100, 4096, 128, False), (3, 40000, 64, False)])
-def test_gemm32_edges(M, N, K, split):
+def test_gemm32_edges(M, N, K, split, monkeypatch):
     """Rows and columns past the last 128 x 128 tile, 16-row blocks past M, rows of C that are not 16-byte aligned, whole
     tiles and tiles in slices of K behind them."""
     from llm_map_reduce_summarizer_amd.ops import hip
+    monkeypatch.setattr(hip, "gemm32_small", lambda *_: False)
     assert (hip.gemm32_splits(M, N, K // 32)[1] > 1) == split
+    x, w = rnd(M, K, seed=1), rnd(N, K, seed=2)
+    got = hip.gemm32(dev(x), dev(w)).double().cpu()
+    # each of the K products and sums rounds by at most 2^-24 of the sum of magnitudes
+    bound = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert got.shape == (M, N) and bool(((got - x.double() @ w.double().T).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 16, 32), (64, 130, 192), (33, 65, 288), (257, 1, 128), (520, 8192, 192), (300, 1023, 512)])
+def test_gemm32_short_k(M, N, K):
+    """The 64 x 64 tiles: rows and columns past the last tile, against 64 bits; the larger tiles give the same up to rounding."""
+    from llm_map_reduce_summarizer_amd.ops import hip
+    assert hip.gemm32_small(M, N, K // 32)
     x, w = rnd(M, K, seed=1), rnd(N, K, seed=2)
     got = hip.gemm32(dev(x), dev(w)).double().cpu()
     # each of the K products and sums rounds by at most 2^-24 of the sum of magnitudes
