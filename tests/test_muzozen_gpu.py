@@ -340,6 +340,18 @@ def test_delta_portions_token_by_token(copies, dim, rows):
     assert max(delta_portions(H, 32, dim, vdim, F32, lens)) < 1e-5
 
 
+@pytest.mark.parametrize("H,dim,lens,staged", [(32, 128, [1, 2] + [3] * 4, False), (32, 128, [1] + [2] * 64, False),
+                                               (32, 128, [1] + [3] * 64, True), (4, 24, [6, 1, 6], False), (4, 24, [1, 7], True),
+                                               (4, 200, [2, 2], False), (4, 200, [2, 3], True)])
+def test_delta_short_portions(H, dim, lens, staged, monkeypatch):
+    """Portions of a few rows run in one launch, longer ones with their rows staged ahead; right either way."""
+    from llm_map_reduce_summarizer_amd.ops import hip
+    ran, fn = [], hip._fn
+    monkeypatch.setattr(hip, "_fn", lambda name: ran.append(name) or fn(name))
+    assert max(delta_portions(H, 2, dim, 20, F32, lens)) < 1e-5
+    assert ("mrsum_delta_portion" in ran) == staged and ("mrsum_gated_norm" in ran) == staged
+
+
 def test_delta_portions_unaligned():
     """Output rows and norm weights that are not 16-byte aligned: the separate norm does not take them, so portions run with
     the norm in the same launch."""
