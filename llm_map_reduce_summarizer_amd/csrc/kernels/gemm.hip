@@ -140,6 +140,18 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmArgs a) {
 #endif
     __shared__ __attribute__((aligned(1024))) char lds[NS * HALF];
     const int tid = threadIdx.x, lane = tid & 63;
+    auto stamp = [&] {  // at every end of the kernel
+#ifdef MRSUM_CLOCK_STAMPS
+        // in-kernel clock = shader ticks / 100 MHz ticks (MI355X_MICROARCH.md, DVFS give-back item 6); lane 0's
+        // vector store to a buffer no other code reads
+        __syncthreads();
+        if (tid == 0) {
+            const unsigned long long clk = __builtin_amdgcn_s_memtime() - clk0, rt = __builtin_amdgcn_s_memrealtime() - rt0;
+            a.stamps[2 * blockIdx.x] = clk;
+            a.stamps[2 * blockIdx.x + 1] = rt;
+        }
+#endif
+    };
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = w >> 2, wc = w & 3;
     int tm, tn;
@@ -341,6 +353,7 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmArgs a) {
                             *reinterpret_cast<f32x4*>(out + (size_t)rl * a.N + 128 * (v >> 1) + 16 * (v & 1)) =
                                 acc[qm][b][v >> 1][v & 1];
                 }
+            stamp();
             return;
         }
         if (slice >= 0) {
@@ -354,6 +367,7 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmArgs a) {
 #pragma unroll
                     for (int v = 0; v < 4; ++v) out[((qm * 4 + b) * 4 + v) * 512] = acc[qm][b][v >> 1][v & 1];
                 }
+            stamp();
             return;
         }
     }
@@ -475,16 +489,7 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmArgs a) {
             if (ok) *reinterpret_cast<u32x4*>(reinterpret_cast<bf16*>(a.c) + (size_t)m * a.ldc + col) = val;
         }
     }
-#ifdef MRSUM_CLOCK_STAMPS
-    // in-kernel clock = shader ticks / 100 MHz ticks (MI355X_MICROARCH.md, DVFS give-back item 6); lane 0's
-    // vector store to a buffer no other code reads
-    __syncthreads();
-    if (tid == 0) {
-        const unsigned long long clk = __builtin_amdgcn_s_memtime() - clk0, rt = __builtin_amdgcn_s_memrealtime() - rt0;
-        a.stamps[2 * blockIdx.x] = clk;
-        a.stamps[2 * blockIdx.x + 1] = rt;
-    }
-#endif
+    stamp();
 }
 
 // Adds the slices of the split tiles and runs the epilogue.  One workgroup per (tile, 2 x 16 rows): the four vectors

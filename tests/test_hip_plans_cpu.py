@@ -1,10 +1,17 @@
 """Host-side work lists and launch plans of the HIP ops (no GPU needed): the prefill-attention item list
 covers every query row of every sequence exactly once at each GQA ratio, heaviest blocks first, and the
 decode-attention split plan keeps its measured choices (ops/hip.py)."""
+import glob
+import importlib.util
+import os
+import re
+
 import pytest
 import torch
 
 from llm_map_reduce_summarizer_amd.ops import hip
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 @pytest.mark.parametrize("group", [1, 2, 4, 8, 3, 5, 16])
@@ -152,3 +159,30 @@ def test_row_attention_of_short_portions(portions, hkv, tiles, monkeypatch):
     (903, 4096, 4096, False)])
 def test_fp32_gemm_of_short_k(M, N, K, small):
     assert hip.gemm32_small(M, N, K // 32) == small
+
+
+def c_parameters():
+    """Entry point -> number of its parameters, from the kernels' sources."""
+    found = {}
+    for f in glob.glob(os.path.join(ROOT, "llm_map_reduce_summarizer_amd", "csrc", "kernels", "*.hip")):
+        with open(f) as fh:
+            for name, pars in re.findall(r"MRSUM_API int (\w+)\(([^)]*)\)\s*\{", fh.read()):
+                found[name] = len([p for p in pars.split(",") if p.strip()])
+    return found
+
+
+def test_signatures_match_the_kernels():
+    """ctypes checks nothing: a signature with another number of arguments reads the rest from the stack."""
+    pars = c_parameters()
+    assert {n: len(t) for n, t in hip._SIGS.items()} == {n: pars[n] for n in hip._SIGS}
+
+
+def test_gemm_clock_passes_what_the_gemm_takes():
+    spec = importlib.util.spec_from_file_location("gemm_clock", os.path.join(ROOT, "tools", "gemm_clock.py"))
+    tool = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(tool)
+    x, w, c = torch.zeros(3, 64), torch.zeros(16, 64), torch.zeros(3, 16)
+    args = [a.value for a in tool.gemm_args(x, w, c, 99)]
+    assert len(args) == c_parameters()["mrsum_gemm"] and args[6:9] == [3, 16, 64]
+    # GLU parameters, no tiles in slices, the stream
+    assert args[15:] == [float("inf"), 1.0, 0.0, 0, 1, None, 0, 99]

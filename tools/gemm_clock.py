@@ -17,16 +17,30 @@ import sys
 import time
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+sys.path.insert(0, ROOT)
 SRC = os.path.join(ROOT, "llm_map_reduce_summarizer_amd", "csrc", "kernels", "gemm.hip")
 LIB = os.path.join(ROOT, "llm_map_reduce_summarizer_amd", "_native", "diag", "libmrsum_gemm_clock.so")
 SHAPES = {"qkv": (6144, 4096), "o": (4096, 4096), "gate_up": (28672, 4096), "down": (4096, 14336)}
 
 
 def build():
+    from llm_map_reduce_summarizer_amd import _stamp
     os.makedirs(os.path.dirname(LIB), exist_ok=True)
-    subprocess.check_call(["/opt/rocm/bin/hipcc", "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
-                           "-DMRSUM_CLOCK_STAMPS", SRC, "-o", LIB])
+    flags = [f for f in _stamp.HIP_FLAGS if not f.startswith("-Rpass")]
+    subprocess.check_call(["/opt/rocm/bin/hipcc"] + flags + ["-shared", "-DMRSUM_CLOCK_STAMPS", SRC, "-o", LIB])
     print("built", LIB)
+
+
+def gemm_args(x, w, c, stream):
+    """Arguments of mrsum_gemm for c = x w^T in bf16, every tile whole; refused if the entry point takes others."""
+    from llm_map_reduce_summarizer_amd.ops import hip
+    (M, K), N = x.shape, w.shape[0]
+    args = (x.data_ptr(), K, w.data_ptr(), K, c.data_ptr(), N, M, N, K, 0, hip.GEMM_EPI_BF16, None, None, 0, 0,
+            *hip.SWIGLU, 0, 1, None, 0, stream)
+    types = hip._SIGS["mrsum_gemm"]
+    if len(args) != len(types):
+        raise TypeError("mrsum_gemm takes %d arguments, not %d" % (len(types), len(args)))
+    return [t(v) for t, v in zip(types, args)]
 
 
 def main():
@@ -39,12 +53,12 @@ def main():
     if a.build:
         return build()
     import torch
+    from llm_map_reduce_summarizer_amd.ops import hip
     lib = ctypes.CDLL(LIB)
-    vp, ci = ctypes.c_void_p, ctypes.c_int
-    lib.mrsum_gemm.argtypes = [vp, ci, vp, ci, vp, ci, ci, ci, ci, ci, ci, vp, vp, ci, ci, vp]
-    lib.mrsum_gemm_stamps.argtypes = [vp, ci]
+    lib.mrsum_gemm.argtypes = hip._SIGS["mrsum_gemm"]
+    lib.mrsum_gemm_stamps.argtypes = [ctypes.c_void_p, ctypes.c_int]
     dev = torch.device("cuda:0")
-    stream = vp(torch.cuda.current_stream().cuda_stream)
+    stream = torch.cuda.current_stream().cuda_stream
     for role in a.roles.split(","):
         N, K = SHAPES[role]
         M = a.M
@@ -53,9 +67,10 @@ def main():
         w = (torch.randn(N, K, generator=g) * 0.02).to(torch.bfloat16).to(dev)
         c = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
 
+        args = gemm_args(x, w, c, stream)
+
         def run():
-            rc = lib.mrsum_gemm(x.data_ptr(), K, w.data_ptr(), K, c.data_ptr(), N, M, N, K, 0, 0, None, None, 0, 0,
-                                stream)
+            rc = lib.mrsum_gemm(*args)
             assert rc == 0, rc
 
         flop = 2.0 * M * N * K
