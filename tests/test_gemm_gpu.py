@@ -169,6 +169,51 @@ def test_gemm_split_tail(M, N, K, epi):
     assert bool(((out.double() - y).abs() <= 2.0 ** -8 * y.abs() + 1e-4).all())
 
 
+@pytest.mark.parametrize("M,N,K,two", [(1, 48, 4096, False), (300, 1040, 4224, False), (257, 528, 2176, True), (4097, 4096, 4096, False),
+                                       (2100, 4096, 12288, True)])
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_gemm_fp8_split_tail(M, N, K, two, swiglu):
+    """The 8-bit product in slices of K, row and column scales behind the added slices; a slice border inside the low term of
+    two-term rows and between the terms."""
+    assert hip.gemm_splits(M, N, (2 if two else 1) * K // 128)[1] > 1
+    g = torch.Generator().manual_seed(18)
+    f8 = lambda *s: (torch.randn(*s, generator=g) * 8).to(torch.float8_e4m3fn)  # noqa: E731
+    xq, w = f8(M, (2 if two else 1) * K), Fp8Weight(f8(N, K).to(DEV), (torch.rand(N, generator=g) / 64 + 1 / 64).to(DEV))
+    xs = (torch.rand(M, generator=g) + 0.5) / K ** 0.5 / 8
+    n0 = N // 32 * 32 if swiglu else N
+    w = Fp8Weight(w.q[:n0].contiguous(), w.scale[:n0].contiguous())
+    out = hip.gemm_fp8(xq.to(DEV), xs.to(DEV), w, swiglu=swiglu, group_m=hip.GEMM_GROUP_M)
+    assert torch.equal(out, hip.gemm_fp8(xq.to(DEV), xs.to(DEV), w, swiglu=swiglu, group_m=hip.GEMM_GROUP_M))
+    x = xq.to(DEV).double()
+    x = (x[:, :K] + x[:, K:] / 16 if two else x) * xs.to(DEV).double()[:, None]
+    wd = w.q.double() * w.scale.double()[:, None]
+    y = x @ wd.t()
+    # sums of K exact products in fp32 (a few roundings of 2^-24 of the largest partial sum each), one bf16 rounding
+    slack = K * 2.0 ** -24 * (x.abs() @ wd.abs().t())
+    if swiglu:
+        h, e = y.reshape(M, -1, 2, 8), slack.reshape(M, -1, 2, 8)
+        gate, up = h[:, :, 0], h[:, :, 1]
+        y = (torch.nn.functional.silu(gate) * up).reshape(M, -1)
+        slack = (1.1 * e[:, :, 0] * up.abs() + gate.abs() * e[:, :, 1]).reshape(M, -1)  # |silu'| <= 1.1, |silu| <= |gate|
+    assert bool(((out.double() - y).abs() <= 2.0 ** -8 * y.abs() + slack).all())
+
+
+@pytest.mark.parametrize("epi", ["bf16", "swiglu", "gelu", "f32"])
+def test_gemm_split_tail_strided(epi):
+    """Slices of K into columns of wider rows, as whole tiles write them."""
+    M, N, K = 300, 544, 2048
+    assert hip.gemm_splits(M, N, K // 64)[1] > 1
+    big, w = _rand(M, K + 64, seed=20, scale=0.5), _rand(N, K, seed=21, scale=0.03)
+    x, n = big[:, 32:32 + K], N // 2 if epi == "swiglu" else N
+    kw = {} if epi == "bf16" else {epi: True}
+    want = hip.gemm(x.contiguous(), w, **kw)
+    for off in (0, 4):
+        rows = torch.full((M, n + 16), 7.0, dtype=want.dtype, device=DEV)
+        hip.gemm(x, w, out=rows[:, off:off + n], **kw)
+        assert torch.equal(rows[:, off:off + n], want)
+        assert bool((rows[:, :off] == 7).all() and (rows[:, off + n:] == 7).all())
+
+
 @pytest.mark.parametrize("K", [64, 2048])
 def test_gemm_swiglu_small_gates(K):
     """sigmoid(gate) below the smallest normal number (gates under -87.3) times a large up value, one launch (K 64) and

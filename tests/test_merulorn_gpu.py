@@ -167,13 +167,16 @@ def test_state_space_scan(heads, P, N, groups, dtype):
             b += n
 
 
-@pytest.mark.parametrize("copies,dtype,N", [(1, F32, 24), (2, F32, 24), (4, F32, 7), (1, BF, 260 - 12)])
-def test_state_space_portions_token_by_token(copies, dtype, N):
-    """Portions around the 16 rows that the stepped kernel stages at a time, few and many (segment, head) pairs (one, two
-    and four state rows per lane group), and the 16-bit head size that the chunked form does not take."""
+@pytest.mark.parametrize("copies,dtype,N,rows", [(1, F32, 24, 1), (2, F32, 24, 2), (4, F32, 7, 4), (2, F32, 128, 2), (4, F32, 128, 4),
+                                                 (2, F32, 200, 2), (1, BF, 260 - 12, 4)])
+def test_state_space_portions_token_by_token(copies, dtype, N, rows):
+    """Portions around the 16 rows that the stepped kernel stages at a time, and the 16-bit head size that the chunked form
+    does not take; ``rows`` state rows per lane group: one up to 512 workgroups at one row each, two up to 1024, then four."""
     from llm_map_reduce_summarizer_amd import ops
     from llm_map_reduce_summarizer_amd.ops import hip
     heads, P, groups = 64, 20 if dtype == F32 else 136, 2
+    one = -(-P // 16) * heads * 4 * copies
+    assert rows == (1 if one <= 512 else 2 if one <= 1024 else 4)
     lens = [1, 15, 16, 17, 33] * copies
     assert not (dtype == BF and hip.ssm_chunk_ok(P, N))
     T, Cp = sum(lens), heads * P + 2 * groups * N + (-(2 * groups * N)) % 8
