@@ -9,7 +9,7 @@
 // K-tile is 16 LDS reads for 128 instructions of 32 cycles, and the matrix cores set the time (1.7 us a K-tile) once a CU
 // has work.  16-row blocks past M are skipped.  903 x 28672 x 4096: 2310 (64 x 64 tiles, loads between barriers) -> 1650
 // us, 129 TFLOP/s of 157 and 146 counting the rows that pad the last tile.  Tiles that would leave CUs idle run in slices
-// of K (ops/hip.py gemm32_splits), whose fp32 sums a second launch adds in slice order.
+// of K (ops/hip.py gemm32_splits), whose fp32 sums a second launch adds in slice order.  Short K runs in 64 x 64 tiles.
 #include "common.h"
 
 #include <type_traits>
