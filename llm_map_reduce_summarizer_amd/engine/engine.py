@@ -50,9 +50,9 @@ def _always() -> bool:
 
 def _token_ids(toks: Sequence[int], vocab: int) -> np.ndarray:
     """The ids as int32, checked to be non-empty and in range."""
+    if not isinstance(toks, (list, tuple)):  # read once; array() would take bytes for memory
+        toks = list(toks)
     try:
-        if isinstance(toks, (bytes, bytearray)):  # array() would take them for memory
-            raise TypeError
         a = np.frombuffer(array("q", toks), dtype=np.int64) if len(toks) else None  # 20 ns an id
     except (TypeError, OverflowError):  # ids that are not plain integers
         a = [int(t) for t in toks]

@@ -425,7 +425,20 @@ def test_window_rule():
     assert e._window([40, 7], True) == 16  # a feeder / stream hook / interleaved prefill wants sync points
 
 
-@pytest.mark.parametrize("toks,want", [([5, 0, 99], [5, 0, 99]), ((7,), [7]), (range(3), [0, 1, 2]), ([2.0, True], [2, 1]),
+class _Once:
+    """Token ids that can be read once, as a stream's next tokens."""
+
+    def __init__(self, ids):
+        self.n, self.it = len(ids), iter(ids)
+
+    def __len__(self):
+        return self.n
+
+    def __iter__(self):
+        return self.it
+
+
+@pytest.mark.parametrize("toks,want", [(_Once([2.0, 3.0, 4.0]), [2, 3, 4]), (_Once([7, 8]), [7, 8]), ([5, 0, 99], [5, 0, 99]), ((7,), [7]), (range(3), [0, 1, 2]), ([2.0, True], [2, 1]),
                                        (np.array([4, 9], dtype=np.uint8), [4, 9]), (torch.tensor([3, 98]), [3, 98]),
                                        (b"\x01\x02", [1, 2]), (["6"], [6]), ([], None), ([100], None), ([-1], None),
                                        ([1 << 70], None), ([1 << 40], None), ([-(1 << 70)], None)])
