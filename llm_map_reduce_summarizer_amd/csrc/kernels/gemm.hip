@@ -1,8 +1,8 @@
-// Large-M GEMM on the matrix cores (prefill projections, LM head over many rows):
+// Large-M fp8 GEMM on the matrix cores (prefill projections of 8-bit models), and the entry point of both tile GEMMs:
 //
 //     C[M, N] = X[M, K] . W[N, K]^T            X = activations, W = weights, both K-contiguous
 //
-//   * bf16 x bf16 on v_mfma_f32_16x16x32_bf16, or
+//   * bf16 x bf16 runs in gemm_bf16.hip;
 //   * OCP e4m3fn x e4m3fn on v_mfma_scale_f32_16x16x128_f8f6f4 with unit block scales (E8M0 127): the
 //     block-scaled form runs at twice the bf16 rate (MI355X_MICROARCH.md "Matrix cores"), so the plain
 //     per-row quantisation (activation row scale sx[m] x weight row scale sw[n]) is applied in the
@@ -15,7 +15,7 @@
 //
 // Structure (cdna_hip_programming.md §5 "The 256^2 8-phase template", re-derived for this layout):
 //   * one 256 x 256 output tile per 512-thread workgroup (8 waves, one workgroup per CU), K-tiles of 128
-//     bytes per row (64 bf16 | 128 e4m3); the XCD-aware bijective tile remap + grouped raster keeps
+//     bytes per row (128 e4m3); the XCD-aware bijective tile remap + grouped raster keeps
 //     the ~32 tiles an XCD runs at a time on 4 X row-panels x 8 W row-panels (L2 reuse).
 //   * LDS: 2 buffers x 4 half-tile images of 128 rows x 128 B (X rows 0-127, W rows 0-127, W rows
 //     128-255, X rows 128-255 -- the order the phases first read them) = 128 KiB in ONE __shared__
@@ -29,8 +29,8 @@
 //     X half qm and W half qn, so the four phases of a K-tile need the half-tiles in the order
 //     X0 W0 | W1 | X1 | -- and a half-tile can be staged LOOK = 6 half-tiles (1.5 K-tiles) ahead of
 //     the phase that first reads it.  Per phase: R = fragment ds_reads + stage one half-tile (2 DMA
-//     per lane) + counted s_waitcnt vmcnt(8) (never 0 in the main loop), raw s_barrier, M = 16 bf16 (8
-//     fp8) MFMAs between s_setprio(1/0), raw s_barrier.  Waves 4-7 run one barrier (half a phase)
+//     per lane) + counted s_waitcnt vmcnt(8) (never 0 in the main loop), raw s_barrier, M = 8
+//     MFMAs between s_setprio(1/0), raw s_barrier.  Waves 4-7 run one barrier (half a phase)
 //     behind waves 0-3 (stagger), so one wave of each SIMD reads LDS while its partner computes.
 //   * hazards (derived for the staggered schedule, which is the stricter one): the wait at the end of
 //     R_P covers every half-tile phase P+1 reads, before the barrier the lagging group passes ahead
@@ -40,15 +40,11 @@
 //   * the MFMA computes the transposed tile (A = W fragment, B = X fragment) so each lane ends with 4
 //     consecutive output columns of one row: 8-byte bf16 stores, and the fused SwiGLU epilogue of the
 //     [8 gate | 8 up]-interleaved gate_up weight is a lane-xor-32 exchange.
-//   * split tail: tiles behind the last whole round of 256 (all of them where M and N are small) would leave most CUs
-//     idle for a full K loop, so each is cut into S slices of K.  A slice writes its fp32 accumulators to scratch in
-//     register order (lane-contiguous 16-B stores) and gemm_tail_kernel adds them in slice order and runs the
-//     epilogue: a second launch and no ticket, so results do not depend on arrival and concurrent streams share
-//     nothing.  Which S: ops/hip.py gemm_splits.
-//   * M32 variant: the same ring, phases and quadrants on 32x32 MFMA tiles (v_mfma_f32_32x32x16_bf16 /
-//     v_mfma_scale_f32_32x32x64_f8f6f4); a lane then holds 4 register groups of 4 consecutive columns,
+//   * split tail: as in gemm_bf16.hip, with this kernel's register order.
+//   * M32 variant: the same ring, phases and quadrants on 32x32 MFMA tiles
+//     (v_mfma_scale_f32_32x32x64_f8f6f4); a lane then holds 4 register groups of 4 consecutive columns,
 //     and the SwiGLU gate / up halves of a 16-column group sit in adjacent groups of the same lane.
-#include "common.h"
+#include "gemm.h"
 
 #include <type_traits>
 
@@ -57,35 +53,7 @@ constexpr int HALF = 16384;
 constexpr int TILE = 4 * HALF;
 constexpr int LOOK = 6;
 
-enum { GEPI_BF16 = 0, GEPI_SWIGLU = 1, GEPI_GELU = 2, GEPI_F32 = 3 };
-
 typedef int i32x8 __attribute__((ext_vector_type(8)));
-
-struct GemmArgs {
-    const char* x;
-    const char* w;
-    void* c;
-    const float* sx;  // fp8: per-row activation scale [M]
-    const float* sw;  // fp8: per-row weight scale [N]
-    int ldx_b, ldw_b, ldc;  // X / W row strides in bytes, C row stride in elements
-    int M, N, kb;           // kb = K-tiles (128 bytes of every row each)
-    int kbw;                // W's K-tiles: kb, or kb / 2 for two-term X (X tiles kt >= kbw re-read W tile kt - kbw)
-    int tiles_m, tiles_n, group_m;
-    int whole;    // raster positions below it run whole, the others in ``splits`` slices of K each
-    int splits;
-    float* part;  // [tiles - whole][splits][TILE_F] fp32 accumulators of the slices
-    int slabs;    // GEPI_F32, every tile split: part is [splits][M][N] rows instead, for a consumer that adds the slabs
-    GluArgs glu;  // GEPI_SWIGLU
-#ifdef MRSUM_CLOCK_STAMPS
-    unsigned long long* stamps;  // diagnostic build only (tools/gemm_clock.py): [grid][2] shader / 100 MHz ticks
-#endif
-};
-
-template <int N>
-__device__ __forceinline__ void vm_wait() {
-    static_assert(N >= 0 && N < 64, "vmcnt range");
-    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
 
 __device__ __forceinline__ void vm_wait_rt(int n) {
     if (n >= 12) vm_wait<12>();
@@ -102,56 +70,17 @@ __device__ __forceinline__ void bar() {
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 }
-
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
-
-__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, char* dst, int voff, int soff) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)dst, 16, voff, soff, 0, 0);
-}
-
-constexpr int TILE_F = 256 * 256;  // accumulators of one tile
-
-// bijective XCD remap: blocks b, b+8, ... (one XCD's) get consecutive positions
-__device__ __forceinline__ int xcd_position(int bid, int nwg) {
-    const int xcd = bid & 7, local = bid >> 3, q = nwg >> 3, r = nwg & 7;
-    return (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + local;
-}
-
-// grouped raster of group_m tile rows
-__device__ __forceinline__ void tile_of(int p, int tiles_m, int tiles_n, int group_m, int& tm, int& tn) {
-    const int gsz = group_m * tiles_n;
-    const int g = p / gsz, first = g * group_m;
-    const int gm = min(tiles_m - first, group_m);
-    const int within = p - g * gsz;
-    tm = first + within % gm;
-    tn = within / gm;
-}
 }  // namespace
 
-template <bool FP8, int EPI, int NS, bool LEPI, bool M32>
+template <int EPI, int NS, bool LEPI, bool M32>
 __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmArgs a) {
     // NS = half-tile slots of the LDS ring: half-tile h (K-tile h / 4, part h % 4) lives in slot h % NS.
     // NS = 8 (128 KiB, 2 K-tiles): staged LK = 6 ahead; NS = 10 (160 KiB): LK = 8 ahead.  A slot is
     // restaged at phase h + NS - LK >= 2 phases after the last phase that read half-tile h (<= h).
     constexpr int LK = NS - 2;
     static_assert(NS * HALF <= 160 * 1024 && NS * HALF >= 2 * TILE, "LDS ring size");
-#ifdef MRSUM_CLOCK_STAMPS
-    const unsigned long long clk0 = __builtin_amdgcn_s_memtime(), rt0 = __builtin_amdgcn_s_memrealtime();
-#endif
     __shared__ __attribute__((aligned(1024))) char lds[NS * HALF];
     const int tid = threadIdx.x, lane = tid & 63;
-    auto stamp = [&] {  // at every end of the kernel
-#ifdef MRSUM_CLOCK_STAMPS
-        // in-kernel clock = shader ticks / 100 MHz ticks (MI355X_MICROARCH.md, DVFS give-back item 6); lane 0's
-        // vector store to a buffer no other code reads
-        __syncthreads();
-        if (tid == 0) {
-            const unsigned long long clk = __builtin_amdgcn_s_memtime() - clk0, rt = __builtin_amdgcn_s_memrealtime() - rt0;
-            a.stamps[2 * blockIdx.x] = clk;
-            a.stamps[2 * blockIdx.x + 1] = rt;
-        }
-#endif
-    };
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = w >> 2, wc = w & 3;
     int tm, tn;
@@ -254,40 +183,21 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmArgs a) {
     auto mfma_q = [&](int qm, int qn, const u32x4 (&wf)[4], int xsc) {
         __builtin_amdgcn_s_setprio(1);
         if constexpr (M32) {
-            if constexpr (FP8) {
 #pragma unroll
-                for (int s = 0; s < 2; ++s)
+            for (int s = 0; s < 2; ++s)
 #pragma unroll
-                    for (int b = 0; b < 2; ++b)
-                        acc32[qm][b][qn] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
-                            cat8(wf[2 * s], wf[2 * s + 1]), cat8(xf[4 * b + 2 * s], xf[4 * b + 2 * s + 1]),
-                            acc32[qm][b][qn], 0, 0, 0, 127, 0, xsc);
-            } else {
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-#pragma unroll
-                    for (int b = 0; b < 2; ++b)
-                        acc32[qm][b][qn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                            __builtin_bit_cast(bf16x8, wf[r]), __builtin_bit_cast(bf16x8, xf[4 * b + r]),
-                            acc32[qm][b][qn], 0, 0, 0);
-            }
+                for (int b = 0; b < 2; ++b)
+                    acc32[qm][b][qn] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+                        cat8(wf[2 * s], wf[2 * s + 1]), cat8(xf[4 * b + 2 * s], xf[4 * b + 2 * s + 1]),
+                        acc32[qm][b][qn], 0, 0, 0, 127, 0, xsc);
         } else {
 #pragma unroll
             for (int i = 0; i < 2; ++i)
 #pragma unroll
-                for (int b = 0; b < 4; ++b) {
-                    if constexpr (FP8) {
-                        acc[qm][b][qn][i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-                            cat8(wf[2 * i], wf[2 * i + 1]), cat8(xf[2 * b], xf[2 * b + 1]), acc[qm][b][qn][i],
-                            0, 0, 0, 127, 0, xsc);
-                    } else {
-#pragma unroll
-                        for (int ks = 0; ks < 2; ++ks)
-                            acc[qm][b][qn][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                                __builtin_bit_cast(bf16x8, wf[2 * i + ks]), __builtin_bit_cast(bf16x8, xf[2 * b + ks]),
-                                acc[qm][b][qn][i], 0, 0, 0);
-                    }
-                }
+                for (int b = 0; b < 4; ++b)
+                    acc[qm][b][qn][i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                        cat8(wf[2 * i], wf[2 * i + 1]), cat8(xf[2 * b], xf[2 * b + 1]), acc[qm][b][qn][i], 0, 0, 0,
+                        127, 0, xsc);
         }
         __builtin_amdgcn_s_setprio(0);
     };
@@ -306,7 +216,7 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmArgs a) {
     };
     auto slot = [&](int kt, int part) -> const char* { return lds + ((4 * kt + part) % NS) * HALF; };
     auto ktile = [&](int kt, auto tail) {
-        const int xsc = FP8 && kt0 + kt >= a.kbw ? 123 : 127;  // E8M0 2^-4 on the lo half of two-term X
+        const int xsc = kt0 + kt >= a.kbw ? 123 : 127;  // E8M0 2^-4 on the lo half of two-term X
         // phase 0: quadrant (0, 0) -- X0, W0
         read_x(slot(kt, 0));
         read_w(slot(kt, 1), wf0);
@@ -339,23 +249,6 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmArgs a) {
     if (wr == 0) bar();
 
     if constexpr (!M32) {
-        if (EPI == GEPI_F32 && a.slabs) {
-            float* out = a.part + ((size_t)slice * a.M + m0) * a.N + n0 + 32 * wc + 4 * (lane >> 4);
-#pragma unroll
-            for (int qm = 0; qm < 2; ++qm)
-#pragma unroll
-                for (int b = 0; b < 4; ++b) {
-                    const int rl = 128 * qm + 64 * wr + 16 * b + (lane & 15);
-                    if (rl >= xrows) continue;
-#pragma unroll
-                    for (int v = 0; v < 4; ++v)
-                        if (32 * wc + 128 * (v >> 1) + 16 * (v & 1) < wrows)
-                            *reinterpret_cast<f32x4*>(out + (size_t)rl * a.N + 128 * (v >> 1) + 16 * (v & 1)) =
-                                acc[qm][b][v >> 1][v & 1];
-                }
-            stamp();
-            return;
-        }
         if (slice >= 0) {
             // accumulator vector v of this lane at [v][thread]; 16-row blocks past M are skipped
             f32x4* out = reinterpret_cast<f32x4*>(a.part + ((size_t)(pos - a.whole) * a.splits + slice) * TILE_F) + tid;
@@ -367,7 +260,6 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmArgs a) {
 #pragma unroll
                     for (int v = 0; v < 4; ++v) out[((qm * 4 + b) * 4 + v) * 512] = acc[qm][b][v >> 1][v & 1];
                 }
-            stamp();
             return;
         }
     }
@@ -379,10 +271,8 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmArgs a) {
     constexpr int RB = EPI == GEPI_SWIGLU ? 256 : 512;
     // fp8: v *= activation row scale x weight row scales of tile columns c4 .. c4+3
     auto scale4 = [&](f32x4& v, float rs, int c4) {
-        if constexpr (FP8) {
-            const float4 s4 = *reinterpret_cast<const float4*>(a.sw + min(n0 + c4, a.N - 4));
-            v[0] *= rs * s4.x; v[1] *= rs * s4.y; v[2] *= rs * s4.z; v[3] *= rs * s4.w;
-        }
+        const float4 s4 = *reinterpret_cast<const float4*>(a.sw + min(n0 + c4, a.N - 4));
+        v[0] *= rs * s4.x; v[1] *= rs * s4.y; v[2] *= rs * s4.z; v[3] *= rs * s4.w;
     };
     auto silu_mul = [&](const f32x4& g, const f32x4& u) {
         f32x4 r;
@@ -393,15 +283,6 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmArgs a) {
     // 4 bf16 outputs of tile row rl at byte cbyte of the output tile row; gcol = first weight column of
     // the 16-column group they come from (N % 16 == 0, so the group is wholly in or out of range)
     auto store4 = [&](int rl, int cbyte, f32x4 v, int gcol) {
-        if constexpr (EPI == GEPI_GELU) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) v[j] = gelu_tanh<bf16>(v[j]);
-        }
-        if constexpr (EPI == GEPI_F32) {
-            if (m0 + rl < a.M && n0 + gcol < a.N)
-                *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.c) + (size_t)(m0 + rl) * a.ldc + n0 + (cbyte >> 1)) = v;
-            return;
-        }
         const uint2 pk = make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
         if constexpr (LEPI) {
             *reinterpret_cast<uint2*>(lds + rl * RB + (((cbyte >> 4) ^ (rl & 7)) << 4) + (cbyte & 15)) = pk;
@@ -420,8 +301,7 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmArgs a) {
 #pragma unroll
             for (int b = 0; b < 2; ++b) {
                 const int rl = 128 * qm + 64 * wr + 32 * b + (lane & 31);
-                float rs = 1.f;
-                if constexpr (FP8) rs = a.sx[min(m0 + rl, a.M - 1)];
+                const float rs = a.sx[min(m0 + rl, a.M - 1)];
 #pragma unroll
                 for (int qn = 0; qn < 2; ++qn) {
                     const int cb = 128 * qn + 32 * wc;
@@ -456,8 +336,7 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmArgs a) {
 #pragma unroll
             for (int b = 0; b < 4; ++b) {
                 const int rl = 128 * qm + 64 * wr + 16 * b + (lane & 15);
-                float rs = 1.f;
-                if constexpr (FP8) rs = a.sx[min(m0 + rl, a.M - 1)];
+                const float rs = a.sx[min(m0 + rl, a.M - 1)];
 #pragma unroll
                 for (int qn = 0; qn < 2; ++qn)
 #pragma unroll
@@ -489,12 +368,11 @@ __global__ __launch_bounds__(512, 1) void gemm_kernel(const GemmArgs a) {
             if (ok) *reinterpret_cast<u32x4*>(reinterpret_cast<bf16*>(a.c) + (size_t)m * a.ldc + col) = val;
         }
     }
-    stamp();
 }
 
 // Adds the slices of the split tiles and runs the epilogue.  One workgroup per (tile, 2 x 16 rows): the four vectors
 // that every lane of gemm_kernel holds for one of its eight row blocks.
-template <bool FP8, int EPI>
+template <int EPI>
 __global__ __launch_bounds__(512) void gemm_tail_kernel(const GemmArgs a) {
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, wr = w >> 2, wc = w & 3, g4 = lane >> 4;
     const int t = blockIdx.x >> 3, rb = blockIdx.x & 7;
@@ -512,15 +390,12 @@ __global__ __launch_bounds__(512) void gemm_tail_kernel(const GemmArgs a) {
         for (int j = 0; j < 4; ++j) v[j] += in[j * 512];
     }
     const int m = r0 + (lane & 15);
-    float rs = 1.f;
-    if constexpr (FP8) rs = a.sx[min(m, a.M - 1)];
+    const float rs = a.sx[min(m, a.M - 1)];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int cb = n0 + 128 * (j >> 1) + 32 * wc + 16 * (j & 1);  // 16-column block, wholly in or out of range
-        if constexpr (FP8) {
-            const float4 s4 = *reinterpret_cast<const float4*>(a.sw + min(cb + 4 * g4, a.N - 4));
-            v[j][0] *= rs * s4.x; v[j][1] *= rs * s4.y; v[j][2] *= rs * s4.z; v[j][3] *= rs * s4.w;
-        }
+        const float4 s4 = *reinterpret_cast<const float4*>(a.sw + min(cb + 4 * g4, a.N - 4));
+        v[j][0] *= rs * s4.x; v[j][1] *= rs * s4.y; v[j][2] *= rs * s4.z; v[j][3] *= rs * s4.w;
         int col = cb + 4 * g4;
         if constexpr (EPI == GEPI_SWIGLU) {  // the up columns sit in lane xor 32
             f32x4 up;
@@ -529,16 +404,10 @@ __global__ __launch_bounds__(512) void gemm_tail_kernel(const GemmArgs a) {
 #pragma unroll
             for (int k = 0; k < 4; ++k) v[j][k] = glu(v[j][k], up[k], a.glu);
             col = (cb >> 1) + 4 * g4;
-        } else if constexpr (EPI == GEPI_GELU) {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) v[j][k] = gelu_tanh<bf16>(v[j][k]);
         }
         if (m >= a.M || cb >= a.N || (EPI == GEPI_SWIGLU && lane >= 32)) continue;
-        if constexpr (EPI == GEPI_F32)
-            *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.c) + (size_t)m * a.ldc + col) = v[j];
-        else
-            *reinterpret_cast<uint2*>(reinterpret_cast<bf16*>(a.c) + (size_t)m * a.ldc + col) =
-                make_uint2(pack2(v[j][0], v[j][1]), pack2(v[j][2], v[j][3]));
+        *reinterpret_cast<uint2*>(reinterpret_cast<bf16*>(a.c) + (size_t)m * a.ldc + col) =
+            make_uint2(pack2(v[j][0], v[j][1]), pack2(v[j][2], v[j][3]));
     }
 }
 
@@ -562,7 +431,7 @@ MRSUM_API int mrsum_gemm_stamps(unsigned long long* host, int max_words) {
 // whole / splits / part: tiles from raster position ``whole`` on run in ``splits`` slices of K through ``part``
 // [tiles - whole][splits][65536] fp32 (splits 1: none, part unused;
 // 16x16 MFMA tiles only).  slabs (epi 3, whole 0): the slices stay apart, in part [splits][M][N]; c unused.
-// Requirements (checked by the Python wrapper too): K % 64 (bf16) / K % 128 (fp8), N % 16, 16-byte
+// Requirements (checked by the Python wrapper too): K % 64 and K > 0 (bf16) / K % 128 (fp8), N % 16, 16-byte
 // aligned rows.
 MRSUM_API int mrsum_gemm(const void* x, int ldx, const void* w, int ldw, void* c, int ldc, int M, int N, int K,
                          int fp8, int epi, const float* sx, const float* sw, int group_m, int split, float glu_limit,
@@ -574,7 +443,7 @@ MRSUM_API int mrsum_gemm(const void* x, int ldx, const void* w, int ldw, void* c
     if ((size_t)256 * ldx * es >= (1u << 31) || (size_t)256 * ldw * es >= (1u << 31)) return (int)hipErrorInvalidValue;
     if (epi < GEPI_BF16 || epi > GEPI_F32 || (epi >= GEPI_GELU && (fp8 || ((group_m >> 8) & 1))))
         return (int)hipErrorInvalidValue;
-    if (fp8 && (!sx || !sw)) return (int)hipErrorInvalidValue;
+    if (fp8 ? !sx || !sw : K < 64) return (int)hipErrorInvalidValue;
     GemmArgs a;
     a.x = (const char*)x; a.w = (const char*)w; a.c = c; a.sx = sx; a.sw = sw;
     a.ldx_b = ldx * es; a.ldw_b = ldw * es; a.ldc = ldc;
@@ -584,11 +453,11 @@ MRSUM_API int mrsum_gemm(const void* x, int ldx, const void* w, int ldw, void* c
     a.kbw = a.kb;
     if (split) a.kb *= 2;  // X K-tiles: hi then lo
     a.tiles_m = ceil_div(M, 256); a.tiles_n = ceil_div(N, 256);
-    // group_m bits 0-7: tile rows per raster group (0 = 4); bit 8: 32x32 MFMA tiles instead of 16x16.
-    // Measured (profiles/r3_gemm_mfma32_experiment.jsonl, same box, interleaved): 32x32 is 0-9 % slower on
-    // the 8B bf16 projections and about equal on the 70B fp8 qkv / o / down, so 16x16 stays the default;
-    // the fp8 gate_up + SwiGLU GEMM gains 1.7-3.8 % at M = 4k-32k and takes it (ops/hip.py gemm_fp8).
-    const bool m32 = (group_m >> 8) & 1;
+    // group_m bits 0-7: tile rows per raster group (0 = 4); bit 8 (fp8): 32x32 MFMA tiles instead of 16x16.
+    // Measured (profiles/r3_gemm_mfma32_experiment.jsonl, same box, interleaved): 32x32 is
+    // about equal on the 70B fp8 qkv / o / down, so 16x16 stays the default;
+    // the gate_up + SwiGLU GEMM gains 1.7-3.8 % at M = 4k-32k and takes it (ops/hip.py gemm_fp8).
+    const bool m32 = fp8 && ((group_m >> 8) & 1);
     group_m &= 255;
     a.group_m = group_m > 0 ? group_m : 4;
     const int tiles = a.tiles_m * a.tiles_n;
@@ -600,49 +469,39 @@ MRSUM_API int mrsum_gemm(const void* x, int ldx, const void* w, int ldw, void* c
     a.slabs = slabs;
     if (slabs && (epi != GEPI_F32 || splits <= 1 || whole || N % 16)) return (int)hipErrorInvalidValue;
     const int rest = tiles - a.whole;
-    const dim3 grid(a.whole + rest * a.splits), block(512);
+    if (!fp8) {
 #ifdef MRSUM_CLOCK_STAMPS
-    static unsigned long long* stamps = nullptr;
-    static size_t nstamps = 0;
-    if (nstamps < 2 * grid.x) {
-        if (stamps) (void)hipFree(stamps);
-        nstamps = 2 * grid.x;
-        if (hipMalloc(&stamps, nstamps * 8) != hipSuccess) return (int)hipErrorOutOfMemory;
-    }
-    a.stamps = stamps;
-    g_stamps = stamps;
-    g_nstamps = 2 * (int)grid.x;
+        const size_t wgs = gemm_bf16_grid(a);
+        static unsigned long long* stamps = nullptr;
+        static size_t nstamps = 0;
+        if (nstamps < 2 * wgs) {
+            if (stamps) (void)hipFree(stamps);
+            nstamps = 2 * wgs;
+            if (hipMalloc(&stamps, nstamps * 8) != hipSuccess) return (int)hipErrorOutOfMemory;
+        }
+        a.stamps = stamps;
+        g_stamps = stamps;
+        g_nstamps = 2 * (int)wgs;
 #endif
+        gemm_bf16_launch(a, epi, s);
+        return (int)hipGetLastError();
+    }
+    const dim3 grid(a.whole + rest * a.splits), block(512);
     // measured (profiles/r2_gemm_variants_ab.jsonl, r2_gemm_ring10_ab.jsonl): the staggered 8-slot ring
     // (LOOK 6) with the LDS-staged epilogue is the fastest; the 2-phase / 10-slot rings and the
     // unstaggered schedule lost 5-25 %.  The register epilogue remains for outputs that are not 16-B
     // aligned (strided views).
     const bool lepi = ldc % 8 == 0 && (uintptr_t)c % 16 == 0;
-#define GEMM_LAUNCH(F, E)                                                          \
-    if (m32) {                                                                     \
-        if (lepi) gemm_kernel<F, E, 8, true, true><<<grid, block, 0, s>>>(a);      \
-        else gemm_kernel<F, E, 8, false, true><<<grid, block, 0, s>>>(a);          \
-    } else {                                                                       \
-        if (lepi) gemm_kernel<F, E, 8, true, false><<<grid, block, 0, s>>>(a);     \
-        else gemm_kernel<F, E, 8, false, false><<<grid, block, 0, s>>>(a);         \
-        if (rest) gemm_tail_kernel<F, E><<<rest * 8, block, 0, s>>>(a);            \
+#define GEMM_LAUNCH(E)                                                          \
+    if (m32) {                                                                  \
+        if (lepi) gemm_kernel<E, 8, true, true><<<grid, block, 0, s>>>(a);      \
+        else gemm_kernel<E, 8, false, true><<<grid, block, 0, s>>>(a);          \
+    } else {                                                                    \
+        if (lepi) gemm_kernel<E, 8, true, false><<<grid, block, 0, s>>>(a);     \
+        else gemm_kernel<E, 8, false, false><<<grid, block, 0, s>>>(a);         \
+        if (rest) gemm_tail_kernel<E><<<rest * 8, block, 0, s>>>(a);            \
     }
-    if (fp8) {
-        if (epi == GEPI_SWIGLU) { GEMM_LAUNCH(true, GEPI_SWIGLU) } else { GEMM_LAUNCH(true, GEPI_BF16) }
-    } else {
-        if (epi == GEPI_SWIGLU) {
-            GEMM_LAUNCH(false, GEPI_SWIGLU)
-        } else if (epi == GEPI_GELU) {
-            if (lepi) gemm_kernel<false, GEPI_GELU, 8, true, false><<<grid, block, 0, s>>>(a);
-            else gemm_kernel<false, GEPI_GELU, 8, false, false><<<grid, block, 0, s>>>(a);
-            if (rest) gemm_tail_kernel<false, GEPI_GELU><<<rest * 8, block, 0, s>>>(a);
-        } else if (epi == GEPI_F32) {
-            gemm_kernel<false, GEPI_F32, 8, false, false><<<grid, block, 0, s>>>(a);
-            if (rest && !slabs) gemm_tail_kernel<false, GEPI_F32><<<rest * 8, block, 0, s>>>(a);
-        } else {
-            GEMM_LAUNCH(false, GEPI_BF16)
-        }
-    }
+    if (epi == GEPI_SWIGLU) { GEMM_LAUNCH(GEPI_SWIGLU) } else { GEMM_LAUNCH(GEPI_BF16) }
 #undef GEMM_LAUNCH
     return (int)hipGetLastError();
 }

@@ -10,7 +10,7 @@ Every GPU op is a hand-written gfx950 kernel, GEMMs included: decode-shaped
 projections on the weight-streaming MFMA kernels (stream_gemm.hip /
 skinny_gemm.hip, fused split-K / SwiGLU / RoPE epilogues), everything with
 more rows (prefill projections, the LM head over many rows) on the 256 x 256
-MFMA GEMM (gemm.hip; bf16 or OCP fp8).  No vendor BLAS on the hot path.
+MFMA GEMMs (gemm_bf16.hip, OCP fp8 in gemm.hip).  No vendor BLAS on the hot path.
 """
 
 from __future__ import annotations

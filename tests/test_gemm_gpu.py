@@ -1,4 +1,4 @@
-"""Large-M MFMA GEMM (csrc/kernels/gemm.hip) vs a plain PyTorch fp32 reference.
+"""Large-M MFMA GEMMs (csrc/kernels/gemm_bf16.hip, gemm.hip) vs a plain PyTorch fp32 reference.
 
 Covers ragged M (tiles past M), N tails (a vocab shard that is not a multiple of 256),
 strided activations, both epilogues (LDS-staged 16-B row stores for aligned outputs, register
@@ -167,6 +167,33 @@ def test_gemm_split_tail(M, N, K, epi):
         y = torch.nn.functional.gelu(y, approximate="tanh")
     # one bf16 rounding (2^-9 relative) behind fp32 sums; the activations' fp32 exponentials add far less
     assert bool(((out.double() - y).abs() <= 2.0 ** -8 * y.abs() + 1e-4).all())
+
+
+@pytest.mark.parametrize("K", [64, 128, 192, 384, 704])
+@pytest.mark.parametrize("epi", ["bf16", "swiglu", "gelu", "f32"])
+@pytest.mark.parametrize("off", [0, 4])
+def test_gemm_tile_after_tile(K, epi, off):
+    """More tiles than CUs, so that requests run on into the next tile: K-tiles from one (a tile per workgroup) over two
+    (every request past the tile's own) to more than the ring's images, ragged last rows and columns, into columns of
+    wider rows, 16-byte aligned (counted stores) and not."""
+    M, N = 4100, 4128
+    x, w = _rand(M, K, seed=22, scale=0.5, offset=0.02), _rand(N, K, seed=23, scale=0.05, offset=0.001)
+    n, dtype = N // 2 if epi == "swiglu" else N, torch.float32 if epi == "f32" else torch.bfloat16
+    rows = torch.full((M, n + 16), 7.0, dtype=dtype, device=DEV)
+    out = rows[:, off:off + n]
+    for _ in range(2):
+        hip.gemm(x, w, out=out, **({} if epi == "bf16" else {epi: True}))
+    y = x.double() @ w.double().t()
+    slack = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    if epi == "swiglu":
+        h, e = y.reshape(M, -1, 2, 8), slack.reshape(M, -1, 2, 8)
+        y = (torch.nn.functional.silu(h[:, :, 0]) * h[:, :, 1]).reshape(M, -1)
+        slack = (1.1 * e[:, :, 0] * h[:, :, 1].abs() + h[:, :, 0].abs() * e[:, :, 1]).reshape(M, -1)  # |silu'| <= 1.1
+    elif epi == "gelu":
+        y, slack = torch.nn.functional.gelu(y, approximate="tanh"), 1.2 * slack + 1e-5  # |gelu'| < 1.2; its fp32 exponential
+    # sums of K exact products in fp32, then one bf16 rounding
+    assert bool(((out.double() - y).abs() <= (0 if epi == "f32" else 2.0 ** -8) * y.abs() + slack).all())
+    assert bool((rows[:, :off] == 7).all() and (rows[:, off + n:] == 7).all())
 
 
 @pytest.mark.parametrize("M,N,K,two", [(1, 48, 4096, False), (300, 1040, 4224, False), (257, 528, 2176, True), (4097, 4096, 4096, False),

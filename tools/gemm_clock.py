@@ -1,10 +1,10 @@
 #!/usr/bin/env python3
-"""In-kernel clock of the bf16 prefill GEMM (gemm.hip) under sustained load, against its wall-clock TF/s and
+"""In-kernel clock of the bf16 prefill GEMM (gemm_bf16.hip) under sustained load, against its wall-clock TF/s and
 hipBLASLt's (torch.matmul) on the same shapes.
 
 MFMA-dense loops on random data run well under the 2.4 GHz the 2.5 PF/s bf16 peak is quoted at
 (MI355X_MICROARCH.md, 'DVFS give-back'), so the useful ceiling of a GEMM is peak x (held clock / 2.4 GHz).
-A diagnostic build of gemm.hip (-DMRSUM_CLOCK_STAMPS: s_memtime / s_memrealtime around each workgroup,
+A diagnostic build of it (-DMRSUM_CLOCK_STAMPS: s_memtime / s_memrealtime around each workgroup,
 stored by one lane to a buffer nothing else reads) measures that clock after >= 2 s of back-to-back
 launches.  The production library is not touched: ``--build`` writes _native/diag/libmrsum_gemm_clock.so."""
 import argparse
@@ -18,7 +18,8 @@ import time
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 sys.path.insert(0, ROOT)
-SRC = os.path.join(ROOT, "llm_map_reduce_summarizer_amd", "csrc", "kernels", "gemm.hip")
+KERNELS = os.path.join(ROOT, "llm_map_reduce_summarizer_amd", "csrc", "kernels")
+SRC = [os.path.join(KERNELS, f) for f in ("gemm.hip", "gemm_bf16.hip")]
 LIB = os.path.join(ROOT, "llm_map_reduce_summarizer_amd", "_native", "diag", "libmrsum_gemm_clock.so")
 SHAPES = {"qkv": (6144, 4096), "o": (4096, 4096), "gate_up": (28672, 4096), "down": (4096, 14336)}
 
@@ -27,7 +28,7 @@ def build():
     from llm_map_reduce_summarizer_amd import _stamp
     os.makedirs(os.path.dirname(LIB), exist_ok=True)
     flags = [f for f in _stamp.HIP_FLAGS if not f.startswith("-Rpass")]
-    subprocess.check_call(["/opt/rocm/bin/hipcc"] + flags + ["-shared", "-DMRSUM_CLOCK_STAMPS", SRC, "-o", LIB])
+    subprocess.check_call(["/opt/rocm/bin/hipcc"] + flags + ["-shared", "-DMRSUM_CLOCK_STAMPS"] + SRC + ["-o", LIB])
     print("built", LIB)
 
 
