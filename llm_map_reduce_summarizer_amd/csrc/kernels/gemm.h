@@ -13,10 +13,11 @@ struct GemmArgs {
     int ldx_b, ldw_b, ldc;  // X / W row strides in bytes, C row stride in elements
     int M, N, kb;           // kb = K-tiles (128 bytes of every row each)
     int kbw;                // fp8, W's K-tiles: kb, or kb / 2 for two-term X (X tiles kt >= kbw re-read W tile kt - kbw)
+    int rows;  // of a tile: 256, bf16 also 128, 160, 192, 224
     int tiles_m, tiles_n, group_m;
     int whole;    // raster positions below it run whole, the others in ``splits`` slices of K each
     int splits;
-    float* part;  // [tiles - whole][splits][TILE_F] fp32 accumulators of the slices
+    float* part;  // [tiles - whole][splits][rows * 256] fp32 accumulators of the slices
     int slabs;    // GEPI_F32, every tile split: part is [splits][M][N] rows instead, for a consumer that adds the slabs
     GluArgs glu;  // GEPI_SWIGLU
 #ifdef MRSUM_CLOCK_STAMPS

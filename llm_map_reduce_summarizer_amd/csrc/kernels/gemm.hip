@@ -429,8 +429,8 @@ MRSUM_API int mrsum_gemm_stamps(unsigned long long* host, int max_words) {
 // fp32 for epi 3 (both bf16 operands only).  fp8: x, w are e4m3fn bytes,
 // sx [M] / sw [N] fp32 row scales; split: x is two-term [hi | lo] of 2K bytes per row over w's K.
 // whole / splits / part: tiles from raster position ``whole`` on run in ``splits`` slices of K through ``part``
-// [tiles - whole][splits][65536] fp32 (splits 1: none, part unused;
-// 16x16 MFMA tiles only).  slabs (epi 3, whole 0): the slices stay apart, in part [splits][M][N]; c unused.
+// [tiles - whole][splits][rows * 256] fp32 (splits 1: none, part unused;
+// 16x16 MFMA tiles only).  group_m bits 9 - 12: rows of a tile / 32 (0: 256; bf16 also 128, 160, 192, 224).  slabs (epi 3, whole 0): the slices stay apart, in part [splits][M][N]; c unused.
 // Requirements (checked by the Python wrapper too): K % 64 and K > 0 (bf16) / K % 128 (fp8), N % 16, 16-byte
 // aligned rows.
 MRSUM_API int mrsum_gemm(const void* x, int ldx, const void* w, int ldw, void* c, int ldc, int M, int N, int K,
@@ -444,6 +444,8 @@ MRSUM_API int mrsum_gemm(const void* x, int ldx, const void* w, int ldw, void* c
     if (epi < GEPI_BF16 || epi > GEPI_F32 || (epi >= GEPI_GELU && (fp8 || ((group_m >> 8) & 1))))
         return (int)hipErrorInvalidValue;
     if (fp8 ? !sx || !sw : K < 64) return (int)hipErrorInvalidValue;
+    const int rows = (group_m >> 9) & 15 ? 32 * ((group_m >> 9) & 15) : 256;
+    if (rows != 256 && (fp8 || rows < 128 || rows > 256)) return (int)hipErrorInvalidValue;
     GemmArgs a;
     a.x = (const char*)x; a.w = (const char*)w; a.c = c; a.sx = sx; a.sw = sw;
     a.ldx_b = ldx * es; a.ldw_b = ldw * es; a.ldc = ldc;
@@ -452,7 +454,8 @@ MRSUM_API int mrsum_gemm(const void* x, int ldx, const void* w, int ldw, void* c
     if (split && (!fp8 || ldx < 2 * K)) return (int)hipErrorInvalidValue;
     a.kbw = a.kb;
     if (split) a.kb *= 2;  // X K-tiles: hi then lo
-    a.tiles_m = ceil_div(M, 256); a.tiles_n = ceil_div(N, 256);
+    a.rows = rows;
+    a.tiles_m = ceil_div(M, rows); a.tiles_n = ceil_div(N, 256);
     // group_m bits 0-7: tile rows per raster group (0 = 4); bit 8 (fp8): 32x32 MFMA tiles instead of 16x16.
     // Measured (profiles/r3_gemm_mfma32_experiment.jsonl, same box, interleaved): 32x32 is
     // about equal on the 70B fp8 qkv / o / down, so 16x16 stays the default;

@@ -275,3 +275,42 @@ def test_gemm_slabs(M, N, K):
     bound = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
     assert bool(((parts.double().sum(0) - x.double() @ w.double().t()).abs() <= bound).all())
     assert hip.gemm_slabs(x[:, :64], w[:, :64]) is None and hip.gemm_slabs(_rand(4097, K), _rand(4096, K)) is None
+
+
+@pytest.mark.parametrize("rows", [128, 160, 192, 224])
+@pytest.mark.parametrize("epi", ["bf16", "swiglu", "gelu", "f32"])
+@pytest.mark.parametrize("M,N,K,splits", [(1, 32, 64, 1), (129, 288, 128, 1), (449, 544, 704, 3), (4100, 4128, 192, 1), (4100, 4128, 320, 1)])
+def test_gemm_tile_rows(monkeypatch, rows, epi, M, N, K, splits):
+    """Tiles of fewer rows than 256: one K-tile and two (past the end of which the loop asks for nothing that is read), ragged
+    rows and columns, slices of K, and tile after tile with few and more K-tiles.  Whole tiles add a row's products in the
+    same order at every height, so they have the bits of 256 rows; slices are held to the bound of fp32 sums."""
+    x, w = _rand(M, K, seed=24, scale=0.5, offset=0.02), _rand(N, K, seed=25, scale=0.05, offset=0.001)
+    kw = {} if epi == "bf16" else {epi: True}
+
+    def run(rows, splits):
+        tiles = -(-M // rows) * -(-N // 256)
+        whole = tiles if splits == 1 else 0
+        monkeypatch.setattr(hip, "gemm_splits", lambda *_: (whole, splits, (tiles - whole) * splits * rows * 256, rows))
+        return hip.gemm(x, w, **kw)
+    want, got = run(256, 1), run(rows, splits)
+    assert torch.equal(got, run(rows, splits))
+    if splits == 1:
+        assert torch.equal(got, want)
+    else:
+        # fp32 sums of K exact products, either way off by at most K 2^-24 of the sum of magnitudes; gate and up (|silu'| <=
+        # 1.1) or gelu (< 1.2) pass that on; then one bf16 rounding each
+        slack = 2.4 * K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+        if epi == "swiglu":
+            h, e = (x.double() @ w.double().t()).reshape(M, -1, 2, 8).abs(), slack.reshape(M, -1, 2, 8)
+            slack = (e[:, :, 0] * h[:, :, 1] + h[:, :, 0] * e[:, :, 1]).reshape(M, -1)
+        rounding = 0 if epi == "f32" else 2.0 ** -7
+        assert bool(((got.double() - want.double()).abs() <= rounding * want.double().abs() + slack + 1e-30).all())
+
+
+@pytest.mark.parametrize("M", [1, 100, 129, 300, 522, 903, 2000, 7615])
+@pytest.mark.parametrize("N,K", [(32, 64), (1536, 4096), (4096, 22528), (28672, 4096)])
+def test_gemm_plan_is_one_the_kernel_takes(M, N, K):
+    whole, splits, room, rows = hip.gemm_splits(M, N, K // 64)
+    tiles = -(-M // rows) * -(-N // 256)
+    assert rows in (128, 160, 192, 224, 256) and splits >= 1 and room == (tiles - whole) * splits * rows * 256
+    assert whole == tiles if splits == 1 else 0 <= whole < tiles and whole % hip.N_CU == 0 and K // 64 // splits >= 4
