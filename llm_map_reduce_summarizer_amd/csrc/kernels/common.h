@@ -220,6 +220,12 @@ __device__ __forceinline__ float gelu_tanh(float z) {
 }
 
 
+// bijective XCD remap: blocks b, b+8, ... (one XCD's) get consecutive positions
+__device__ __forceinline__ int xcd_position(int bid, int nwg) {
+    const int xcd = bid & 7, local = bid >> 3, q = nwg >> 3, r = nwg & 7;
+    return (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + local;
+}
+
 // Sums over aligned groups of 16 lanes without LDS traffic.
 template <int CTRL>
 __device__ __forceinline__ float dpp(float v) {

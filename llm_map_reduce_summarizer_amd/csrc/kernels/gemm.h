@@ -45,12 +45,6 @@ __device__ __forceinline__ void vm_wait() {
     __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
 }
 
-// bijective XCD remap: blocks b, b+8, ... (one XCD's) get consecutive positions
-__device__ __forceinline__ int xcd_position(int bid, int nwg) {
-    const int xcd = bid & 7, local = bid >> 3, q = nwg >> 3, r = nwg & 7;
-    return (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + local;
-}
-
 // grouped raster of group_m tile rows
 __device__ __forceinline__ void tile_of(int p, int tiles_m, int tiles_n, int group_m, int& tm, int& tn) {
     const int gsz = group_m * tiles_n;

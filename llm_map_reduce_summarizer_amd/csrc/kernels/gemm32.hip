@@ -2,20 +2,25 @@
 //
 //     C[M, N] = X[M, K] . W[N, K]^T        K % 32 == 0
 //
-// 128 x 128 output tile per 256-thread workgroup, two workgroups per CU; wave (wr, wc) owns 64 x 64 outputs as 4 x 4
-// blocks, or for M <= 64 (LOW) wave w 64 x 32, so that all four SIMDs have work (64 x 28672 x 4096: 248 -> 145 us; a form
-// of its own: a branch cost the others 9 %).  K-tiles of 32 (128 bytes a row) arrive by LDS-DMA in two buffers, chunk c of
-// row r at c ^ ((r >> 1) & 7) (conflict-free b128 fragment reads); a fragment's four floats feed four instructions, so a
-// K-tile is 16 LDS reads for 128 instructions of 32 cycles, and the matrix cores set the time (1.7 us a K-tile) once a CU
-// has work.  16-row blocks past M are skipped.  903 x 28672 x 4096: 2310 (64 x 64 tiles, loads between barriers) -> 1650
-// us, 129 TFLOP/s of 157 and 146 counting the rows that pad the last tile.  Tiles that would leave CUs idle run in slices
-// of K (ops/hip.py gemm32_splits), whose fp32 sums a second launch adds in slice order.  Short K runs in 64 x 64 tiles.
+// A tile of up to 128 rows x 128 columns per 256-thread workgroup, two workgroups per CU; wave w owns all rows x columns
+// [32 w, 32 w + 32), so that the four SIMDs have the same work at any number of 16-row blocks (in quarters of 64 x 64 a tile
+// of 22 rows took as long as a full one: two of the SIMDs did its work).  The rows are dealt to the row tiles evenly.
+// What bounds it is the matrix cores: a K-tile of 32 (128 bytes a row) is 128 instructions of 32 cycles a wave, 1.7 us, for 20
+// LDS reads.  Images arrive by LDS-DMA, chunk c of row r at c ^ ((r >> 1) & 7) (conflict-free b128 fragment reads); the one
+// wait and barrier of a K-tile stands in its middle, with the second half's fragments in registers, and the next
+// K-tile's first ones are read behind the second half's products: both workgroups of a CU, which run in step, would else stop
+// for their reads together (128 x 128 tiles, 480 -> 500 us with the reads ahead of the products they feed).
+// us, four quarters and two barriers -> this: 903 x 28672 x 4096 1646 -> 1500 (141 TFLOP/s of 155), 300 x 28672 x 4096 667 ->
+// 535, 150 x 18560 x 4096 305 -> 196, 70 x 4096 x 8192 73 -> 54, 508 x 28672 x 4096 832 -> 826.
+// Tiles that would leave CUs idle run in slices of K (ops/hip.py _gemm32_plan), whose fp32 sums a second launch adds in slice
+// order.  Short K runs in 64 x 64 tiles.
 #include "common.h"
 
 #include <type_traits>
 
 namespace {
-constexpr int T32 = 128, STAGE = T32 * 128;  // bytes of one operand's K-tile
+constexpr int T32 = 128, STAGE = T32 * 128;  // bytes of W's K-tile
+constexpr int LDS_BYTES = 80 * 1024;         // two workgroups on a CU
 
 struct Gemm32Args {
     const float* x;
@@ -47,134 +52,187 @@ __device__ __forceinline__ void store_c(const Gemm32Args& a, int m, int n, const
 }
 }  // namespace
 
-template <bool LOW>
-__global__ __launch_bounds__(256, 2) void gemm32_kernel(const Gemm32Args a) {
-    __shared__ __attribute__((aligned(1024))) char lds[4 * STAGE];  // [buffer][x | w]
+// Row tile tm of column tile tn: an even share of the 16-row blocks, so that no tile is nearly empty beside full ones; which
+// ones are a block taller changes from column to column, as two tall ones on a CU would set the time of all.
+__device__ __forceinline__ void rows_of(const Gemm32Args& a, int tm, int tn, int& b0, int& nb) {
+    const int blocks = (a.M + 15) >> 4, turn = (tn + (tn >> 2) + (tn >> 4)) % a.tiles_m;
+    b0 = (int)(((long long)blocks * tm + turn) / a.tiles_m);
+    nb = (int)(((long long)blocks * (tm + 1) + turn) / a.tiles_m) - b0;
+}
+
+// K-tiles [kt0, kt1) of a tile of NB row blocks; acc[row block][column block]
+template <int NB>
+__device__ __forceinline__ void k_loop(const Gemm32Args& a, char* lds, int m0, int n0, int kt0, int kt1, f32x4 (&acc)[8][2]) {
     typedef __attribute__((address_space(3))) void* lds_ptr;
+    constexpr int XB = NB * 2048, IMAGE = XB + STAGE, XI = (NB + 1) / 2;  // a K-tile of X; of both; pieces of X a wave
+    constexpr int D = LDS_BYTES / IMAGE < 4 ? LDS_BYTES / IMAGE : 4;
+    static_assert(D >= 2 && (D - 1) * (4 + XI) < 64, "K-tiles in flight");
     const int tid = threadIdx.x, lane = tid & 63;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6), wr = w >> 1, wc = w & 1;
-    int p = blockIdx.x, slice = -1, kt0 = 0, kt1 = a.kb;
-    if (p >= a.whole) {
-        const int rest = a.tiles_m * a.tiles_n - a.whole;
-        slice = (p - a.whole) / rest;
-        p -= slice * rest;
-        kt0 = a.kb * slice / a.splits;
-        kt1 = a.kb * (slice + 1) / a.splits;
-    }
-    int tm, tn;
-    tile32(a, p, tm, tn);
-    const int m0 = tm * T32, n0 = tn * T32, xrows = min(a.M - m0, T32), wrows = min(a.N - n0, T32);
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int xrows = min(a.M - m0, 16 * NB), wrows = min(a.N - n0, T32);
     const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(a.x + (size_t)m0 * a.ldx), (short)0, xrows * a.ldx * 4, 0x00020000);
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(a.w + (size_t)n0 * a.ldw), (short)0, wrows * a.ldw * 4, 0x00020000);
-    // staging: wave w fills rows 32 w .. 32 w + 31 of both operands, 8 rows per instruction; rows past M / N are
-    // dropped by the descriptor (their LDS rows feed sums that are not stored)
-    const int row = 32 * w + (lane >> 3);
-    const int ch0 = ((lane & 7) ^ ((lane >> 4) & 7)) << 4, ch1 = ((lane & 7) ^ ((4 + (lane >> 4)) & 7)) << 4;
-    auto stage = [&](int kt, int buf) {
-        char* dst = lds + buf * 2 * STAGE + w * 4096;
+    // staging: 8 rows per instruction, wave w rows 32 w .. 32 w + 31 of W and every fourth piece of X (behind the last one
+    // that one again, so that all waves count alike); rows past M / N are dropped by the descriptor (their LDS rows feed
+    // sums that are not stored)
+    int vw[4], vx[XI], dx[XI];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int ch = i & 1 ? ch1 : ch0;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr)(dst + i * 1024), 16, (row + 8 * i) * a.ldx * 4 + ch,
-                                                     kt * 128, 0, 0);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr)(dst + STAGE + i * 1024), 16,
-                                                     (row + 8 * i) * a.ldw * 4 + ch, kt * 128, 0, 0);
-        }
+    for (int i = 0; i < 4; ++i) {
+        const int r = 32 * w + 8 * i + (lane >> 3);
+        vw[i] = r * a.ldw * 4 + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
+    }
+#pragma unroll
+    for (int i = 0; i < XI; ++i) {
+        const int p = min(w + 4 * i, 2 * NB - 1), r = 8 * p + (lane >> 3);
+        vx[i] = r * a.ldx * 4 + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
+        dx[i] = STAGE + p * 1024;
+    }
+    auto stage = [&](int kt, int buf) {
+        char* dst = lds + buf * IMAGE;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr)(dst + (4 * w + i) * 1024), 16, vw[i], kt * 128, 0, 0);
+#pragma unroll
+        for (int i = 0; i < XI; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr)(dst + dx[i]), 16, vx[i], kt * 128, 0, 0);
     };
     int lo[2];
 #pragma unroll
     for (int r = 0; r < 2; ++r) lo[r] = (lane & 15) * 128 + (((4 * r + (lane >> 4)) ^ ((lane >> 1) & 7)) << 4);
-    constexpr int NC = LOW ? 2 : 4;
-    f32x4 acc[4][NC];  // [row block][column block]
+    f32x4 xf[2][NB], wf[2][2];  // fragments of the two halves of a K-tile
+    auto read = [&](int r, int buf) {
+        const char* ws = lds + buf * IMAGE + w * 4096;
+        const char* xs = lds + buf * IMAGE + STAGE;
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
+        for (int i = 0; i < 2; ++i) wf[r][i] = *reinterpret_cast<const f32x4*>(ws + i * 2048 + lo[r]);
 #pragma unroll
-        for (int i = 0; i < NC; ++i) acc[b][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int rbase = LOW ? 0 : 64 * wr, cbase = LOW ? 32 * w : 64 * wc;  // this wave's outputs
-    const int nb = min(4, (xrows - rbase + 15) >> 4);                     // its row blocks (<= 0: none)
-    auto compute = [&](int buf, auto all) {
-        const char* xs = lds + buf * 2 * STAGE + rbase * 128;
-        const char* ws = lds + buf * 2 * STAGE + STAGE + cbase * 128;
-#pragma unroll
-        for (int r = 0; r < 2; ++r) {
-            f32x4 xf[4], wf[NC];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if (i < NC) wf[i] = *reinterpret_cast<const f32x4*>(ws + i * 2048 + lo[r]);
-                xf[i] = *reinterpret_cast<const f32x4*>(xs + i * 2048 + lo[r]);
-            }
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                if (!decltype(all)::value && b >= nb) break;
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-#pragma unroll
-                    for (int i = 0; i < NC; ++i)
-                        acc[b][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[i][j], xf[b][j], acc[b][i], 0, 0, 0);
-            }
-        }
+        for (int b = 0; b < NB; ++b) xf[r][b] = *reinterpret_cast<const f32x4*>(xs + b * 2048 + lo[r]);
+        __builtin_amdgcn_sched_barrier(0);
     };
-    auto bar = [] {
+    auto products = [&](int r) {
+#pragma unroll
+        for (int b = 0; b < NB; b += 2)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int q = b; q < b + 2 && q < NB; ++q)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+                        acc[q][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[r][i][j], xf[r][q][j], acc[q][i], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    constexpr int PER = 4 + XI;  // requests of a wave for a K-tile
+    // this wave's fragments are in registers and its pieces of the oldest K-tile but ``ahead`` have arrived, and so in all
+    auto meet = [](auto ahead) {
+        constexpr int N = decltype(ahead)::value * PER;
+        __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (0 << 8) | ((N >> 4) << 14));
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
-    stage(kt0, 0);
-    for (int kt = kt0, buf = 0; kt < kt1; ++kt, buf ^= 1) {
-        if (kt + 1 < kt1) {
-            stage(kt + 1, buf ^ 1);
-            __builtin_amdgcn_s_waitcnt(8 | (7 << 4) | (15 << 8));  // vmcnt(8): all but the tile just asked for
-        } else {
-            __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));
-        }
-        bar();
-        if (nb == 4) compute(buf, std::true_type{});
-        else if (nb > 0) compute(buf, std::false_type{});
-        bar();
+#pragma unroll
+    for (int d = 0; d < D; ++d) stage(min(kt0 + d, kt1 - 1), d);
+    meet(std::integral_constant<int, D - 1>{});
+    read(0, 0);
+    for (int kt = kt0, buf = 0; kt < kt1; ++kt) {
+        read(1, buf);
+        products(0);
+        meet(std::integral_constant<int, D - 2>{});
+        stage(min(kt + D, kt1 - 1), buf);  // past the end the last one again, which nothing reads
+        buf = buf + 1 == D ? 0 : buf + 1;
+        read(0, buf);
+        products(1);
+    }
+    __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));  // nothing may arrive in LDS that another workgroup has by then
+}
+
+__global__ __launch_bounds__(256, 2) void gemm32_kernel(const Gemm32Args a) {
+    __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // an XCD's workgroups take neighbouring tiles: they share W's panels, and each XCD has taller and lower tiles alike
+    int p = blockIdx.x, slice = -1, kt0 = 0, kt1 = a.kb;
+    if (p < a.whole) {
+        p = xcd_position(p, a.whole);
+    } else {
+        const int rest = a.tiles_m * a.tiles_n - a.whole;
+        p = xcd_position(p - a.whole, rest * a.splits);
+        slice = p / rest;
+        p += a.whole - slice * rest;
+        kt0 = a.kb * slice / a.splits;
+        kt1 = a.kb * (slice + 1) / a.splits;
+    }
+    int tm, tn, b0, nb;
+    tile32(a, p, tm, tn);
+    rows_of(a, tm, tn, b0, nb);
+    const int m0 = b0 * 16, n0 = tn * T32;
+    f32x4 acc[8][2];
+#pragma unroll
+    for (int b = 0; b < 8; ++b)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) acc[b][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    switch (nb) {
+        case 1: k_loop<1>(a, lds, m0, n0, kt0, kt1, acc); break;
+        case 2: k_loop<2>(a, lds, m0, n0, kt0, kt1, acc); break;
+        case 3: k_loop<3>(a, lds, m0, n0, kt0, kt1, acc); break;
+        case 4: k_loop<4>(a, lds, m0, n0, kt0, kt1, acc); break;
+        case 5: k_loop<5>(a, lds, m0, n0, kt0, kt1, acc); break;
+        case 6: k_loop<6>(a, lds, m0, n0, kt0, kt1, acc); break;
+        case 7: k_loop<7>(a, lds, m0, n0, kt0, kt1, acc); break;
+        default: k_loop<8>(a, lds, m0, n0, kt0, kt1, acc); break;
     }
     if (slice >= 0) {
         f32x4* out = reinterpret_cast<f32x4*>(a.part + ((size_t)(p - a.whole) * a.splits + slice) * (T32 * T32)) + tid;
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
+        for (int b = 0; b < 8; ++b)
             if (b < nb)
 #pragma unroll
-                for (int i = 0; i < NC; ++i) out[(b * 4 + i) * 256] = acc[b][i];
+                for (int i = 0; i < 2; ++i) out[(b * 2 + i) * 256] = acc[b][i];
         return;
     }
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
+    for (int b = 0; b < 8; ++b)
+        if (b < nb)
 #pragma unroll
-        for (int i = 0; i < NC; ++i)
-            store_c(a, m0 + rbase + 16 * b + (lane & 15), n0 + cbase + 16 * i + 4 * (lane >> 4), acc[b][i]);
+            for (int i = 0; i < 2; ++i)
+                store_c(a, m0 + 16 * b + (lane & 15), n0 + 32 * w + 16 * i + 4 * (lane >> 4), acc[b][i]);
 }
 
 // adds the slices of the split tiles; one workgroup per (tile, 2 x 16 rows)
-template <bool LOW>
 __global__ __launch_bounds__(256) void gemm32_tail_kernel(const Gemm32Args a) {
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, t = blockIdx.x >> 2, b = blockIdx.x & 3;
-    int tm, tn;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, t = blockIdx.x >> 2, b = 2 * (blockIdx.x & 3);
+    int tm, tn, b0, nb;
     tile32(a, a.whole + t, tm, tn);
-    constexpr int NC = LOW ? 2 : 4;
-    const int m = tm * T32 + (LOW ? 0 : 64 * (w >> 1)) + 16 * b, n = tn * T32 + (LOW ? 32 * w : 64 * (w & 1));
-    if (m >= a.M) return;
-    const f32x4* in = reinterpret_cast<const f32x4*>(a.part + (size_t)t * a.splits * (T32 * T32)) + b * 4 * 256 + tid;
-    f32x4 v[NC];
+    rows_of(a, tm, tn, b0, nb);
+    if (b >= nb) return;
+    const f32x4* in = reinterpret_cast<const f32x4*>(a.part + (size_t)t * a.splits * (T32 * T32)) + b * 2 * 256 + tid;
+    f32x4 v[4];
+    const int n = b + 1 < nb ? 4 : 2;
 #pragma unroll
-    for (int i = 0; i < NC; ++i) v[i] = in[i * 256];
-    for (int s = 1; s < a.splits; ++s) {
-        in += T32 * T32 / 4;
+    for (int i = 0; i < 4; ++i) v[i] = in[min(i, n - 1) * 256];
+    for (int s = 1; s < a.splits; s += 4) {  // four slices in flight
+        f32x4 p[4][4];
 #pragma unroll
-        for (int i = 0; i < NC; ++i) v[i] += in[i * 256];
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) p[k][i] = in[(size_t)min(s + k, a.splits - 1) * (T32 * T32 / 4) + min(i, n - 1) * 256];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (s + k < a.splits)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] += p[k][i];
     }
 #pragma unroll
-    for (int i = 0; i < NC; ++i) store_c(a, m + (lane & 15), n + 16 * i + 4 * (lane >> 4), v[i]);
+    for (int i = 0; i < 4; ++i)
+        if (i < n)
+            store_c(a, 16 * (b0 + b + (i >> 1)) + (lane & 15), tn * T32 + 32 * w + 16 * (i & 1) + 4 * (lane >> 4), v[i]);
 }
 
 // Short K: 64 x 64 tiles, loads and products in turns, wave w rows [16 w, 16 w + 16).  A K-tile takes half the time that a
-// lone workgroup of the larger tiles takes, and four times as many workgroups share a small product (256 x 4096 x 256: 22 us
-// in 128 x 128 tiles, 12 here); from K 512 on the larger tiles' rate leads.  Which one: ops/hip.py gemm32_small.
+// lone workgroup of the larger tiles takes, and four times as many workgroups share a small product (700 x 8192 x 192: 31 us
+// in 128 x 128 tiles, 26 here); from K 512 on the larger tiles' rate leads.  Which one: ops/hip.py gemm32_small.
 constexpr int TS = 64, LDS32 = 32 + 4;  // tile, padded row of a K-tile
 
 __global__ __launch_bounds__(256) void gemm32_small_kernel(const float* __restrict__ x, int ldx, const float* __restrict__ w,
@@ -238,12 +296,7 @@ MRSUM_API int mrsum_gemm32(const float* x, int ldx, const float* w, int ldw, flo
     a.whole = splits > 1 ? whole : tiles;
     a.splits = splits > 1 ? splits : 1;
     const int rest = tiles - a.whole;
-    if (M <= 64) {
-        gemm32_kernel<true><<<a.whole + rest * a.splits, 256, 0, s>>>(a);
-        if (rest) gemm32_tail_kernel<true><<<rest * 4, 256, 0, s>>>(a);
-    } else {
-        gemm32_kernel<false><<<a.whole + rest * a.splits, 256, 0, s>>>(a);
-        if (rest) gemm32_tail_kernel<false><<<rest * 4, 256, 0, s>>>(a);
-    }
+    gemm32_kernel<<<a.whole + rest * a.splits, 256, 0, s>>>(a);
+    if (rest) gemm32_tail_kernel<<<rest * 4, 256, 0, s>>>(a);
     return (int)hipGetLastError();
 }

@@ -494,6 +494,20 @@ def test_gemm32_edges(M, N, K, split, monkeypatch):
     assert got.shape == (M, N) and bool(((got - x.double() @ w.double().T).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("M", [16, 31, 48, 65, 80, 90, 100, 127, 128, 129, 145, 263, 1040])
+@pytest.mark.parametrize("N,K", [(130, 32), (2062, 96), (390, 512)])
+def test_gemm32_row_blocks(M, N, K, monkeypatch):
+    """Every number of 16-row blocks in a tile, tiles of unequal heights that change from column to column, K-tiles fewer than
+    the images in flight and more, whole tiles and (K 512) slices of K."""
+    from llm_map_reduce_summarizer_amd.ops import hip
+    monkeypatch.setattr(hip, "gemm32_small", lambda *_: False)
+    x, w = rnd(M, K, seed=1), rnd(N, K, seed=2)
+    got = hip.gemm32(dev(x), dev(w)).double().cpu()
+    # each of the K products and sums rounds by at most 2^-24 of the sum of magnitudes
+    bound = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert got.shape == (M, N) and bool(((got - x.double() @ w.double().T).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(65, 16, 32), (64, 130, 192), (33, 65, 288), (257, 1, 128), (520, 8192, 192), (300, 1023, 512)])
 def test_gemm32_short_k(M, N, K):
     """The 64 x 64 tiles: rows and columns past the last tile, against 64 bits; the larger tiles give the same up to rounding."""
