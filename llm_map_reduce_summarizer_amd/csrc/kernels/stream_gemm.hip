@@ -73,6 +73,13 @@ constexpr int ring_slots(int mt, int wpb, int halves) {
 // slot's x share falls with its W rows: N 128256, K 4096, 128 x rows: 299 us at 64 W rows, 254 at 128.
 constexpr int slot_halves(int mt, int wpb) { return mt > 4 && ring_slots(mt, wpb, 2) < 3 ? 1 : 2; }
 
+// Grids of many rounds (the LM head): workgroups of 64 W rows with rings so shallow that two share a CU, whose loads run on
+// through each other's barriers, first waits and epilogues.  N 128256, us, one deep ring -> two: K 4096, 16 rows 185 -> 177, 32
+// 197 -> 188 (one row 186 either way); 39 rows, whose slots leave such rings two slots, 208 stays (214), up to K 1024:
+// K 256, 1 row 23.5 -> 13.4, 64 rows 33 -> 20, K 1024 65 -> 56.  One round gains nothing: it has a ring per CU to fill.
+constexpr int SHALLOW_MAX_K = 1024;
+constexpr int shallow_slots(int mt) { return mt <= 2 ? 3 : 2; }
+
 // deferred-RMSNorm operands (see the header); all null / zero for a plain GEMM
 struct NormArgs {
     const float* ssq;  // consumer: [M][ssq_tiles] row sums of squares of x per producer column tile
@@ -381,7 +388,7 @@ __device__ __forceinline__ void stream_epilogue(f32x4 (&acc)[MT], char* lds, flo
 // NTW: weight pieces loaded with the nontemporal policy (aux = 2): decode weights are read once per
 // step by one CU (MI355X_MICROARCH.md "nt-weights"); the x pieces keep the default policy (re-read by
 // every column tile from L2).
-template <int MT, int EPI, int WPB, bool NTW>
+template <int MT, int EPI, int WPB, bool NTW, bool SHALLOW = false>
 __global__ __launch_bounds__(64 * WPB, 1) void stream_gemm_kernel(const bf16* __restrict__ x, int ldx,
                                                                   const bf16* __restrict__ W, int K, int M,
                                                                   void* __restrict__ out, int ldo, int kper,
@@ -393,7 +400,8 @@ __global__ __launch_bounds__(64 * WPB, 1) void stream_gemm_kernel(const bf16* __
     constexpr int XP = H * BM / 8;               // x pieces per slot
     constexpr int XI = (XP + WPB - 1) / WPB;     // x pieces per wave (padded)
     constexpr int NI = 2 * H + XI;               // DMA instructions per wave per slot
-    constexpr int XTRA = lds_extra(MT, WPB, H), D = ring_slots(MT, WPB, H);
+    constexpr int XTRA = lds_extra(MT, WPB, H), D = SHALLOW ? shallow_slots(MT) : ring_slots(MT, WPB, H);
+    static_assert(!SHALLOW || (MT <= 4 && 2 * (D * SLOT + XTRA) <= 160 * 1024), "two on a CU");
     static_assert(D >= 3 || MT <= 4, "ring too shallow");
     __shared__ __attribute__((aligned(1024))) char lds[D * SLOT + XTRA];
     float* const s_ss = reinterpret_cast<float*>(lds + (MT > 4 ? 0 : D * SLOT + 1024));  // consumer row-norm partials
@@ -518,6 +526,24 @@ MRSUM_API int mrsum_stream_gemm(const void* x, int ldx, const void* W, int N, in
     auto P = (float*)parts;
 #define L(MT_, EPI_, WPB_)                                                                                   \
     stream_gemm_kernel<MT_, EPI_, WPB_, true><<<grid, block, 0, s>>>(X, ldx, Wp, K, M, out, ldo, kper, P, counters, e)
+#define LS(MT_, EPI_)                                                                                        \
+    stream_gemm_kernel<MT_, EPI_, 4, true, true><<<grid, block, 0, s>>>(X, ldx, Wp, K, M, out, ldo, kper, P, counters, e)
+#define SHALLOW_BY_EPI(MT_)                                      \
+    if (epi == EPI_BF16) LS(MT_, EPI_BF16);                      \
+    else if (epi == EPI_F32_PARTIAL) LS(MT_, EPI_F32_PARTIAL);   \
+    else LS(MT_, EPI_SWIGLU);
+    if (wpb == 4 && mt <= 4 && grid.x * grid.y > 512 && (mt <= 2 || kper <= SHALLOW_MAX_K) &&
+        (epi == EPI_BF16 || epi == EPI_F32_PARTIAL || epi == EPI_SWIGLU)) {
+        switch (mt) {
+            case 1: SHALLOW_BY_EPI(1); break;
+            case 2: SHALLOW_BY_EPI(2); break;
+            case 3: SHALLOW_BY_EPI(3); break;
+            default: SHALLOW_BY_EPI(4); break;
+        }
+        return (int)hipGetLastError();
+    }
+#undef SHALLOW_BY_EPI
+#undef LS
 #define BY_WPB(MT_, EPI_)                          \
     switch (wpb) {                                 \
         case 4: L(MT_, EPI_, 4); break;            \

@@ -441,6 +441,28 @@ def test_stream_gemm(M, wpb, K):
            g * torch.sigmoid(g) * u, 2e-2)
 
 
+@pytest.mark.parametrize("M,K", [(1, 128), (16, 256), (17, 1152), (32, 2048), (33, 256), (64, 1024)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_stream_gemm_many_rounds(M, K, norm):
+    """Grids of more than two rounds share CUs in pairs with shallow rings (K blocks fewer than the ring's slots, as many and
+    more): the bits of the same columns from grids of one round, whose rings are deep."""
+    n = 64 * 514
+    x, w = _rand(M, K, seed=64), _rand(n, K, scale=0.05, seed=65)
+    half, kw = n // 2, {}
+    if norm:
+        kw["norm"] = ((x.float() ** 2).view(M, 32, -1).sum(-1).contiguous(), 1e-5)
+
+    def run(w, epi):
+        n = w.shape[0]
+        shape = {hip.EPI_BF16: (M, n), hip.EPI_F32_PARTIAL: (1, M, n), hip.EPI_SWIGLU: (M, n // 2)}[epi]
+        o = torch.empty(shape, dtype=torch.float32 if epi == hip.EPI_F32_PARTIAL else torch.bfloat16, device=DEV)
+        return hip._stream_gemm(x, w, o, epi, 1, shape[-1], 4, **kw)
+    for epi in (hip.EPI_BF16, hip.EPI_F32_PARTIAL, hip.EPI_SWIGLU):
+        assert torch.equal(run(w, epi), torch.cat([run(w[:half], epi), run(w[half:], epi)], -1))
+    if not norm:
+        _close(run(w, hip.EPI_F32_PARTIAL)[0], x.float() @ w.float().t(), 1e-3, 1e-3)
+
+
 @pytest.mark.parametrize("M", [1, 10, 39, 64])
 @pytest.mark.parametrize("N,K,wpb,S", [(3584, 4096, 7, 8), (7168, 4096, 7, 4), (448, 1024, 4, 2), (896, 512, 8, 4)])
 def test_stream_swiglu_split(M, N, K, wpb, S):
