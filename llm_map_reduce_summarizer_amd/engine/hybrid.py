@@ -195,8 +195,8 @@ class HybridModel:
         return workspaces(self._mixers(), B, max_ctx, self.device)
 
     def pass_items(self, lens: Sequence[int]):
-        """Prefill-attention work lists of a pass's portions, per distinct kernel form."""
-        return work_items(self._mixers(), lens, self.device)
+        """Prefill-attention work lists of a pass's portions, on the host, per distinct kernel form."""
+        return work_items(self._mixers(), lens)
 
     # ------------------------------------------------------------------ forward
     def _embed(self, b, kv) -> torch.Tensor:

@@ -352,10 +352,10 @@ def workspaces(mixers, B: int, max_ctx: int, device) -> Dict[object, object]:
     return out
 
 
-def work_items(mixers, lens, device) -> Dict[object, object]:
+def work_items(mixers, lens) -> Dict[object, object]:
     out: Dict[object, object] = {}
     for m in mixers if lens else ():
         e = m.pass_items(lens)
         if e is not None and e[0] not in out:
-            out[e[0]] = e[1]().to(device, non_blocking=True)
+            out[e[0]] = e[1]().numpy()
     return out

@@ -252,7 +252,9 @@ class LlamaModel:
         return ops.decode_workspace(B, self.hq, self.hkv, self.hd, max_ctx, self.device, kv8)
 
     def pass_items(self, lens):
-        return ops.prefill_items(lens, self.hq // self.hkv).to(self.device, non_blocking=True)
+        """Prefill-attention work list of a pass, on the host, by GQA ratio."""
+        r = self.hq // self.hkv
+        return {r: ops.prefill_items(lens, r).numpy()}
 
     def forward_pass(self, x, kv, gather: bool = True, logits: bool = True) -> Optional[torch.Tensor]:
         """One packed pass of LLMEngine._pass_inputs; logits of the rows ``x.last_rows``."""

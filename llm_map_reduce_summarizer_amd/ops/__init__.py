@@ -15,6 +15,7 @@ MFMA GEMMs (gemm_bf16.hip, OCP fp8 in gemm.hip).  No vendor BLAS on the hot path
 
 from __future__ import annotations
 
+import numpy as np
 import torch
 
 from . import reference
@@ -339,15 +340,23 @@ class PortionContext:
     row ``slots[i]``) has ``ctx[i]`` = prefix + portion rows, gathered to rows [base[i], base[i] + ctx[i])."""
 
     def __init__(self, lens, prefix, slots, device):
-        from itertools import accumulate
         self.ctx = [p + n for p, n in zip(prefix, lens)]
-        base = [0] + list(accumulate(self.ctx))
-        self.rows = base[-1]
-        i32 = lambda v: torch.tensor(v, dtype=torch.int32).to(device, non_blocking=True)  # noqa: E731
-        self.base, self.prefix = i32(base), i32(list(prefix))
+        base = np.concatenate(([0], np.cumsum(self.ctx))).astype(np.int32)
+        self.rows = int(base[-1])
         # one entry per 64-token page: (block-table row, page of the sequence, destination row, rows)
-        self.pages = i32([(s, p, b + 64 * p, min(64, c - 64 * p)) for s, b, c in zip(slots, base, self.ctx)
-                          for p in range(-(-c // 64))])
+        n = [-(-c // 64) for c in self.ctx]
+        page = np.concatenate([np.arange(k, dtype=np.int32) for k in n] or [np.zeros(0, np.int32)])
+        pages = np.stack((np.repeat(np.asarray(slots, np.int32), n), page, np.repeat(base[:-1], n) + 64 * page,
+                          np.minimum(64, np.repeat(np.asarray(self.ctx, np.int32), n) - 64 * page)), 1).astype(np.int32)
+        parts, at = (pages.reshape(-1), base, np.asarray(list(prefix), np.int32)), [0]
+        for v in parts:  # one copy; pieces at multiples of 256 bytes
+            at.append(at[-1] + -(-v.size // 64) * 64)
+        buf = np.zeros(at[-1], np.int32)
+        for k, v in zip(at, parts):
+            buf[k: k + v.size] = v
+        d = torch.from_numpy(buf).to(device, non_blocking=True)
+        self.pages, self.base, self.prefix = (d[k: k + v.size] for k, v in zip(at, parts))
+        self.pages = self.pages.view(-1, 4)
         self.prefix_host, self.slot_host = list(prefix), list(slots)
 
 

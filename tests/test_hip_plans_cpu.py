@@ -6,6 +6,7 @@ import importlib.util
 import os
 import re
 
+import numpy as np
 import pytest
 import torch
 
@@ -186,3 +187,21 @@ def test_gemm_clock_passes_what_the_gemm_takes():
     assert len(args) == c_parameters()["mrsum_gemm"] and args[6:9] == [3, 16, 64]
     # GLU parameters, no tiles in slices, the stream
     assert args[15:] == [float("inf"), 1.0, 0.0, 0, 1, None, 0, 99]
+
+
+@pytest.mark.parametrize("lens", [[1], [300, 64], [0, 65, 4096, 4096, 1, 700], [64] * 40])
+def test_block_items_of_few_and_many_blocks(lens):
+    """Work lists built from tuples (few blocks) and from arrays are the same list: latest blocks first, then by sequence."""
+    want = sorted(((-qb, i) for i, n in enumerate(lens) for qb in range(0, n, 64)), key=lambda e: e[0])
+    got = hip.block_items(lens, 64)
+    assert got.dtype == torch.int32 and got.tolist() == [[i, -qb] for qb, i in want]
+
+
+def test_token_ids_of_one_and_many():
+    from llm_map_reduce_summarizer_amd.engine.engine import _token_ids
+    for toks in ([7], (7,), [7, 9], range(3), np.arange(4)):
+        ids = _token_ids(toks, 10)
+        assert ids.dtype == np.int32 and ids.tolist() == list(toks)
+    for toks in ([], [10], [-1], [3, 10], [2 ** 70], [-(2 ** 70)]):
+        with pytest.raises(ValueError):
+            _token_ids(toks, 10)
