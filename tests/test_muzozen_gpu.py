@@ -294,6 +294,34 @@ def test_delta_rule(H, G, dim, vdim, dtype, monkeypatch):
             b = e
 
 
+def test_delta_chunks_in_grids_of_both_kinds():
+    """The heads of a key head in one block each while the grid is small, one after the other beyond: the same bits."""
+    from llm_map_reduce_summarizer_amd import ops
+    from llm_map_reduce_summarizer_amd.engine import mixers
+    from llm_map_reduce_summarizer_amd.engine.config import DeltaSpec
+    H, G, dim, vdim, n, L = 16, 4, 32, 16, 72, 63
+    m = mixers.DeltaMixer(DeltaSpec(H, G, dim, vdim, 2), torch.device(DEV), BF)
+    cols = [0]
+
+    def take(k):
+        at = cols[0]
+        cols[0] = -(-(at + k) // 8) * 8
+        return at
+    m.columns(take)
+    m.col = 0
+    x, u = dev(rnd(n * L, m.channels, std=0.8).to(BF)), dev(rnd(n * L, -(-cols[0] // 16) * 16, seed=1, std=1.5).to(BF))
+    small = [dev(rnd(k, seed=2 + j)) for j, k in enumerate((H, H, vdim))]
+
+    def run(lo, hi):
+        state = torch.zeros(n + 1, H, vdim, dim, device=DEV)
+        a = torch.zeros((hi - lo) * L, m.width, dtype=BF, device=DEV)
+        ops.delta_mix(x[lo * L: hi * L].contiguous(), u[lo * L: hi * L].contiguous(), m, -small[0].exp(), small[1] - 3, small[2],
+                      1e-3, state, segments([L] * (hi - lo), list(range(1, hi - lo + 1)), [0] * (hi - lo)), a)
+        return a, state[1: hi - lo + 1]
+    (a, s), (b, t), (c, v) = run(0, n), run(0, n // 2), run(n // 2, n)
+    assert torch.equal(a, torch.cat((b, c))) and torch.equal(s, torch.cat((t, v))) and bool(a.float().abs().sum() > 0)
+
+
 def delta_portions(H, G, dim, vdim, dtype, lens, off=0):
     """Both sides of one delta_mix over segments of ``lens`` rows; ``off``: first element of ``a`` and the norm weights in
     their storage.  Returns (rows, states) errors."""
