@@ -314,3 +314,15 @@ def test_gemm_plan_is_one_the_kernel_takes(M, N, K):
     tiles = -(-M // rows) * -(-N // 256)
     assert rows in (128, 160, 192, 224, 256) and splits >= 1 and room == (tiles - whole) * splits * rows * 256
     assert whole == tiles if splits == 1 else 0 <= whole < tiles and whole % hip.N_CU == 0 and K // 64 // splits >= 4
+
+
+@pytest.mark.parametrize("M", [64, 65, 128, 129])
+@pytest.mark.parametrize("N", [48896, 49152, 65536, 65792])
+def test_lm_heads_of_65_to_128_rows(M, N):
+    """``linear`` and ``logits32`` on both sides of the row counts and widths at which the tile GEMM takes over."""
+    x, w = _rand(M, 256, seed=26, scale=0.5), _rand(N, 256, seed=27, scale=0.05)
+    y = x.double() @ w.double().t()
+    slack = 256 * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())  # fp32 sums; bf16 results round once
+    assert bool(((hip.linear(x, w).double() - y).abs() <= 2.0 ** -8 * y.abs() + slack).all())
+    got = hip.logits32(x, w)
+    assert got.dtype == torch.float32 and bool(((got.double() - y).abs() <= slack).all())
