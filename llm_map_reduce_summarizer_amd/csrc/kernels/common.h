@@ -100,14 +100,6 @@ __device__ __forceinline__ float glu(float g, float u, const GluArgs& a) {
     u = fminf(fmaxf(u, -a.limit), a.limit);
     return g / (1.f + __expf(-a.alpha * g)) * (u + a.shift);
 }
-// The same for values that leave as 16-bit in kernels that the division's dozen instructions cost: the hardware reciprocal
-// (1 ulp), of the denominator times 2^-32, whose reciprocal is a normal number for every finite exponential.
-__device__ __forceinline__ float glu16(float g, float u, const GluArgs& a) {
-    g = fminf(g, a.limit);
-    u = fminf(fmaxf(u, -a.limit), a.limit);
-    const float r = __builtin_amdgcn_rcpf(fmaf(__expf(-a.alpha * g), 0x1p-32f, 0x1p-32f));
-    return g * 0x1p-32f * r * (u + a.shift);
-}
 
 // Attention output form: head h of row t goes to columns [h * pitch, (h + 1) * pitch) of the row, times
 // gate[t * gate_ld + h] when a gate is given.

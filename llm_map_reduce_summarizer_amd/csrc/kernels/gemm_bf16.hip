@@ -238,11 +238,13 @@ struct Lane {
 };
 
 // The outputs of column group q from a row block's accumulators v[j] (W block j).
+// GLU divides: the hardware reciprocal is 1 - 2 % of the kernel faster (18234 x 28672 x 4096 2954 -> 2900 us, 305 rows 69.8 ->
+// 69.0) but a bit less exact, and scaled to reach every exponential it loses the bits of gates under 2^-94.
 template <int EPI>
 __device__ __forceinline__ void outputs(const f32x4 (&v)[8], int q, const GluArgs& ga, float (&o)[8]) {
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
-        if constexpr (EPI == GEPI_SWIGLU) o[r] = glu16(v[4 * q + (r >> 2)][r & 3], v[4 * q + 2 + (r >> 2)][r & 3], ga);
+        if constexpr (EPI == GEPI_SWIGLU) o[r] = glu(v[4 * q + (r >> 2)][r & 3], v[4 * q + 2 + (r >> 2)][r & 3], ga);
         else o[r] = v[2 * q + (r >> 2)][r & 3];
         if constexpr (EPI == GEPI_GELU) o[r] = gelu_tanh<bf16>(o[r]);
     }

@@ -255,6 +255,21 @@ def test_gemm_swiglu_small_gates(K):
     assert bool(((out - want).abs() <= 2.0 ** -8 * want.abs()).all())
 
 
+@pytest.mark.parametrize("K", [64, 2048])
+@pytest.mark.parametrize("up", [2.0 ** 100, 1.0])
+def test_gemm_swiglu_tiny_gates(K, up):
+    """Gates of 2^-90 to 2^-126, whose half is the product with sigmoid(gate) = 1/2, in one launch (K 64) and in slices of K
+    (2048): exact in fp32 down to the smallest normal number, and no scaling on the way may lose bits of it."""
+    assert (hip.gemm_splits(8, 32, K // 64)[1] > 1) == (K == 2048)
+    gate = torch.tensor([s * f * 2.0 ** -e for e in (90, 100, 110, 125) for s, f in ((1, 1.0), (-1, 1.9921875))], dtype=torch.float64)
+    x, w = torch.zeros(8, K, dtype=torch.bfloat16), torch.zeros(32, K, dtype=torch.bfloat16)
+    x[range(8), range(8)] = 1
+    w[:, :8] = torch.where(torch.arange(32)[:, None] % 16 < 8, gate, torch.tensor(up, dtype=torch.float64))
+    out = hip.gemm(x.to(DEV), w.to(DEV), swiglu=True).cpu().double()
+    # gate, up and half their product have 8 bits: nothing rounds
+    assert torch.equal(out, (gate / 2 * up)[:, None].expand(8, 16))
+
+
 @pytest.mark.parametrize("M", [128, 129, 256, 257])
 def test_stream_parts_beyond_tall_tiles(M):
     """linear_parts gives the slabs it is asked for at any row count; consumers that add however many there are get one
