@@ -285,6 +285,7 @@ MRSUM_API int mrsum_gemm32(const float* x, int ldx, const float* w, int ldw, flo
     if (K % 32 || ldx % 4 || ldw % 4 || (uintptr_t)x % 16 || (uintptr_t)w % 16 || (size_t)T32 * ldx * 4 >= (1u << 31) ||
         (size_t)T32 * ldw * 4 >= (1u << 31))
         return (int)hipErrorInvalidValue;
+    if (splits && K < 32) return (int)hipErrorInvalidValue;  // the tiles ask for their first K-tiles ahead
     if (splits == 0) {
         if (ceil_div(M, TS) > 65535) return (int)hipErrorInvalidValue;
         gemm32_small_kernel<<<dim3(ceil_div(N, TS), ceil_div(M, TS)), 256, 0, s>>>(x, ldx, w, ldw, c, ldc, M, N, K);

@@ -162,6 +162,12 @@ def test_fp32_gemm_of_short_k(M, N, K, small):
     assert hip.gemm32_small(M, N, K // 32) == small
 
 
+def test_fp32_tiles_refuse_an_empty_k():
+    """The tiles ask for their first K-tile before they look whether there is one; the entry point refuses K 0 on the host."""
+    invalid = 1  # hipErrorInvalidValue
+    assert hip._fn("mrsum_gemm32")(None, 0, None, 0, None, 16, 4, 16, 0, 0, 1, None, None) == invalid
+
+
 def c_parameters():
     """Entry point -> number of its parameters, from the kernels' sources."""
     found = {}

@@ -508,6 +508,13 @@ def test_gemm32_row_blocks(M, N, K, monkeypatch):
     assert got.shape == (M, N) and bool(((got - x.double() @ w.double().T).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("M", [0, 4, 64, 65])
+def test_gemm32_of_empty_k(M):
+    from llm_map_reduce_summarizer_amd.ops import hip
+    got = hip.gemm32(dev(torch.zeros(M, 0)), dev(torch.zeros(130, 0)))
+    assert got.shape == (M, 130) and bool((got == 0).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(65, 16, 32), (64, 130, 192), (33, 65, 288), (257, 1, 128), (520, 8192, 192), (300, 1023, 512)])
 def test_gemm32_short_k(M, N, K):
     """The 64 x 64 tiles: rows and columns past the last tile, against 64 bits; the larger tiles give the same up to rounding."""
