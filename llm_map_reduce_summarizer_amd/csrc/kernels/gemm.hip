@@ -430,7 +430,8 @@ MRSUM_API int mrsum_gemm_stamps(unsigned long long* host, int max_words) {
 // sx [M] / sw [N] fp32 row scales; split: x is two-term [hi | lo] of 2K bytes per row over w's K.
 // whole / splits / part: tiles from raster position ``whole`` on run in ``splits`` slices of K through ``part``
 // [tiles - whole][splits][rows * 256] fp32 (splits 1: none, part unused;
-// 16x16 MFMA tiles only).  group_m bits 9 - 12: rows of a tile / 32 (0: 256; bf16 also 128, 160, 192, 224).  slabs (epi 3, whole 0): the slices stay apart, in part [splits][M][N]; c unused.
+// 16x16 MFMA tiles only).  group_m bits 9 - 12: rows of a tile / 32 (0: 256; bf16 also 128, 160, 192, 224).  slabs (epi 3,
+// whole 0): the slices stay apart, in part [splits][M][N]; c unused.
 // Requirements (checked by the Python wrapper too): K % 64 and K > 0 (bf16) / K % 128 (fp8), N % 16, 16-byte
 // aligned rows.
 MRSUM_API int mrsum_gemm(const void* x, int ldx, const void* w, int ldw, void* c, int ldc, int M, int N, int K,
@@ -456,7 +457,7 @@ MRSUM_API int mrsum_gemm(const void* x, int ldx, const void* w, int ldw, void* c
     if (split) a.kb *= 2;  // X K-tiles: hi then lo
     a.rows = rows;
     a.tiles_m = ceil_div(M, rows); a.tiles_n = ceil_div(N, 256);
-    // group_m bits 0-7: tile rows per raster group (0 = 4); bit 8 (fp8): 32x32 MFMA tiles instead of 16x16.
+    // group_m bits 0-7: tile rows per raster group (0 = 4); bit 8: fp8 on 32x32 MFMA tiles instead of 16x16 (bf16 has one form).
     // Measured (profiles/r3_gemm_mfma32_experiment.jsonl, same box, interleaved): 32x32 is
     // about equal on the 70B fp8 qkv / o / down, so 16x16 stays the default;
     // the gate_up + SwiGLU GEMM gains 1.7-3.8 % at M = 4k-32k and takes it (ops/hip.py gemm_fp8).

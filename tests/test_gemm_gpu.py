@@ -104,8 +104,8 @@ def test_gemm_fp8(M, N, K, swiglu):
 @pytest.mark.parametrize("swiglu", [False, True])
 @pytest.mark.parametrize("aligned", [True, False])
 def test_gemm_mfma32_variant(fp8, swiglu, aligned):
-    """The 32x32-MFMA tile variant (group_m bit 8; measured slower for bf16, not the default --
-    profiles/r3_gemm_mfma32_experiment.jsonl) against fp32, ragged M and an N % 32 == 16 tail."""
+    """The 32x32-MFMA tile variant (group_m bit 8) of the 8-bit GEMM against fp32, ragged M and an N % 32 == 16 tail; bf16 has one
+    form of tile and gives the bits of a call without it."""
     M, N, K = 777, 1040 if not swiglu else 1056, 1024
     x = _rand(M, K, seed=10, scale=0.5, offset=0.02)
     wb = _rand(N, K, seed=11, scale=0.03, offset=0.001)
@@ -119,6 +119,7 @@ def test_gemm_mfma32_variant(fp8, swiglu, aligned):
         y = (xq.float() * xs[:, None]) @ w.dequant().t()
     else:
         hip.gemm(x, wb, out=out, swiglu=swiglu, group_m=4 | 256)
+        assert torch.equal(out, hip.gemm(x, wb, swiglu=swiglu, group_m=4))
         y = x.float() @ wb.float().t()
     torch.cuda.synchronize()
     if swiglu:

@@ -195,6 +195,21 @@ def test_gemm_clock_passes_what_the_gemm_takes():
     assert args[15:] == [float("inf"), 1.0, 0.0, 0, 1, None, 0, 99]
 
 
+@pytest.mark.parametrize("group_m", [None, 4, 4 | 256, 4 | 512, 255 << 9, -1])
+def test_tile_rows_are_those_of_the_plan(group_m, monkeypatch):
+    """The caller's raster choice shares a word with the tile's rows, which the scratch of the slices is sized for."""
+    M, N, K = 305, 4096, 4096
+    whole, splits, room, rows = hip.gemm_splits(M, N, K // 64)
+    assert splits > 1 and rows < 256
+    passed = []
+    monkeypatch.setattr(hip, "_fn", lambda name: lambda *a: passed.append(a) or 0)
+    monkeypatch.setattr(hip, "_stream", lambda: 0)
+    hip._gemm(None, K, None, K, torch.zeros(M, N, dtype=torch.bfloat16), M, N, K, 0, hip.GEMM_EPI_BF16, None, None, group_m)
+    word = passed[0][13]
+    assert word >> 9 == rows // 32 and word & 511 == (4 if group_m is None else group_m) & 511
+    assert passed[0][18:20] == (whole, splits)
+
+
 @pytest.mark.parametrize("lens", [[1], [300, 64], [0, 65, 4096, 4096, 1, 700], [64] * 40])
 def test_block_items_of_few_and_many_blocks(lens):
     """Work lists built from tuples (few blocks) and from arrays are the same list: latest blocks first, then by sequence."""

@@ -3,6 +3,7 @@
 group_m bit 8 of mrsum_gemm) vs the 16x16 tiles.  First a numerics check of the 32x32 variant against fp32
 (bf16 / fp8, plain / SwiGLU, ragged M, N % 32 == 16, strided output for the register epilogue), then an
 interleaved timing A/B in one process.  One JSON line per check / (shape, variant).
+The bf16 GEMM has one form of tile by now and ignores the bit: its lines time the same kernel twice.
 
     python tools/exp_gemm_m32.py [--ms 4096,16384] [--fp8-model llama3-70b]
 """

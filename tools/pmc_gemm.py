@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """A few prefill GEMM launches for rocprofv3 --pmc passes (tools/gpu_r3_pmc_gemm.sh): Llama-3-8B o
 (4096 x 4096) and gate_up + SwiGLU (28672 x 4096) at M = 16384 in bf16, each on the 16x16 and the 32x32
-MFMA tiles, and the 70B fp8 gate_up + SwiGLU at M = 8192 on both tile shapes."""
+MFMA tiles (bf16 by now has one form and runs it twice), and the 70B fp8 gate_up + SwiGLU at M = 8192 on both tile shapes."""
 import os
 import sys
 
