@@ -21,7 +21,7 @@
 //     was and the first half of W(t + 3), which goes where W(t) was; its second half is asked for in step 0 of t + 1.  W,
 //     which comes from further away where rows are few, has one and a half K-tiles to arrive, X one (of few rows two).
 //     Requests two K-tiles ahead in a common ring of five images left the last of W half a K-tile: 305 x 28672 x 4096
-//     91 us, 80 in tiles of 160 rows; so 87 and 72, and W past the caches (nt, up to 192 rows: no other round reads it) 70.
+//     91 us, 80 in tiles of 160 rows; so 87 and 72, and W past the caches (nt, where no other round reads it) 70.
 //   * the workgroups stay for all their tiles, and the requests run on into the next tile (or slice of K), whose first
 //     K-tiles arrive while the epilogue runs.  The epilogue keeps out of LDS for that: W's rows are dealt to the MFMA
 //     rows so that a lane ends with 8 consecutive output columns (gate and up of the same columns for GLU) of a row, one
@@ -109,17 +109,24 @@ constexpr int WGS = 256;          // one workgroup per CU
 // step 1 asks for X and the first half of W, step 0 of the next K-tile for W's second half
 #define ASK1_8 DX(0), DX(1), DX(2), DX(3), DX(4), DX(5), DX(6), DXL(7), DW(0), DW(1), DW(2), DW(3)
 #define ASK1_7 DX(0), DX(1), DX(2), DX(3), DX(4), DX(5), DXL(6), DW(0), DW(1), DW(2), DW(3),
-#define ASK1_6 DX(0), DX(1), DX(2), DX(3), DX(4), DXL(5), DWN(0), DWN(1), DWN(2), DWN(3), ,
-#define ASK1_5 DX(0), DX(1), DX(2), DX(3), DXL(4), DWN(0), DWN(1), DWN(2), DWN(3), , ,
-#define ASK1_4 DX(0), DX(1), DX(2), DXL(3), DWN(0), DWN(1), DWN(2), DWN(3), , , ,
+#define ASK1_6 DX(0), DX(1), DX(2), DX(3), DX(4), DXL(5), DW(0), DW(1), DW(2), DW(3), ,
+#define ASK1_5 DX(0), DX(1), DX(2), DX(3), DXL(4), DW(0), DW(1), DW(2), DW(3), , ,
+#define ASK1_4 DX(0), DX(1), DX(2), DXL(3), DW(0), DW(1), DW(2), DW(3), , , ,
 #define ASK0_8 , DW(4), , DW(5), , DW(6), , DW(7), , , ,
 #define ASK0_7 ASK0_8
-#define ASK0_6 , DWN(4), , DWN(5), , DWN(6), , DWN(7), , , ,
-#define ASK0_5 ASK0_6
-#define ASK0_4 ASK0_6
+#define ASK0_6 ASK0_8
+#define ASK0_5 ASK0_8
+#define ASK0_4 ASK0_8
+// with W past the caches
+#define ASK1_6N DX(0), DX(1), DX(2), DX(3), DX(4), DXL(5), DWN(0), DWN(1), DWN(2), DWN(3), ,
+#define ASK1_5N DX(0), DX(1), DX(2), DX(3), DXL(4), DWN(0), DWN(1), DWN(2), DWN(3), , ,
+#define ASK1_4N DX(0), DX(1), DX(2), DXL(3), DWN(0), DWN(1), DWN(2), DWN(3), , , ,
+#define ASK0_6N , DWN(4), , DWN(5), , DWN(6), , DWN(7), , , ,
+#define ASK0_5N ASK0_6N
+#define ASK0_4N ASK0_6N
 #define EXPAND(...) __VA_ARGS__
-#define STEP0(NB, M, off) READ_AT("xlo1", "wlo1") "s_add_u32 m0, %[tw], %[ldsw4]\n" EXPAND(STEP_##NB EXPAND((M, 0, 1, off, ASK0_##NB)))
-#define STEP1(NB, off) READ_AT("xlo0", "wlo0") "s_add_u32 m0, %[tx], %[ldsx]\n" EXPAND(STEP_##NB EXPAND((MF, 1, 0, off, ASK1_##NB)))
+#define STEP0(NB, ASK, M, off) READ_AT("xlo1", "wlo1") "s_add_u32 m0, %[tw], %[ldsw4]\n" EXPAND(STEP_##NB EXPAND((M, 0, 1, off, ASK0_##ASK)))
+#define STEP1(NB, ASK, off) READ_AT("xlo0", "wlo0") "s_add_u32 m0, %[tx], %[ldsx]\n" EXPAND(STEP_##NB EXPAND((MF, 1, 0, off, ASK1_##ASK)))
 #define READ_X_4 RX(0, 0) RX(0, 1) RX(0, 2) RX(0, 3)
 #define READ_X_5 READ_X_4 RX(0, 4)
 #define READ_X_6 READ_X_5 RX(0, 5)
@@ -130,20 +137,20 @@ constexpr int WGS = 256;          // one workgroup per CU
     "s_cmp_lg_u32 %[" k "], %[" ke "]\ns_cbranch_scc1 " label "f\n"                         \
     "s_mov_b64 " r0 ", " n0 "\ns_mov_b64 " r1 ", " n1 "\n"                                  \
     "s_mov_b32 %[" k "], %[k0n]\ns_mov_b32 %[" ke "], %[ken]\n" label ":\n"
-#define K_LOOP(NB, off)                                                                     \
+#define K_LOOP(NB, ASK, off)                                                                \
     "s_barrier\n" READ_AT("xlo0", "wlo0") READ_X_##NB                                       \
     RW(0, 0, off) RW(0, 1, off) RW(0, 2, off) RW(0, 3, off)                                 \
     RW(0, 4, off) RW(0, 5, off) RW(0, 6, off) RW(0, 7, off)                                 \
-    "s_waitcnt lgkmcnt(0)\n" STEP0(NB, MZ, off)                                             \
+    "s_waitcnt lgkmcnt(0)\n" STEP0(NB, ASK, MZ, off)                                        \
     "s_waitcnt vmcnt(%[w0]) lgkmcnt(0)\ns_branch 2f\n"                                      \
-    "1:\ns_waitcnt lgkmcnt(0)\n" STEP0(NB, MF, off)                                         \
+    "1:\ns_waitcnt lgkmcnt(0)\n" STEP0(NB, ASK, MF, off)                                    \
     "s_waitcnt vmcnt(%[w1]) lgkmcnt(0)\n2:\ns_barrier\n"                                    \
     "s_mov_b32 %[tx], %[sx]\ns_mov_b32 %[tw], %[sw]\n"                                      \
     NEXT("sx", "%[xi]", "%[xe]") NEXT("sw", "0x8000", "0x18000")                            \
     "s_add_u32 %[kw], %[kw], 0x80\n"                                                        \
     FOLLOW("kx", "kex", "s[64:65]", "s[66:67]", "s[72:73]", "s[74:75]", "3")                \
     FOLLOW("kw", "kew", "s[68:69]", "s[70:71]", "s[76:77]", "s[78:79]", "4")                \
-    STEP1(NB, off)                                                                          \
+    STEP1(NB, ASK, off)                                                                     \
     "s_add_u32 %[kx], %[kx], 0x80\ns_sub_u32 %[n], %[n], 1\ns_cmp_lg_u32 %[n], 0\n"         \
     "s_cbranch_scc1 1b\ns_waitcnt lgkmcnt(0)\ns_nop 15\n"
 // the W row of MFMA row a = lane & 15 of block j is OFF(j) + (8 or 16) (a >> 2) + (a & 3)
@@ -275,8 +282,8 @@ __device__ __forceinline__ void store_rows(const GemmArgs& a, const Lane<NB>& l,
 }  // namespace
 
 // WIDE: rows of C are 16-byte aligned and 256 of them stay below 2 GiB, so that a whole tile leaves through a buffer
-// descriptor in a fixed number of 16-byte stores, which the next tile's first wait can count past.
-template <int EPI, bool WIDE, int NB>
+// descriptor in a fixed number of 16-byte stores, which the next tile's first wait can count past.  NT: W past the caches.
+template <int EPI, bool WIDE, int NB, bool NT>
 __global__ __launch_bounds__(256, 1) void gemm_bf16_kernel(const GemmArgs a) {
     static_assert(!(WIDE && EPI == GEPI_F32), "fp32 rows leave by store_rows");
 #ifdef MRSUM_CLOCK_STAMPS
@@ -366,12 +373,13 @@ __global__ __launch_bounds__(256, 1) void gemm_bf16_kernel(const GemmArgs a) {
       [vw1] "v"(vw[1]), [vw2] "v"(vw[2]), [vw3] "v"(vw[3]), [vw4] "v"(vw[4]), [vw5] "v"(vw[5]), [vw6] "v"(vw[6]),     \
       [vw7] "v"(vw[7])                                                                                                \
     : CLOBBERS
-#define RUN_K(NB_)                                                                        \
-    if constexpr (NB == NB_) {                                                            \
-        if constexpr (GLU) asm volatile(K_LOOP(NB_, OFF_GLU) K_LOOP_OPERANDS(NB_));       \
-        else asm volatile(K_LOOP(NB_, OFF_ROWS) K_LOOP_OPERANDS(NB_));                    \
+#define RUN_K(NB_, ASK, NT_)                                                              \
+    if constexpr (NB == NB_ && NT == NT_) {                                               \
+        if constexpr (GLU) asm volatile(K_LOOP(NB_, ASK, OFF_GLU) K_LOOP_OPERANDS(NB_));  \
+        else asm volatile(K_LOOP(NB_, ASK, OFF_ROWS) K_LOOP_OPERANDS(NB_));               \
     }
-            RUN_K(4) RUN_K(5) RUN_K(6) RUN_K(7) RUN_K(8)
+            RUN_K(4, 4N, true) RUN_K(5, 5N, true) RUN_K(6, 6N, true)
+            RUN_K(4, 4, false) RUN_K(5, 5, false) RUN_K(6, 6, false) RUN_K(7, 7, false) RUN_K(8, 8, false)
         }
 
         const Lane<NB> l = {t.m0, t.n0, wr, wc, lane & 15, lane >> 4};
@@ -495,25 +503,36 @@ int gemm_bf16_grid(const GemmArgs& a) {
     return a.kb / a.splits < 3 ? nu : std::min(nu, WGS);
 }
 
-template <int NB>
-static void launch_rows(const GemmArgs& a, int epi, hipStream_t s) {
+template <int NB, bool NT>
+static void launch_form(const GemmArgs& a, int epi, hipStream_t s) {
     const dim3 grid(gemm_bf16_grid(a));
     const int rest = a.tiles_m * a.tiles_n - a.whole;
     const bool wide = a.ldc % 8 == 0 && (uintptr_t)a.c % 16 == 0 && (size_t)256 * a.ldc * 2 < (1u << 31);
 #define GEMM_LAUNCH(E)                                                                \
     {                                                                                 \
-        if (wide) gemm_bf16_kernel<E, true, NB><<<grid, 256, 0, s>>>(a);              \
-        else gemm_bf16_kernel<E, false, NB><<<grid, 256, 0, s>>>(a);                  \
+        if (wide) gemm_bf16_kernel<E, true, NB, NT><<<grid, 256, 0, s>>>(a);          \
+        else gemm_bf16_kernel<E, false, NB, NT><<<grid, 256, 0, s>>>(a);              \
         if (rest) gemm_bf16_tail_kernel<E, NB><<<rest * NB, 256, 0, s>>>(a);          \
     }
     if (epi == GEPI_SWIGLU) GEMM_LAUNCH(GEPI_SWIGLU)
     else if (epi == GEPI_GELU) GEMM_LAUNCH(GEPI_GELU)
     else if (epi == GEPI_BF16) GEMM_LAUNCH(GEPI_BF16)
     else {
-        gemm_bf16_kernel<GEPI_F32, false, NB><<<grid, 256, 0, s>>>(a);
+        gemm_bf16_kernel<GEPI_F32, false, NB, NT><<<grid, 256, 0, s>>>(a);
         if (rest && !a.slabs) gemm_bf16_tail_kernel<GEPI_F32, NB><<<rest * NB, 256, 0, s>>>(a);
     }
 #undef GEMM_LAUNCH
+}
+
+// W of up to 192 rows goes past the caches where all row tiles of a column are neighbours in the raster, so that no later
+// round reads it again.  us, through the caches -> past them: 305 x 24576 x 4096 (2 row tiles) 67.6 -> 64.2, 600 x 8192 x 4096
+// (4) 47.4 -> 46.5; but 903 x 24576 x 4096 (5) 149 -> 156, 903 x 8192 x 4096 (8) 57 -> 63, 1300 x 6144 x 4096 (9) 61 -> 68, 4096 x
+// 2176 x 4096 (26) 61 -> 70.
+template <int NB>
+static void launch_rows(const GemmArgs& a, int epi, hipStream_t s) {
+    if constexpr (NB <= 6)
+        if (a.tiles_m <= a.group_m) return launch_form<NB, true>(a, epi, s);
+    launch_form<NB, false>(a, epi, s);
 }
 
 void gemm_bf16_launch(const GemmArgs& a, int epi, hipStream_t s) {
