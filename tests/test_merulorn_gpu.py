@@ -508,6 +508,20 @@ def test_gemm32_row_blocks(M, N, K, monkeypatch):
     assert got.shape == (M, N) and bool(((got - x.double() @ w.double().T).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("M,N,K", [(3, 130, 22528), (72, 130, 22528), (128, 130, 22528), (70, 1030, 6144)])
+def test_gemm32_error_does_not_grow_with_k(M, N, K, monkeypatch):
+    """One workgroup adds all of K in chains of 512 products and less, however long K is."""
+    from llm_map_reduce_summarizer_amd.ops import hip
+    monkeypatch.setattr(hip, "gemm32_small", lambda *_: False)
+    monkeypatch.setattr(hip, "gemm32_splits", lambda M, N, kb: (-(-M // 128) * -(-N // 128), 1, 0))
+    x, w = rnd(M, K, seed=1), rnd(N, K, seed=2)
+    y = x.double() @ w.double().T
+    err = (hip.gemm32(dev(x), dev(w)).double().cpu() - y).norm() / y.norm()
+    # a chain's i-th sum has the size of i of its products and rounds by at most 2^-24 of that, with random signs: sqrt(n / 2) 2^-24
+    # of the chain's sum for n products; the sums of the chains in the same way
+    assert err <= ((512 + K / 256) / 2) ** 0.5 * 2.0 ** -24
+
+
 @pytest.mark.parametrize("M", [0, 4, 64, 65])
 def test_gemm32_of_empty_k(M):
     from llm_map_reduce_summarizer_amd.ops import hip
