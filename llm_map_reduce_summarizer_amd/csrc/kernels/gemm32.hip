@@ -182,7 +182,9 @@ __global__ __launch_bounds__(256, 2) void gemm32_kernel(const Gemm32Args a) {
         p = xcd_position(p, a.whole);
     } else {
         const int rest = a.tiles_m * a.tiles_n - a.whole;
-        p = xcd_position(p - a.whole, rest * a.splits);
+        // short K: the slices of a tile on different XCDs.  us, one range of K to an XCD -> this: 508 x 2048 x 768 28.7 -> 25.4, 256 x
+        // 4096 x 768 28.6 -> 25.9, 903 x 2048 x 512 31.9 -> 28.1; at K 1536 it costs up to 7 % (400 x 4096: 52 -> 56)
+        p = a.kb > 32 ? xcd_position(p - a.whole, rest * a.splits) : p - a.whole;
         slice = p / rest;
         p += a.whole - slice * rest;
         kt0 = a.kb * slice / a.splits;
