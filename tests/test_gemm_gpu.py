@@ -147,7 +147,7 @@ def test_gemm_graph_capture():
 @pytest.mark.parametrize("epi", ["bf16", "swiglu", "gelu", "f32"])
 def test_gemm_split_tail(M, N, K, epi):
     """Tiles behind the last whole round run in slices of K that a second launch adds: one tile of one row, a ragged
-    last slice, few tiles, 16 sliced tiles behind a whole round, and two rounds of thirds; repeated calls are the same bits."""
+    last slice, few tiles, some sliced tiles behind a whole round, and two rounds of thirds; repeated calls are the same bits."""
     assert hip.gemm_splits(M, N, K // 64)[1] > 1
     x, w = _rand(M, K, seed=12, scale=0.5, offset=0.02), _rand(N, K, seed=13, scale=0.03, offset=0.001)
     if epi == "swiglu":
@@ -203,12 +203,14 @@ def test_gemm_tile_after_tile(K, epi, off):
 def test_gemm_fp8_split_tail(M, N, K, two, swiglu):
     """The 8-bit product in slices of K, row and column scales behind the added slices; a slice border inside the low term of
     two-term rows and between the terms."""
-    assert hip.gemm_splits(M, N, (2 if two else 1) * K // 128)[1] > 1
     g = torch.Generator().manual_seed(18)
     f8 = lambda *s: (torch.randn(*s, generator=g) * 8).to(torch.float8_e4m3fn)  # noqa: E731
     xq, w = f8(M, (2 if two else 1) * K), Fp8Weight(f8(N, K).to(DEV), (torch.rand(N, generator=g) / 64 + 1 / 64).to(DEV))
     xs = (torch.rand(M, generator=g) + 0.5) / K ** 0.5 / 8
     n0 = N // 32 * 32 if swiglu else N
+    kb = (2 if two else 1) * K // 128
+    splits = hip.gemm_splits_fp8(M, n0, kb)[1]
+    assert splits > 1 and (not two or any(kb // 2 < kb * i // splits for i in range(splits)))
     w = Fp8Weight(w.q[:n0].contiguous(), w.scale[:n0].contiguous())
     out = hip.gemm_fp8(xq.to(DEV), xs.to(DEV), w, swiglu=swiglu, group_m=hip.GEMM_GROUP_M)
     assert torch.equal(out, hip.gemm_fp8(xq.to(DEV), xs.to(DEV), w, swiglu=swiglu, group_m=hip.GEMM_GROUP_M))
