@@ -546,19 +546,19 @@ void gemm_bf16_launch(const GemmArgs& a, int epi, hipStream_t s) {
 }
 
 // Rows of a tile, raster position from which tiles run in slices of K, and the slices (1: none do) of an M x N product of kb
-// K-tiles: the cheapest by a model of the kernel, fitted to all row counts and slices of 14 shapes (N 1536 - 28672, K 512 -
-// 22528) at 23 row counts from 130 to 7615, of which it loses 1.5 % on average.  256 rows at their best slices are 9 %
-// slower on average: M 305, N 28672, K 4096 86 us (160 rows: 71), M 1967, N 4096, K 4096 68 (128: 55); at M 130 - 1000 the gain
-// is 5 - 20 %, from 4000 rows on nothing.
+// K-tiles: the cheapest by a model of the kernel, fitted to 21 shapes (N 1024 - 28672, K 512 - 22528) at 47 row counts from 3 to
+// 7615.  There and at 6 other shapes it loses 1 % on average against the best height and slices, 20 % at most (200 x 28672 x 4096
+// with GLU: 72 us in 224 rows and two slices, 60 in 128 whole).  256 rows at their best slices are 17 % slower on average at M 130 -
+// 1000, 11 % up to 4000 and 4 % beyond: M 305, N 28672, K 4096 91 us (160 rows: 67), M 1967, N 4096, K 4096 68 (128: 56).
 MRSUM_API int mrsum_gemm_plan(int M, int N, int kb, int* out) {
     // us a K-tile: few workgroups at work, and all CUs (the clock that power allows, and what all ask of memory)
-    struct Height { int rows; float alone, full; };
-    static constexpr Height H[5] = {{256, .99f, 1.38f}, {224, .88f, 1.23f}, {192, .82f, 1.15f}, {160, .78f, 1.02f}, {128, .72f, .92f}};
+    struct Height { int rows; float few, full; };
+    static constexpr Height H[5] = {{256, .962f, 1.294f}, {224, .928f, 1.157f}, {192, .867f, 1.059f}, {160, .783f, .958f}, {128, .472f, .884f}};
     const int tn = ceil_div(N, 256);
     float best = INFINITY;
     for (const Height& h : H) {
         const int tm = ceil_div(M, h.rows), tiles = tm * tn, rest = tiles % WGS;
-        const float epilogue = 3.9f * h.rows / 256;
+        const float epilogue = 3.13f * h.rows / 256;
         // slices below 32 K-tiles: a whole loop is as short as the second launch, and a row's sum the same whichever rows
         // run with it.  They fill one round, or two with up to three a tile.
         const int most = kb < 32 || !rest ? 1 : std::min(std::max(WGS / rest, std::min(3, 2 * WGS / rest)), kb / 4);
@@ -566,10 +566,13 @@ MRSUM_API int mrsum_gemm_plan(int M, int N, int kb, int* out) {
             const float ks = (float)kb / s;
             const int n = rest * s, last = n % WGS;
             float t = (tiles / WGS) * (kb * h.full + epilogue) + (n / WGS) * (ks * h.full + epilogue);
-            if (last) t += ks * (h.alone + (h.full - h.alone) * std::max(0.f, last / (float)WGS - .21f) / .79f) + epilogue;
+            const float load = last ? last / (float)WGS : 1.f;
+            if (last) t += ks * (h.few + (h.full - h.few) * load) + epilogue;
+            // a round of stores on the last CUs: 903 x 8192 x 512 17.6 us, 13.0 in 192 tiles
+            if (s == 1) t += 7.1f * std::max(0.f, load - .764f);
             if (s > 1) {  // the second launch, and accumulators written and read again: dearer beyond what the L2s hold
                 const float mb = (float)n * (16 * ceil_div(M, 16)) / tm * 1024e-6f;
-                t += 1.3f + .62f * s + .167f * mb + .13f * std::max(0.f, mb - 29.5f);
+                t += 3.4f + .44f * s + .12f * mb + .178f * std::max(0.f, mb - 28.7f);
             }
             if (t < best) {
                 best = t;

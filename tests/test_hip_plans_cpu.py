@@ -177,6 +177,19 @@ def recorded(name):
         return [json.loads(line) for line in f if not line.startswith("#")]
 
 
+def test_tile_gemm_plan_by_its_record():
+    """What the rule takes was timed, is what the record says, and is near the best of each shape: 20 % at most, 1 % on average
+    (whether or not the rule was fitted to the shape)."""
+    losses = {True: [], False: []}
+    for e in recorded("gemm_rows.jsonl"):
+        _, splits, _, rows = hip.gemm_splits(e["M"], e["N"], e["K"] // 64)
+        took = "%d/%d" % (rows, splits)
+        assert took == e["rule"] and took in e["us"], e
+        losses[e["fit"]].append(e["us"][took] / min(e["us"].values()) - 1)
+        assert losses[e["fit"]][-1] <= 0.2, e
+    assert len(losses[True]) > 400 and len(losses[False]) > 100 and all(sum(v) / len(v) <= 0.012 for v in losses.values())
+
+
 def test_fp32_gemm_slices_by_their_record():
     """What the rule takes was timed, is what the record says, and is near the best of each shape: 12 % at most (16 rows of 4096 x
     22528, whose slices are bound by reads that the rule does not tell apart), 1 % on average."""
