@@ -715,10 +715,12 @@ MRSUM_API int mrsum_delta_chunk(const void* x, int ldx, int xk, int xv, const vo
         return (int)hipErrorInvalidValue;
     const DeltaArgs a{ProjSrc{u, S, (size_t)T * ld, ld}, b_at, a_at, 0, dt_bias, a_neg, nullptr, 0.f,
                       1.f / sqrtf((float)N), ldx, xk, xv, 0, 0, 0, heads, kv_heads, P, N, N};
-    // the heads of a key head one after the other share its dot products; while all of them fit the chip at once (four blocks a
-    // CU), a block each is over sooner: 16 key heads of 2, us, 2 chunks 17.2 -> 11.9, 12 chunks 17.5 -> 13.1, 32 chunks 22.7 -> 18.5
-    const int rep = heads / kv_heads;
-    const dim3 g1(kv_heads, n_chunks, (long long)heads * n_chunks <= 1024 ? rep : 1), g2(heads, ceil_div(P, 16 * wpb), n_segs);
+    // The heads of a key head one after the other share its dot products; while all of them fit the chip at once (four blocks a
+    // CU), a block each is over sooner.  16 key heads of 2, N 128, us, 2 chunks 16.0 -> 10.5, 32 chunks 21.1 -> 18.6, but 40 chunks
+    // 24.2 -> 25.3.  Of N above 128 a CU takes two: 16 chunks 21.1 -> 17.4, 20 chunks 22.9 -> 26.2; with four heads to a key head
+    // two rounds of blocks still lead: 8 key heads, 20 chunks 30.6 -> 25.2, 32 chunks 31.3 -> 28.9, but 40 chunks 35.2 -> 39.7.
+    const int rep = heads / kv_heads, most = N > 128 ? std::min(256 * rep, 1024) : 1024;
+    const dim3 g1(kv_heads, n_chunks, (long long)heads * n_chunks <= most ? rep : 1), g2(heads, ceil_div(P, 16 * wpb), n_segs);
 #define DC_P(NB_, W_)                                                                                                     \
     delta_chunk_pair_kernel<NB_, W_><<<g2, 128 * W_, 0, s>>>((const bf16*)x, a, (const int4*)segs, slots, pos0,              \
                                                             (const uint4*)frags, vec, state, y, y0)

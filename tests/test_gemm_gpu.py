@@ -147,7 +147,7 @@ def test_gemm_graph_capture():
 @pytest.mark.parametrize("epi", ["bf16", "swiglu", "gelu", "f32"])
 def test_gemm_split_tail(M, N, K, epi):
     """Tiles behind the last whole round run in slices of K that a second launch adds: one tile of one row, a ragged
-    last slice, few tiles, some sliced tiles behind a whole round, and two rounds of thirds; repeated calls are the same bits."""
+    last slice, few tiles, 16 sliced tiles behind a whole round, and two rounds of thirds; repeated calls are the same bits."""
     assert hip.gemm_splits(M, N, K // 64)[1] > 1
     x, w = _rand(M, K, seed=12, scale=0.5, offset=0.02), _rand(N, K, seed=13, scale=0.03, offset=0.001)
     if epi == "swiglu":

@@ -322,6 +322,33 @@ def test_delta_chunks_in_grids_of_both_kinds():
     assert torch.equal(a, torch.cat((b, c))) and torch.equal(s, torch.cat((t, v))) and bool(a.float().abs().sum() > 0)
 
 
+@pytest.mark.parametrize("H,G,n", [(16, 8, 36), (16, 4, 72)])
+def test_delta_chunks_of_wide_heads_in_grids_of_both_kinds(H, G, n):
+    """The same where a CU takes two blocks: n chunks are past the limit for two and four heads of 256 to a key head, halves not."""
+    from llm_map_reduce_summarizer_amd import ops
+    from llm_map_reduce_summarizer_amd.engine import mixers
+    from llm_map_reduce_summarizer_amd.engine.config import DeltaSpec
+    m = mixers.DeltaMixer(DeltaSpec(H, G, 256, 16, 2), torch.device(DEV), BF)
+    cols = [0]
+
+    def take(k):
+        at = cols[0]
+        cols[0] = -(-(at + k) // 8) * 8
+        return at
+    m.columns(take)
+    m.col = 0
+    x, u = dev(rnd(n * 64, m.channels, std=0.8).to(BF)), dev(rnd(n * 64, -(-cols[0] // 16) * 16, seed=1, std=1.5).to(BF))
+    small = [dev(rnd(k, seed=2 + j)) for j, k in enumerate((H, H, 16))]
+
+    def run(lo, hi):
+        state, a = torch.zeros(n + 1, H, 16, 256, device=DEV), torch.zeros((hi - lo) * 64, m.width, dtype=BF, device=DEV)
+        ops.delta_mix(x[lo * 64: hi * 64].contiguous(), u[lo * 64: hi * 64].contiguous(), m, -small[0].exp(), small[1] - 3, small[2],
+                      1e-3, state, segments([64] * (hi - lo), list(range(1, hi - lo + 1)), [0] * (hi - lo)), a)
+        return a, state[1: hi - lo + 1]
+    whole, halves = run(0, n), [run(0, n // 2), run(n // 2, n)]
+    assert all(torch.equal(w, torch.cat(h)) for w, h in zip(whole, zip(*halves))) and bool(whole[0].float().abs().sum() > 0)
+
+
 def delta_portions(H, G, dim, vdim, dtype, lens, off=0):
     """Both sides of one delta_mix over segments of ``lens`` rows; ``off``: first element of ``a`` and the norm weights in
     their storage.  Returns (rows, states) errors."""
