@@ -295,6 +295,18 @@ def test_gemm_slabs(M, N, K):
     assert hip.gemm_slabs(x[:, :64], w[:, :64]) is None and hip.gemm_slabs(_rand(4097, K), _rand(4096, K)) is None
 
 
+@pytest.mark.parametrize("M,N,K", [(1967, 4096, 4096), (2400, 4096, 14336), (1569, 4096, 4096), (2048, 4096, 4096)])
+def test_gemm_slabs_of_whole_tiles(M, N, K):
+    """Row counts whose lower tiles run whole: consumers of slabs still get the product in fp32, as one slab."""
+    from llm_map_reduce_summarizer_amd import ops
+    assert hip.gemm_splits(M, N, K // 64)[1] == 1 and hip.gemm_splits_fp8(M, N, K // 64)[1] > 1
+    x, w = _rand(M, K, seed=28, scale=0.5), _rand(N, K, seed=29, scale=0.03)
+    parts = ops.project(x, w, "o")
+    assert parts.shape == (1, M, N) and parts.dtype == torch.float32
+    bound = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())  # fp32 sums of K exact products
+    assert bool(((parts[0].double() - x.double() @ w.double().t()).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("rows", [128, 160, 192, 224])
 @pytest.mark.parametrize("epi", ["bf16", "swiglu", "gelu", "f32"])
 @pytest.mark.parametrize("M,N,K,splits", [(1, 32, 64, 1), (129, 288, 128, 1), (449, 544, 704, 3), (4100, 4128, 192, 1), (4100, 4128, 320, 1)])
