@@ -168,6 +168,21 @@ def test_fp32_gemm_of_short_k(M, N, K, small):
     assert hip.gemm32_small(M, N, K // 32) == small
 
 
+def test_wide_heads_keep_the_outputs_they_took(monkeypatch):
+    """The tile GEMM takes a head's 65 - 128 rows only into rows that it can store; others stay with the stream GEMM."""
+    ran = []
+    monkeypatch.setattr(hip, "gemm", lambda x, w, out=None, **kw: ran.append("tile") or out)
+    monkeypatch.setattr(hip, "_stream_gemm", lambda x, w, out, *a, **kw: ran.append("stream") or out)
+    M, N, K = 66, 49152, 256
+    x, w, room = (torch.empty(n, dtype=torch.bfloat16) for n in (M * K, N * K, M * N + 4))
+    x, w = x.view(M, K), w.view(N, K)
+    assert hip.tile_head(M, N)
+    for off in (0, 4, 1, 2):  # elements of 2 bytes
+        hip.linear(x, w, out=room[off: off + M * N].view(M, N))
+    hip.linear(x, w)
+    assert ran == ["tile", "tile", "stream", "stream", "tile"]
+
+
 def recorded(name):
     """Lines of a record under profiles/; some machines get the tree without them."""
     path = os.path.join(ROOT, "profiles", name)
