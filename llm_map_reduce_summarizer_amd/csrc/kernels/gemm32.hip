@@ -10,8 +10,9 @@
 // wait and barrier of a K-tile stands in its middle, with the second half's fragments in registers, and the next
 // K-tile's first ones are read behind the second half's products: both workgroups of a CU, which run in step, would else stop
 // for their reads together (128 x 128 tiles, 480 -> 500 us with the reads ahead of the products they feed).
-// us, four quarters and two barriers -> this: 903 x 28672 x 4096 1646 -> 1500 (141 TFLOP/s of 155), 300 x 28672 x 4096 667 ->
-// 535, 150 x 18560 x 4096 305 -> 196, 70 x 4096 x 8192 73 -> 54, 508 x 28672 x 4096 832 -> 826.
+// us, four quarters, two barriers and one chain of sums -> this: 903 x 28672 x 4096 1653 -> 1530 (139 TFLOP/s of 155), 300 x
+// 28672 x 4096 668 -> 567, 150 x 18560 x 4096 306 -> 199, 70 x 4096 x 8192 74 -> 55, 508 x 28672 x 4096 833 -> 844.  A workgroup
+// costs 1 us more than there, which short calls of full tiles see: 128 x 2048 x 768 17.8 -> 19.4, 64 x 8192 x 384 13.3 -> 15.2.
 // Tiles that would leave CUs idle run in slices of K (ops/hip.py _gemm32_plan), whose fp32 sums a second launch adds in slice
 // order.  Short K runs in 64 x 64 tiles.
 #include "common.h"

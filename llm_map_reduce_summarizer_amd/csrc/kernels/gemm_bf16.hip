@@ -35,8 +35,8 @@
 //     nothing.  Rows of a tile and slices: mrsum_gemm_plan.
 //
 // Measured, eight waves (two 64 KiB tiles of LDS, two barriers a quarter of a K-tile) -> this, us: 18234 x 28672 x 4096 with
-// GLU 3498 -> 2982 (1436 TFLOP/s), 18234 x 4096 x 14336 1592 -> 1419 (1509), 18234 x 6144 x 4096 694 -> 640, 1967 x 18432 x
-// 4096 with gelu 249 -> 225.  The large ones run at the clock that the card's power allows (1.8 - 1.9 of 2.4 GHz): requests
+// GLU 3439 -> 3015 (1420 TFLOP/s), 18234 x 4096 x 14336 1546 -> 1421 (1507), 18234 x 6144 x 4096 685 -> 640, 1967 x 18432 x
+// 4096 with gelu 258 -> 238.  The large ones run at the clock that the card's power allows (1.8 - 1.9 of 2.4 GHz): requests
 // earlier or later, or reads closer together, change them by less than 1 %.
 #include "gemm.h"
 

@@ -74,9 +74,9 @@ constexpr int ring_slots(int mt, int wpb, int halves) {
 constexpr int slot_halves(int mt, int wpb) { return mt > 4 && ring_slots(mt, wpb, 2) < 3 ? 1 : 2; }
 
 // Grids of many rounds (the LM head): workgroups of 64 W rows with rings so shallow that two share a CU, whose loads run on
-// through each other's barriers, first waits and epilogues.  N 128256, us, one deep ring -> two: K 4096, 16 rows 185 -> 177, 32
-// 197 -> 188 (one row 186 either way); 39 rows, whose slots leave such rings two slots, 208 stays (214), up to K 1024:
-// K 256, 1 row 23.5 -> 13.4, 64 rows 33 -> 20, K 1024 65 -> 56.  One round gains nothing: it has a ring per CU to fill.
+// through each other's barriers, first waits and epilogues.  N 128256, us, one deep ring -> two: K 4096, 1 row 186 -> 181, 16
+// rows 192 -> 190, 32 209 -> 200; more rows, whose slots leave such rings two slots, only up to K 1024:
+// K 256, 1 row 23.4 -> 13.0, 64 rows 34 -> 23, K 1024 67 -> 60.  One round gains nothing: it has a ring per CU to fill.
 constexpr int SHALLOW_MAX_K = 1024;
 constexpr int shallow_slots(int mt) { return mt <= 2 ? 3 : 2; }
 
