@@ -12,7 +12,7 @@
 // for their reads together (128 x 128 tiles, 480 -> 500 us with the reads ahead of the products they feed).
 // us, four quarters, two barriers and one chain of sums -> this: 903 x 28672 x 4096 1653 -> 1530 (139 TFLOP/s of 155), 300 x
 // 28672 x 4096 668 -> 567, 150 x 18560 x 4096 306 -> 199, 70 x 4096 x 8192 74 -> 55, 508 x 28672 x 4096 833 -> 844.  A workgroup
-// costs 1 us more than there, which short calls of full tiles see: 128 x 2048 x 768 17.8 -> 19.4, 64 x 8192 x 384 13.3 -> 15.2.
+// costs 1 us more than there, which short calls of full tiles see: 128 x 2048 x 768 17.8 -> 18.6, 64 x 8192 x 384 13.3 -> 14.5.
 // Tiles that would leave CUs idle run in slices of K (ops/hip.py _gemm32_plan), whose fp32 sums a second launch adds in slice
 // order.  Short K runs in 64 x 64 tiles.
 #include "common.h"
@@ -39,8 +39,14 @@ struct Gemm32Args {
     float* part;        // [tiles - whole][splits][128 * 128]
 };
 
-// grouped raster: 8 tile rows of one tile column are neighbours
+// grouped raster: 8 tile rows of one tile column are neighbours.  A lone row tile needs no division, which are chains of some 40
+// instructions ahead of a workgroup's first load: 20 x 8192 x 512 13.7 -> 13.1 us with this and the same in rows_of.
 __device__ __forceinline__ void tile32(const Gemm32Args& a, int p, int& tm, int& tn) {
+    if (a.tiles_m == 1) {
+        tm = 0;
+        tn = p;
+        return;
+    }
     const int gsz = 8 * a.tiles_n, g = p / gsz, first = 8 * g, gm = min(a.tiles_m - first, 8), within = p - g * gsz;
     tm = first + within % gm;
     tn = within / gm;
@@ -62,6 +68,11 @@ __device__ __forceinline__ void store_c(const Gemm32Args& a, int m, int n, const
 // Row tile tm of column tile tn: an even share of the 16-row blocks, so that no tile is nearly empty beside full ones; which
 // ones are a block taller changes from column to column, as two tall ones on a CU would set the time of all.
 __device__ __forceinline__ void rows_of(const Gemm32Args& a, int tm, int tn, int& b0, int& nb) {
+    if (a.tiles_m == 1) {
+        b0 = 0;
+        nb = (a.M + 15) >> 4;
+        return;
+    }
     const int blocks = (a.M + 15) >> 4, turn = (tn + (tn >> 2) + (tn >> 4)) % a.tiles_m;
     b0 = (int)(((long long)blocks * tm + turn) / a.tiles_m);
     nb = (int)(((long long)blocks * (tm + 1) + turn) / a.tiles_m) - b0;
