@@ -12,7 +12,7 @@
 // for their reads together (128 x 128 tiles, 480 -> 500 us with the reads ahead of the products they feed).
 // us, four quarters, two barriers and one chain of sums -> this: 903 x 28672 x 4096 1653 -> 1530 (139 TFLOP/s of 155), 300 x
 // 28672 x 4096 668 -> 567, 150 x 18560 x 4096 306 -> 199, 70 x 4096 x 8192 74 -> 55, 508 x 28672 x 4096 833 -> 844.  A workgroup
-// costs 1 us more than there, which short calls of full tiles see: 128 x 2048 x 768 17.8 -> 18.6, 64 x 8192 x 384 13.3 -> 14.5.
+// costs 1 us more than there, which short calls of full tiles see: 128 x 2048 x 768 17.7 -> 18.3, 64 x 8192 x 384 13.3 -> 14.5.
 // Tiles that would leave CUs idle run in slices of K (ops/hip.py _gemm32_plan), whose fp32 sums a second launch adds in slice
 // order.  Short K runs in 64 x 64 tiles.
 #include "common.h"
@@ -25,9 +25,11 @@ constexpr int LDS_BYTES = 80 * 1024;         // two workgroups on a CU
 // K-tiles whose products one chain of accumulations adds; the chains' sums are added in order, so that the error does not
 // grow with K nor depend on how many slices a plan takes.  Relative error (2-norm, random operands), one chain -> this: K 4096
 // 1.15e-6 -> 4.1e-7 (2.3e-7 of low tiles, whose slices may be four K-tiles long), K 22528 2.35e-6 -> 4.2e-7, for 1 % of the time
-// (2 % at 20 - 64 rows).
+// (2 % at 20 - 64 rows).  Tall tiles of at most 16 K-tiles are one chain and run without the sums (gemm32_kernel<true>), which
+// would be 5 - 9 % of so short a loop: 1200 x 16384 x 256 97.5 -> 89.2 us, 1500 x 8192 x 192 49.7 -> 46.0, 256 x 1024 x 512 17.4 -> 16.9.
+constexpr int LONG_RUN = 16;
 template <int NB>
-constexpr int RUN = NB > 4 ? 16 : 4;
+constexpr int RUN = NB > 4 ? LONG_RUN : 4;
 
 struct Gemm32Args {
     const float* x;
@@ -78,8 +80,8 @@ __device__ __forceinline__ void rows_of(const Gemm32Args& a, int tm, int tn, int
     nb = (int)(((long long)blocks * (tm + 1) + turn) / a.tiles_m) - b0;
 }
 
-// K-tiles [kt0, kt1) of a tile of NB row blocks; acc[row block][column block]
-template <int NB>
+// K-tiles [kt0, kt1) of a tile of NB row blocks; acc[row block][column block].  ONE: there are at most LONG_RUN of them
+template <int NB, bool ONE>
 __device__ __forceinline__ void k_loop(const Gemm32Args& a, char* lds, int m0, int n0, int kt0, int kt1, f32x4 (&acc)[8][2]) {
     typedef __attribute__((address_space(3))) void* lds_ptr;
     constexpr int XB = NB * 2048, IMAGE = XB + STAGE, XI = (NB + 1) / 2;  // a K-tile of X; of both; pieces of X a wave
@@ -154,13 +156,8 @@ __device__ __forceinline__ void k_loop(const Gemm32Args& a, char* lds, int m0, i
     for (int d = 0; d < D; ++d) stage(min(kt0 + d, kt1 - 1), d);
     meet(std::integral_constant<int, D - 1>{});
     read(0, 0);
-    f32x4 sum[NB][2];
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) sum[b][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int kt = kt0, buf = 0; kt < kt1;) {
-        for (const int end = min(kt + RUN<NB>, kt1); kt < end; ++kt) {
+    auto chain = [&](int& kt, int end, int& buf) {
+        for (; kt < end; ++kt) {
             read(1, buf);
             products(0);
             meet(std::integral_constant<int, D - 2>{});
@@ -169,21 +166,35 @@ __device__ __forceinline__ void k_loop(const Gemm32Args& a, char* lds, int m0, i
             read(0, buf);
             products(1);
         }
+    };
+    int kt = kt0, buf = 0;
+    if constexpr (ONE && RUN<NB> == LONG_RUN) {
+        chain(kt, kt1, buf);
+    } else {
+        f32x4 sum[NB][2];
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                sum[b][i] += acc[b][i];
-                acc[b][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-            }
+            for (int i = 0; i < 2; ++i) sum[b][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        while (kt < kt1) {
+            chain(kt, min(kt + RUN<NB>, kt1), buf);
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    sum[b][i] += acc[b][i];
+                    acc[b][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+        }
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) acc[b][i] = sum[b][i];
     }
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) acc[b][i] = sum[b][i];
     __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));  // nothing may arrive in LDS that another workgroup has by then
 }
 
+template <bool ONE>
 __global__ __launch_bounds__(256, 2) void gemm32_kernel(const Gemm32Args a) {
     __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -212,14 +223,14 @@ __global__ __launch_bounds__(256, 2) void gemm32_kernel(const Gemm32Args a) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) acc[b][i] = f32x4{0.f, 0.f, 0.f, 0.f};
     switch (nb) {
-        case 1: k_loop<1>(a, lds, m0, n0, kt0, kt1, acc); break;
-        case 2: k_loop<2>(a, lds, m0, n0, kt0, kt1, acc); break;
-        case 3: k_loop<3>(a, lds, m0, n0, kt0, kt1, acc); break;
-        case 4: k_loop<4>(a, lds, m0, n0, kt0, kt1, acc); break;
-        case 5: k_loop<5>(a, lds, m0, n0, kt0, kt1, acc); break;
-        case 6: k_loop<6>(a, lds, m0, n0, kt0, kt1, acc); break;
-        case 7: k_loop<7>(a, lds, m0, n0, kt0, kt1, acc); break;
-        default: k_loop<8>(a, lds, m0, n0, kt0, kt1, acc); break;
+        case 1: k_loop<1, ONE>(a, lds, m0, n0, kt0, kt1, acc); break;
+        case 2: k_loop<2, ONE>(a, lds, m0, n0, kt0, kt1, acc); break;
+        case 3: k_loop<3, ONE>(a, lds, m0, n0, kt0, kt1, acc); break;
+        case 4: k_loop<4, ONE>(a, lds, m0, n0, kt0, kt1, acc); break;
+        case 5: k_loop<5, ONE>(a, lds, m0, n0, kt0, kt1, acc); break;
+        case 6: k_loop<6, ONE>(a, lds, m0, n0, kt0, kt1, acc); break;
+        case 7: k_loop<7, ONE>(a, lds, m0, n0, kt0, kt1, acc); break;
+        default: k_loop<8, ONE>(a, lds, m0, n0, kt0, kt1, acc); break;
     }
     if (slice >= 0) {
         f32x4* out = reinterpret_cast<f32x4*>(a.part + ((size_t)(p - a.whole) * a.splits + slice) * (T32 * T32)) + tid;
@@ -335,7 +346,10 @@ MRSUM_API int mrsum_gemm32(const float* x, int ldx, const float* w, int ldw, flo
     a.whole = splits > 1 ? whole : tiles;
     a.splits = splits > 1 ? splits : 1;
     const int rest = tiles - a.whole;
-    gemm32_kernel<<<a.whole + rest * a.splits, 256, 0, s>>>(a);
+    if (ceil_div(a.kb, a.whole ? 1 : a.splits) <= LONG_RUN)
+        gemm32_kernel<true><<<a.whole + rest * a.splits, 256, 0, s>>>(a);
+    else
+        gemm32_kernel<false><<<a.whole + rest * a.splits, 256, 0, s>>>(a);
     if (rest) gemm32_tail_kernel<<<rest * 4, 256, 0, s>>>(a);
     return (int)hipGetLastError();
 }

@@ -522,6 +522,19 @@ def test_gemm32_error_does_not_grow_with_k(M, N, K, monkeypatch):
     assert err <= ((512 + K / 256) / 2) ** 0.5 * 2.0 ** -24
 
 
+@pytest.mark.parametrize("M", [64, 65, 100, 128, 300])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_gemm32_of_one_chain_and_more(M, splits, monkeypatch):
+    """512 products in the longest slice are one chain; with 32 more, which are zeros here, the sums of two: the same bits."""
+    from llm_map_reduce_summarizer_amd.ops import hip
+    N, tiles = 390, -(-M // 128) * 4
+    monkeypatch.setattr(hip, "gemm32_small", lambda *_: False)
+    monkeypatch.setattr(hip, "gemm32_splits", lambda M, N, kb: (tiles if splits == 1 else 0, splits, tiles * splits * 16384))
+    zeros = lambda t: torch.cat([torch.cat([s, torch.zeros(len(t), 32)], 1) for s in t.split(512, 1)], 1)
+    x, w = rnd(M, 512 * splits, seed=1), rnd(N, 512 * splits, seed=2)
+    assert torch.equal(hip.gemm32(dev(x), dev(w)), hip.gemm32(dev(zeros(x)), dev(zeros(w))))
+
+
 @pytest.mark.parametrize("M", [0, 4, 64, 65])
 def test_gemm32_of_empty_k(M):
     from llm_map_reduce_summarizer_amd.ops import hip
