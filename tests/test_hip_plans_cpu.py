@@ -219,13 +219,13 @@ def test_fp32_gemm_slices_by_their_record():
 
 
 def test_fp32_gemm_of_short_k_by_its_record():
-    """The rule is the record's, and takes what is 0.5 % from the faster of the two on average, 25 % at most but for one call of 4 us."""
+    """The rule is the record's, and takes what is 0.5 % from the faster of the two on average, 28 % at most (33 x 4096 x 32, 1 us)."""
     losses = []
     for e in recorded("gemm32_short_k.jsonl"):
         assert hip.gemm32_small(e["M"], e["N"], e["K"] // 32) == e["rule"], e
         if e["K"] <= 512:
             losses.append((e["small"] if e["rule"] else e["large"]) / min(e["small"], e["large"]) - 1)
-            assert losses[-1] <= (0.31 if (e["M"], e["N"], e["K"]) == (33, 4096, 32) else 0.26), e
+            assert losses[-1] <= 0.29, e
     assert len(losses) > 1300 and sum(losses) / len(losses) <= 0.006
 
 
