@@ -15,70 +15,16 @@
 // costs 1 us more than there, which short calls of full tiles see: 128 x 2048 x 768 17.7 -> 18.3, 64 x 8192 x 384 13.3 -> 14.5.
 // Tiles that would leave CUs idle run in slices of K (ops/hip.py _gemm32_plan), whose fp32 sums a second launch adds in slice
 // order.  Short K runs in 64 x 64 tiles.
-#include "common.h"
+#include "gemm32.h"
 
 #include <type_traits>
 
 namespace {
 constexpr int T32 = 128, STAGE = T32 * 128;  // bytes of W's K-tile
 constexpr int LDS_BYTES = 80 * 1024;         // two workgroups on a CU
-// K-tiles whose products one chain of accumulations adds; the chains' sums are added in order, so that the error does not
-// grow with K nor depend on how many slices a plan takes.  Relative error (2-norm, random operands), one chain -> this: K 4096
-// 1.15e-6 -> 4.1e-7 (2.3e-7 of low tiles, whose slices may be four K-tiles long), K 22528 2.35e-6 -> 4.2e-7, for 1 % of the time
-// (2 % at 20 - 64 rows).  Tall tiles of at most 16 K-tiles are one chain and run without the sums (gemm32_kernel<true>), which
-// would be 5 - 9 % of so short a loop: 1200 x 16384 x 256 97.5 -> 89.2 us, 1500 x 8192 x 192 49.7 -> 46.0, 256 x 1024 x 512 17.4 -> 16.9.
-constexpr int LONG_RUN = 16;
 template <int NB>
 constexpr int RUN = NB > 4 ? LONG_RUN : 4;
-
-struct Gemm32Args {
-    const float* x;
-    const float* w;
-    float* c;
-    int ldx, ldw, ldc, M, N, kb;  // kb: K-tiles
-    int tiles_m, tiles_n;
-    int whole, splits;  // raster positions from ``whole`` on run in ``splits`` slices of K
-    float* part;        // [tiles - whole][splits][128 * 128]
-};
-
-// grouped raster: 8 tile rows of one tile column are neighbours.  A lone row tile needs no division, which are chains of some 40
-// instructions ahead of a workgroup's first load: 20 x 8192 x 512 13.7 -> 13.1 us with this and the same in rows_of.
-__device__ __forceinline__ void tile32(const Gemm32Args& a, int p, int& tm, int& tn) {
-    if (a.tiles_m == 1) {
-        tm = 0;
-        tn = p;
-        return;
-    }
-    const int gsz = 8 * a.tiles_n, g = p / gsz, first = 8 * g, gm = min(a.tiles_m - first, 8), within = p - g * gsz;
-    tm = first + within % gm;
-    tn = within / gm;
-}
-
-__device__ __forceinline__ void store_c(const Gemm32Args& a, int m, int n, const f32x4& v) {
-    if (m >= a.M) return;
-    float* o = a.c + (size_t)m * a.ldc + n;
-    if (n + 4 <= a.N && a.ldc % 4 == 0 && (uintptr_t)a.c % 16 == 0) {
-        *reinterpret_cast<f32x4*>(o) = v;
-    } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if (n + j < a.N) o[j] = v[j];
-    }
-}
 }  // namespace
-
-// Row tile tm of column tile tn: an even share of the 16-row blocks, so that no tile is nearly empty beside full ones; which
-// ones are a block taller changes from column to column, as two tall ones on a CU would set the time of all.
-__device__ __forceinline__ void rows_of(const Gemm32Args& a, int tm, int tn, int& b0, int& nb) {
-    if (a.tiles_m == 1) {
-        b0 = 0;
-        nb = (a.M + 15) >> 4;
-        return;
-    }
-    const int blocks = (a.M + 15) >> 4, turn = (tn + (tn >> 2) + (tn >> 4)) % a.tiles_m;
-    b0 = (int)(((long long)blocks * tm + turn) / a.tiles_m);
-    nb = (int)(((long long)blocks * (tm + 1) + turn) / a.tiles_m) - b0;
-}
 
 // K-tiles [kt0, kt1) of a tile of NB row blocks; acc[row block][column block].  ONE: there are at most LONG_RUN of them
 template <int NB, bool ONE>
@@ -196,6 +142,7 @@ __device__ __forceinline__ void k_loop(const Gemm32Args& a, char* lds, int m0, i
 
 template <bool ONE>
 __global__ __launch_bounds__(256, 2) void gemm32_kernel(const Gemm32Args a) {
+    if (a.inexact && !*a.inexact) return;
     __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -215,7 +162,7 @@ __global__ __launch_bounds__(256, 2) void gemm32_kernel(const Gemm32Args a) {
     }
     int tm, tn, b0, nb;
     tile32(a, p, tm, tn);
-    rows_of(a, tm, tn, b0, nb);
+    rows_of(a, (a.M + 15) >> 4, tm, tn, b0, nb);
     const int m0 = b0 * 16, n0 = tn * T32;
     f32x4 acc[8][2];
 #pragma unroll
@@ -251,10 +198,11 @@ __global__ __launch_bounds__(256, 2) void gemm32_kernel(const Gemm32Args a) {
 
 // adds the slices of the split tiles; one workgroup per (tile, 2 x 16 rows)
 __global__ __launch_bounds__(256) void gemm32_tail_kernel(const Gemm32Args a) {
+    if (a.inexact && !*a.inexact) return;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, t = blockIdx.x >> 2, b = 2 * (blockIdx.x & 3);
     int tm, tn, b0, nb;
     tile32(a, a.whole + t, tm, tn);
-    rows_of(a, tm, tn, b0, nb);
+    rows_of(a, (a.M + 15) >> 4, tm, tn, b0, nb);
     if (b >= nb) return;
     const f32x4* in = reinterpret_cast<const f32x4*>(a.part + (size_t)t * a.splits * (T32 * T32)) + b * 2 * 256 + tid;
     f32x4 v[4];
@@ -326,10 +274,8 @@ __global__ __launch_bounds__(256) void gemm32_small_kernel(const float* __restri
     }
 }
 
-// x [M][ldx], w [N][ldw], c [M][ldc]; tiles from raster position ``whole`` on in ``splits`` slices of K through ``part``
-// [tiles - whole][splits][16384] (splits 1: none, part unused); splits 0: 64 x 64 tiles
-MRSUM_API int mrsum_gemm32(const float* x, int ldx, const float* w, int ldw, float* c, int ldc, int M, int N, int K,
-                           int whole, int splits, float* part, hipStream_t s) {
+int gemm32_launch(const float* x, int ldx, const float* w, int ldw, float* c, int ldc, int M, int N, int K, int whole, int splits,
+                  float* part, int* inexact, hipStream_t s) {
     if (M <= 0 || N <= 0) return 0;
     if (K % 32 || ldx % 4 || ldw % 4 || (uintptr_t)x % 16 || (uintptr_t)w % 16 || (size_t)T32 * ldx * 4 >= (1u << 31) ||
         (size_t)T32 * ldw * 4 >= (1u << 31))
@@ -340,7 +286,7 @@ MRSUM_API int mrsum_gemm32(const float* x, int ldx, const float* w, int ldw, flo
         gemm32_small_kernel<<<dim3(ceil_div(N, TS), ceil_div(M, TS)), 256, 0, s>>>(x, ldx, w, ldw, c, ldc, M, N, K);
         return (int)hipGetLastError();
     }
-    Gemm32Args a{x, w, c, ldx, ldw, ldc, M, N, K / 32, ceil_div(M, T32), ceil_div(N, T32), 0, 1, part};
+    Gemm32Args a{x, w, c, ldx, ldw, ldc, M, N, K / 32, ceil_div(M, T32), ceil_div(N, T32), 0, 1, part, inexact};
     const int tiles = a.tiles_m * a.tiles_n;
     if (splits > 1 && (whole < 0 || whole >= tiles || splits > a.kb || !part)) return (int)hipErrorInvalidValue;
     a.whole = splits > 1 ? whole : tiles;
@@ -352,4 +298,11 @@ MRSUM_API int mrsum_gemm32(const float* x, int ldx, const float* w, int ldw, flo
         gemm32_kernel<false><<<a.whole + rest * a.splits, 256, 0, s>>>(a);
     if (rest) gemm32_tail_kernel<<<rest * 4, 256, 0, s>>>(a);
     return (int)hipGetLastError();
+}
+
+// x [M][ldx], w [N][ldw], c [M][ldc]; tiles from raster position ``whole`` on in ``splits`` slices of K through ``part``
+// [tiles - whole][splits][16384] (splits 1: none, part unused); splits 0: 64 x 64 tiles
+MRSUM_API int mrsum_gemm32(const float* x, int ldx, const float* w, int ldw, float* c, int ldc, int M, int N, int K,
+                           int whole, int splits, float* part, hipStream_t s) {
+    return gemm32_launch(x, ldx, w, ldw, c, ldc, M, N, K, whole, splits, part, nullptr, s);
 }

@@ -1,0 +1,357 @@
+// fp32 GEMM of many rows on the bf16 matrix instruction (v_mfma_f32_16x16x32_bf16), with no bit of an operand left out:
+//
+//     C[M, N] = X[M, K] . W[N, K]^T        K % 32 == 0
+//
+// An fp32 value is the exact sum of three bf16 terms, its 24 bits in groups of eight.  Where W's values are bf16 ones (weights of a
+// 16-bit checkpoint, widened), X . W is the sum of three products of bf16 operands, each of which the instruction forms exactly and
+// adds in fp32: sixteen times the fp32 instruction's rate, for three times the products.  W stays 32 bits wide in memory and is
+// looked at as it is read; if a value has lower bits, or is infinite (an infinity times a term of 0 is no number), a flag is set and the
+// fp32 instruction's form (gemm32.hip), which is launched behind and otherwise returns at once, makes the whole result.  A workgroup
+// that sees it in its first K-tile stops there, so that W with 24 bits cost the launches, about 10 us.
+//
+// Relative error (2-norm, random operands, K 4096 - 22528, chains of 16 K-tiles on both): 2.4e-7, the fp32 instruction 4.1e-7, as one
+// sum takes the products of 32 columns and not of four.
+//
+// What bounds it: the arrival of the tiles, and the card's power.  A workgroup of four waves has up to 160 rows x 256 columns of
+// outputs, one wave a SIMD with 80 x 128; larger ones do not fit in the registers beside the sums of finished chains.  A K-tile of 32 is
+// 1920 cycles of products, 120 KiB of LDS reads and 62 KiB of requests, and takes 1.6 - 1.7 us (1.2 PFLOP/s in bf16, 0.9 us with the
+// requests left out, 1.7 PFLOP/s at the clock that the power then allows).
+//   * X's terms are made by a launch ahead (10 bytes a value), in the order that fragments are read in: 1 KiB pieces of
+//     consecutive lanes, by LDS-DMA and by ds_read_b128 alike.
+//   * W arrives by LDS-DMA too, 8 rows x 128 bytes an instruction; loaded by the lanes that use it (16 rows x 64 bytes) it took
+//     three times as many cache accesses and as long (20608 columns, 300 rows: 181 us, 165 here).
+//   * every product has an instruction or three of other work behind it: it keeps the matrix core busy for 16 cycles and the
+//     wave for four.
+// us, fp32 instruction -> this: 903 x 28672 x 4096 1560 -> 600, 903 x 4096 x 14336 809 -> 341, 300 x 20608 x 4096 436 -> 165, 160 x
+// 28672 x 4096 302 -> 155 (where W's arrival is all).  Which rows and shapes: ops/hip.py gemm32_terms.
+#include "gemm32.h"
+
+#include <type_traits>
+
+namespace {
+constexpr int TN = 256;                 // columns of a tile
+constexpr int MAX_NB = 5;               // its 32-row units
+constexpr int BLOCK = 3072;             // bytes of a K-tile of 32 of 16 rows of X: [term][lane][16]
+constexpr int WI = TN * 128, WS = 3;    // bytes of W's K-tile, and how many are in LDS; behind them X's
+constexpr int x_slots(int nb) { return nb <= 3 ? 3 : 2; }
+constexpr int LDS_BYTES = WS * WI + 2 * 2 * MAX_NB * BLOCK;
+constexpr int SLOT = MAX_NB * 32 * TN;  // scratch floats of a slice of a tile
+static_assert(LDS_BYTES + 16 <= 160 * 1024 && x_slots(3) * 2 * 3 * BLOCK <= 2 * 2 * MAX_NB * BLOCK, "LDS");
+
+typedef __attribute__((address_space(3))) void* lds_ptr;
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer(const void* p, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, bytes, 0x00020000);
+}
+
+__device__ __forceinline__ uint32_t high_halves(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302); }
+
+// v - its first term; infinities leave none
+__device__ __forceinline__ uint32_t below(uint32_t v) {
+    const float top = __uint_as_float(v & 0xffff0000u);
+    return (v & 0x7f800000u) == 0x7f800000u ? 0u : __float_as_uint(__uint_as_float(v) - top);
+}
+}  // namespace
+
+// X's terms, laid out as the matrix instruction reads them: [M / 16][K / 32][term][lane][8], lane (r, g) holding row r, k 4 g .. and
+// 16 + 4 g ..  Rows past M are zeros.
+__global__ __launch_bounds__(256) void terms32_kernel(const float* __restrict__ x, int ldx, char* __restrict__ out, int M, int kb,
+                                                      int pieces, int* inexact) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *inexact = 0;
+    const int lane = threadIdx.x & 63, p = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (p >= pieces) return;
+    const int block = p / kb, kt = p - block * kb, m = block * 16 + (lane & 15);
+    u32x4 v[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+    if (m < M) {
+        const u32x4* in = reinterpret_cast<const u32x4*>(x + (size_t)m * ldx + kt * 32) + (lane >> 4);
+        v[0] = in[0];
+        v[1] = in[4];
+    }
+    u32x4 t[3];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        uint32_t a[2][3];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const uint32_t u = v[i >> 1][2 * (i & 1) + j], r = below(u);
+            a[j][0] = (u & 0x7fffffffu) > 0x7f800000u ? u | 0x00400000u : u;  // a NaN whose bits are all low
+            a[j][1] = r;
+            a[j][2] = below(r);
+        }
+#pragma unroll
+        for (int k = 0; k < 3; ++k) t[k][i] = high_halves(a[0][k], a[1][k]);
+    }
+    u32x4* o = reinterpret_cast<u32x4*>(out + (size_t)p * BLOCK) + lane;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) o[64 * k] = t[k];
+}
+
+namespace {
+// Outputs of (row block b, column block i) of a tile of nb 32-row units: row lane & 15, columns 4 (lane >> 4) ..
+__device__ __forceinline__ void store_terms(const Gemm32Args& a, int u0, int nb, int n0, int b, int i, const f32x4& v) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    store_c(a, 32 * u0 + 16 * (nb * (w >> 1) + b) + (lane & 15), n0 + 128 * (w & 1) + 16 * i + 4 * (lane >> 4), v);
+}
+
+// K-tiles [kt0, kt1) of 32 NB rows from 32 u0 on and columns n0 ..; wave (wr, wc) has half of the rows and 128 columns: acc[row
+// block][column block].  False: W has bits below its bf16 values, and the sums are not made.
+template <int NB>
+__device__ __forceinline__ bool terms_loop(const Gemm32Args& a, char* lds, int u0, int n0, int kt0, int kt1, f32x4 (&acc)[NB][8]) {
+    constexpr int XI = 2 * NB * BLOCK, PX = (6 * NB + 3) / 4, XS = x_slots(NB);
+    const int tid = threadIdx.x, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6), wr = w >> 1, wc = w & 1;
+    const __amdgpu_buffer_rsrc_t rx = buffer(reinterpret_cast<const char*>(a.x) + (size_t)u0 * 2 * a.kb * BLOCK, 2 * NB * a.kb * BLOCK);
+    const __amdgpu_buffer_rsrc_t rw = buffer(a.w + (size_t)n0 * a.ldw, min(a.N - n0, TN) * a.ldw * 4);
+    // pieces of 1 KiB.  X: a term of a row block, every fourth one (behind the last that one again); W: 8 rows of this wave's 64,
+    // position lane & 7 of row r taking chunk (lane & 7) ^ ((r >> 1) & 7); behind row N the last one again
+    int vx[PX], dx[PX], vw[8];
+#pragma unroll
+    for (int i = 0; i < PX; ++i) {
+        const int p = min(w + 4 * i, 6 * NB - 1);
+        vx[i] = (p / 3) * a.kb * BLOCK + p % 3 * 1024 + lane * 16;
+        dx[i] = WS * WI + p * 1024;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int r = 64 * w + 8 * i + (lane >> 3);
+        vw[i] = min(r, a.N - n0 - 1) * a.ldw * 4 + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
+    }
+    auto stage_x = [&](int kt, int slot, int i) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr)(lds + slot * XI + dx[i]), 16, vx[i], kt * BLOCK, 0, 0);
+    };
+    auto stage_w = [&](int kt, int slot, int i) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr)(lds + slot * WI + (8 * w + i) * 1024), 16, vw[i], kt * 128, 0, 0);
+    };
+    const int wlo = (128 * wc + r16) * 128 + ((g ^ (r16 >> 1)) << 4), xlo = WS * WI + wr * NB * BLOCK + lane * 16;
+    auto read_w = [&](u32x4 (&q)[2], int slot, int i, int h) {
+        q[h] = *reinterpret_cast<const u32x4*>(lds + slot * WI + (h ? wlo ^ 64 : wlo) + i * 2048);
+    };
+    auto read_x = [&](u32x4 (&x)[3], int slot, int b, int k) {
+        x[k] = *reinterpret_cast<const u32x4*>(lds + slot * XI + xlo + b * BLOCK + k * 1024);
+    };
+    // first terms of a pair of W's values; ``low`` gathers the bits below them, ``top`` the largest size
+    uint32_t low = 0;
+    float top = 0.f;
+    auto first = [&](const u32x4 (&q)[2], u32x4& f, int i) {
+        const uint32_t u = q[i >> 1][2 * (i & 1)], v = q[i >> 1][2 * (i & 1) + 1];
+        uint32_t d = high_halves(u, v);
+        low |= u | v;
+        top = fmaxf(fmaxf(top, fabsf(__uint_as_float(u))), fabsf(__uint_as_float(v)));
+        asm volatile("" : "+v"(d), "+v"(low), "+v"(top));  // here, and not where they are used
+        f[i] = d;
+    };
+    auto any = [&] { return __ballot((low & 0xffffu) != 0 || top == __builtin_inff()) != 0; };
+    // The products are written out so that a block's sums stay in their registers (left to the compiler, they are copied from
+    // one set to another every K-tile, and spilled).  The waits that it would put between them and other uses of these registers
+    // stand at the ends of a K-tile.
+    auto mfma = [](const u32x4& f, const u32x4& x, f32x4& c) {
+        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(f), "v"(x));
+    };
+    // this wave has read what it wanted, and all but its last N requests have arrived; and so in all waves
+    auto meet = [](auto ahead) {
+        constexpr int N = decltype(ahead)::value;
+        __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (0 << 8) | ((N >> 4) << 14));
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    const int last = kt1 - 1;
+#pragma unroll
+    for (int d = 0; d < WS; ++d) {
+        if (d < 2)
+#pragma unroll
+            for (int i = 0; i < PX; ++i) stage_x(min(kt0 + d, last), d, i);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) stage_w(min(kt0 + d, last), d, i);
+    }
+    meet(std::integral_constant<int, 8>{});  // all but the third W
+    u32x4 wf[8], x0[3];
+    f32x4 sum[NB][8];
+    int* seen = reinterpret_cast<int*>(lds + LDS_BYTES);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        u32x4 q[2];
+        read_w(q, 0, i, 0);
+        read_w(q, 0, i, 1);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) first(q, wf[i], j);
+    }
+    const bool odd = any();
+    if (lane == 0) seen[w] = odd;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) read_x(x0, 0, 0, k);
+    meet(std::integral_constant<int, 8>{});
+    if (seen[0] | seen[1] | seen[2] | seen[3]) {  // most W that are not bf16 values show it here
+        if (tid == 0) atomicOr(a.inexact, 1);
+        __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));
+        return false;
+    }
+    if constexpr (XS == 3)
+#pragma unroll
+        for (int i = 0; i < PX; ++i) stage_x(min(kt0 + 2, last), 2, i);
+    // requests behind X of the next K-tile and W of the one after it, at a K-tile's meeting
+    constexpr int AHEAD = 8 + (XS == 3 ? PX : 0);
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            acc[b][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+            sum[b][i] = acc[b][i];
+        }
+    int sx = 0, sw = 1;  // slots of X(t) and W(t + 1)
+    // A K-tile: 24 products a row block, and an instruction or three of other work behind each, which takes the time of four:
+    // reads of X a row block ahead, reads and conversion of the next K-tile's W, behind the meeting requests.
+    auto step = [&](int kt) {
+        u32x4 x[2][3], wn[8], q[8][2];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) x[0][k] = x0[k];
+        const int pw = sw == 0 ? WS - 1 : sw - 1;  // where the W of this K-tile was
+        int px = 0;
+        asm volatile("s_nop 3");
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            if (b == NB - 1) {
+                meet(std::integral_constant<int, AHEAD>{});
+                px = sx;
+                sx = sx + 1 == XS ? 0 : sx + 1;
+                sw = sw + 1 == WS ? 0 : sw + 1;
+            }
+#pragma unroll
+            for (int m = 0; m < 24; ++m) {
+                mfma(wf[m & 7], x[b & 1][2 - (m >> 3)], acc[b][m & 7]);
+                if (m < 3) read_x(x[(b + 1) & 1], sx, b < NB - 1 ? b + 1 : 0, m);
+                const int s = 24 * b + m;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const int at = 3 * (NB - 1) * i;
+                    if (s == at) read_w(q[i], sw, i, 0);
+                    if (s == at + 1) read_w(q[i], sw, i, 1);
+                    if (s >= at + 14 && s < at + 18) first(q[i], wn[i], s - at - 14);
+                    if (s == at + 2) stage_w(min(kt + WS, last), pw, i);
+                }
+                if (b == NB - 1 && m >= 4 && m < 4 + PX) stage_x(min(kt + XS, last), px, m - 4);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        asm volatile("s_nop 15\ns_nop 15");
+#pragma unroll
+        for (int i = 0; i < 8; ++i) wf[i] = wn[i];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) x0[k] = x[NB & 1][k];
+    };
+    for (int kt = kt0; kt < kt1;) {  // chains
+        for (const int end = min(kt + LONG_RUN, kt1); kt < end; ++kt) step(kt);
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int i = 0; i < 8; i += 4) {
+                asm volatile("s_nop 7" : "+a"(acc[b][i]), "+a"(acc[b][i + 1]), "+a"(acc[b][i + 2]), "+a"(acc[b][i + 3]));
+#pragma unroll
+                for (int j = i; j < i + 4; ++j) {
+                    sum[b][j] += acc[b][j];
+                    acc[b][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+                asm volatile("" : "+a"(acc[b][i]), "+a"(acc[b][i + 1]), "+a"(acc[b][i + 2]), "+a"(acc[b][i + 3]));
+            }
+    }
+    if (any() && lane == 0) atomicOr(a.inexact, 1);
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc[b][i] = sum[b][i];
+    __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));  // nothing may arrive in LDS that another workgroup has by then
+    return true;
+}
+
+template <int NB>
+__device__ __forceinline__ void terms_tile(const Gemm32Args& a, char* lds, int u0, int n0, int kt0, int kt1, f32x4* part) {
+    f32x4 acc[NB][8];
+    if (!terms_loop<NB>(a, lds, u0, n0, kt0, kt1, acc)) return;
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            if (part) part[(b * 8 + i) * 256 + tid] = acc[b][i];
+            else store_terms(a, u0, NB, n0, b, i, acc[b][i]);
+        }
+}
+}  // namespace
+
+__global__ __launch_bounds__(256, 1) void gemm32_terms_kernel(const Gemm32Args a) {
+    __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES + 16];
+    int p = blockIdx.x, slice = -1, kt0 = 0, kt1 = a.kb;
+    if (p < a.whole) {
+        p = xcd_position(p, a.whole);
+    } else {
+        const int rest = a.tiles_m * a.tiles_n - a.whole;
+        p = xcd_position(p - a.whole, rest * a.splits);
+        slice = p / rest;
+        p += a.whole - slice * rest;
+        kt0 = a.kb * slice / a.splits;
+        kt1 = a.kb * (slice + 1) / a.splits;
+    }
+    int tm, tn, u0, nu;
+    tile32(a, p, tm, tn);
+    rows_of(a, (a.M + 31) >> 5, tm, tn, u0, nu);
+    f32x4* part = slice < 0 ? nullptr : reinterpret_cast<f32x4*>(a.part + ((size_t)(p - a.whole) * a.splits + slice) * SLOT);
+    switch (nu) {
+        case 2: terms_tile<2>(a, lds, u0, tn * TN, kt0, kt1, part); break;
+        case 3: terms_tile<3>(a, lds, u0, tn * TN, kt0, kt1, part); break;
+        case 4: terms_tile<4>(a, lds, u0, tn * TN, kt0, kt1, part); break;
+        default: terms_tile<5>(a, lds, u0, tn * TN, kt0, kt1, part); break;
+    }
+}
+
+// adds the slices of the split tiles; one workgroup per (tile, 2 x 16 rows)
+__global__ __launch_bounds__(256) void gemm32_terms_tail_kernel(const Gemm32Args a) {
+    const int tid = threadIdx.x, t = blockIdx.x / MAX_NB, b = blockIdx.x % MAX_NB;
+    int tm, tn, u0, nu;
+    tile32(a, a.whole + t, tm, tn);
+    rows_of(a, (a.M + 31) >> 5, tm, tn, u0, nu);
+    if (b >= nu) return;
+    const f32x4* in = reinterpret_cast<const f32x4*>(a.part + (size_t)t * a.splits * SLOT) + b * 8 * 256 + tid;
+    f32x4 v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = in[i * 256];
+    for (int s = 1; s < a.splits; s += 2) {  // two slices in flight
+        f32x4 q[2][8];
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) q[k][i] = in[(size_t)min(s + k, a.splits - 1) * (SLOT / 4) + i * 256];
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            if (s + k < a.splits)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[i] += q[k][i];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) store_terms(a, u0, nu, tn * TN, b, i, v[i]);
+}
+
+MRSUM_API int mrsum_gemm32_terms(const float* x, int ldx, const float* w, int ldw, float* c, int ldc, int M, int N, int K,
+                                 int tiles_m, int whole, int splits, int whole32, int splits32, void* terms, float* part,
+                                 hipStream_t s) {
+    const int units = ceil_div(M, 32), kb = K / 32, tn = ceil_div(N, TN);
+    if (M <= 32 || N <= 0 || K < 32 || K % 32 || ldx % 4 || ldw % 4 || (uintptr_t)x % 16 || (uintptr_t)w % 16 || !terms ||
+        (uintptr_t)terms % 16 || tiles_m < 1 || units / tiles_m < 2 || ceil_div(units, tiles_m) > MAX_NB ||
+        (size_t)TN * ldw * 4 >= (1u << 31) || (size_t)2 * MAX_NB * kb * BLOCK >= (1u << 31))
+        return (int)hipErrorInvalidValue;
+    const long long tiles = (long long)tiles_m * tn;
+    if (splits < 1 || splits > kb || whole < 0 || whole > tiles || (splits > 1 && whole < tiles && !part) || splits32 < 1 ||
+        tiles * std::max(splits, MAX_NB) >= (1ll << 31) || 2ll * units * kb >= (1ll << 31))
+        return (int)hipErrorInvalidValue;
+    const int pieces = 2 * units * kb;
+    int* inexact = reinterpret_cast<int*>(static_cast<char*>(terms) + (size_t)pieces * BLOCK);
+    Gemm32Args a{static_cast<const float*>(terms), w, c, 0, ldw, ldc, M, N, kb, tiles_m, tn, (int)tiles, 1, part, inexact};
+    if (splits > 1) {
+        a.whole = whole;
+        a.splits = splits;
+    }
+    const int rest = (int)tiles - a.whole;
+    terms32_kernel<<<ceil_div(pieces, 4), 256, 0, s>>>(x, ldx, static_cast<char*>(terms), M, kb, pieces, inexact);
+    gemm32_terms_kernel<<<a.whole + rest * a.splits, 256, 0, s>>>(a);
+    if (rest) gemm32_terms_tail_kernel<<<rest * MAX_NB, 256, 0, s>>>(a);
+    return gemm32_launch(x, ldx, w, ldw, c, ldc, M, N, K, whole32, splits32, part, inexact, s);
+}

@@ -229,6 +229,36 @@ def test_fp32_gemm_of_short_k_by_its_record():
     assert len(losses) > 1300 and sum(losses) / len(losses) <= 0.006
 
 
+def test_fp32_gemm_in_terms_by_its_record():
+    """The plan is the record's and near the best of each shape; the rule takes terms only where they are no slower than the fp32
+    instruction by more than 4 %, and loses 1.5 % on average against the best plan of the two."""
+    plans, losses = [], []
+    for e in recorded("gemm32_terms.jsonl"):
+        plan = hip.gemm32_terms(e["M"], e["N"], e["K"] // 32)
+        assert (plan is not None) == e["rule"], e
+        best = min(e["us"].values())
+        took = e["fp32"]
+        if e["M"] > 64:
+            assert "%d/%d/%d" % hip._gemm32_terms_plan(e["M"], e["N"], e["K"] // 32)[:3] == e["plan"], e
+            plans.append(e["us"][e["plan"]] / best - 1)
+            assert plans[-1] <= 0.21, e
+        if e["rule"]:
+            assert "%d/%d/%d" % plan[:3] == e["plan"]
+            took = e["us"][e["plan"]]
+            assert took <= 1.04 * e["fp32"], e
+        if e["M"] > 64:
+            losses.append(took / min(best, e["fp32"]) - 1)
+    assert len(plans) > 300 and sum(plans) / len(plans) <= 0.015 and sum(losses) / len(losses) <= 0.016
+
+
+@pytest.mark.parametrize("M,K,tiles,whole,splits", [(32, 512, 1, 1, 1), (65, 0, 1, 1, 1), (65, 512, 2, 1, 1), (161, 512, 1, 1, 1),
+                                                    (65, 512, 1, 0, 17), (65, 512, 1, 2, 1), (65, 528, 1, 1, 1), (65, 512, 0, 0, 1)])
+def test_fp32_terms_refuse_what_their_tiles_cannot_hold(M, K, tiles, whole, splits):
+    invalid, buffer = 1, 1 << 20  # hipErrorInvalidValue; never read
+    assert hip._fn("mrsum_gemm32_terms")(buffer, K, buffer, K, buffer, 16, M, 16, K, tiles, whole, splits, 1, 1, buffer, buffer,
+                                         None) == invalid
+
+
 def test_fp32_tiles_refuse_an_empty_k():
     """The tiles ask for their first K-tile before they look whether there is one; the entry point refuses K 0 on the host."""
     invalid = 1  # hipErrorInvalidValue

@@ -565,6 +565,77 @@ def test_gemm32_unaligned_storage(M, off_x, off_w):
     assert torch.equal(hip.gemm32(x, w), hip.gemm32(x.clone(), w.clone()))
 
 
+# row tiles of every height (2 - 5 units of 32 rows), unequal ones, rows and columns past the last tile, whole tiles and slices, one
+# K-tile in a slice, odd numbers of them, chains of 16 and one more
+TERMS = [(65, 130, 512, (1, 1, 1)), (96, 390, 544, (1, 2, 1)), (160, 256, 1056, (1, 0, 16)), (161, 1023, 608, (2, 3, 5)),
+         (250, 2062, 544, (4, 9, 2)), (300, 4100, 512, (3, 0, 3)), (903, 515, 96, (6, 18, 1))]
+
+
+@pytest.mark.parametrize("M,N,K,plan", TERMS)
+def test_gemm32_in_terms(M, N, K, plan, monkeypatch):
+    """W of bf16 values: three exact terms of X, sums in fp32.  W with one value that has more bits, in the first K-tile or the
+    last: what the fp32 instruction gives."""
+    from llm_map_reduce_summarizer_amd.ops import hip
+    scratch = (plan[0] * -(-N // 256) - plan[1]) * plan[2] * 40960
+    x, w = rnd(M, K, seed=1), rnd(N, K, seed=2, dtype=BF).float()
+    x[3], x[5] = x[3] * 2.0 ** -90, x[5] * 2.0 ** 90
+    full = {}
+    for at in ((0, 0), (N - 1, K - 1)):
+        v = w.clone()
+        v[at] += 2.0 ** -20 * v[at]
+        full[at] = v
+    monkeypatch.setattr(hip, "gemm32_small", lambda *_: False)
+    monkeypatch.setattr(hip, "gemm32_terms", lambda *_: None)
+    want = {at: hip.gemm32(dev(x), dev(v)) for at, v in full.items()}
+    monkeypatch.setattr(hip, "gemm32_terms", lambda *_: (*plan, scratch))
+    got = hip.gemm32(dev(x), dev(w)).double().cpu()
+    # a sum rounds by at most 2^-24 of the sum of magnitudes, and there are at most K of them
+    bound = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert got.shape == (M, N) and bool(((got - x.double() @ w.double().T).abs() <= bound).all())
+    for at, v in full.items():
+        assert torch.equal(hip.gemm32(dev(x), dev(v)), want[at])
+
+
+def test_gemm32_in_terms_of_infinities():
+    """Infinities and NaN in X and W make what fp32 products and sums make of them."""
+    from llm_map_reduce_summarizer_amd.ops import hip
+    M, N, K = 300, 4096, 4096
+    assert hip.gemm32_terms(M, N, K // 32)
+    inf, nan = float("inf"), float("nan")
+    x, w = rnd(M, K, seed=1), rnd(N, K, seed=2, dtype=BF).float()
+    x[7, 9], x[8, 4095], x[299, 0] = inf, -inf, nan
+    x[20] = torch.full((K,), 1, dtype=torch.int32).add_(0x7f800000).view(F32)  # NaN whose bits are all low
+    for odd in (False, True):
+        if odd:
+            w[11, 5], w[4095, 4095], w[77, 2048] = inf, -inf, nan
+        want, got = x.double() @ w.double().T, hip.gemm32(dev(x), dev(w)).cpu()
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+        assert torch.equal(got[want.isinf()].double(), want[want.isinf()])
+        ok = want.isfinite()
+        assert float((got.double() - want)[ok].norm() / want[ok].norm()) < 1e-6
+
+
+def test_gemm32_in_terms_of_many_rows(monkeypatch):
+    """Terms beyond their buffer's size are made for a part of the rows at a time; replays of a captured product give the same."""
+    from llm_map_reduce_summarizer_amd.ops import hip
+    M, N, K = 700, 1024, 1024
+    x, w = dev(rnd(M, K, seed=1)), dev(rnd(N, K, seed=2, dtype=BF).float())
+    monkeypatch.setattr(hip, "gemm32_terms", lambda m, n, kb: (-(-m // 160), -(-m // 160) * 4, 1, 0))
+    want = hip.gemm32(x, w)
+    monkeypatch.setattr(hip, "GEMM32_TERMS_BYTES", 300 * K * 6)
+    assert torch.equal(hip.gemm32(x, w), want)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = hip.gemm32(x, w)
+    for scale in (1, 2, 4):
+        got.zero_()
+        x.mul_(scale)
+        want = want * scale  # powers of two
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+
+
 def test_gemm32_deep():
     """K beyond what 31-bit offsets over a tile's rows reach."""
     from llm_map_reduce_summarizer_amd.ops import hip
