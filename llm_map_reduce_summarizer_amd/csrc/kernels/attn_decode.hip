@@ -360,8 +360,17 @@ __device__ __forceinline__ u32x4 ld_kv(const T* p) {
 // cache is fp8 slabs, bit 1 = the V cache is; KVM 2 ("fp8v": bf16 K, fp8 V) stages K with the bf16
 // mapping and V with the slab mapping, each into its own LDS tile.
 // HL: the softmax weights enter the value product as two bf16 terms (hi + lo, 16 bits of mantissa) instead of one.
+// Which forms keep ONE tile in flight in registers, so that 128 of them are enough and four workgroups fit a CU, in place of two
+// tiles and three workgroups: a workgroup's step from tile to tile is a chain (pages -> LDS -> scores -> weights -> sums, two
+// barriers), and a fourth chain beside it hides more of it than a second tile in flight (at 1024 workgroups 128 KiB of bf16
+// pages are on the way to a CU, or 66 KiB of 8-bit ones, 192 and 99 before).  8 kv heads of 4 query heads, us with their plans' splits and
+// the merge, before -> this: 8-bit cache, 92 rows of 4600 163 -> 155, 39 rows 79 -> 77, 64 of 2000 58 -> 53, 92 of 600 49 -> 43, one of
+// 13500 17.0 -> 16.2; bf16, 92 of 4600 277 -> 269, 39 rows 122 -> 119, 64 of 2000 85 -> 80, 92 of 600 60 -> 44, one of 32000 33.0 -> 31.9.
+// The others would spill at 128: a bf16 K cache beside an 8-bit V one, rotated q of eight and more heads.
+constexpr bool four_a_cu(int G, bool rope, int kvm) { return kvm == 3 || (kvm == 0 && (!rope || G <= 4)); }
+
 template <int G, bool ROPE, bool NT = false, int KVM = 0, bool HL = false>
-__global__ __launch_bounds__(256, 3) void attn_decode_mfma_kernel(
+__global__ __launch_bounds__(256, four_a_cu(G, ROPE, KVM) ? 4 : 3) void attn_decode_mfma_kernel(
     const bf16* __restrict__ q, int q_stride, bf16* __restrict__ kc, bf16* __restrict__ vc,
     const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ positions,
     float* __restrict__ part_o, float* __restrict__ part_ml, int Hkv, int S, float scale_log2, RopeArgs ra,
@@ -421,7 +430,7 @@ __global__ __launch_bounds__(256, 3) void attn_decode_mfma_kernel(
     // branch around the loads) so hipcc keeps them in flight.
     // (issued first by every split, the one holding the new token included: its new K/V row reaches
     // the tile through the LDS patch, so the page loads need not wait for the slab sums)
-    // TWO tiles in flight: register sets A (kreg/vreg) and B (kreg2/vreg2) alternate; the (up to two)
+    // ONE tile in flight, or two: register sets A (kreg/vreg) and B (kreg2/vreg2) alternate; the (up to two)
     // loads past the last tile stay unconditional but read the scratch page 0, which every workgroup's
     // overshoot shares and so stays in L2 (re-reading the workgroup's own last tile cost ~9 % extra HBM
     // traffic at B=39, PMC FETCH_SIZE).
@@ -449,8 +458,9 @@ __global__ __launch_bounds__(256, 3) void attn_decode_mfma_kernel(
             _Pragma("unroll") for (int i = 0; i < 4; ++i) VR[i] = ld_kv<NT>(vc + base_ + (size_t)16 * i * D); \
         }                                                                                           \
     }
+    constexpr bool ONE = four_a_cu(G, ROPE, KVM);
     KV_ISSUE(kreg, vreg, ksc, vsc, 0)
-    KV_ISSUE(kreg2, vreg2, ksc2, vsc2, 1)
+    if constexpr (!ONE) KV_ISSUE(kreg2, vreg2, ksc2, vsc2, 1)
     // ROPE: the q rows of this group (and, for the split holding the new token, its K and V rows)
     // summed over the SP slabs by ALL 256 threads in one round of independent loads into an fp32
     // LDS image (aliasing the K/V tile buffers, which are first written after it is consumed):
@@ -604,7 +614,7 @@ __global__ __launch_bounds__(256, 3) void attn_decode_mfma_kernel(
         }                                                                                                       \
     }
     KV_WRITE(kreg, vreg, ksc, vsc, 0)
-    KV_ISSUE(kreg, vreg, ksc, vsc, 2)
+    KV_ISSUE(kreg, vreg, ksc, vsc, ONE ? 1 : 2)
 
     f32x4 o[8];
 #pragma unroll
@@ -654,14 +664,29 @@ __global__ __launch_bounds__(256, 3) void attn_decode_mfma_kernel(
             }
         }
     };
-    // LDS holds tile t; set B carries tile t + 1 and set A tile t + 2 (two tiles in flight while a tile
-    // is scored); unrolled by two so every register array is indexed statically.  (Four sets in flight at
+    // LDS holds tile t; set A carries tile t + 1 (four_a_cu), or set B tile t + 1 and set A tile t + 2 (two tiles in flight while a
+    // tile is scored); unrolled by two so every register array is indexed statically.  (Four sets in flight at
     // one workgroup per CU measured SLOWER in round 5: B=1 at 13.5k +1.5-2.5 %, the TP=8 shard +10 %, the
     // overshoot loads past a short split's last tile outweighing the deeper queue: r5_attn_deep_ab.jsonl; again
     // in round 6, r6_attn_deep_ring_insitu.jsonl.  Nor did 4 staging waves beside the 4 scoring ones over two
     // LDS tile buffers: the loaders wait on the page loads, r6_attn_stamps.jsonl.)
     ST(0)
-    for (int t = 0; t < ntiles; t += 2) {
+    if constexpr (ONE) {
+        for (int t = 0; t < ntiles; ++t) {
+            compute(t);
+            ST(1)
+            __syncthreads();
+            ST(2)
+            if (t + 1 < ntiles) {
+                KV_WRITE(kreg, vreg, ksc, vsc, t + 1)
+                KV_ISSUE(kreg, vreg, ksc, vsc, t + 2)
+                ST(3)
+                __syncthreads();
+                ST(4)
+            }
+        }
+    }
+    for (int t = ONE ? ntiles : 0; t < ntiles; t += 2) {
         compute(t);
         ST(1)
         __syncthreads();

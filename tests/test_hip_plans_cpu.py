@@ -58,6 +58,16 @@ def test_decode_attn_plan_measured_choices():
     assert not fused and s == 64
 
 
+@pytest.mark.parametrize("batch,ctx,splits", [(17, 4608, 7), (39, 4608, 3), (64, 2048, 2), (92, 4608, 1), (300, 4608, 1),
+                                              (20, 128, 1), (20, 32768, 6)])
+def test_decode_attn_plan_is_one_round_of_four_workgroups_a_cu(batch, ctx, splits):
+    assert hip.decode_attn_plan(batch, 8, ctx) == (splits, False)
+    # eight query heads a kv head (three a CU), 8-bit caches (the bytes they store), up to 128 groups
+    for other in (dict(group=8), dict(kv8="fp8v"), dict(kv8="fp8")):
+        assert hip.decode_attn_plan(batch, 8, ctx, **other) == hip.decode_attn_plan_bf16(batch, 8, ctx)
+    assert hip.decode_attn_plan(16, 8, ctx) == hip.decode_attn_plan_bf16(16, 8, ctx)
+
+
 def test_decode_attn_plan_class1_six_fused_splits():
     # the <= 12k context class (level-1 reduce at ~6k), per graph bucket: 6 fused splits, in situ
     # (profiles/r4_attn_plans_insitu_class1.jsonl): batch 5 (bucket 8) and batch 10 (bucket 16) faster than 4

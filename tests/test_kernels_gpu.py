@@ -254,6 +254,35 @@ def test_attn_decode(hq, hkv, splits, fused, kv8):
         assert int(ws.counters.abs().sum()) == 0
 
 
+@pytest.mark.parametrize("kv8", ["bf16", "fp8"])
+@pytest.mark.parametrize("gate", [False, True])
+def test_attn_decode_pages_of_a_split(kv8, gate):
+    """One to six pages in a split, the last of one key or all, in the form that keeps one page in flight; with a gate the softmax
+    weights in two terms (bf16)."""
+    hq, hkv, d, page = 8, 2, 128, 64
+    ctxs = [1, 63, 64, 65, 128, 129, 192, 193, 256, 257, 320, 321, 384]
+    B, g = len(ctxs), torch.Generator().manual_seed(17)
+    kc = torch.randn(60, hkv, page, d, generator=g).to(torch.bfloat16).to(DEV)
+    vc = torch.randn(60, hkv, page, d, generator=g).to(torch.bfloat16).to(DEV)
+    kc, vc = _kv_format(kc, vc, kv8)
+    bt = torch.zeros(B, 6, dtype=torch.int32)
+    perm, used = torch.randperm(59, generator=g) + 1, 0
+    for b, c in enumerate(ctxs):
+        n = -(-c // page)
+        bt[b, :n] = perm[used:used + n]
+        used += n
+    bt, pos = bt.to(DEV), torch.tensor([c - 1 for c in ctxs], dtype=torch.int32, device=DEV)
+    q, sc = _rand(B, (hq + 2 * hkv) * d, seed=18), 1.0 / math.sqrt(d)
+    want = reference.attn_decode(q, kc, vc, bt, pos, hq, hkv, d, page, sc)
+    factors = torch.rand(B, hq, generator=g).to(DEV) if gate else None
+    if gate:
+        want = (want.view(B, hq, d).float() * factors[:, :, None]).view(B, -1)
+    for splits in (1, 2, 6):
+        ws = hip.DecodeWorkspace(B, hq, d, splits, DEV, hkv)
+        ws.part_o.fill_(float("nan"))
+        _close(hip.attn_decode(q, kc, vc, bt, pos, hq, hkv, d, page, sc, workspace=ws, gate=factors), want, 2e-2)
+
+
 @pytest.mark.parametrize("splits,fused", [(64, False), (160, False), (256, False), (256, True)])
 def test_attn_decode_many_splits_one_kv_head(splits, fused):
     """A TP shard's single kv head at a long context split up to the merge's 256 ways (decode_attn_plan's
