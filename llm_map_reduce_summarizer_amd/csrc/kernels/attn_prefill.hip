@@ -2,15 +2,26 @@
 //
 // Packed batch: qkv [T, row_stride] bf16 (Q heads, then K heads, then V
 // heads, D=128 each, already rotated by rope_kv), cu_seqlens [nseq+1].
-// Work item = (sequence, query block of 256/G positions) x KV HEAD, G = Hq / Hkv: the 8 waves
-// of a workgroup run all G query heads of their kv head (wave w: head kvh*G + w%G, rows 32(w/G)..+32), so a
-// staged K/V tile always feeds 256 query rows, and the causal diagonal of a block is only 256/G rows deep
+// Work item = (sequence, query block of 256/G positions) x KV HEAD, G = Hq / Hkv: 8 waves run all G query heads
+// of their kv head (head kvh*G + w%G, rows 32(w/G)..+32), so the causal diagonal of a block is only 256/G rows deep
 // (64 for Llama-3-8B, 32 for 70B: waves idle on masked diagonal tiles far less than with 256-row blocks of
 // one head).  Items are listed by the host heaviest-first (blocks late in a sequence do the most key tiles).
 //
-// Workgroup: 8 waves (one per CU, 2 per SIMD at ~216 VGPRs).  K/V tiles go through a two-stage LDS ring with
-// one barrier per tile: right after barrier t every wave writes tile t+1 (loaded into registers one tile
-// earlier) into the other stage and issues the global loads of tile t+2, then consumes tile t.  The LDS
+// bf16 caches and packed rows: two workgroups of four waves run an item, each half of its positions (half of its heads
+// where G is eight), and two share a CU (64 KiB of LDS and at most 218 VGPRs each).  K/V tiles go by LDS-DMA through a
+// two-stage ring with one barrier per tile: behind barrier t the loads of tile t+1 into the other stage are issued, then
+// tile t is consumed.  The loop is bound by the chain QK^T -> softmax -> P.V of a wave; two workgroups that meet at
+// barriers of their own fill each other's gaps, where the eight waves of one all stood at the same barrier, and a small
+// prompt is over twice the CUs.  Against one workgroup of eight waves that staged through registers, in us, 32 / 8 heads
+// (bits the same): paged 1 x 305 14.0 -> 10.2, 1 x 2000 61.3 -> 53.1, 2 x 4096 253.7 -> 242.5 (with two-term weights
+// 345 -> 333.5), 5 x 4000 630 -> 595, 1 x 16000 2008 -> 1966; packed 13.7 -> 10.1, 60.1 -> 52.5, 250.5 -> 243,
+// 623 -> 596, 1985 -> 1969; 32 / 32 heads 5 x 4000 703 -> 652, 32 / 4 heads 596 -> 573.
+//
+// fp8 caches: one workgroup of 8 waves an item (one per CU, 2 per SIMD at ~216 VGPRs); right after barrier t every wave
+// converts and writes tile t+1 (loaded into registers one tile earlier) into the other stage and issues the global loads
+// of tile t+2, then consumes tile t.
+//
+// The LDS
 // operand reads run ahead of their MFMAs under sched_group_barrier (8 fragments deep, counted lgkmcnt
 // waits; hipcc otherwise sank each read next to its MFMA behind an lgkmcnt(0)).  GQA packing + ring +
 // read-ahead: 8 x 4k 728 -> 873 TF/s, 1 x 32k 839 -> 1092, 70B heads 1 x 32k 874 -> 1100
@@ -53,11 +64,9 @@
 
 namespace {
 constexpr int D = 128;
-constexpr int NW = 8;             // waves per workgroup, 32 query rows each
-constexpr int NTHR = 64 * NW;
-constexpr int SROWS = NTHR / 16;  // tile rows staged per load round (16 lanes x 16 B per 256-B row)
+constexpr int NW = 8;             // waves of a work item, 32 query rows each: one workgroup, or two of four
 constexpr int BN = 64;            // keys per tile
-constexpr int SIT = BN / SROWS;   // load rounds per 64-row tile
+constexpr int waves(int kvm) { return kvm ? 8 : 4; }
 constexpr int STAGE = 2 * BN * 256;  // bytes of one ring stage: K tile | V tile
 constexpr float RESCALE_LOG2 = 8.0f;  // deferred-rescale threshold (log2 units), see the softmax
 
@@ -97,14 +106,26 @@ struct PagedKV {
 // heads", one per query head, each reading the K/V columns of its real kv head h / gq (gq = Hq / Hkv):
 // no K/V reuse across the group inside a workgroup, but any ratio works.  Hg = Hkv and gq = 1 otherwise.
 // HL: the softmax weights enter the value product as two bf16 terms (hi + lo) instead of one.
+// 1 KiB from p to LDS: lane l's 16 bytes at byte offset `off` to dst + 16 l
+__device__ __forceinline__ void dma_1k(const bf16* p, int bytes, int off, char* dst) {
+    typedef __attribute__((address_space(3))) void* lds_ptr;
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(p), (short)0, bytes, 0x00020000);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr)dst, 16, off, 0, 0, 0);
+}
+
 template <bool PAGED, int G, int KVM = 0, bool HL = false>
-__global__ __launch_bounds__(NTHR, 1) void attn_prefill_kernel(const bf16* __restrict__ qkv, int row_stride,
+__global__ __launch_bounds__(64 * waves(KVM), waves(KVM) == 4 ? 2 : 1) void attn_prefill_kernel(const bf16* __restrict__ qkv, int row_stride,
                                                               const int* __restrict__ cu_seqlens,
                                                               const int2* __restrict__ items,
                                                               bf16* __restrict__ out, int out_stride, int Hq,
                                                               int Hkv, int Hg, int gq, float scale_log2, PagedKV pk,
-                                                              int kv_major, AttnEpi ep) {
-    constexpr int BMP = 32 * (NW / G);  // query positions per workgroup
+                                                              int kv_major, int n_items, AttnEpi ep) {
+    constexpr int WV = waves(KVM), PARTS = NW / WV;  // waves of this workgroup, workgroups of a work item
+    constexpr int NTHR = 64 * WV, SROWS = NTHR / 16, SIT = BN / SROWS;  // staging: tile rows of a round, rounds
+    constexpr bool DMA = KVM == 0;
+    static_assert(PAGED || DMA, "packed rows are bf16");
+    constexpr int HW = G < WV ? G : WV;  // heads of this workgroup: of eight, each of an item's workgroups takes four
+    constexpr int BMP = 32 * (WV / HW);  // query positions per workgroup
     // two-stage ring of [K tile | V tile]: tile t+1 is written into the other stage while tile t is
     // consumed, one barrier per tile
     __shared__ __attribute__((aligned(16))) char lds[2 * STAGE];
@@ -114,16 +135,20 @@ __global__ __launch_bounds__(NTHR, 1) void attn_prefill_kernel(const bf16* __res
     // kv head 0-6's lists (1 x 4k: 580 vs 870 TF/s).  Large grids (kv_major = 1): block b = kv head
     // b / n_items x item b % n_items, so the blocks in flight share one kv head and its K/V stays in the
     // Infinity Cache (39 x 4k: 912 vs 815 TF/s); profiles/r3_attn_prefill_grid_order_ab.jsonl.
-    const int n_items = gridDim.x / Hg;
-    const int item = kv_major ? blockIdx.x % n_items : blockIdx.x / Hg;
+    // The two workgroups of an item are eight blocks apart: on the same XCD, at about the same time.
+    const int block = PARTS == 1 ? blockIdx.x : (blockIdx.x & 7) + 8 * (blockIdx.x >> 4);
+    const int part = PARTS == 1 ? 0 : (blockIdx.x >> 3) & 1;
+    if (PARTS == 2 && block >= n_items * Hg) return;
+    const int item = kv_major ? block % n_items : block / Hg;
     const int2 it = items[item];
-    const int seq = it.x, qblock = it.y;
-    const int kvg = kv_major ? blockIdx.x / n_items : blockIdx.x % Hg;  // head group of this workgroup
+    const int seq = it.x, qblock = it.y + (HW == G ? part * BMP : 0);
+    const int kvg = kv_major ? block / n_items : block % Hg;  // head group of this workgroup
     const int kvh = G == 1 ? kvg / gq : kvg;                             // its real kv head
     const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, r32 = lane & 31;
     const int w = tid >> 6;
-    const int h = G == 1 ? kvg : kvh * G + w % G, rb = w / G;
+    const int h = G == 1 ? kvg : kvh * G + (HW == G ? 0 : part * HW) + w % HW, rb = w / HW;
     const int s0 = cu_seqlens[seq], len = cu_seqlens[seq + 1] - s0;
+    if (PARTS == 2 && qblock >= len) return;
     const bf16* base = qkv + (size_t)s0 * row_stride;
     const int kcol = (Hq + kvh) * D, vcol = (Hq + Hkv + kvh) * D;
     // keys live at absolute positions [0, pre + len); query row qi at pre + qi
@@ -149,9 +174,8 @@ __global__ __launch_bounds__(NTHR, 1) void attn_prefill_kernel(const bf16* __res
     const int kend = pre + min(len, qblock + BMP);
     const int ntiles = (kend + BN - 1) / BN;
 
-    // staging: thread loads rows tid/16 + SROWS i (i < SIT), chunk tid%16.  Named u32x4 registers and
-    // UNCONDITIONAL loads (tile index clamped to the last tile, key clamped to the last row of the
-    // sequence; such rows are masked out of the scores and V rows stay finite) -- a conditional prefetch
+    // staging of fp8 caches: thread loads bf16 rows tid/16 + SROWS i (i < SIT), chunk tid%16.  Named u32x4 registers and
+    // UNCONDITIONAL loads (tile index clamped to the last tile) -- a conditional prefetch
     // made hipcc serialise the loop on vmcnt(0).
     const int st_chunk = tid & 15, st_row0 = tid >> 4;
     u32x4 kreg[SIT], vreg[SIT];
@@ -160,8 +184,37 @@ __global__ __launch_bounds__(NTHR, 1) void attn_prefill_kernel(const bf16* __res
     float ks8 = 1.f, vs8 = 1.f;
     constexpr bool K8 = (KVM & 1) != 0, V8 = (KVM & 2) != 0;
     static_assert(KVM == 0 || NTHR / 8 == BN, "fp8 slab staging: one slab row per 8 threads");
+    // bf16 tiles by LDS-DMA: 4 rows = 1 KiB an instruction, 16 / WV instructions of K and of V a wave; lane l fills position l & 15
+    // of row l >> 4 with the chunk that the swizzle keeps there
+    int page = 0;  // of the tile staged next
+    const int dma_row = (64 / WV) * w + (lane >> 4), pitch = 2 * (PAGED ? D : row_stride);
+    int dma_r[16 / WV], dma_k[16 / WV];
+    const int dma_v = ((lane & 15) ^ ((dma_row & 3) << 2)) * 16;
+#pragma unroll
+    for (int i = 0; i < 16 / WV; ++i) {
+        dma_r[i] = (dma_row + 4 * i) * pitch;
+        dma_k[i] = ((lane & 15) ^ ((dma_row + 4 * i) & 15)) * 16;
+    }
+    auto stage = [&](int t, int st) {
+        char* dst = lds + st + (16 / WV) * __builtin_amdgcn_readfirstlane(w) * 1024;
+        const bf16 *kp, *vp;
+        if constexpr (PAGED) {
+            const size_t pg = (size_t)__builtin_amdgcn_readfirstlane(page) * Hkv * BN * D + head_pg;
+            kp = pk.kc + pg, vp = pk.vc + pg;
+        } else {
+            kp = base + (size_t)t * BN * row_stride + kcol, vp = kp - kcol + vcol;
+        }
+        const int last = (min(BN, len - t * BN) - 1) * pitch;  // behind the sequence's last row that one again
+#pragma unroll
+        for (int i = 0; i < 16 / WV; ++i) {
+            const int r = PAGED ? dma_r[i] : min(dma_r[i], last);
+            dma_1k(kp, BN * pitch, r + dma_k[i], dst + i * 1024);
+            dma_1k(vp, BN * pitch, r + dma_v, dst + BN * 256 + i * 1024);
+        }
+        if constexpr (PAGED) page = btab[min(t + 1, ntiles - 1)];
+    };
 #define LOAD_TILE(t)                                                                              \
-    if constexpr (PAGED && KVM != 0) {                                                            \
+    if constexpr (!DMA) {                                                                         \
         const size_t sb = kv8::slab_off(btab[t], Hkv, kvh);                                       \
         const size_t pg = (size_t)btab[t] * Hkv * BN * D + head_pg + st_chunk * 8;                \
         if constexpr (K8) {                                                                       \
@@ -180,22 +233,9 @@ __global__ __launch_bounds__(NTHR, 1) void attn_prefill_kernel(const bf16* __res
             _Pragma("unroll") for (int i = 0; i < SIT; ++i)                                         \
                 vreg[i] = *reinterpret_cast<const u32x4*>(pk.vc + pg + (size_t)(st_row0 + SROWS * i) * D); \
         }                                                                                         \
-    } else if constexpr (PAGED) {                                                                 \
-        const size_t pg = (size_t)btab[t] * Hkv * BN * D + head_pg + st_chunk * 8;                \
-        _Pragma("unroll") for (int i = 0; i < SIT; ++i) {                                           \
-            kreg[i] = *reinterpret_cast<const u32x4*>(pk.kc + pg + (size_t)(st_row0 + SROWS * i) * D); \
-            vreg[i] = *reinterpret_cast<const u32x4*>(pk.vc + pg + (size_t)(st_row0 + SROWS * i) * D); \
-        }                                                                                         \
-    } else {                                                                                      \
-        _Pragma("unroll") for (int i = 0; i < SIT; ++i) {                                           \
-            const int key = min((t) * BN + st_row0 + SROWS * i, len - 1);                           \
-            const bf16* p = base + (size_t)key * row_stride + st_chunk * 8;                      \
-            kreg[i] = *reinterpret_cast<const u32x4*>(p + kcol);                                 \
-            vreg[i] = *reinterpret_cast<const u32x4*>(p + vcol);                                 \
-        }                                                                                         \
     }
 #define STORE_TILE(st)                                                                            \
-    if constexpr (KVM != 0) {                                                                     \
+    if constexpr (!DMA) {                                                                         \
         u32x4 lo_, hi_;                                                                           \
         if constexpr (K8) {                                                                       \
             kv8::dequant16(kreg[0], ks8, lo_, hi_);                                               \
@@ -213,11 +253,6 @@ __global__ __launch_bounds__(NTHR, 1) void attn_prefill_kernel(const bf16* __res
             _Pragma("unroll") for (int i = 0; i < SIT; ++i)                                         \
                 *reinterpret_cast<u32x4*>(lds + (st) + BN * 256 + v_off(st_row0 + SROWS * i, st_chunk)) = vreg[i]; \
         }                                                                                         \
-    } else                                                                                        \
-    _Pragma("unroll") for (int i = 0; i < SIT; ++i) {                                               \
-        const int row = st_row0 + SROWS * i;                                                         \
-        *reinterpret_cast<u32x4*>(lds + (st) + k_off(row, st_chunk)) = kreg[i];                    \
-        *reinterpret_cast<u32x4*>(lds + (st) + BN * 256 + v_off(row, st_chunk)) = vreg[i];         \
     }
 
     f32x16 o[4];
@@ -225,9 +260,14 @@ __global__ __launch_bounds__(NTHR, 1) void attn_prefill_kernel(const bf16* __res
     for (int dt = 0; dt < 4; ++dt) o[dt] = f32x16{};
     float m = -INFINITY, l = 0.f;
 
-    LOAD_TILE(0);
-    STORE_TILE(0);
-    LOAD_TILE(min(1, ntiles - 1));
+    if constexpr (DMA) {
+        if constexpr (PAGED) page = btab[0];
+        stage(0, 0);
+    } else {
+        LOAD_TILE(0);
+        STORE_TILE(0);
+        LOAD_TILE(min(1, ntiles - 1));
+    }
 
     const int wave_last_q = pre + q0 + 31;  // absolute position of the wave's last row
     // PV operand addressing (loop-invariant parts): lane (g, q4, p4) reads V rows 4(g>>1) + q4 (+8) of each
@@ -245,27 +285,36 @@ __global__ __launch_bounds__(NTHR, 1) void attn_prefill_kernel(const bf16* __res
         const int cur = (t & 1) * STAGE;
         const int kv0 = t * BN;
         const bool act = kv0 <= wave_last_q;  // wave-uniform: tiles wholly above the diagonal are skipped
-        __syncthreads();  // tile t visible in stage t&1; every wave is done with tile t-1 (stage (t+1)&1)
-        STORE_TILE(STAGE - cur);
-        LOAD_TILE(min(t + 2, ntiles - 1));
+        // tile t visible in stage t&1; every wave is done with tile t-1 (stage (t+1)&1)
+        if constexpr (DMA) {
+            __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (0 << 8));  // this wave's pieces of tile t are there, its reads of t - 1 done
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // for the compiler alone
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            if (t + 1 < ntiles) stage(t + 1, STAGE - cur);
+        } else {
+            __syncthreads();
+            STORE_TILE(STAGE - cur);
+            LOAD_TILE(min(t + 2, ntiles - 1));
+        }
         const char* ldsK = lds + cur;
         const char* ldsV = ldsK + BN * 256;
         if (!act) continue;
         // S^T = K Q^T: all 16 K fragments read up front (64 VGPRs, dead after the QK^T MFMAs), so the
         // ds_reads run ahead of the MFMA chain instead of one exposed LDS round trip per MFMA
-        uint4 kf[2][8];
+        u32x4 kf[2][8];
         f32x16 sacc[2];
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
             for (int ks = 0; ks < 8; ++ks)
-                kf[kt][ks] = *reinterpret_cast<const uint4*>(ldsK + k_off(kt * 32 + r32, 2 * ks + half));
+                kf[kt][ks] = *reinterpret_cast<const u32x4*>(ldsK + k_off(kt * 32 + r32, 2 * ks + half));
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt) {
             sacc[kt] = f32x16{};
 #pragma unroll
             for (int ks = 0; ks < 8; ++ks)
-                sacc[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(kf[kt][ks]), qf[ks], sacc[kt], 0, 0, 0);
+                sacc[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kf[kt][ks]), qf[ks], sacc[kt], 0, 0, 0);
         }
         // schedule (cdna_hip_programming.md T19): 8 reads ahead, then one read per MFMA gap -- without it the
         // machine scheduler sinks every read next to its MFMA and waits lgkmcnt(0) before each one
@@ -395,30 +444,31 @@ template <bool PAGED, int G>
 static void launch_g(dim3 grid, hipStream_t s, const bf16* Q, int row_stride, const int* cu, const int2* it, bf16* out,
                      int out_stride, int Hq, int Hkv, int Hg, int gq, float sl, const PagedKV& p, int kv8, const AttnEpi& ep, bool hl) {
     // kv-head-major order from 8 blocks per CU up (measured crossover: 4096 blocks neutral, 19656 kv-major)
-    const int kv_major = grid.x > 8 * 256;
+    const int kv_major = grid.x > 8 * 256, n_items = grid.x / Hg;
+    const dim3 grid2(16 * ((grid.x + 7) / 8));
     if constexpr (PAGED) {
         if (kv8 == 3 || kv8 == 2) {
             if (kv8 == 3)
-                attn_prefill_kernel<PAGED, G, 3><<<grid, NTHR, 0, s>>>(Q, row_stride, cu, it, out, out_stride, Hq,
-                                                                       Hkv, Hg, gq, sl, p, kv_major, ep);
+                attn_prefill_kernel<PAGED, G, 3><<<grid, 64 * waves(3), 0, s>>>(Q, row_stride, cu, it, out, out_stride, Hq,
+                                                                       Hkv, Hg, gq, sl, p, kv_major, n_items, ep);
             else
-                attn_prefill_kernel<PAGED, G, 2><<<grid, NTHR, 0, s>>>(Q, row_stride, cu, it, out, out_stride, Hq,
-                                                                       Hkv, Hg, gq, sl, p, kv_major, ep);
+                attn_prefill_kernel<PAGED, G, 2><<<grid, 64 * waves(3), 0, s>>>(Q, row_stride, cu, it, out, out_stride, Hq,
+                                                                       Hkv, Hg, gq, sl, p, kv_major, n_items, ep);
             return;
         }
         if (hl) {
-            attn_prefill_kernel<PAGED, G, 0, true><<<grid, NTHR, 0, s>>>(Q, row_stride, cu, it, out, out_stride, Hq,
-                                                                         Hkv, Hg, gq, sl, p, kv_major, ep);
+            attn_prefill_kernel<PAGED, G, 0, true><<<grid2, 64 * waves(0), 0, s>>>(Q, row_stride, cu, it, out, out_stride, Hq,
+                                                                         Hkv, Hg, gq, sl, p, kv_major, n_items, ep);
             return;
         }
     }
-    attn_prefill_kernel<PAGED, G, 0><<<grid, NTHR, 0, s>>>(Q, row_stride, cu, it, out, out_stride, Hq, Hkv, Hg,
-                                                                   gq, sl, p, kv_major, ep);
+    attn_prefill_kernel<PAGED, G, 0><<<grid2, 64 * waves(0), 0, s>>>(Q, row_stride, cu, it, out, out_stride, Hq, Hkv, Hg,
+                                                                   gq, sl, p, kv_major, n_items, ep);
 }
 
 static bool packed_ratio(int G) { return G == 1 || G == 2 || G == 4 || G == 8; }
 
-// Query positions per workgroup for a GQA ratio (the host's work list must use the same block size):
+// Query positions per work item for a GQA ratio (the host's work list must use the same block size):
 // 256 / G for the packed ratios, 256 for the per-query-head fallback of any other ratio.
 MRSUM_API int mrsum_attn_prefill_block_m(int Hq, int Hkv) {
     if (Hkv <= 0 || Hq % Hkv || Hq / Hkv > 64) return -1;

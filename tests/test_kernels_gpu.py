@@ -202,6 +202,33 @@ def test_attn_prefill_paged(hq, hkv, spans, kv8):
     _close(o1, o2, 2e-2)
 
 
+@pytest.mark.parametrize("hq,hkv", [(8, 8), (4, 2), (8, 2), (16, 2), (6, 2)])
+@pytest.mark.parametrize("edge", [-1, 0, 1])
+def test_attn_prefill_halves_of_an_item(hq, hkv, edge):
+    """Two workgroups run the query block of a work item: sequences that end before, at and behind the first one's last
+    position (the second has no row, or one), in the first block and in a later one, over packed rows and over pages."""
+    from llm_map_reduce_summarizer_amd.ops import PagedPrefill
+    d, block = 128, hip.prefill_block_m(hq // hkv)
+    lens = [block // 2 + edge, block + edge, 3 * block // 2 + edge, 65]
+    qkv, sc = _rand(sum(lens), (hq + 2 * hkv) * d, seed=13), 1.0 / math.sqrt(d)
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32, device=DEV)
+    want = reference.attn_prefill(qkv, cu, hq, hkv, d, sc)
+    _close(hip.attn_prefill(qkv, cu, hq, hkv, d, sc), want, 2e-2)
+    pages = [-(-n // 64) for n in lens]
+    kc, vc = (torch.full((sum(pages) + 1, hkv, 64, d), 7.0, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    bt, page = torch.zeros(len(lens), max(pages), dtype=torch.int32), sum(pages)
+    for i, n in enumerate(lens):
+        rows = qkv[int(cu[i]):int(cu[i]) + n].view(n, hq + 2 * hkv, d).transpose(0, 1)
+        for p in range(pages[i]):
+            m = min(64, n - 64 * p)
+            kc[page, :, :m], vc[page, :, :m] = rows[hq:hq + hkv, 64 * p:64 * p + m], rows[hq + hkv:, 64 * p:64 * p + m]
+            bt[i, p], page = page, page - 1
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)  # noqa: E731
+    slots, pre = list(range(len(lens))), [0] * len(lens)
+    pp = PagedPrefill(bt.to(DEV), i32(slots), i32(pre), slots, pre, kc, vc)
+    _close(hip.attn_prefill(qkv, cu, hq, hkv, d, sc, paged=pp), want, 2e-2)
+
+
 @pytest.mark.parametrize("hq", [4, 8])
 def test_attn_prefill_spike(hq):
     """A key far larger than the rest forces the online-softmax rescale path mid-sequence."""
