@@ -24,8 +24,8 @@ from __future__ import annotations
 import functools
 import logging
 import os
+import struct
 import time
-from array import array
 from dataclasses import dataclass, field
 from types import SimpleNamespace
 from typing import Dict, List, Optional, Sequence, Tuple
@@ -50,18 +50,18 @@ def _always() -> bool:
 
 def _token_ids(toks: Sequence[int], vocab: int) -> np.ndarray:
     """The ids as int32, checked to be non-empty and in range."""
-    if not isinstance(toks, (list, tuple)):  # read once; array() would take bytes for memory
+    if not isinstance(toks, (list, tuple)):  # read once
         toks = list(toks)
     if len(toks) == 1 and type(toks[0]) is int and 0 <= toks[0] < vocab:  # a decoded row: 5 us less than below
         return np.array(toks, dtype=np.int32)
-    try:
-        a = np.frombuffer(array("q", toks), dtype=np.int64) if len(toks) else None  # 20 ns an id
-    except (TypeError, OverflowError):  # ids that are not plain integers
+    try:  # 9 ns an id, 18 by way of an array
+        a = np.frombuffer(struct.pack("%di" % len(toks), *toks), dtype=np.int32) if len(toks) else None
+    except struct.error:  # ids that are not plain integers, or far out of range
         a = [int(t) for t in toks]
-        a = None if min(a) < 0 or max(a) >= vocab else np.asarray(a)
-    if a is None or int(a.min()) < 0 or int(a.max()) >= vocab:
+        a = None if min(a) < 0 or max(a) >= vocab else np.asarray(a, dtype=np.int32)
+    if a is None or int(a.view(np.uint32).max()) >= vocab:  # (negative ids are large ones)
         raise ValueError("empty step entry or token id out of range")
-    return a.astype(np.int32)
+    return a
 
 
 class _Upload:
@@ -433,7 +433,7 @@ class LLMEngine:
             rows = [int(cu[k + 1]) - 1 for k in range(len(spans)) if sample is None or sample[k]]
         up = _Upload()
         at = {"ids": up.add(np.concatenate([np.asarray(s.prompt[b:e], dtype=np.int32) for s, (b, e) in zip(seqs, spans)])),
-              "positions": up.add(np.concatenate([np.arange(b, e, dtype=np.int32) for b, e in spans])),
+              "positions": up.add(np.arange(cu[-1], dtype=np.int32) - np.repeat(cu[:-1] - np.asarray(pre, dtype=np.int32), lens)),
               "seq_idx": up.add(np.repeat(np.asarray(slots, dtype=np.int32), lens)), "cu_seqlens": up.add(cu),
               "last_rows": up.add(rows, np.int64)}
         recurrent = self.model.recurrent
@@ -744,12 +744,13 @@ class LLMEngine:
             b = len(s.prompt)
             if b + len(toks) > self.max_model_len:
                 raise ValueError("request of %d tokens exceeds max_model_len %d" % (b + len(toks), self.max_model_len))
-            need = self.kv.pages_for(b + len(toks)) - len(s.pages)
-            if need > self.kv.alloc.available():
-                raise MemoryError("KV cache exhausted: %d pages needed, %d free" % (need, self.kv.alloc.available()))
             held = len(s.pages)
-            self._hold(s, need)
-            self._stepped[rid] = s
+            need = self.kv.pages_for(b + len(toks)) - held
+            if need > 0 and need > self.kv.alloc.available():
+                raise MemoryError("KV cache exhausted: %d pages needed, %d free" % (need, self.kv.alloc.available()))
+            if need or rid not in self._stepped:  # (most decoded rows need nothing)
+                self._hold(s, need)
+                self._stepped[rid] = s
             if need:
                 pages.append((s.pf_slot * self.max_pages + held, s.pages[held:]))
             s.prompt = toks if b == 0 else np.concatenate((s.prompt, toks))  # (stepped requests keep their ids as an array)

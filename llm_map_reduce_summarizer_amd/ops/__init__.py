@@ -18,7 +18,7 @@ from __future__ import annotations
 import numpy as np
 import torch
 
-from . import reference
+from . import hip, reference
 from .reference import Fp8Weight
 
 def _use_hip(t) -> bool:
@@ -27,7 +27,6 @@ def _use_hip(t) -> bool:
 
 def _impl(t):
     if _use_hip(t):
-        from . import hip
         return hip
     return reference
 
@@ -51,7 +50,6 @@ def rmsnorm(x, w, eps, out=None, quant=False):
     if w is None:
         w = unit_gain(x.shape[-1], x.device)
     if quant and out is None and _quant_ok(x):
-        from . import hip
         return QuantRows(*hip.rmsnorm_fp8(x, w, eps, split=quant == "split"))
     return _impl(x).rmsnorm(x, w, eps, out)
 
@@ -76,7 +74,6 @@ class NormRows:
         return (self.ssq, self.eps)
 
     def materialize(self):
-        from . import hip
         return hip.rmsnorm(self.h, unit_gain(self.h.shape[1], self.h.device), self.eps)
 
 
@@ -108,7 +105,6 @@ def _quant_ok(x) -> bool:
     """Prefill rows that every fp8 consumer sends to the fp8 MFMA GEMM (above the stream kernels' rows)."""
     if not _use_hip(x):
         return False
-    from . import hip
     return x.shape[0] > max(hip.STREAM_MAX_M, hip.STREAM_MAX_M_SWIGLU) and x.shape[1] % 16 == 0
 
 
@@ -144,7 +140,6 @@ def linear(x, w):
     otherwise; ``w`` may be an Fp8Weight (W8A16 decode kernel / fp8 MFMA GEMM at prefill sizes).
     ``x`` may be a NormRows (the LM head after the last layer)."""
     if isinstance(x, NormRows):
-        from . import hip
         M, K = x.shape
         if isinstance(w, Fp8Weight):
             if hip.fp8_stream_cfg(M, w.shape[0], K, splits=1) is not None:
@@ -154,7 +149,6 @@ def linear(x, w):
         x = x.materialize()
     if isinstance(w, Fp8Weight):
         if _use_hip(x):
-            from . import hip
             return hip.fp8_linear(x, w)
         return reference.linear(x, w)
     return _impl(x).linear(x, w)
@@ -163,7 +157,6 @@ def linear(x, w):
 def linear_parts(x, w, splits=None):
     """fp32 split-K partial slabs [S, M, N] of x @ w^T, consumed by add_rmsnorm_parts."""
     if _use_hip(x):
-        from . import hip
         return hip.linear_parts(x, w, splits)
     return reference.linear_parts(x, w, splits or 1)
 
@@ -198,7 +191,6 @@ class PagedPrefill:
 def attn_prefill(qkv, cu_seqlens, hq, hkv, d, scale, out=None, paged=None, **kw):
     """``gate`` fp32 [T, hq] and ``pitch`` (GPU): per-head output factors and the width of one head in ``out``."""
     if _use_hip(qkv):
-        from . import hip
         return hip.attn_prefill(qkv, cu_seqlens, hq, hkv, d, scale, out, paged=paged, **kw)
     if paged is not None:
         return reference.attn_prefill_paged(qkv, cu_seqlens, hq, hkv, d, scale, paged, out)
@@ -210,11 +202,9 @@ def attn_decode(q, kcache, vcache, block_tables, positions, hq, hkv, d, page, sc
     """``q``: bf16 rows [B, hq * d] (already rotated, K/V already in the cache) or a QKVParts.  ``gate`` / ``pitch``
     (bf16 rows on the GPU): as attn_prefill."""
     if isinstance(q, QKVParts):
-        from . import hip
         return hip.attn_decode_rope(q.parts, q.cos_sin, kcache, vcache, block_tables, positions, hq, hkv, d,
                                     page, scale, out, workspace=workspace)
     if _use_hip(q):
-        from . import hip
         return hip.attn_decode(q, kcache, vcache, block_tables, positions, hq, hkv, d, page, scale, out,
                                workspace=workspace, gate=gate, pitch=pitch)
     return reference.attn_decode(q, kcache, vcache, block_tables, positions, hq, hkv, d, page, scale, out)
@@ -268,7 +258,6 @@ def project(x, w, role):
     a whole product ("o", "down"), and always in fp32 mode; else 16-bit rows [T, N] of the MFMA GEMM."""
     if not _use_hip(x):
         return reference.project(x, w)
-    from . import hip
     if x.dtype == torch.float32:
         return hip.gemm32(x, w)[None]
     M, (N, K) = x.shape[0], w.shape
@@ -404,38 +393,32 @@ def latent_out(o, m, w_uv, a, col):
 
 def latent_decode(q, cache, block_tables, positions, heads, rank, page, scale, workspace):
     """Split-K attention of decoded tokens over the cached rows (GPU): unmerged partial sums, see latent_out_parts."""
-    from . import hip
     return hip.latent_decode(q, cache, block_tables, positions, heads, rank, page, scale, workspace)
 
 
 def latent_out_parts(parts, m, w_uv, a, col):
     """latent_out of latent_decode's partial sums, merged on the way in (GPU)."""
-    from . import hip
     return hip.latent_out_parts(parts, m, w_uv, a, col)
 
 
 def latent_gather(cache, ctx, block_tables, width, page):
     """The cached rows of a pass's sequences side by side [ctx.rows, width], zeros behind the row (GPU)."""
-    from . import hip
     return hip.latent_gather(cache, ctx, block_tables, width, page)
 
 
 def latent_expand(lat, w_kv):
     """Gathered latents -> unrotated keys and values of every head (GPU)."""
-    from . import hip
     x = lat[:, : w_kv.shape[1]]
     return hip.gemm(x, w_kv)
 
 
 def latent_rope(q, first, m, cs, positions):
     """Query rows from ``first`` on with their rotated parts turned (GPU): bf16 [T - first, H * qw]."""
-    from . import hip
     return hip.latent_rope(q, first, m, cs, positions)
 
 
 def latent_prefill(q, kv, lat, ctx, m, cu, lens, items, scale, out, col):
     """Causal attention of prompt portions over expanded keys and values (GPU); heads at out[:, col + h * vp :]."""
-    from . import hip
     return hip.latent_prefill(q, kv, lat, ctx, m, cu, lens, items, scale, out, col)
 
 
@@ -451,7 +434,6 @@ def delta_mix(x, u, m, a_neg, dt_bias, norm, eps, state, segs, a):
 
 def sample(logits, st):
     if _use_hip(logits):
-        from . import hip
         return hip.sample(logits, st)
     n = logits.shape[0]
     toks = reference.sample_tokens(logits, st.temps[:n], st.seeds[:n], st.positions[:n])
@@ -460,7 +442,6 @@ def sample(logits, st):
 
 def sample_tp(logits, st, tok_offset, max_reduce):
     """Vocab-parallel sampling over this rank's logits shard (GPU only; see hip.sample_tp)."""
-    from . import hip
     return hip.sample_tp(logits, st, tok_offset, max_reduce)
 
 
@@ -521,7 +502,6 @@ class QKVParts:
         self.hq, self.hkv, self.d, self.page = hq, hkv, d, page
 
     def materialize(self):
-        from . import hip
         return hip.rope_kv_parts(self.parts, self.positions, self.seq_idx, self.block_tables, self.kcache,
                                  self.vcache, self.cos_sin, self.hq, self.hkv, self.d, self.page)
 
@@ -535,13 +515,11 @@ def qkv_rope(x, wqkv, positions, seq_idx, block_tables, kcache, vcache, cos_sin,
     ``defer`` on the GPU decode path, a QKVParts for attn_decode's fused RoPE + KV write.  ``x`` may
     be a NormRows (deferred RMSNorm of the previous layer's down projection)."""
     if isinstance(x, QuantRows):
-        from . import hip
         qkv = hip.fp8_linear(x.pair, wqkv)
         hip.rope_kv(qkv, positions, seq_idx, block_tables, kcache, vcache, cos_sin, hq, hkv, d, page)
         return qkv
     xt = x.h if isinstance(x, NormRows) else x
     if _use_hip(xt) and isinstance(wqkv, Fp8Weight):
-        from . import hip
         if x.shape[0] <= hip.SKINNY_MAX_M:
             parts = _fp8_parts(hip, x, wqkv, "qkv", None)
             if _defer_ok(hip, defer, x, hq, hkv, d, page):
@@ -552,7 +530,6 @@ def qkv_rope(x, wqkv, positions, seq_idx, block_tables, kcache, vcache, cos_sin,
         hip.rope_kv(qkv, positions, seq_idx, block_tables, kcache, vcache, cos_sin, hq, hkv, d, page)
         return qkv
     if _use_hip(xt):
-        from . import hip
         p = hip.plan("qkv", x.shape[0], wqkv.shape[0], wqkv.shape[1])
         if p[0] != "gemm":
             parts = _plan_parts(hip, p, x, wqkv, None)
@@ -658,7 +635,6 @@ def proj_add_rmsnorm(a, w, residual, ln, eps, role="o", all_reduce=None, quant=F
     all-reduce) the decode path runs the projection's split-K slabs straight into one fused
     all-reduce + residual add + RMSNorm kernel."""
     if _use_hip(a):
-        from . import hip
         if ln is None and a.shape[0] <= hip.SKINNY_MAX_M:
             # TP: the producer all-reduces its own tiles (TP push) when the group's buffers take the rows
             ok = getattr(all_reduce, "push_ok", None)
@@ -680,7 +656,6 @@ def proj_add_rmsnorm(a, w, residual, ln, eps, role="o", all_reduce=None, quant=F
     if ln is None:
         ln = unit_gain(residual.shape[1], residual.device)
     if _use_hip(a) and isinstance(w, Fp8Weight):
-        from . import hip
         if a.shape[0] <= hip.SKINNY_MAX_M:
             fused = _fused_ar(all_reduce, a.shape[0], residual.shape[1])
             parts = _fp8_parts(hip, a, w, role, 1 if (all_reduce and not fused) else None)
@@ -696,7 +671,6 @@ def proj_add_rmsnorm(a, w, residual, ln, eps, role="o", all_reduce=None, quant=F
             return QuantRows(*hip.rmsnorm_fp8(o, ln, eps, residual=residual, split=quant == "split"))
         return hip.add_rmsnorm(o, residual, ln, eps)
     if _use_hip(a):
-        from . import hip
         fused = _fused_ar(all_reduce, a.shape[0], residual.shape[1])
         one = 1 if (all_reduce and not fused) else None  # a plain all-reduce takes one slab
         if not all_reduce and not quant and a.shape[0] > hip.STREAM_TALL_M:
@@ -737,16 +711,13 @@ def gate_up_swiglu(x, wgu, glu=None):
     """silu(gate) * up (``glu`` = (limit, alpha, shift): the clamped form, bf16 weights) of the fused,
     [8 gate | 8 up]-blocked gate_up projection; ``x`` may be a NormRows (deferred RMSNorm) or QuantRows (fp8 prefill rows quantised by the norm)."""
     if isinstance(x, QuantRows):
-        from . import hip
         return hip.fp8_linear_swiglu(x.pair, wgu)
     xt = x.h if isinstance(x, NormRows) else x
     if _use_hip(xt) and isinstance(wgu, Fp8Weight):
-        from . import hip
         if isinstance(x, NormRows) and hip.fp8_swiglu_takes_norm(x.shape[0], wgu.shape[0], x.shape[1]):
             return hip.fp8_linear_swiglu(x.h, wgu, norm=x.norm)
         return hip.fp8_linear_swiglu(rows(x), wgu)
     if _use_hip(xt):
-        from . import hip
         p = hip.plan("gate_up", x.shape[0], wgu.shape[0], wgu.shape[1])
         nr = isinstance(x, NormRows) and p[0] in ("stream", "stream_split", "skinny")
         xin, norm = (x.h, x.norm) if nr else (rows(x), None)
