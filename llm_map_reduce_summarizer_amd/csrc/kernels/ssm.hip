@@ -5,8 +5,9 @@
 // slot holds.  Projections arrive as 16-bit rows or fp32 split-K slabs (common.h ProjSrc).
 //
 //   conv_silu    xBC columns -> silu(conv) rows of width C; the slot keeps the last taps - 1 inputs
-//   ssm_step     S = exp(a dt) S + dt x B^T, y = S C + D x, token by token with S^T in registers (decode; prompt portions of
-//                fp32 models and of head sizes the chunked form does not take, with the rows ahead staged in LDS)
+//   ssm_step     S = exp(a dt) S + dt x B^T, y = S C + D x, token by token with S^T in registers (decode; short prompt
+//                portions of fp32 models and those of head sizes the chunked forms do not take, with the rows ahead staged
+//                in LDS)
 //   gated_norm   y silu(z), RMS norm in equal parts, weight, mixer scale -> the output projection's input columns
 //
 // State S^T is [slots][heads][vdim][N4] fp32 (N4: state size rounded up to 4, zeros past it).

@@ -285,6 +285,22 @@ def c_parameters():
     return found
 
 
+@pytest.mark.parametrize("rows,heads,vdim,chunks", [
+    # token by token and in chunks, us (state 128)
+    ([24], 128, 64, False),        # 10.7, 15.2
+    ([64], 128, 64, True),         # 19.2, 16.8
+    ([900], 128, 64, True),        # 228, 76
+    ([40] * 8, 128, 64, False),    # 51, 59
+    ([80] * 8, 128, 64, False),    # 87, 95
+    ([128] * 8, 128, 64, True),    # 128, 99
+    ([1200] * 4, 128, 64, True),   # 559, 340
+    ([900], 24, 64, True),         # 209, 72
+    ([64] * 40, 128, 128, False),  # 519, 556
+    ([], 128, 64, False)])
+def test_fp32_scan_in_chunks(rows, heads, vdim, chunks):
+    assert hip.ssm_chunk32_rows(rows, heads, vdim) == chunks
+
+
 def test_signatures_match_the_kernels():
     """ctypes checks nothing: a signature with another number of arguments reads the rest from the stack."""
     pars = c_parameters()
