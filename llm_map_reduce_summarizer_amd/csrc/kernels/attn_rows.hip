@@ -159,9 +159,10 @@ MRSUM_API int mrsum_attn_rows(const void* q, const void* kc, const void* vc, con
 // ------------------------------------------------------------------------------------------------ prompt portions
 // The same attention for many rows of few sequences, on the fp32 matrix instruction.  The row kernel reads every key
 // from memory for every (row, head): 1088 us for 900 rows of 32 heads of 128 over 8 kv heads, 4380 over 576-wide latents.
-// Here (183 and 755 us, 36 TFLOP/s; the exponentials and their exchange are the rest) 64 (row, head) pairs -- RB
-// consecutive rows of HB heads of one kv head -- share key and value tiles of 32 in LDS (two buffers, the next tile on its
-// way in registers), a wave for 16 pairs.
+// Here (163 and 520 us; bound by the chain of the block with the most keys, 5.5 us a tile of which its products are 1.7) 64
+// (row, head) pairs -- RB consecutive rows of HB heads of one kv head -- share key and value tiles of 32 in LDS (two buffers,
+// the next tile on its way in registers), a wave for 16 pairs.  With the page ids read when a tile is fetched, its loads
+// behind tests of the row and two barriers a tile, 183 and 758 (16-bit caches 201 and 915, now 167 and 570).
 //
 // Scores are computed transposed, S^T = K Q^T: lane (pair = lane & 15, g = lane >> 4) holds the scores of keys 4 g .. 4 g
 // + 3 of a 16-key block, which is how the second product O^T = V^T P^T takes its right operand, so weights stay in
@@ -179,10 +180,10 @@ __global__ __launch_bounds__(256, NQ <= 8 ? 2 : 1) void attn_portion_kernel(
     constexpr int TPR = 256 / KT, FK = (NQ * 4 + TPR - 1) / TPR, FV = SHARED ? 1 : (NV * 4 + TPR - 1) / TPR;
     __shared__ __attribute__((aligned(16))) float s_k[2][KT][LK];
     __shared__ __attribute__((aligned(16))) float s_v[SHARED ? 1 : 2][SHARED ? 1 : KT][LV];
-    __shared__ int s_bad[2];  // the tile holds a value that is not finite
+    __shared__ int s_bad[3];  // tile i (slot i % 3, of SHARED i % 2) holds a value that is not finite
     const int tid = threadIdx.x, lane = tid & 63, j16 = lane & 15, g4 = lane >> 4;
     const int gh = H / G, hblocks = (gh + HB - 1) / HB, g = blockIdx.y / hblocks, h0 = blockIdx.y % hblocks * HB;
-    const int t0 = blockIdx.x * RB, tend = min(rows, t0 + RB);
+    const int t0 = (gridDim.x - 1 - blockIdx.x) * RB, tend = min(rows, t0 + RB);  // the last rows, with the most keys, first
     const int pair = 16 * (tid >> 6) + j16, trow = t0 + pair / HB, hh = h0 + pair % HB;
     const bool valid = pair < RB * HB && trow < tend && hh < gh;
     const int t = valid ? trow : t0, head = g * gh + (valid ? hh : h0), pos = positions[t];
@@ -206,45 +207,43 @@ __global__ __launch_bounds__(256, NQ <= 8 ? 2 : 1) void attn_portion_kernel(
         while (b < tend && seq_idx[b] == seq) last = max(last, positions[b++]);
         const bool mine = valid && t >= a && t < b;
         const int* bt = block_tables + (size_t)seq * bt_stride;
+        // keys past the last one are read as that (masked), columns past the row as its end and zeroed on the way into LDS
+        int page = bt[min(lr, last) / ROW_PAGE];  // of this thread's row of the tile fetched next
         auto fetch = [&](int k0) {
-            const int key = k0 + lr;
-            const bool in = key <= last;
-            const size_t slab = in ? ((size_t)bt[key / ROW_PAGE] * G + g) * ROW_PAGE + key % ROW_PAGE : 0;
+            const int key = min(k0 + lr, last);
+            const size_t slab = ((size_t)page * G + g) * ROW_PAGE + key % ROW_PAGE;
+            page = bt[min(k0 + KT + lr, last) / ROW_PAGE];
 #pragma unroll
-            for (int i = 0; i < FK; ++i) {
-                const int c = lc + 4 * TPR * i;
-                fk[i] = in && c < dk ? ld4(kc + slab * dk + c) : make_float4(0.f, 0.f, 0.f, 0.f);
-            }
+            for (int i = 0; i < FK; ++i) fk[i] = ld4(kc + slab * dk + min(lc + 4 * TPR * i, dk - 4));
             if constexpr (!SHARED) {
 #pragma unroll
-                for (int i = 0; i < FV; ++i) {
-                    const int c = lc + 4 * TPR * i;
-                    fv[i] = in && c < dv ? ld4(vc + slab * ldv + c) : make_float4(0.f, 0.f, 0.f, 0.f);
-                }
+                for (int i = 0; i < FV; ++i) fv[i] = ld4(vc + slab * ldv + min(lc + 4 * TPR * i, dv - 4));
             }
         };
-        auto put = [&](int buf) {
+        auto put = [&](int buf, int slot) {
             bool bad = false;
 #pragma unroll
             for (int i = 0; i < FK; ++i) {
+                if (lc + 4 * TPR * i >= dk) fk[i] = make_float4(0.f, 0.f, 0.f, 0.f);
                 if (lc + 4 * TPR * i < NQ * 16) *reinterpret_cast<float4*>(&s_k[buf][lr][lc + 4 * TPR * i]) = fk[i];
                 if (SHARED && lc + 4 * TPR * i < dv) bad |= !(fabsf(fk[i].x) + fabsf(fk[i].y) + fabsf(fk[i].z) + fabsf(fk[i].w) < INFINITY);
             }
             if constexpr (!SHARED) {
 #pragma unroll
                 for (int i = 0; i < FV; ++i) {
+                    if (lc + 4 * TPR * i >= dv) fv[i] = make_float4(0.f, 0.f, 0.f, 0.f);
                     if (lc + 4 * TPR * i < NV * 16) *reinterpret_cast<float4*>(&s_v[buf][lr][lc + 4 * TPR * i]) = fv[i];
                     bad |= !(fabsf(fv[i].x) + fabsf(fv[i].y) + fabsf(fv[i].z) + fabsf(fv[i].w) < INFINITY);
                 }
             }
-            if (bad) s_bad[buf] = 1;
+            if (bad) s_bad[slot] = 1;
         };
-        if (tid < 2) s_bad[tid] = 0;
+        if (tid < 3) s_bad[tid] = 0;
         fetch(0);
         __syncthreads();
-        put(0);
+        put(0, 0);
         __syncthreads();
-        for (int k0 = 0, buf = 0; k0 <= last; k0 += KT, buf ^= 1) {
+        for (int k0 = 0, buf = 0, slot = 0; k0 <= last; k0 += KT, buf ^= 1) {
             const bool more = k0 + KT <= last;
             if (more) fetch(k0 + KT);
             f32x4 s[KT / 16];
@@ -293,7 +292,7 @@ __global__ __launch_bounds__(256, NQ <= 8 ? 2 : 1) void attn_portion_kernel(
                     l += s[kb][i];
                 }
             auto vrow = [&](int k) -> const float* { return SHARED ? s_k[buf][k] : s_v[SHARED ? 0 : buf][SHARED ? 0 : k]; };
-            if (!s_bad[buf]) {
+            if (!s_bad[SHARED ? buf : slot]) {
 #pragma unroll
                 for (int kb = 0; kb < KT / 16; ++kb)
 #pragma unroll
@@ -323,9 +322,16 @@ __global__ __launch_bounds__(256, NQ <= 8 ? 2 : 1) void attn_portion_kernel(
                                 for (int i = 0; i < 4; ++i) o[c][i] += p * vrow(k)[16 * c + 4 * g4 + i];
                 }
             }
-            if (tid == 0) s_bad[buf ^ 1] = 0;
-            __syncthreads();
-            if (more) put(buf ^ 1);
+            if constexpr (SHARED) {  // (registers are full there: the form below spills)
+                if (tid == 0) s_bad[buf ^ 1] = 0;
+                __syncthreads();
+                if (more) put(buf ^ 1, buf ^ 1);
+            } else {  // the other buffer and the slot after the next were last read before the barrier ahead of this tile
+                const int next = slot == 2 ? 0 : slot + 1;
+                if (more) put(buf ^ 1, next);
+                if (tid == 0) s_bad[3 - slot - next] = 0;
+                slot = next;
+            }
             __syncthreads();
         }
         a = b;

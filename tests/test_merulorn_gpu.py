@@ -532,6 +532,31 @@ def test_row_attention_portions(H, G, dk, dv, dtype, monkeypatch):
         assert bool((got[odd] == float("inf")).all())
 
 
+@pytest.mark.parametrize("key", [31, 32, 65, 97, 130])
+@pytest.mark.parametrize("dk,dv", [(128, 128), (64, 40)])
+def test_row_attention_portions_infinite_value_of_a_tile(key, dk, dv, monkeypatch):
+    """An infinite value in each of the slots that take turns as flags of a tile: rows before it leave it alone."""
+    from llm_map_reduce_summarizer_amd import ops
+    from llm_map_reduce_summarizer_amd.ops import hip
+    monkeypatch.setattr(hip, "PORTION_PAIRS", 0)
+    H, G, n, page = 8, 2, 170, 64
+    kc, vc = rnd(4, G, page, dk, seed=1), rnd(4, G, page, dv, seed=2)
+    vc[1 + key // page, :, key % page, 3] = float("inf")
+    i32 = [torch.arange(n).int(), torch.zeros(n, dtype=torch.int32), torch.tensor([[1, 2, 3]], dtype=torch.int32)]
+    q, gate = rnd(n, H * dk, seed=3, std=2.0), torch.sigmoid(rnd(n, H, seed=4))
+    got = torch.zeros(n, H * dv, device=DEV)
+    ops.attn_rows(dev(q), dev(kc), dev(vc), *map(dev, i32), H, G, dv, page, dk ** -0.5, dev(gate), got, singles=0)
+    vc[1 + key // page, :, key % page, 3] = 0
+    want = torch.zeros(n, H * dv)
+    ops.attn_rows(q, kc, vc, *i32, H, G, dv, page, dk ** -0.5, gate, want)
+    hit = torch.zeros(n, H, dv, dtype=torch.bool)
+    hit[key:, :, 3] = True
+    hit, got = hit.view(n, -1), got.cpu()
+    assert bool((got[hit] == float("inf")).all())
+    # as above
+    assert rel(got[~hit], want[~hit]) < 2e-6
+
+
 @pytest.mark.parametrize("M,N,K,split", [(1, 130, 1024, True), (17, 1023, 2048, True), (129, 2062, 512, True),
                                          (500, 8200, 256, True), (1100, 4096, 128, False), (3, 40000, 64, False)])
 def test_gemm32_edges(M, N, K, split, monkeypatch):
