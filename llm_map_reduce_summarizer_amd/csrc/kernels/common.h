@@ -177,6 +177,17 @@ struct SegArgs {
     const int* pos0;
 };
 
+// The recurrent state of a decoded token: read once, written once.  Nontemporal both ways, it streams: 128 heads of 64 x 128,
+// 32 rows (268 MB) 61 -> 53 us, 92 rows 170 -> 136 (5.7 TB/s; either way alone 155 and 167), 8 rows 23 -> 18, one row that
+// stays in a cache from token to token 6.3 -> 6.0.
+__device__ __forceinline__ float4 load_state4(const float* p) {
+    const f32x4 v = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p));
+    return make_float4(v[0], v[1], v[2], v[3]);
+}
+__device__ __forceinline__ void store_state4(float* p, const float4& v) {
+    __builtin_nontemporal_store(f32x4{v.x, v.y, v.z, v.w}, reinterpret_cast<f32x4*>(p));
+}
+
 __device__ __forceinline__ void load8(const float* p, float* f) {
     const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
     f[0] = a.x; f[1] = a.y; f[2] = a.z; f[3] = a.w; f[4] = b.x; f[5] = b.y; f[6] = b.z; f[7] = b.w;

@@ -38,7 +38,7 @@ __global__ __launch_bounds__(NT, R <= 8 ? 4 : 1) void delta_step_kernel(const T*
         for (int v = 0; v < NV; ++v) {
             const int p = r + RP * i, n = 4 * (l + LPR * v);
             S[i][v] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (cont && p < a.P && n < a.N4) S[i][v] = *reinterpret_cast<const float4*>(st + (size_t)p * a.N4 + n);
+            if (cont && p < a.P && n < a.N4) S[i][v] = load_state4(st + (size_t)p * a.N4 + n);
         }
     const bool whole = a.N % 4 == 0 && a.ldx % 4 == 0 && a.xk % 4 == 0;
     const float an = a.a_neg[head], db = a.dt_bias[head];
@@ -137,7 +137,7 @@ __global__ __launch_bounds__(NT, R <= 8 ? 4 : 1) void delta_step_kernel(const T*
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             const int p = r + RP * i, n = 4 * (l + LPR * v);
-            if (p < a.P && n < a.N4) *reinterpret_cast<float4*>(st + (size_t)p * a.N4 + n) = S[i][v];
+            if (p < a.P && n < a.N4) store_state4(st + (size_t)p * a.N4 + n, S[i][v]);
         }
 }
 

@@ -282,7 +282,7 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(const T* __restrict__ xbc
         for (int v = 0; v < NV; ++v) {
             const int p = p0 + RP * i, n = 4 * (l + LPR * v);
             S[i][v] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (cont && p < a.P && n < a.N4) S[i][v] = *reinterpret_cast<const float4*>(st + (size_t)p * a.N4 + n);
+            if (cont && p < a.P && n < a.N4) S[i][v] = load_state4(st + (size_t)p * a.N4 + n);
         }
     for (int t = b; t < e; ++t) {
         const float dt = softplus(proj_at<PARTS>(a.u, t, a.dt_at + head) + db);
@@ -321,7 +321,7 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(const T* __restrict__ xbc
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             const int p = p0 + RP * i, n = 4 * (l + LPR * v);
-            if (p < a.P && n < a.N4) *reinterpret_cast<float4*>(st + (size_t)p * a.N4 + n) = S[i][v];
+            if (p < a.P && n < a.N4) store_state4(st + (size_t)p * a.N4 + n, S[i][v]);
         }
 }
 
