@@ -297,6 +297,46 @@ __device__ __forceinline__ void gelu_piece(const ProjSrc& src, const GeluJob& j,
     store8(reinterpret_cast<T*>(j.out) + (size_t)t * j.ldo + c, v);
 }
 
+// The short causal convolution of a segment of one row t: 4 channels from c on (C in all), whose history it advances.
+template <bool PARTS, typename T, int TAPS>
+__device__ __forceinline__ void conv_step4(const ProjSrc& src, int at, const float* __restrict__ kernel,
+                                           const float* __restrict__ bias, float* __restrict__ state, const SegArgs& sg,
+                                           T* __restrict__ out, int C, int t, int c) {
+    const bool cont = sg.pos0[t] > 0;
+    float* st = state + (size_t)sg.slots[t] * (TAPS - 1) * C + c;
+    float4 win[TAPS], kw[TAPS];
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) kw[j] = *reinterpret_cast<const float4*>(kernel + (size_t)j * C + c);
+#pragma unroll
+    for (int j = 0; j < TAPS - 1; ++j) {
+        win[j] = *reinterpret_cast<const float4*>(st + (size_t)j * C);
+        if (!cont) win[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    float4 x = proj4<PARTS>(src, t, at + c);
+    if constexpr (PARTS && sizeof(T) == 2)
+        x = make_float4((float)(T)x.x, (float)(T)x.y, (float)(T)x.z, (float)(T)x.w);
+    win[TAPS - 1] = x;
+    float4 a = *reinterpret_cast<const float4*>(bias + c);
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) {
+        a.x += kw[j].x * win[j].x; a.y += kw[j].y * win[j].y; a.z += kw[j].z * win[j].z; a.w += kw[j].w * win[j].w;
+    }
+#pragma unroll
+    for (int j = 0; j < TAPS - 1; ++j) *reinterpret_cast<float4*>(st + (size_t)j * C) = win[j + 1];
+    a.x *= logistic_for<T>(a.x); a.y *= logistic_for<T>(a.y); a.z *= logistic_for<T>(a.z); a.w *= logistic_for<T>(a.w);
+    store4(out + (size_t)t * C + c, a);
+}
+
+// ... of all rows and channels, taken along by a kernel with few rows in blocks of its own (C = 0: nothing).
+struct ConvJob {
+    int at, C;
+    const float* kernel;  // [taps][C]
+    const float* bias;
+    float* state;
+    SegArgs sg;
+    void* out;  // [T][C]
+};
+
 static inline bool gelu_job_ok(const GeluJob& j, int S, int ld) {
     return j.n == 0 || (S >= 1 && j.n > 0 && j.out && j.at >= 0 && j.at % 8 == 0 && j.n % 8 == 0 && j.ldo % 8 == 0 && j.at + j.n <= ld);
 }

@@ -51,11 +51,22 @@ __device__ __forceinline__ void head_pad(T* base, size_t head_stride, int heads,
 // A thread holds CH 8-column pieces of the token's q | k | v columns in registers (sections start at multiples of 8
 // and are padded to them, so a piece belongs to one section; the biases of padding columns are zero, and so are the
 // projections).
-template <bool PARTS, typename T, int CH>
+//
+// CONV: blocks behind the rows' are those of a convolution of four taps over other columns of the same projection.  Either
+// alone is a launch of 5 - 6 us that fills a part of the chip; together they take 6.
+template <bool PARTS, typename T, int CH, bool CONV = false>
 __global__ __launch_bounds__(1024) void qkv_prep_kernel(ProjSrc src, QkvPrep a, T* __restrict__ q, T* __restrict__ kc,
-                                                        T* __restrict__ vc, float* __restrict__ gate) {
+                                                        T* __restrict__ vc, float* __restrict__ gate, int rows, ConvJob job) {
     __shared__ float red[64];
     const int t = blockIdx.x, tid = threadIdx.x, nt = blockDim.x;
+    if constexpr (CONV) {
+        if (t >= rows) {
+            const int per = (job.C / 4 + nt - 1) / nt, i = t - rows, c = 4 * (i % per * nt + tid);
+            if (c < job.C)
+                conv_step4<PARTS, T, 4>(src, job.at, job.kernel, job.bias, job.state, job.sg, (T*)job.out, job.C, i / per, c);
+            return;
+        }
+    }
     const int nq = a.H * a.dim, nk = a.G * a.dim, nv = a.G * a.vdim;
     const int pq = (nq + 7) / 8, pk = (nk + 7) / 8, pieces = pq + pk + (nv + 7) / 8;
     const int pos = a.positions[t];
@@ -124,13 +135,19 @@ __global__ __launch_bounds__(1024) void qkv_prep_kernel(ProjSrc src, QkvPrep a, 
 
 template <bool PARTS, typename T>
 static int launch_qkv_prep(const ProjSrc& p, const QkvPrep& a, void* q, void* kc, void* vc, float* gate, int rows,
-                           hipStream_t s) {
+                           const ConvJob& job, hipStream_t s) {
     const int pieces = (a.H * a.dim + 7) / 8 + (a.G * a.dim + 7) / 8 + (a.G * a.vdim + 7) / 8;
     // few rows: one piece per thread (all loads in flight); many rows: 256-thread blocks
     int nt = rows <= 512 ? std::min(1024, ceil_div(pieces, 64) * 64) : 256;
     if (pieces > 8 * nt) nt = 1024;
     const int ch = ceil_div(pieces, nt);
-#define QP(C) qkv_prep_kernel<PARTS, T, C><<<rows, nt, 0, s>>>(p, a, (T*)q, (T*)kc, (T*)vc, gate)
+    if (job.C) {
+        if (ch > 1) return (int)hipErrorInvalidValue;
+        qkv_prep_kernel<PARTS, T, 1, true><<<rows + rows * ceil_div(job.C / 4, nt), nt, 0, s>>>(p, a, (T*)q, (T*)kc, (T*)vc, gate,
+                                                                                                rows, job);
+        return (int)hipGetLastError();
+    }
+#define QP(C) qkv_prep_kernel<PARTS, T, C><<<rows, nt, 0, s>>>(p, a, (T*)q, (T*)kc, (T*)vc, gate, rows, job)
     if (ch <= 1) QP(1);
     else if (ch <= 2) QP(2);
     else if (ch <= 3) QP(3);
@@ -142,19 +159,26 @@ static int launch_qkv_prep(const ProjSrc& p, const QkvPrep& a, void* q, void* kc
 }
 
 // src: S = 0 bf16 rows [T][ld], S >= 1 fp32 slabs [S][T][ld].  f32: q / caches fp32 (slabs only), else bf16.
+// conv_n > 0: the convolution (as mrsum_conv_silu, four taps, one row per segment) of as many columns from conv_at on
+// besides; at most 512 rows and 8192 columns of q, k and v then.
 MRSUM_API int mrsum_qkv_prep(const void* src, int S, int ld, int T, int f32, void* q, void* kc, void* vc, float* gate,
                              int H, int G, int dim, int vdim, int dk, int dv, int cq, int ck, int cv, int cg,
                              const float* bias, const float* qn, const float* kn, float eps, float out_scale,
                              float coef, float every, const int* positions, const int* seq_idx, const int* block_tables,
-                             int bt_stride, int page, hipStream_t s) {
+                             int bt_stride, int page, int conv_at, int conv_n, const float* kernel, const float* conv_bias,
+                             float* state, const int* slots, const int* pos0, void* conv_out, hipStream_t s) {
     if (T <= 0) return 0;
+    if (conv_n < 0 || (conv_n && (T > 512 || conv_n % 8 || conv_at % 8 || conv_at < 0 || conv_at + conv_n > ld || !kernel ||
+                                  !conv_bias || !state || !slots || !pos0 || !conv_out)))
+        return (int)hipErrorInvalidValue;
     if (H <= 0 || G <= 0 || H % G || dk < dim || dv < vdim || dk % 8 || dv % 8 || (cq | ck | cv) % 8 || ld % 8 ||
         page <= 0 || (f32 && S < 1))
         return (int)hipErrorInvalidValue;
     const QkvPrep a{H, G, dim, vdim, dk, dv, cq, ck, cv, cg, bias, qn, kn, eps, out_scale, coef, every,
                     positions, seq_idx, block_tables, bt_stride, page};
     const ProjSrc p{src, S, (size_t)T * ld, ld};
-    if (f32) return launch_qkv_prep<true, float>(p, a, q, kc, vc, gate, T, s);
-    if (S) return launch_qkv_prep<true, bf16>(p, a, q, kc, vc, gate, T, s);
-    return launch_qkv_prep<false, bf16>(p, a, q, kc, vc, gate, T, s);
+    const ConvJob job{conv_at, conv_n, kernel, conv_bias, state, SegArgs{nullptr, nullptr, slots, pos0}, conv_out};
+    if (f32) return launch_qkv_prep<true, float>(p, a, q, kc, vc, gate, T, job, s);
+    if (S) return launch_qkv_prep<true, bf16>(p, a, q, kc, vc, gate, T, job, s);
+    return launch_qkv_prep<false, bf16>(p, a, q, kc, vc, gate, T, job, s);
 }

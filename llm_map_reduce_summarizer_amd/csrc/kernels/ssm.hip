@@ -94,7 +94,7 @@ __global__ __launch_bounds__(256) void conv_silu_kernel(ProjSrc src, int at, con
     }
 }
 
-// one row per segment (decode): one thread per 4 channels, which advances their history too
+// one row per segment (decode)
 template <bool PARTS, typename T, int TAPS>
 __global__ __launch_bounds__(64) void conv_step_kernel(ProjSrc src, int at, const float* __restrict__ kernel,
                                                        const float* __restrict__ bias, float* __restrict__ state,
@@ -107,30 +107,7 @@ __global__ __launch_bounds__(64) void conv_step_kernel(ProjSrc src, int at, cons
             return;
         }
     }
-    if (c >= C) return;
-    const bool cont = sg.pos0[t] > 0;
-    float* st = state + (size_t)sg.slots[t] * (TAPS - 1) * C + c;
-    float4 win[TAPS], kw[TAPS];
-#pragma unroll
-    for (int j = 0; j < TAPS; ++j) kw[j] = *reinterpret_cast<const float4*>(kernel + (size_t)j * C + c);
-#pragma unroll
-    for (int j = 0; j < TAPS - 1; ++j) {
-        win[j] = *reinterpret_cast<const float4*>(st + (size_t)j * C);
-        if (!cont) win[j] = make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-    float4 x = proj4<PARTS>(src, t, at + c);
-    if constexpr (PARTS && sizeof(T) == 2)
-        x = make_float4((float)(T)x.x, (float)(T)x.y, (float)(T)x.z, (float)(T)x.w);
-    win[TAPS - 1] = x;
-    float4 a = *reinterpret_cast<const float4*>(bias + c);
-#pragma unroll
-    for (int j = 0; j < TAPS; ++j) {
-        a.x += kw[j].x * win[j].x; a.y += kw[j].y * win[j].y; a.z += kw[j].z * win[j].z; a.w += kw[j].w * win[j].w;
-    }
-#pragma unroll
-    for (int j = 0; j < TAPS - 1; ++j) *reinterpret_cast<float4*>(st + (size_t)j * C) = win[j + 1];
-    a.x *= logistic_for<T>(a.x); a.y *= logistic_for<T>(a.y); a.z *= logistic_for<T>(a.z); a.w *= logistic_for<T>(a.w);
-    store4(out + (size_t)t * C + c, a);
+    if (c < C) conv_step4<PARTS, T, TAPS>(src, at, kernel, bias, state, sg, out, C, t, c);
 }
 
 // any number of taps: one thread, one row x 8 channels.  STEP: one row per segment, the state is advanced here.

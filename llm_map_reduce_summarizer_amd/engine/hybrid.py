@@ -215,6 +215,10 @@ class HybridModel:
             u = ops.project(x, la.w.w_in, "qkv")
             if la.ssm is None and la.k_mix < la.k_out:
                 a[:, la.k_mix:].zero_()
+        if la.attn is not None and la.ssm is not None and gelu is None and b.segs.cu is None:  # decoded rows
+            xbc = la.attn.run(i, u, a, b, kv, self.cfg.rms_eps, beside=la.ssm)
+            la.ssm.run(i, u, a, b, kv, self.cfg.rms_eps, xbc=xbc)
+            return ops.project(a, la.w.w_o, "o")
         for m in la.mixers:
             if gelu is not None and m.takes_gelu:
                 m.run(i, u, a, b, kv, self.cfg.rms_eps, gelu)

@@ -124,15 +124,17 @@ class AttnMixer(Mixer):
         r = self.spec.heads // self.spec.kv_heads
         return r, lambda: ops.prefill_items(lens, r)
 
-    def run(self, i, u, a, b, kv, eps, gelu=None) -> None:
+    def run(self, i, u, a, b, kv, eps, gelu=None, beside=None):
+        """``beside``: the layer's state-space mixer, whose convolution goes with the preparation of q, k and v; returns its
+        rows."""
         sp, w, page, T = self.spec, self.w, kv.page, a.shape[0]
         kc, vc = kv.k[i], kv.v[i]
-        q, gate = ops.qkv_prep(u, self, w.qkv_bias, w.q_norm, w.k_norm, eps, self.scale, b.positions, b.seq_idx,
-                               b.tables, kc, vc, page, self.dtype)
+        q, gate, *conv = ops.qkv_prep(u, self, w.qkv_bias, w.q_norm, w.k_norm, eps, self.scale, b.positions, b.seq_idx,
+                                      b.tables, kc, vc, page, self.dtype, beside and beside.conv_args(i, b, kv))
         if not self.mfma:
             ops.attn_rows(q, kc, vc, b.positions, b.seq_idx, b.tables, sp.heads, sp.kv_heads, self.vp, page, sp.scale,
                           gate, a, b.n_decode, b.portions)
-            return
+            return conv[0] if conv else None
         nd = b.n_decode
         if nd:
             ops.attn_decode(q[:nd], kc, vc, b.decode_tables, b.positions, sp.heads, sp.kv_heads, MFMA_HEAD, page,
@@ -142,6 +144,7 @@ class AttnMixer(Mixer):
             ops.attn_prefill(q[nd:], b.cu_portions, sp.heads, sp.kv_heads, MFMA_HEAD, sp.scale, out=a[nd:],
                              paged=b.paged.layer(kc, vc), seqlens=b.portion_lens,
                              items=b.items[sp.heads // sp.kv_heads], gate=gate[nd:], pitch=self.vp)
+        return conv[0] if conv else None
 
 
 class SSMMixer(Mixer):
@@ -179,9 +182,14 @@ class SSMMixer(Mixer):
         s = self.spec
         return (up(s.channels, 8), s.conv, s.heads, s.vdim, s.state)
 
-    def run(self, i, u, a, b, kv, eps, gelu=None) -> None:
+    def conv_args(self, i, b, kv):
+        return self.xbc, self.w.conv, self.w.conv_b, kv.state.conv[i], b.segs
+
+    def run(self, i, u, a, b, kv, eps, gelu=None, xbc=None) -> None:
+        """``xbc``: the convolved rows, if the layer's attention has run the convolution."""
         s, w, st = self.spec, self.w, kv.state
-        xbc = ops.conv_silu(u, self.xbc, w.conv, w.conv_b, st.conv[i], b.segs, self.dtype, gelu)
+        if xbc is None:
+            xbc = ops.conv_silu(u, *self.conv_args(i, b, kv), self.dtype, gelu)
         y = ops.ssm_scan(xbc, u, self.dt, w.dt_bias, w.a_neg, w.d_skip, st.ssm[i], b.segs, s.heads, s.vdim, s.state,
                          s.groups)
         ops.gated_norm(y, u, self.z, w.ssm_norm, s.norm_groups, eps, self.scale, a, self.col)

@@ -283,9 +283,9 @@ def logits32(x, w):
 
 
 def qkv_prep(u, al, bias, q_norm, k_norm, eps, out_scale, positions, seq_idx, block_tables, kcache, vcache, page,
-             dtype):
+             dtype, conv=None):
     return _impl(u).qkv_prep(u, al, bias, q_norm, k_norm, eps, out_scale, positions, seq_idx, block_tables, kcache,
-                             vcache, page, dtype)
+                             vcache, page, dtype, conv)
 
 
 def attn_rows(q, kcache, vcache, positions, seq_idx, block_tables, hq, hkv, pitch, page, scale, gate, out, singles=None,

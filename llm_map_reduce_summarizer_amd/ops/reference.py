@@ -445,9 +445,10 @@ def project_glu(x, w_gu, limit: float, alpha: float, shift: float) -> torch.Tens
 
 
 def qkv_prep(u, al, bias, q_norm, k_norm, eps: float, out_scale: float, positions, seq_idx, block_tables, kcache,
-             vcache, page: int, dtype):
+             vcache, page: int, dtype, conv=None):
     """Bias, whole-projection q / k norm, query temperature; K / V rows into the paged cache.  Returns (q [T, H * dk]
-    with zero-padded heads, gate fp32 [T, H] = out_scale * sigmoid(gate column), or out_scale without a gate)."""
+    with zero-padded heads, gate fp32 [T, H] = out_scale * sigmoid(gate column), or out_scale without a gate), and with
+    ``conv`` (arguments of conv_silu behind u, without dtype) the convolved rows."""
     sp, r = al.spec, rows32(u)
     T, H, G = r.shape[0], sp.heads, sp.kv_heads
     pos, rows = positions[:T].long(), seq_idx[:T].long()
@@ -472,7 +473,8 @@ def qkv_prep(u, al, bias, q_norm, k_norm, eps: float, out_scale: float, position
     gate = torch.full((T, H), out_scale, dtype=torch.float32, device=r.device)
     if sp.head_gate:
         gate *= torch.sigmoid(r[:, al.g: al.g + H])
-    return qo.reshape(T, H * al.dk), gate
+    qo = qo.reshape(T, H * al.dk)
+    return (qo, gate) if conv is None else (qo, gate, conv_silu(u, *conv, dtype))
 
 
 def attn_rows(q, kcache, vcache, positions, seq_idx, block_tables, hq: int, hkv: int, pitch: int, page: int,

@@ -301,6 +301,42 @@ def test_gated_group_norm(n, groups):
         assert (out[:, :col] == 3).all() and not out[:, col + n:].any()
 
 
+@pytest.mark.parametrize("T,H,dim,C,taps", [(1, 8, 128, 24, 4), (5, 6, 40, 4 * 448, 4), (33, 8, 128, 4 * 1024 + 8, 4), (3, 64, 128, 64, 4),
+                                            (2, 8, 128, 64, 3), (513, 2, 32, 40, 4)])
+def test_convolution_beside_qkv(T, H, dim, C, taps, monkeypatch):
+    """Decoded rows' convolution in the blocks behind those of q, k and v: less than one, whole and partial blocks a row; in a
+    launch of its own beyond 8192 columns, 512 rows or at other than four taps.  The same bits either way."""
+    from types import SimpleNamespace
+    from llm_map_reduce_summarizer_amd import ops
+    from llm_map_reduce_summarizer_amd.ops import hip
+    G, page, i32 = 2, 64, dict(dtype=torch.int32, device=DEV)
+    spec = SimpleNamespace(heads=H, kv_heads=G, dim=dim, vdim=dim, q_temp=None, head_gate=True)
+    al = SimpleNamespace(spec=spec, q=0, k=H * dim, v=(H + G) * dim, g=(H + 2 * G) * dim, dk=dim, dv=dim)
+    at = al.g + -(-H // 8) * 8
+    u = rnd(T, at + C, std=0.5)
+    bias, kernel, cb = rnd(at + C, seed=2), rnd(taps, C, seed=3), rnd(C, seed=4)
+    one = (torch.arange(T, **i32), torch.arange(T, **i32), torch.arange(1, T + 1, **i32)[:, None].contiguous())
+    pos = one[0] % page
+    segs = ops.Segments(torch.arange(T, **i32).flip(0).contiguous(), pos)
+    calls, plain = [], hip.conv_silu
+    monkeypatch.setattr(hip, "conv_silu", lambda *a, **k: calls.append(1) or plain(*a, **k))
+    for src, dt, _ in forms(u):
+        got = []
+        for beside in (False, True):
+            state = dev(rnd(T, taps - 1, C, seed=5))
+            kc, vc = (torch.zeros(T + 1, G, page, dim, dtype=dt, device=DEV) for _ in range(2))
+            conv = (at, dev(kernel), dev(cb), state, segs)
+            calls.clear()
+            q, gate, *rows = ops.qkv_prep(src, al, dev(bias), None, None, 1e-5, 1.0, pos, one[1], one[2], kc, vc, page, dt,
+                                          conv if beside else None)
+            if not beside:
+                rows = [ops.conv_silu(src, *conv, dt)]
+            else:
+                assert len(calls) == (0 if taps == 4 and T <= 512 and H * dim <= 4096 else 1)
+            got.append((q, gate, kc, vc, rows[0], state))
+        assert all(torch.equal(x, y) for x, y in zip(*got))
+
+
 ATTN = [(8, 2, 128, 128), (6, 2, 40, 56), (4, 4, 64, 96), (16, 1, 96, 128), (10, 2, 24, 16), (2, 1, 136, 200)]
 
 
