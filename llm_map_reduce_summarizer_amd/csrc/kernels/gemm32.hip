@@ -55,11 +55,14 @@ __device__ __forceinline__ void k_loop(const Gemm32Args& a, char* lds, int m0, i
         vx[i] = r * a.ldx * 4 + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
         dx[i] = STAGE + p * 1024;
     }
+    // Up to 48 rows are one row of tiles: W is read once, nontemporal (aux 2).  us, K 4096: 4 x 128256 399 -> 369 (5.7 TB/s), 2 x
+    // 14336 56 -> 52, 4 x 4096 19.6 -> 18.3; 4 x 4096 x 14336 51 -> 47.
+    constexpr int NT = NB <= 3 ? 2 : 0;
     auto stage = [&](int kt, int buf) {
         char* dst = lds + buf * IMAGE;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr)(dst + (4 * w + i) * 1024), 16, vw[i], kt * 128, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr)(dst + (4 * w + i) * 1024), 16, vw[i], kt * 128, 0, NT);
 #pragma unroll
         for (int i = 0; i < XI; ++i)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr)(dst + dx[i]), 16, vx[i], kt * 128, 0, 0);
