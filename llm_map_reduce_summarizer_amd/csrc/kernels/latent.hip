@@ -209,7 +209,7 @@ __global__ __launch_bounds__(MODE == 2 ? HM_THREADS : 256) void head_product_ker
         }
         return;
     }
-    const int ldx = a.K + 8;
+    const int ldx = a.K + (sizeof(T) == 2 ? 8 : 4);  // 16 rows' pieces of 16 bytes in different banks
     if constexpr (MODE == 2) {
         __shared__ float sw[HM_ROWS][256];  // weights of the splits, the common denominator divided out
         __shared__ int s_n[HM_ROWS];        // splits in use: the leading ones
@@ -337,23 +337,33 @@ __global__ __launch_bounds__(MODE == 2 ? HM_THREADS : 256) void head_product_ker
                        make_float4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]));
         }
     } else {
-        const float* w = reinterpret_cast<const float*>(a.w) + (size_t)h * a.N * a.K;
-        const int rg = tid >> 6;  // rows 4 rg .. + 4
-        for (int nn = 0; nn < HP_COLS; nn += 64) {
-            const int n = blockIdx.x * HP_COLS + nn + (tid & 63);
-            if (n >= a.N) break;
-            float acc[4] = {0.f, 0.f, 0.f, 0.f};
-            for (int k = 0; k < a.K; k += 4) {
-                const float4 wk = *reinterpret_cast<const float4*>(w + (size_t)n * a.K + k);
+        // a wave has 32 columns, as above, on the fp32 matrix instruction, in four chains.  (With a thread to a column every wave
+        // read all weights and added K products in one chain.  1079 rows of 32 heads, K 128 to 512 columns 260 -> 77 us, K 512 to 128
+        // 316 -> 91; bound by the weights, which every 16 rows read again from the L2s.)
+        const int wv = tid >> 6, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
+        const float* w = reinterpret_cast<const float*>(a.w) + (size_t)h * a.N * a.K + 4 * g;
+        const int n0 = blockIdx.x * HP_COLS + 32 * wv;
+        const float* w0 = w + (size_t)min(n0 + r16, a.N - 1) * a.K;
+        const float* w1 = w + (size_t)min(n0 + 16 + r16, a.N - 1) * a.K;
+        const float* xr = reinterpret_cast<const float*>(sx) + r16 * ldx + 4 * g;
+        f32x4 acc[2][4];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float4 xk = *reinterpret_cast<const float4*>(sx + (4 * rg + r) * ldx + k);
-                    acc[r] += wk.x * xk.x + wk.y * xk.y + wk.z * xk.z + wk.w * xk.w;
-                }
+        for (int e = 0; e < 4; ++e) acc[0][e] = acc[1][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+        for (int k = 0; k < a.K; k += 16) {
+            const f32x4 xf = *reinterpret_cast<const f32x4*>(xr + k);
+            const f32x4 f0 = *reinterpret_cast<const f32x4*>(w0 + k), f1 = *reinterpret_cast<const f32x4*>(w1 + k);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                acc[0][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(f0[e], xf[e], acc[0][e], 0, 0, 0);
+                acc[1][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(f1[e], xf[e], acc[1][e], 0, 0, 0);
             }
+        }
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (4 * rg + r < nr) out[(size_t)(r0 + 4 * rg + r) * a.ldo + h * a.os + n] = (T)acc[r];
+        for (int i = 0; i < 2; ++i) {
+            const int n = n0 + 16 * i + 4 * g;  // N % 8 == 0
+            const f32x4 y = (acc[i][0] + acc[i][1]) + (acc[i][2] + acc[i][3]);
+            if (r16 < nr && n < a.N) *reinterpret_cast<f32x4*>(out + (size_t)(r0 + r16) * a.ldo + h * a.os + n) = y;
         }
     }
 }

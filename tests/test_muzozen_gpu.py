@@ -227,6 +227,24 @@ def test_latent_kernels_of_real_sizes_are_the_fused_ones():
 DELTA = [(4, 2, 128, 128), (3, 3, 24, 40), (2, 1, 64, 136), (6, 2, 32, 16), (2, 2, 200, 112), (3, 1, 5, 7), (2, 1, 256, 64)]
 
 
+@pytest.mark.parametrize("rows,H,xk,K,N", [(1, 3, 24, 32, 8), (15, 2, 96, 96, 136), (16, 2, 128, 128, 128), (17, 5, 40, 64, 24),
+                                            (33, 2, 512, 512, 40), (70, 1, 576, 576, 264)])
+def test_head_product_of_fp32(rows, H, xk, K, N):
+    """Row blocks of 16 and column blocks of 32, 128 and what is left of them, depths past the operand, two slabs."""
+    from llm_map_reduce_summarizer_amd.ops import hip
+    xs, os = xk + 8, N + 8
+    x, w = rnd(2, rows + 3, H * xs, seed=1), torch.zeros(H, N, K)
+    w[:, :, :xk] = rnd(H, N, xk, seed=2)
+    out = torch.full((rows, H * os), 7.0, device=DEV)
+    xd, wd = dev(x), dev(w)
+    hip._head_product(xd.data_ptr(), 2, H * xs, rows + 3, rows, xs, xk, wd, out, os, H)
+    got = out.cpu().view(rows, H, os)
+    v = x.double().sum(0)[:rows].view(rows, H, xs)[:, :, :xk]
+    want = torch.einsum("thk,hnk->thn", v, w[:, :, :xk].double())
+    # fp32 sums of two slabs and of up to 576 products in four chains: a few 2^-24 of the terms' norm
+    assert rel(got[:, :, :N], want) < 1e-6 and (got[:, :, N:] == 7).all()
+
+
 @pytest.mark.parametrize("H,G,dim,vdim", DELTA)
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_delta_rule(H, G, dim, vdim, dtype, monkeypatch):
