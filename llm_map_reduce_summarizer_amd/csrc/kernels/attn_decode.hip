@@ -752,7 +752,9 @@ __global__ __launch_bounds__(256, four_a_cu(G, ROPE, KVM) ? 4 : 3) void attn_dec
 
 // KV page loads are nontemporal from 64 (sequence, kv head) groups up -- measured, step at 4k context:
 // B=39 x 8 kv heads 7.02-7.05 vs 7.18-7.26 ms with the default policy; B <= 10 0.7-1 % slower with nt
-// (profiles/r1_decode_nt_ab.jsonl)
+// (profiles/r1_decode_nt_ab.jsonl).  So they are for one row whose splits fill the chip: in a step of 8 layers that row's keys
+// are gone from the caches by the next.  us a launch, 32 / 8 heads over 13500 keys 19.7 -> 18.2, 32000 32 -> 28.3; decode steps of one
+// row over 13500, 25278 and 32000 keys 1059 -> 1048, 1140 -> 1120 and 1012 -> 998, over 4526 the same; 3 - 7 rows lost 0.5 - 1 %
 constexpr int NT_MIN_GROUPS = 64;
 
 static bool decode_packed(int G) { return G == 1 || G == 2 || G == 4 || G == 8 || G == 16; }
@@ -788,7 +790,7 @@ static int launch_mfma(const void* q, int q_stride, const void* kcache, const vo
                                                                      (bf16*)out, out_stride, Hc, gq, ep)
 #define MFMA_L(G_, R_)                                                                                        \
     do {                                                                                                      \
-        const bool nt_ = B * Hkv >= NT_MIN_GROUPS;                                                            \
+        const bool nt_ = B * Hkv >= NT_MIN_GROUPS || (B == 1 && S * Hkv >= 256);                              \
         if (kv8 == 3) { if (nt_) MFMA_K(G_, R_, true, 3, false); else MFMA_K(G_, R_, false, 3, false); }                    \
         else if (kv8 == 2) { if (nt_) MFMA_K(G_, R_, true, 2, false); else MFMA_K(G_, R_, false, 2, false); }               \
         else if (!R_ && hl) { if (nt_) MFMA_K(G_, false, true, 0, true); else MFMA_K(G_, false, false, 0, true); }  \

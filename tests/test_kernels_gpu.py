@@ -310,6 +310,28 @@ def test_attn_decode_pages_of_a_split(kv8, gate):
         _close(hip.attn_decode(q, kc, vc, bt, pos, hq, hkv, d, page, sc, workspace=ws, gate=factors), want, 2e-2)
 
 
+@pytest.mark.parametrize("kv8", ["bf16", "fp8"])
+@pytest.mark.parametrize("ctx", [64 * 33, 64 * 40 - 1])
+def test_attn_decode_of_one_row(kv8, ctx):
+    """One row on either side of the 256 workgroups from which its pages are read past the caches: the same bits as the same
+    row beside another."""
+    hq, hkv, d, page = 32, 8, 128, 64
+    n, g = -(-ctx // page), torch.Generator().manual_seed(23)
+    kc = torch.randn(n + 1, hkv, page, d, generator=g).to(torch.bfloat16).to(DEV)
+    vc = torch.randn(n + 1, hkv, page, d, generator=g).to(torch.bfloat16).to(DEV)
+    kc, vc = _kv_format(kc, vc, kv8)
+    bt = (torch.randperm(n, generator=g) + 1).to(torch.int32).view(1, n).to(DEV)
+    pos = torch.tensor([ctx - 1], dtype=torch.int32, device=DEV)
+    q, sc = _rand(1, (hq + 2 * hkv) * d, seed=24), 1.0 / math.sqrt(d)
+    want = reference.attn_decode(q, kc, vc, bt, pos, hq, hkv, d, page, sc)
+    for splits in (31, 32):
+        two = hip.attn_decode(q.repeat(2, 1), kc, vc, bt.repeat(2, 1), pos.repeat(2), hq, hkv, d, page, sc,
+                              workspace=hip.DecodeWorkspace(2, hq, d, splits, DEV, hkv))
+        got = hip.attn_decode(q, kc, vc, bt, pos, hq, hkv, d, page, sc, workspace=hip.DecodeWorkspace(1, hq, d, splits, DEV, hkv))
+        _close(got, want, 2e-2)
+        assert torch.equal(got[0], two[0]) and torch.equal(got[0], two[1])
+
+
 @pytest.mark.parametrize("splits,fused", [(64, False), (160, False), (256, False), (256, True)])
 def test_attn_decode_many_splits_one_kv_head(splits, fused):
     """A TP shard's single kv head at a long context split up to the merge's 256 ways (decode_attn_plan's
