@@ -235,7 +235,7 @@ def decode_workspace(B, hq, hkv, d, max_ctx, device, kv8=False):
     """Split-K buffers of the decode attention for ``B`` rows whose contexts reach ``max_ctx`` (GPU only)."""
     from .hip import DecodeWorkspace, decode_attn_plan, decode_groups
     ng = decode_groups(hq, hkv)  # kv heads, or query heads for odd GQA ratios
-    s, fused = decode_attn_plan(B, ng, max_ctx, kv8=kv8, group=hq // ng)
+    s, fused = decode_attn_plan(B, ng, max_ctx, kv8=kv8)
     return DecodeWorkspace(B, hq, d, s, device, ng, fused_combine=fused)
 
 
