@@ -54,9 +54,11 @@ def _token_ids(toks: Sequence[int], vocab: int) -> np.ndarray:
         toks = list(toks)
     if len(toks) == 1 and type(toks[0]) is int and 0 <= toks[0] < vocab:  # a decoded row: 5 us less than below
         return np.array(toks, dtype=np.int32)
+    a = np.empty(len(toks), dtype=np.int32) if len(toks) else None
     try:  # 9 ns an id, 18 by way of an array
-        a = np.frombuffer(struct.pack("%di" % len(toks), *toks), dtype=np.int32) if len(toks) else None
-    except struct.error:  # ids that are not plain integers, or far out of range
+        if a is not None:
+            struct.pack_into("%di" % len(toks), a, 0, *toks)
+    except (struct.error, TypeError, OverflowError):  # ids that are not plain integers, or far out of range
         a = [int(t) for t in toks]
         a = None if min(a) < 0 or max(a) >= vocab else np.asarray(a, dtype=np.int32)
     if a is None or int(a.view(np.uint32).max()) >= vocab:  # (negative ids are large ones)
