@@ -205,6 +205,10 @@ __global__ __launch_bounds__(256, NQ <= 8 ? 2 : 1) void attn_portion_kernel(
         const int seq = seq_idx[a];
         int b = a + 1, last = positions[a];
         while (b < tend && seq_idx[b] == seq) last = max(last, positions[b++]);
+        if (last < 0) {  // no key for any of these rows: nothing of theirs is read
+            a = b;
+            continue;
+        }
         const bool mine = valid && t >= a && t < b;
         const int* bt = block_tables + (size_t)seq * bt_stride;
         // keys past the last one are read as that (masked), columns past the row as its end and zeroed on the way into LDS

@@ -568,6 +568,32 @@ def test_row_attention_portions(H, G, dk, dv, dtype, monkeypatch):
         assert bool((got[odd] == float("inf")).all())
 
 
+@pytest.mark.parametrize("H,G,dk,dv", [(8, 2, 128, 128), (4, 1, 576, 512)])
+def test_row_attention_portions_without_keys(H, G, dk, dv, monkeypatch):
+    """Rows before position 0 have no keys: a run of them in blocks of their own, or between others, reads nothing and
+    leaves the others as they are without it."""
+    from llm_map_reduce_summarizer_amd.ops import hip
+    monkeypatch.setattr(hip, "PORTION_PAIRS", 0)
+    page, lens = 64, [70, 100, 41]
+    n = sum(lens)
+    kc = dev(rnd(6, G, page, dk, seed=1))
+    vc = dev(rnd(6, G, page, dv, seed=2)) if dv == dk else kc
+    pos = torch.cat([torch.arange(70), torch.full((100,), -1), torch.arange(41)]).int()
+    seq = torch.repeat_interleave(torch.arange(3), torch.tensor(lens)).int()
+    tables = dev(torch.tensor([[1, 2], [0, 0], [3, 4]], dtype=torch.int32))
+    q, gate = dev(rnd(n, H * dk, seed=3)), dev(torch.ones(n, H))
+
+    def run(rows):
+        out = torch.zeros(len(rows), H * dv, device=DEV)
+        i = dev(torch.tensor(rows))
+        hip._rows_attention(q[i].contiguous(), kc, vc, dev(pos)[i].contiguous(), dev(seq)[i].contiguous(), tables, H, G, dk, dv,
+                            dk if vc is kc else dv, dv, dk ** -0.5, gate[i].contiguous(), out, 0, None, "rows")
+        return out
+    held = [i for i in range(n) if pos[i] >= 0]
+    got = run(list(range(n)))
+    assert torch.equal(got[held], torch.cat([run(held[:70]), run(held[70:])])) and bool(got[70:170].isnan().all())
+
+
 @pytest.mark.parametrize("key", [31, 32, 65, 97, 130])
 @pytest.mark.parametrize("dk,dv", [(128, 128), (64, 40)])
 def test_row_attention_portions_infinite_value_of_a_tile(key, dk, dv, monkeypatch):
