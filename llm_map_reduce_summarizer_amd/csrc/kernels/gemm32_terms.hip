@@ -5,9 +5,10 @@
 // An fp32 value is the exact sum of three bf16 terms, its 24 bits in groups of eight.  Where W's values are bf16 ones (weights of a
 // 16-bit checkpoint, widened), X . W is the sum of three products of bf16 operands, each of which the instruction forms exactly and
 // adds in fp32: sixteen times the fp32 instruction's rate, for three times the products.  W stays 32 bits wide in memory and is
-// looked at as it is read; if a value has lower bits, or is infinite (an infinity times a term of 0 is no number), a flag is set and the
-// fp32 instruction's form (gemm32.hip), which is launched behind and otherwise returns at once, makes the whole result.  A workgroup
-// that sees it in its first K-tile stops there, so that W with 24 bits cost the launches, about 10 us.
+// looked at as it is read.  If a value has lower bits, is infinite (an infinity times a term of 0 is no number) or smaller than bf16's
+// normal numbers (whose products the instruction forms with fewer bits), or if X has a value whose lowest bits would be finer than
+// bf16's (below 2^-110), a flag is set and the fp32 instruction's form (gemm32.hip), which is launched behind and otherwise returns
+// at once, makes the whole result.  A workgroup that sees it in its first K-tile or its rows of X stops there.
 //
 // Relative error (2-norm, random operands, K 4096 - 22528, chains of 16 K-tiles on both): 2.4e-7, the fp32 instruction 4.1e-7, as one
 // sum takes the products of 32 columns and not of four.
@@ -46,6 +47,11 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer(const void* p, int byte
 
 __device__ __forceinline__ uint32_t high_halves(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302); }
 
+// Values that terms hold short: a bf16 ends at 2^-133 and so do the lowest bits of x from 2^-110 up; below bf16's smallest normal
+// number the products of w have fewer bits (x 2^20 times 2^-133: 7e-6 off).
+constexpr uint32_t X_LEAST = (127 - 110) << 23;
+constexpr uint32_t W_LEAST = 2 * 0x0080;  // of 2 d, d without its sign
+
 // v - its first term; infinities leave none
 __device__ __forceinline__ uint32_t below(uint32_t v) {
     const float top = __uint_as_float(v & 0xffff0000u);
@@ -54,10 +60,15 @@ __device__ __forceinline__ uint32_t below(uint32_t v) {
 }  // namespace
 
 // X's terms, laid out as the matrix instruction reads them: [M / 16][K / 32][term][lane][8], lane (r, g) holding row r, k 4 g .. and
-// 16 + 4 g ..  Rows past M are zeros.
+// 16 + 4 g ..  Rows past M are zeros.  ``inexact`` is cleared; behind it, on 16 bytes, a byte for each [M / 16][K / 32] says
+// whether X has a value there that is not the sum of its terms, and zeros up to a multiple of four.
 __global__ __launch_bounds__(256) void terms32_kernel(const float* __restrict__ x, int ldx, char* __restrict__ out, int M, int kb,
                                                       int pieces, int* inexact) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) *inexact = 0;
+    char* small = reinterpret_cast<char*>(inexact) + 16;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        *inexact = 0;
+        for (int i = pieces; i % 4; ++i) small[i] = 0;
+    }
     const int lane = threadIdx.x & 63, p = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (p >= pieces) return;
     const int block = p / kb, kt = p - block * kb, m = block * 16 + (lane & 15);
@@ -68,12 +79,14 @@ __global__ __launch_bounds__(256) void terms32_kernel(const float* __restrict__ 
         v[1] = in[4];
     }
     u32x4 t[3];
+    bool least = false;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         uint32_t a[2][3];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const uint32_t u = v[i >> 1][2 * (i & 1) + j], r = below(u);
+            least |= (u & 0x7fffffffu) - 1 < X_LEAST - 1;
             a[j][0] = (u & 0x7fffffffu) > 0x7f800000u ? u | 0x00400000u : u;  // a NaN whose bits are all low
             a[j][1] = r;
             a[j][2] = below(r);
@@ -84,17 +97,19 @@ __global__ __launch_bounds__(256) void terms32_kernel(const float* __restrict__ 
     u32x4* o = reinterpret_cast<u32x4*>(out + (size_t)p * BLOCK) + lane;
 #pragma unroll
     for (int k = 0; k < 3; ++k) o[64 * k] = t[k];
+    const bool any = __ballot(least) != 0;
+    if (lane == 0) small[p] = any;
 }
 
 namespace {
-// Outputs of (row block b, column block i) of a tile of nb 32-row units: row lane & 15, columns 4 (lane >> 4) ..
+// Outputs of (row block b, column block i ^ 4 wr) of a tile of nb 32-row units: row lane & 15, columns 4 (lane >> 4) ..
 __device__ __forceinline__ void store_terms(const Gemm32Args& a, int u0, int nb, int n0, int b, int i, const f32x4& v) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    store_c(a, 32 * u0 + 16 * (nb * (w >> 1) + b) + (lane & 15), n0 + 128 * (w & 1) + 16 * i + 4 * (lane >> 4), v);
+    store_c(a, 32 * u0 + 16 * (nb * (w >> 1) + b) + (lane & 15), n0 + 128 * (w & 1) + 16 * (i ^ 4 * (w >> 1)) + 4 * (lane >> 4), v);
 }
 
 // K-tiles [kt0, kt1) of 32 NB rows from 32 u0 on and columns n0 ..; wave (wr, wc) has half of the rows and 128 columns: acc[row
-// block][column block].  False: W has bits below its bf16 values, and the sums are not made.
+// block][column block ^ 4 wr], as the two waves of the same columns look at the first four each.  False: some value is not the sum of its terms, and the sums are not made.
 template <int NB>
 __device__ __forceinline__ bool terms_loop(const Gemm32Args& a, char* lds, int u0, int n0, int kt0, int kt1, f32x4 (&acc)[NB][8]) {
     constexpr int XI = 2 * NB * BLOCK, PX = (6 * NB + 3) / 4, XS = x_slots(NB);
@@ -122,25 +137,34 @@ __device__ __forceinline__ bool terms_loop(const Gemm32Args& a, char* lds, int u
     auto stage_w = [&](int kt, int slot, int i) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr)(lds + slot * WI + (8 * w + i) * 1024), 16, vw[i], kt * 128, 0, 0);
     };
-    const int wlo = (128 * wc + r16) * 128 + ((g ^ (r16 >> 1)) << 4), xlo = WS * WI + wr * NB * BLOCK + lane * 16;
+    const int wlo = (128 * wc + r16) * 128 + ((g ^ (r16 >> 1)) << 4), wl[2] = {wlo + wr * 8192, wlo - wr * 8192}, xlo = WS * WI + wr * NB * BLOCK + lane * 16;
     auto read_w = [&](u32x4 (&q)[2], int slot, int i, int h) {
-        q[h] = *reinterpret_cast<const u32x4*>(lds + slot * WI + (h ? wlo ^ 64 : wlo) + i * 2048);
+        q[h] = *reinterpret_cast<const u32x4*>(lds + slot * WI + (h ? wl[i >> 2] ^ 64 : wl[i >> 2]) + i * 2048);
     };
     auto read_x = [&](u32x4 (&x)[3], int slot, int b, int k) {
         x[k] = *reinterpret_cast<const u32x4*>(lds + slot * XI + xlo + b * BLOCK + k * 1024);
     };
-    // first terms of a pair of W's values; ``low`` gathers the bits below them, ``top`` the largest size
-    uint32_t low = 0;
+    // First terms of a pair of W's values.  ``look``: and what they leave out, in this wave's half of the columns that it shares with
+    // another one: ``low`` gathers the bits below them, ``top`` the largest size, ``least`` the smallest one but zero (as 2 d - 1).
+    uint32_t low = 0, least = 0xffffffff;
     float top = 0.f;
-    auto first = [&](const u32x4 (&q)[2], u32x4& f, int i) {
+    auto first = [&](const u32x4 (&q)[2], u32x4& f, int i, bool look) {
         const uint32_t u = q[i >> 1][2 * (i & 1)], v = q[i >> 1][2 * (i & 1) + 1];
-        uint32_t d = high_halves(u, v);
-        low |= u | v;
-        top = fmaxf(fmaxf(top, fabsf(__uint_as_float(u))), fabsf(__uint_as_float(v)));
-        asm volatile("" : "+v"(d), "+v"(low), "+v"(top));  // here, and not where they are used
+        uint32_t d = high_halves(u, v), e;
+        if (look) {
+            low |= u | v;
+            top = fmaxf(fmaxf(top, fabsf(__uint_as_float(u))), fabsf(__uint_as_float(v)));
+            // (the compiler would put a wait on either side of such a minimum between written-out lines)
+            asm volatile("v_pk_mad_u16 %1, %0, %5, %6\n\tv_pk_min_u16 %2, %2, %1"
+                         : "+v"(d), "=&v"(e), "+v"(least), "+v"(low), "+v"(top) : "s"(0x00020002), "v"(0xffffffff));
+        } else {
+            asm volatile("" : "+v"(d));  // here, and not where they are used
+        }
         f[i] = d;
     };
-    auto any = [&] { return __ballot((low & 0xffffu) != 0 || top == __builtin_inff()) != 0; };
+    auto any = [&] {
+        return __ballot((low & 0xffffu) != 0 || top == __builtin_inff() || min(least & 0xffffu, least >> 16) < W_LEAST - 1) != 0;
+    };
     // The products are written out so that a block's sums stay in their registers (left to the compiler, they are copied from
     // one set to another every K-tile, and spilled).  The waits that it would put between them and other uses of these registers
     // stand at the ends of a K-tile.
@@ -156,6 +180,10 @@ __device__ __forceinline__ bool terms_loop(const Gemm32Args& a, char* lds, int u
         asm volatile("" ::: "memory");
     };
     const int last = kt1 - 1;
+    // whether X has such values in this tile's rows
+    const int* words = a.inexact + 4 + (2 * u0 * a.kb >> 2);
+    const int nwords = (2 * (u0 + NB) * a.kb + 3 >> 2) - (2 * u0 * a.kb >> 2);
+    const int small[2] = {words[min(tid, nwords - 1)], words[min(tid + 256, nwords - 1)]};
 #pragma unroll
     for (int d = 0; d < WS; ++d) {
         if (d < 2)
@@ -164,6 +192,8 @@ __device__ __forceinline__ bool terms_loop(const Gemm32Args& a, char* lds, int u
 #pragma unroll
         for (int i = 0; i < 8; ++i) stage_w(min(kt0 + d, last), d, i);
     }
+    int more = 0;
+    for (int i = tid + 512; i < nwords; i += 256) more |= words[i];
     meet(std::integral_constant<int, 8>{});  // all but the third W
     u32x4 wf[8], x0[3];
     f32x4 sum[NB][8];
@@ -174,9 +204,11 @@ __device__ __forceinline__ bool terms_loop(const Gemm32Args& a, char* lds, int u
         read_w(q, 0, i, 0);
         read_w(q, 0, i, 1);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) first(q, wf[i], j);
+        for (int j = 0; j < 4; ++j) {
+            first(q, wf[i], j, i < 4);
+        }
     }
-    const bool odd = any();
+    const bool odd = any() || __ballot((small[0] | small[1] | more) != 0) != 0;
     if (lane == 0) seen[w] = odd;
 #pragma unroll
     for (int k = 0; k < 3; ++k) read_x(x0, 0, 0, k);
@@ -226,7 +258,7 @@ __device__ __forceinline__ bool terms_loop(const Gemm32Args& a, char* lds, int u
                     const int at = 3 * (NB - 1) * i;
                     if (s == at) read_w(q[i], sw, i, 0);
                     if (s == at + 1) read_w(q[i], sw, i, 1);
-                    if (s >= at + 14 && s < at + 18) first(q[i], wn[i], s - at - 14);
+                    if (s >= at + 14 && s < at + 18) first(q[i], wn[i], s - at - 14, i < 4);
                     if (s == at + 2) stage_w(min(kt + WS, last), pw, i);
                 }
                 if (b == NB - 1 && m >= 4 && m < 4 + PX) stage_x(min(kt + XS, last), px, m - 4);

@@ -736,6 +736,84 @@ def test_gemm32_in_terms(M, N, K, plan, monkeypatch):
         assert torch.equal(hip.gemm32(dev(x), dev(v)), want[at])
 
 
+# every tile height over more than one chain of 16 K-tiles, whole and in slices, odd numbers of K-tiles, heights side by side
+HEIGHTS = [(50, 300, 1056, (1, 2, 1)), (50, 300, 1056, (1, 0, 2)), (96, 257, 1280, (1, 2, 1)), (96, 257, 1280, (1, 1, 3)),
+           (120, 256, 1120, (1, 1, 1)), (120, 256, 1120, (1, 0, 5)), (160, 300, 1568, (1, 2, 1)), (160, 300, 1568, (1, 0, 4)),
+           (300, 520, 1088, (3, 9, 1)), (300, 520, 1088, (3, 4, 2)), (903, 515, 96, (6, 18, 1))]
+
+
+def terms_only(hip, monkeypatch, N, plan):
+    """gemm32 in terms by ``plan``; and a function that gives what the fp32 instruction does."""
+    scratch = (plan[0] * -(-N // 256) - plan[1]) * plan[2] * 40960
+    monkeypatch.setattr(hip, "gemm32_small", lambda *_: False)
+    monkeypatch.setattr(hip, "gemm32_terms", lambda *_: (*plan, scratch))
+
+    def instruction(x, w):
+        with monkeypatch.context() as m:
+            m.setattr(hip, "gemm32_terms", lambda *_: None)
+            return hip.gemm32(x, w)
+    return instruction
+
+
+@pytest.mark.parametrize("bits,per_row", [(21, 6), (24, 1)])
+@pytest.mark.parametrize("M,N,K,plan", HEIGHTS)
+def test_gemm32_in_terms_leaves_no_bit_out(M, N, K, plan, bits, per_row, monkeypatch):
+    """X of integers of so many bits and W of few ones: every product and every sum, in any order, is an integer below 2^24 and
+    exact, so the result is, and a term left out is seen."""
+    from llm_map_reduce_summarizer_amd.ops import hip
+    terms_only(hip, monkeypatch, N, plan)
+    g = torch.Generator().manual_seed(5)
+    x = torch.randint(1 << (bits - 1), 1 << bits, (M, K), generator=g) | 1
+    x *= torch.randint(0, 2, (M, K), generator=g) * 2 - 1
+    w = torch.zeros(N, K, dtype=torch.int64)
+    w.scatter_(1, torch.rand(N, K, generator=g).argsort(1)[:, :per_row], 1)
+    w *= torch.randint(0, 2, (N, K), generator=g) * 2 - 1
+    want = (x.double() @ w.double().T).float()
+    assert torch.equal(hip.gemm32(dev(x.float()), dev(w.float())).cpu(), want)
+    # the two upper terms of X alone give other values nearly everywhere
+    top = x.float()
+    for shift in (2.0 ** (bits - 8), 2.0 ** (bits - 16)):
+        hi = torch.trunc(top / shift) * shift
+        top = top - hi
+    assert float(((x.double() - top.double()) @ w.double().T != want).double().mean()) > 0.8
+
+
+@pytest.mark.parametrize("kind", ["bit", "inf", "subnormal"])
+def test_gemm32_in_terms_finds_each_column_of_w(kind, monkeypatch):
+    """Two waves share a tile's columns and look at half of them each: one value that is not its bf16 term, in every block of
+    16 columns, in the first K-tile, in the one behind a chain and in the last."""
+    from llm_map_reduce_summarizer_amd.ops import hip
+    M, N, K = 70, 256, 576
+    instruction = terms_only(hip, monkeypatch, N, (1, 1, 1))
+    x, w = dev(rnd(M, K, seed=1)), dev(rnd(N, K, seed=2, dtype=BF).float())
+    got = hip.gemm32(x, w)
+    assert not torch.equal(got, instruction(x, w)) and rel(got, x.cpu().double() @ w.cpu().double().T) < 1e-6
+    for n in range(0, N, 16):
+        for k in (n % 32, 16 * 32 + 5, K - 1 - n % 3):
+            v = w.clone()
+            at = n + (n // 16 * 5) % 16, k
+            v[at] = {"bit": v[at] * (1 + 2.0 ** -20), "inf": float("inf"), "subnormal": 2.0 ** -130}[kind]
+            assert torch.equal(hip.gemm32(x, v), instruction(x, v)), (n, k)
+
+
+@pytest.mark.parametrize("M,K,tiles,at", [(70, 512, 1, (0, 0)), (70, 512, 1, (69, 511)), (70, 608, 1, (33, 607)), (96, 544, 1, (95, 543)),
+                                          (161, 1056, 2, (97, 1055)), (160, 9632, 1, (159, 9631)), (160, 9632, 1, (3, 7000))])
+def test_gemm32_in_terms_of_values_finer_than_bf16(M, K, tiles, at, monkeypatch):
+    """One value of X whose lowest bits are below bf16's: what the fp32 instruction gives.  Values down to 2^-110 are the sums of
+    their terms, whose own values are subnormal then."""
+    from llm_map_reduce_summarizer_amd.ops import hip
+    N = 256
+    instruction = terms_only(hip, monkeypatch, N, (tiles, tiles, 1))
+    x, w = dev(rnd(M, K, seed=1)), torch.zeros(N, K)
+    w[torch.arange(N), torch.randint(0, K, (N,), generator=torch.Generator().manual_seed(3))] = 1.0
+    w[7], w[7, at[1]] = 0.0, 1.0
+    w, x[at] = dev(w), 2.0 ** -111 * (1 + 2.0 ** -23)
+    assert torch.equal(hip.gemm32(x, w), instruction(x, w))
+    small = (torch.randint(1 << 23, 1 << 24, (M, K), generator=torch.Generator().manual_seed(4)).double() * 2.0 ** -133).float()
+    got = hip.gemm32(dev(small), w).double().cpu()
+    assert torch.equal(got, small.double() @ w.double().cpu().T)
+
+
 def test_gemm32_in_terms_of_infinities():
     """Infinities and NaN in X and W make what fp32 products and sums make of them."""
     from llm_map_reduce_summarizer_amd.ops import hip
