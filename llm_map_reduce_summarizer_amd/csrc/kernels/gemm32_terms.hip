@@ -8,7 +8,10 @@
 // looked at as it is read.  If a value has lower bits, is infinite (an infinity times a term of 0 is no number) or smaller than bf16's
 // normal numbers (whose products the instruction forms with fewer bits), or if X has a value whose lowest bits would be finer than
 // bf16's (below 2^-110), a flag is set and the fp32 instruction's form (gemm32.hip), which is launched behind and otherwise returns
-// at once, makes the whole result.  A workgroup that sees it in its first K-tile or its rows of X stops there.
+// at once, makes the whole result.  A workgroup that sees it in its first K-tile or its rows of X stops there, others when their next
+// chain of 16 K-tiles ends.  What that costs, us: 903 x 28672 x 4096 on the fp32 instruction 1550, by way of here with 24 bits in all of W
+// 1612, in half of its rows 1640 (2100 where nobody asks the others), in half of its columns 1730, in its last value alone 2100; 160 x
+// 6144 x 4096 74, 96, 113, 121, 126.
 //
 // Relative error (2-norm, random operands, K 4096 - 22528, chains of 16 K-tiles on both): 2.4e-7, the fp32 instruction 4.1e-7, as one
 // sum takes the products of 32 columns and not of four.
@@ -37,7 +40,8 @@ constexpr int WI = TN * 128, WS = 3;    // bytes of W's K-tile, and how many are
 constexpr int x_slots(int nb) { return nb <= 3 ? 3 : 2; }
 constexpr int LDS_BYTES = WS * WI + 2 * 2 * MAX_NB * BLOCK;
 constexpr int SLOT = MAX_NB * 32 * TN;  // scratch floats of a slice of a tile
-static_assert(LDS_BYTES + 16 <= 160 * 1024 && x_slots(3) * 2 * 3 * BLOCK <= 2 * 2 * MAX_NB * BLOCK, "LDS");
+constexpr int TAIL = 512 + 3 * 1024;    // and behind these what is known of values that are not the sums of their terms
+static_assert(LDS_BYTES + TAIL <= 160 * 1024 && x_slots(3) * 2 * 3 * BLOCK <= 2 * 2 * MAX_NB * BLOCK, "LDS");
 
 typedef __attribute__((address_space(3))) void* lds_ptr;
 
@@ -60,17 +64,12 @@ __device__ __forceinline__ uint32_t below(uint32_t v) {
 }  // namespace
 
 // X's terms, laid out as the matrix instruction reads them: [M / 16][K / 32][term][lane][8], lane (r, g) holding row r, k 4 g .. and
-// 16 + 4 g ..  Rows past M are zeros.  ``inexact`` is cleared; behind it, on 16 bytes, a byte for each [M / 16][K / 32] says
-// whether X has a value there that is not the sum of its terms, and zeros up to a multiple of four.
+// 16 + 4 g ..  Rows past M are zeros.  ``inexact`` is cleared; 16 bytes behind it, a byte for four pieces says whether X has a value
+// there that is not the sum of its terms, and zeros up to a multiple of 16.
 __global__ __launch_bounds__(256) void terms32_kernel(const float* __restrict__ x, int ldx, char* __restrict__ out, int M, int kb,
                                                       int pieces, int* inexact) {
-    char* small = reinterpret_cast<char*>(inexact) + 16;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        *inexact = 0;
-        for (int i = pieces; i % 4; ++i) small[i] = 0;
-    }
-    const int lane = threadIdx.x & 63, p = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (p >= pieces) return;
+    __shared__ uint32_t s_small[4];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, p = blockIdx.x * 4 + w;
     const int block = p / kb, kt = p - block * kb, m = block * 16 + (lane & 15);
     u32x4 v[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
     if (m < M) {
@@ -79,14 +78,14 @@ __global__ __launch_bounds__(256) void terms32_kernel(const float* __restrict__ 
         v[1] = in[4];
     }
     u32x4 t[3];
-    bool least = false;
+    bool small = false;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         uint32_t a[2][3];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const uint32_t u = v[i >> 1][2 * (i & 1) + j], r = below(u);
-            least |= (u & 0x7fffffffu) - 1 < X_LEAST - 1;
+            small |= (u & 0x7fffffffu) - 1 < X_LEAST - 1;
             a[j][0] = (u & 0x7fffffffu) > 0x7f800000u ? u | 0x00400000u : u;  // a NaN whose bits are all low
             a[j][1] = r;
             a[j][2] = below(r);
@@ -94,22 +93,33 @@ __global__ __launch_bounds__(256) void terms32_kernel(const float* __restrict__ 
 #pragma unroll
         for (int k = 0; k < 3; ++k) t[k][i] = high_halves(a[0][k], a[1][k]);
     }
-    u32x4* o = reinterpret_cast<u32x4*>(out + (size_t)p * BLOCK) + lane;
+    if (p < pieces) {
+        u32x4* o = reinterpret_cast<u32x4*>(out + (size_t)p * BLOCK) + lane;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) o[64 * k] = t[k];
-    const bool any = __ballot(least) != 0;
-    if (lane == 0) small[p] = any;
+        for (int k = 0; k < 3; ++k) o[64 * k] = t[k];
+    }
+    const bool any = __ballot(small) != 0;
+    if (lane == 0) s_small[w] = any;
+    __syncthreads();
+    char* flags = reinterpret_cast<char*>(inexact) + 16;
+    if (threadIdx.x == 0) flags[blockIdx.x] = s_small[0] | s_small[1] | s_small[2] | s_small[3];
+    if (blockIdx.x == 0) {
+        if (threadIdx.x == 0) *inexact = 0;
+        const int i = gridDim.x + threadIdx.x;
+        if (threadIdx.x < 16 && i < (((int)gridDim.x + 15) & ~15)) flags[i] = 0;
+    }
 }
 
 namespace {
-// Outputs of (row block b, column block i ^ 4 wr) of a tile of nb 32-row units: row lane & 15, columns 4 (lane >> 4) ..
+// Outputs of (row block b, column block i ^ wr) of a tile of nb 32-row units: row lane & 15, columns 4 (lane >> 4) ..
 __device__ __forceinline__ void store_terms(const Gemm32Args& a, int u0, int nb, int n0, int b, int i, const f32x4& v) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    store_c(a, 32 * u0 + 16 * (nb * (w >> 1) + b) + (lane & 15), n0 + 128 * (w & 1) + 16 * (i ^ 4 * (w >> 1)) + 4 * (lane >> 4), v);
+    store_c(a, 32 * u0 + 16 * (nb * (w >> 1) + b) + (lane & 15), n0 + 128 * (w & 1) + 16 * (i ^ (w >> 1)) + 4 * (lane >> 4), v);
 }
 
 // K-tiles [kt0, kt1) of 32 NB rows from 32 u0 on and columns n0 ..; wave (wr, wc) has half of the rows and 128 columns: acc[row
-// block][column block ^ 4 wr], as the two waves of the same columns look at the first four each.  False: some value is not the sum of its terms, and the sums are not made.
+// block][column block ^ wr], so that the two waves that have the same columns each look at every other block of them, by the same
+// code.  False: some value is not the sum of its terms, and the sums are not made.
 template <int NB>
 __device__ __forceinline__ bool terms_loop(const Gemm32Args& a, char* lds, int u0, int n0, int kt0, int kt1, f32x4 (&acc)[NB][8]) {
     constexpr int XI = 2 * NB * BLOCK, PX = (6 * NB + 3) / 4, XS = x_slots(NB);
@@ -137,30 +147,33 @@ __device__ __forceinline__ bool terms_loop(const Gemm32Args& a, char* lds, int u
     auto stage_w = [&](int kt, int slot, int i) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr)(lds + slot * WI + (8 * w + i) * 1024), 16, vw[i], kt * 128, 0, 0);
     };
-    const int wlo = (128 * wc + r16) * 128 + ((g ^ (r16 >> 1)) << 4), wl[2] = {wlo + wr * 8192, wlo - wr * 8192}, xlo = WS * WI + wr * NB * BLOCK + lane * 16;
+    const int wlo = (128 * wc + r16) * 128 + ((g ^ (r16 >> 1)) << 4), wl[2] = {wlo + wr * 2048, wlo - wr * 2048};
+    const int xlo = WS * WI + wr * NB * BLOCK + lane * 16;
     auto read_w = [&](u32x4 (&q)[2], int slot, int i, int h) {
-        q[h] = *reinterpret_cast<const u32x4*>(lds + slot * WI + (h ? wl[i >> 2] ^ 64 : wl[i >> 2]) + i * 2048);
+        q[h] = *reinterpret_cast<const u32x4*>(lds + slot * WI + (h ? wl[i & 1] ^ 64 : wl[i & 1]) + i * 2048);
     };
     auto read_x = [&](u32x4 (&x)[3], int slot, int b, int k) {
         x[k] = *reinterpret_cast<const u32x4*>(lds + slot * XI + xlo + b * BLOCK + k * 1024);
     };
-    // First terms of a pair of W's values.  ``look``: and what they leave out, in this wave's half of the columns that it shares with
-    // another one: ``low`` gathers the bits below them, ``top`` the largest size, ``least`` the smallest one but zero (as 2 d - 1).
+    // First terms of a pair of W's values.  ``look``: and what they leave out: ``low`` gathers the bits below them, ``top`` the largest
+    // size, and ``least`` the smallest one but zero, as 2 d - 1, in products of its own (written out, as the compiler would put a
+    // wait on either side of such a minimum between written-out lines).
     uint32_t low = 0, least = 0xffffffff;
     float top = 0.f;
     auto first = [&](const u32x4 (&q)[2], u32x4& f, int i, bool look) {
         const uint32_t u = q[i >> 1][2 * (i & 1)], v = q[i >> 1][2 * (i & 1) + 1];
-        uint32_t d = high_halves(u, v), e;
+        uint32_t d = high_halves(u, v);
         if (look) {
             low |= u | v;
             top = fmaxf(fmaxf(top, fabsf(__uint_as_float(u))), fabsf(__uint_as_float(v)));
-            // (the compiler would put a wait on either side of such a minimum between written-out lines)
-            asm volatile("v_pk_mad_u16 %1, %0, %5, %6\n\tv_pk_min_u16 %2, %2, %1"
-                         : "+v"(d), "=&v"(e), "+v"(least), "+v"(low), "+v"(top) : "s"(0x00020002), "v"(0xffffffff));
-        } else {
-            asm volatile("" : "+v"(d));  // here, and not where they are used
         }
+        asm volatile("" : "+v"(d), "+v"(low), "+v"(top));  // here, and not where they are used
         f[i] = d;
+    };
+    auto smallest = [&](uint32_t d) {
+        uint32_t e;
+        asm volatile("v_pk_mad_u16 %1, %2, %3, %4\n\tv_pk_min_u16 %0, %0, %1"
+                     : "+v"(least), "=&v"(e) : "v"(d), "s"(0x00020002), "v"(0xffffffff));
     };
     auto any = [&] {
         return __ballot((low & 0xffffu) != 0 || top == __builtin_inff() || min(least & 0xffffu, least >> 16) < W_LEAST - 1) != 0;
@@ -180,10 +193,20 @@ __device__ __forceinline__ bool terms_loop(const Gemm32Args& a, char* lds, int u
         asm volatile("" ::: "memory");
     };
     const int last = kt1 - 1;
-    // whether X has such values in this tile's rows
-    const int* words = a.inexact + 4 + (2 * u0 * a.kb >> 2);
-    const int nwords = (2 * (u0 + NB) * a.kb + 3 >> 2) - (2 * u0 * a.kb >> 2);
-    const int small[2] = {words[min(tid, nwords - 1)], words[min(tid + 256, nwords - 1)]};
+    // What X's split has found in this tile's rows (and, to whole 16 bytes, in some next to them) and whether another workgroup has
+    // met something go to LDS ahead of the first K-tile, and are not waited for by themselves.
+    int* heard = reinterpret_cast<int*>(lds + LDS_BYTES);        // word 0: the flag, as it was asked for last
+    int* seen = heard + 64;
+    const volatile int* words = heard + 128;
+    const __amdgpu_buffer_rsrc_t rf = buffer(a.inexact, 4);
+    auto ask = [&] { __builtin_amdgcn_raw_ptr_buffer_load_lds(rf, (lds_ptr)heard, 4, lane ? 4 : 0, 0, 0, 16); };
+    const int flag0 = (2 * u0 * a.kb >> 2) & ~15, flags = ((((a.M + 31) >> 5) * 2 * a.kb + 3 >> 2) + 15 & ~15) - flag0;
+    const int nwords = ((2 * (u0 + NB) * a.kb - 1 >> 2) - flag0 >> 2) + 1;
+    const char* flag = reinterpret_cast<const char*>(a.inexact) + 16 + flag0;
+    if (w == 3)
+        ask();
+    else if (256 * w < nwords)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(buffer(flag, flags), (lds_ptr)(heard + 128 + 256 * w), 16, w * 1024 + lane * 16, 0, 0, 0);
 #pragma unroll
     for (int d = 0; d < WS; ++d) {
         if (d < 2)
@@ -192,12 +215,14 @@ __device__ __forceinline__ bool terms_loop(const Gemm32Args& a, char* lds, int u
 #pragma unroll
         for (int i = 0; i < 8; ++i) stage_w(min(kt0 + d, last), d, i);
     }
-    int more = 0;
-    for (int i = tid + 512; i < nwords; i += 256) more |= words[i];
+    int small = 0;
+    for (int i = tid + 256 * 3; i < nwords; i += 256) small |= reinterpret_cast<const int*>(flag)[i];
     meet(std::integral_constant<int, 8>{});  // all but the third W
+#pragma unroll
+    for (int i = 0; i < 3; ++i) small |= words[min(tid + 256 * i, min(nwords, 768) - 1)];
+    small |= *(volatile int*)heard;
     u32x4 wf[8], x0[3];
     f32x4 sum[NB][8];
-    int* seen = reinterpret_cast<int*>(lds + LDS_BYTES);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         u32x4 q[2];
@@ -205,10 +230,11 @@ __device__ __forceinline__ bool terms_loop(const Gemm32Args& a, char* lds, int u
         read_w(q, 0, i, 1);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            first(q, wf[i], j, i < 4);
+            first(q, wf[i], j, i % 2 == 0);
+            if (i % 2 == 0) smallest(wf[i][j]);
         }
     }
-    const bool odd = any() || __ballot((small[0] | small[1] | more) != 0) != 0;
+    const bool odd = any() || __ballot(small != 0) != 0;
     if (lane == 0) seen[w] = odd;
 #pragma unroll
     for (int k = 0; k < 3; ++k) read_x(x0, 0, 0, k);
@@ -258,7 +284,8 @@ __device__ __forceinline__ bool terms_loop(const Gemm32Args& a, char* lds, int u
                     const int at = 3 * (NB - 1) * i;
                     if (s == at) read_w(q[i], sw, i, 0);
                     if (s == at + 1) read_w(q[i], sw, i, 1);
-                    if (s >= at + 14 && s < at + 18) first(q[i], wn[i], s - at - 14, i < 4);
+                    if (s >= at + 14 && s < at + 18) first(q[i], wn[i], s - at - 14, i % 2 == 0);
+                    if (i % 2 == 0 && s >= at + 18 && s < at + 22) smallest(wn[i][s - at - 18]);
                     if (s == at + 2) stage_w(min(kt + WS, last), pw, i);
                 }
                 if (b == NB - 1 && m >= 4 && m < 4 + PX) stage_x(min(kt + XS, last), px, m - 4);
@@ -271,8 +298,15 @@ __device__ __forceinline__ bool terms_loop(const Gemm32Args& a, char* lds, int u
 #pragma unroll
         for (int k = 0; k < 3; ++k) x0[k] = x[NB & 1][k];
     };
-    for (int kt = kt0; kt < kt1;) {  // chains
-        for (const int end = min(kt + LONG_RUN, kt1); kt < end; ++kt) step(kt);
+    // Chains.  At the end of one the workgroup says what it has met and ends with it if another one has met something: what it stores
+    // then is overwritten.  (Without a branch, and in the loop's bound: around one the compiler moves the sums about and spills.)
+    for (int kt = kt0, stop = kt1; kt < stop;) {
+        const int end = min(kt + LONG_RUN, kt1);
+        for (; kt < end; ++kt) {
+            // the flag arrives ahead of this K-tile's meeting and is read behind it; the next one is asked for LONG_RUN K-tiles later
+            if (kt == end - 1 && end < kt1 && w == 0) ask();
+            step(kt);
+        }
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll
@@ -285,8 +319,9 @@ __device__ __forceinline__ bool terms_loop(const Gemm32Args& a, char* lds, int u
                 }
                 asm volatile("" : "+a"(acc[b][i]), "+a"(acc[b][i + 1]), "+a"(acc[b][i + 2]), "+a"(acc[b][i + 3]));
             }
+        __builtin_amdgcn_raw_buffer_store_b32(1u, rf, any() && lane == 0 ? 0 : 4, 0, 16);  // (at 4: nowhere)
+        if (__builtin_amdgcn_readfirstlane(*(volatile int*)heard) && end < kt1) stop = kt;
     }
-    if (any() && lane == 0) atomicOr(a.inexact, 1);
 #pragma unroll
     for (int b = 0; b < NB; ++b)
 #pragma unroll
@@ -311,7 +346,7 @@ __device__ __forceinline__ void terms_tile(const Gemm32Args& a, char* lds, int u
 }  // namespace
 
 __global__ __launch_bounds__(256, 1) void gemm32_terms_kernel(const Gemm32Args a) {
-    __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES + 16];
+    __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES + TAIL];
     int p = blockIdx.x, slice = -1, kt0 = 0, kt1 = a.kb;
     if (p < a.whole) {
         p = xcd_position(p, a.whole);

@@ -796,6 +796,31 @@ def test_gemm32_in_terms_finds_each_column_of_w(kind, monkeypatch):
             assert torch.equal(hip.gemm32(x, v), instruction(x, v)), (n, k)
 
 
+@pytest.mark.parametrize("M,N,K,plan", [(160, 1500, 2080, (1, 6, 1)), (300, 1024, 1600, (3, 12, 1)), (500, 700, 3200, (4, 6, 3))])
+@pytest.mark.parametrize("n0,n1,k", [(0, 256, 0), (300, 301, 700), (500, 700, 520), (699, 700, 1599)])
+def test_gemm32_in_terms_stops_with_its_neighbours(M, N, K, plan, n0, n1, k, monkeypatch):
+    """Some rows of W have more bits from some column on: tiles that see it, at their start, behind a chain or at their end, and
+    tiles that hear of it from others, whole and in slices, and again when the call is replayed."""
+    from llm_map_reduce_summarizer_amd.ops import hip
+    instruction = terms_only(hip, monkeypatch, N, plan)
+    x, w = dev(rnd(M, K, seed=1)), dev(rnd(N, K, seed=2, dtype=BF).float())
+    clean = hip.gemm32(x, w)
+    v = w.clone()
+    v[n0:n1, k:] *= 1 + 2.0 ** -20
+    want = instruction(x, v)
+    assert not torch.equal(clean, want)
+    buf = w.clone()
+    hip.gemm32(x, buf)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = hip.gemm32(x, buf)
+    for src, res in ((v, want), (w, clean), (v, want), (v, want), (w, clean)):
+        buf.copy_(src)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, res) and torch.equal(hip.gemm32(x, src), res)
+
+
 @pytest.mark.parametrize("M,K,tiles,at", [(70, 512, 1, (0, 0)), (70, 512, 1, (69, 511)), (70, 608, 1, (33, 607)), (96, 544, 1, (95, 543)),
                                           (161, 1056, 2, (97, 1055)), (160, 9632, 1, (159, 9631)), (160, 9632, 1, (3, 7000))])
 def test_gemm32_in_terms_of_values_finer_than_bf16(M, K, tiles, at, monkeypatch):
