@@ -272,6 +272,13 @@ def project(x, w, role):
     return hip.gemm(x, w) if p[0] == "gemm" else _plan_parts(hip, p, x, w, None)
 
 
+def mark_values(*weights):
+    """Notes on fp32 weights on the GPU, laid out once, what their products ask of their values (hip.gemm32)."""
+    for w in weights:
+        if w.dtype == torch.float32 and _use_hip(w):
+            w.bf16_values = hip.bf16_values(w)
+
+
 def project_glu(x, w_gu, limit, alpha, shift):
     """min(g, limit) sigmoid(alpha g) (clamp(u, limit) + shift) of the [8 gate | 8 up]-blocked projection."""
     return _impl(x).project_glu(x, w_gu, limit, alpha, shift)

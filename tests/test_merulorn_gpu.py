@@ -821,6 +821,63 @@ def test_gemm32_in_terms_stops_with_its_neighbours(M, N, K, plan, n0, n1, k, mon
         assert torch.equal(got, res) and torch.equal(hip.gemm32(x, src), res)
 
 
+@pytest.mark.parametrize("at", [(0, 0), (8191, 2047), (8999, 4095)])
+@pytest.mark.parametrize("value,held", [(1.0, True), (0.0, True), (-0.0, True), (2.0 ** -126, True), (1 + 2.0 ** -8, False), (3.0e38, False),
+                                        (2.0 ** -127, False), (-2.0 ** -149, False), (float("inf"), False), (float("nan"), False)])
+def test_weights_of_bf16_values(at, value, held):
+    from llm_map_reduce_summarizer_amd.ops import hip
+    w = torch.randn(9000, 4096, generator=torch.Generator(DEV).manual_seed(1), device=DEV).to(BF).float()
+    w[at] = value
+    assert hip.bf16_values(w) == held and hip.bf16_values(w[at[0]: at[0] + 1, at[1]: at[1] + 1]) == held
+    assert hip.bf16_values(w[:, :1][:0])
+
+
+def entries(hip, monkeypatch):
+    """Names of the entry points called from here on."""
+    names, fn = [], hip._fn
+    monkeypatch.setattr(hip, "_fn", lambda name: names.append(name) or fn(name))
+    return names
+
+
+def test_gemm32_of_weights_known_to_have_more_bits(monkeypatch):
+    """They run on the fp32 instruction alone, as before there were terms; a mark that no longer holds costs no bit."""
+    from llm_map_reduce_summarizer_amd import ops
+    from llm_map_reduce_summarizer_amd.ops import hip
+    x, w = dev(rnd(300, 4096, seed=1)), dev(rnd(4096, 4096, seed=2))
+    names = entries(hip, monkeypatch)
+    got = hip.gemm32(x, w)
+    assert names == ["mrsum_gemm32_terms"]
+    ops.mark_values(w)
+    assert w.bf16_values is False and torch.equal(ops.project(x, w, "o")[0], got) and torch.equal(ops.logits32(x, w), got)
+    assert names[1:] == ["mrsum_gemm32"] * 2
+    v = w.to(BF).float()
+    ops.mark_values(v)
+    assert v.bf16_values is True
+    v.copy_(w)
+    assert torch.equal(hip.gemm32(x, v), got)
+    w.copy_(w.to(BF).float())
+    assert rel(hip.gemm32(x, w).cpu(), x.cpu().double() @ w.cpu().double().T) < 1e-6
+
+
+@pytest.mark.parametrize("model", ["tiny-merulorn", "tiny-muzozen"])
+@pytest.mark.parametrize("more", [False, True])
+def test_models_know_which_weights_are_bf16_values(model, more, monkeypatch):
+    from llm_map_reduce_summarizer_amd.engine.config import get_model_config
+    from llm_map_reduce_summarizer_amd.engine.hybrid import HybridModel
+    plain = HybridModel._random
+
+    def random(self, seed):
+        get = plain(self, seed)
+        return lambda name, shape: get(name, shape).float() * (1 + 2.0 ** -12) if more else get(name, shape)
+    monkeypatch.setattr(HybridModel, "_random", random)
+    m = HybridModel(get_model_config(model), torch.device(DEV), F32)
+    found = [m.lm_head] + [t for la in m.layers for t in (la.w.w_in, la.w.w_o)]
+    found += [la.w.w_gu for la in m.layers if hasattr(la.w, "w_gu")] + [la.latent.w.w_uq for la in m.layers if la.latent is not None]
+    assert len(found) > 4 and [t.bf16_values for t in found] == [not more] * len(found)
+    half = HybridModel(get_model_config(model), torch.device(DEV), BF)
+    assert not hasattr(half.lm_head, "bf16_values")
+
+
 @pytest.mark.parametrize("M,K,tiles,at", [(70, 512, 1, (0, 0)), (70, 512, 1, (69, 511)), (70, 608, 1, (33, 607)), (96, 544, 1, (95, 543)),
                                           (161, 1056, 2, (97, 1055)), (160, 9632, 1, (159, 9631)), (160, 9632, 1, (3, 7000))])
 def test_gemm32_in_terms_of_values_finer_than_bf16(M, K, tiles, at, monkeypatch):
