@@ -26,8 +26,9 @@ template <int NB>
 constexpr int RUN = NB > 4 ? LONG_RUN : 4;
 }  // namespace
 
-// K-tiles [kt0, kt1) of a tile of NB row blocks; acc[row block][column block].  ONE: there are at most LONG_RUN of them
-template <int NB, bool ONE>
+// K-tiles [kt0, kt1) of a tile of NB row blocks; acc[row block][column block].  ONE: there are at most LONG_RUN of them;
+// ONCE: W goes past the caches (gemm32_launch)
+template <int NB, bool ONE, bool ONCE>
 __device__ __forceinline__ void k_loop(const Gemm32Args& a, char* lds, int m0, int n0, int kt0, int kt1, f32x4 (&acc)[8][2]) {
     typedef __attribute__((address_space(3))) void* lds_ptr;
     constexpr int XB = NB * 2048, IMAGE = XB + STAGE, XI = (NB + 1) / 2;  // a K-tile of X; of both; pieces of X a wave
@@ -55,9 +56,7 @@ __device__ __forceinline__ void k_loop(const Gemm32Args& a, char* lds, int m0, i
         vx[i] = r * a.ldx * 4 + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
         dx[i] = STAGE + p * 1024;
     }
-    // Up to 48 rows are one row of tiles: W is read once, nontemporal (aux 2).  us, K 4096: 4 x 128256 399 -> 369 (5.7 TB/s), 2 x
-    // 14336 56 -> 52, 4 x 4096 19.6 -> 18.3; 4 x 4096 x 14336 51 -> 47.
-    constexpr int NT = NB <= 3 ? 2 : 0;
+    constexpr int NT = ONCE ? 2 : 0;  // nontemporal
     auto stage = [&](int kt, int buf) {
         char* dst = lds + buf * IMAGE;
 #pragma unroll
@@ -143,7 +142,7 @@ __device__ __forceinline__ void k_loop(const Gemm32Args& a, char* lds, int m0, i
     __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));  // nothing may arrive in LDS that another workgroup has by then
 }
 
-template <bool ONE>
+template <bool ONE, bool ONCE>
 __global__ __launch_bounds__(256, 2) void gemm32_kernel(const Gemm32Args a) {
     if (a.inexact && !*a.inexact) return;
     __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
@@ -172,16 +171,26 @@ __global__ __launch_bounds__(256, 2) void gemm32_kernel(const Gemm32Args a) {
     for (int b = 0; b < 8; ++b)
 #pragma unroll
         for (int i = 0; i < 2; ++i) acc[b][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    switch (nb) {
-        case 1: k_loop<1, ONE>(a, lds, m0, n0, kt0, kt1, acc); break;
-        case 2: k_loop<2, ONE>(a, lds, m0, n0, kt0, kt1, acc); break;
-        case 3: k_loop<3, ONE>(a, lds, m0, n0, kt0, kt1, acc); break;
-        case 4: k_loop<4, ONE>(a, lds, m0, n0, kt0, kt1, acc); break;
-        case 5: k_loop<5, ONE>(a, lds, m0, n0, kt0, kt1, acc); break;
-        case 6: k_loop<6, ONE>(a, lds, m0, n0, kt0, kt1, acc); break;
-        case 7: k_loop<7, ONE>(a, lds, m0, n0, kt0, kt1, acc); break;
-        default: k_loop<8, ONE>(a, lds, m0, n0, kt0, kt1, acc); break;
+#define LOOP(NB_) k_loop<NB_, ONE, ONCE>(a, lds, m0, n0, kt0, kt1, acc)
+    if constexpr (ONCE) {
+        switch (nb) {
+            case 1: LOOP(1); break;
+            case 2: LOOP(2); break;
+            default: LOOP(3); break;
+        }
+    } else {
+        switch (nb) {
+            case 1: LOOP(1); break;
+            case 2: LOOP(2); break;
+            case 3: LOOP(3); break;
+            case 4: LOOP(4); break;
+            case 5: LOOP(5); break;
+            case 6: LOOP(6); break;
+            case 7: LOOP(7); break;
+            default: LOOP(8); break;
+        }
     }
+#undef LOOP
     if (slice >= 0) {
         f32x4* out = reinterpret_cast<f32x4*>(a.part + ((size_t)(p - a.whole) * a.splits + slice) * (T32 * T32)) + tid;
 #pragma unroll
@@ -295,10 +304,19 @@ int gemm32_launch(const float* x, int ldx, const float* w, int ldw, float* c, in
     a.whole = splits > 1 ? whole : tiles;
     a.splits = splits > 1 ? splits : 1;
     const int rest = tiles - a.whole;
-    if (ceil_div(a.kb, a.whole ? 1 : a.splits) <= LONG_RUN)
-        gemm32_kernel<true><<<a.whole + rest * a.splits, 256, 0, s>>>(a);
-    else
-        gemm32_kernel<false><<<a.whole + rest * a.splits, 256, 0, s>>>(a);
+    // Up to 48 rows are one row of tiles, which read W once a call; W of more than the 256 MiB that the last cache holds is gone by
+    // the next call and goes past the caches.  us through the caches -> past them, the same W again / another one each time, K 4096: 4
+    // x 14336 (224 MiB) 38.2 -> 42.9 / 53.8 -> 49.6, 4 x 16384 (256 MiB) 47.6 -> 55.7 / 60.0 -> 56.4, 4 x 18432 59.7 -> 57.6 / 65.1 ->
+    // 60.2, 4 x 20608 67.3 -> 60.5 / 69.7 -> 62.8; 4 x 4096 15.8 -> 17.2 / 18.4 -> 18.0; 4 x 128256 399 -> 369 (5.7 TB/s).
+    const bool once = M <= 48 && (size_t)N * K * 4 > (256u << 20);
+    const int grid = a.whole + rest * a.splits;
+    if (ceil_div(a.kb, a.whole ? 1 : a.splits) <= LONG_RUN) {
+        if (once) gemm32_kernel<true, true><<<grid, 256, 0, s>>>(a);
+        else gemm32_kernel<true, false><<<grid, 256, 0, s>>>(a);
+    } else {
+        if (once) gemm32_kernel<false, true><<<grid, 256, 0, s>>>(a);
+        else gemm32_kernel<false, false><<<grid, 256, 0, s>>>(a);
+    }
     if (rest) gemm32_tail_kernel<<<rest * 4, 256, 0, s>>>(a);
     return (int)hipGetLastError();
 }

@@ -936,6 +936,22 @@ def test_gemm32_in_terms_of_many_rows(monkeypatch):
         assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 48, 49])
+@pytest.mark.parametrize("K,splits", [(512, 1), (4096, 1), (4096, 3)])
+def test_gemm32_of_weights_that_no_cache_holds(M, K, splits, monkeypatch):
+    """Beyond 256 MiB W is read past the caches, for up to 48 rows: the bits of two products of its halves."""
+    from llm_map_reduce_summarizer_amd.ops import hip
+    N = (1 << 26) // K + 3 * 128 + 5
+    tiles = lambda n: -(-M // 128) * -(-n // 128)  # noqa: E731
+    monkeypatch.setattr(hip, "gemm32_small", lambda *_: False)
+    monkeypatch.setattr(hip, "gemm32_splits", lambda m, n, kb: (tiles(n), 1, 0) if splits == 1 else (0, splits, tiles(n) * splits * 16384))
+    x = dev(rnd(M, K, seed=1))
+    w = torch.randn(N, K, generator=torch.Generator(DEV).manual_seed(2), device=DEV)
+    got, half = hip.gemm32(x, w), N // 256 * 128
+    assert torch.equal(got, torch.cat([hip.gemm32(x, w[:half]), hip.gemm32(x, w[half:])], 1))
+    assert rel(got.cpu(), (x.double() @ w.double().T).cpu()) < 1e-6
+
+
 def test_gemm32_deep():
     """K beyond what 31-bit offsets over a tile's rows reach."""
     from llm_map_reduce_summarizer_amd.ops import hip
