@@ -24,11 +24,14 @@ constexpr int T32 = 128, STAGE = T32 * 128;  // bytes of W's K-tile
 constexpr int LDS_BYTES = 80 * 1024;         // two workgroups on a CU
 template <int NB>
 constexpr int RUN = NB > 4 ? LONG_RUN : 4;
+
+// PAST_CACHES: W goes past the caches (gemm32_launch).  GUARDED: launched behind the terms, and does nothing unless they have met what
+// they hold short (a form of its own: the test of a pointer that is not there cost every other call 0.2 us, 16 x 768 x 768 8.1 -> 7.9)
+enum { PLAIN, PAST_CACHES, GUARDED };
 }  // namespace
 
-// K-tiles [kt0, kt1) of a tile of NB row blocks; acc[row block][column block].  ONE: there are at most LONG_RUN of them;
-// ONCE: W goes past the caches (gemm32_launch)
-template <int NB, bool ONE, bool ONCE>
+// K-tiles [kt0, kt1) of a tile of NB row blocks; acc[row block][column block].  ONE: there are at most LONG_RUN of them
+template <int NB, bool ONE, int FORM>
 __device__ __forceinline__ void k_loop(const Gemm32Args& a, char* lds, int m0, int n0, int kt0, int kt1, f32x4 (&acc)[8][2]) {
     typedef __attribute__((address_space(3))) void* lds_ptr;
     constexpr int XB = NB * 2048, IMAGE = XB + STAGE, XI = (NB + 1) / 2;  // a K-tile of X; of both; pieces of X a wave
@@ -56,7 +59,7 @@ __device__ __forceinline__ void k_loop(const Gemm32Args& a, char* lds, int m0, i
         vx[i] = r * a.ldx * 4 + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
         dx[i] = STAGE + p * 1024;
     }
-    constexpr int NT = ONCE ? 2 : 0;  // nontemporal
+    constexpr int NT = FORM == PAST_CACHES ? 2 : 0;  // nontemporal
     auto stage = [&](int kt, int buf) {
         char* dst = lds + buf * IMAGE;
 #pragma unroll
@@ -142,9 +145,9 @@ __device__ __forceinline__ void k_loop(const Gemm32Args& a, char* lds, int m0, i
     __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));  // nothing may arrive in LDS that another workgroup has by then
 }
 
-template <bool ONE, bool ONCE>
+template <bool ONE, int FORM>
 __global__ __launch_bounds__(256, 2) void gemm32_kernel(const Gemm32Args a) {
-    if (a.inexact && !*a.inexact) return;
+    if (FORM == GUARDED && !*a.inexact) return;
     __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -171,8 +174,8 @@ __global__ __launch_bounds__(256, 2) void gemm32_kernel(const Gemm32Args a) {
     for (int b = 0; b < 8; ++b)
 #pragma unroll
         for (int i = 0; i < 2; ++i) acc[b][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-#define LOOP(NB_) k_loop<NB_, ONE, ONCE>(a, lds, m0, n0, kt0, kt1, acc)
-    if constexpr (ONCE) {
+#define LOOP(NB_) k_loop<NB_, ONE, FORM>(a, lds, m0, n0, kt0, kt1, acc)
+    if constexpr (FORM == PAST_CACHES) {
         switch (nb) {
             case 1: LOOP(1); break;
             case 2: LOOP(2); break;
@@ -209,8 +212,9 @@ __global__ __launch_bounds__(256, 2) void gemm32_kernel(const Gemm32Args a) {
 }
 
 // adds the slices of the split tiles; one workgroup per (tile, 2 x 16 rows)
+template <bool GUARD>
 __global__ __launch_bounds__(256) void gemm32_tail_kernel(const Gemm32Args a) {
-    if (a.inexact && !*a.inexact) return;
+    if (GUARD && !*a.inexact) return;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, t = blockIdx.x >> 2, b = 2 * (blockIdx.x & 3);
     int tm, tn, b0, nb;
     tile32(a, a.whole + t, tm, tn);
@@ -310,14 +314,19 @@ int gemm32_launch(const float* x, int ldx, const float* w, int ldw, float* c, in
     // 60.2, 4 x 20608 67.3 -> 60.5 / 69.7 -> 62.8; 4 x 4096 15.8 -> 17.2 / 18.4 -> 18.0; 4 x 128256 399 -> 369 (5.7 TB/s).
     const bool once = M <= 48 && (size_t)N * K * 4 > (256u << 20);
     const int grid = a.whole + rest * a.splits;
+#define FORMS(ONE)                                                          \
+    if (inexact) gemm32_kernel<ONE, GUARDED><<<grid, 256, 0, s>>>(a);            \
+    else if (once) gemm32_kernel<ONE, PAST_CACHES><<<grid, 256, 0, s>>>(a);  \
+    else gemm32_kernel<ONE, PLAIN><<<grid, 256, 0, s>>>(a)
     if (ceil_div(a.kb, a.whole ? 1 : a.splits) <= LONG_RUN) {
-        if (once) gemm32_kernel<true, true><<<grid, 256, 0, s>>>(a);
-        else gemm32_kernel<true, false><<<grid, 256, 0, s>>>(a);
+        FORMS(true);
     } else {
-        if (once) gemm32_kernel<false, true><<<grid, 256, 0, s>>>(a);
-        else gemm32_kernel<false, false><<<grid, 256, 0, s>>>(a);
+        FORMS(false);
     }
-    if (rest) gemm32_tail_kernel<<<rest * 4, 256, 0, s>>>(a);
+#undef FORMS
+    if (!rest) return (int)hipGetLastError();
+    if (inexact) gemm32_tail_kernel<true><<<rest * 4, 256, 0, s>>>(a);
+    else gemm32_tail_kernel<false><<<rest * 4, 256, 0, s>>>(a);
     return (int)hipGetLastError();
 }
 
