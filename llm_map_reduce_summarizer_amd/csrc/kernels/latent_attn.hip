@@ -268,9 +268,7 @@ struct LatDecode {
 
 // KB: 32-column blocks of a cached row, VB: 128-column blocks of the latent.  Grid (S, ceil(H / 32), B).  Two barriers a
 // page: the next page's registers go to the other LDS stage between them, when every wave is past the page before.
-// ONCE: one workgroup has all heads, so that a page is read once, nontemporal (8 rows over 4096 tokens of 576: a decode step of
-// 8 layers 1032 -> 1021 us).
-template <int KB, int VB, bool ONCE>
+template <int KB, int VB>
 __global__ __launch_bounds__(512, 1) void latent_decode_kernel(const LatDecode a) {
     constexpr int LK = 32 * KB + 8, LP = BN + 8, IT = KB / 2;
     __shared__ __attribute__((aligned(16))) bf16 sk[2][BN * LK];
@@ -311,10 +309,8 @@ __global__ __launch_bounds__(512, 1) void latent_decode_kernel(const LatDecode a
     {                                                                                                   \
         const bf16* pg_ = a.cache + (size_t)id * BN * a.row;                                            \
         id = bt[min((p) + 1, p1 - 1)];                                                                  \
-        _Pragma("unroll") for (int i = 0; i < IT; ++i) {                                                \
-            const u32x4* p_ = reinterpret_cast<const u32x4*>(pg_ + 8 * min(tid + 512 * i, total - 1));  \
-            reg[i] = ONCE ? __builtin_nontemporal_load(p_) : *p_;                                       \
-        }                                                                                               \
+        _Pragma("unroll") for (int i = 0; i < IT; ++i)                                                  \
+            reg[i] = *reinterpret_cast<const u32x4*>(pg_ + 8 * min(tid + 512 * i, total - 1));          \
     }
     f32x4 acc[VB][2];
     float m[2] = {-INFINITY, -INFINITY}, l = 0.f;  // maxima of heads r16, 16 + r16; this lane's share of head 16 hb + r16's sum
@@ -451,12 +447,8 @@ MRSUM_API int mrsum_latent_decode(const void* q, const void* cache, const int* b
     const LatDecode a{(const bf16*)q, (const bf16*)cache, bt, bt_stride, positions, H, rank, row, S,
                       scale * 1.4426950408889634f, po, (float2*)ml};
     const dim3 grid(S, ceil_div(H, DH), B);
-#define LD(KB, VB)                                                               \
-    if (H <= DH) latent_decode_kernel<KB, VB, true><<<grid, 512, 0, s>>>(a);     \
-    else latent_decode_kernel<KB, VB, false><<<grid, 512, 0, s>>>(a)
-    if (rank <= 128 && row <= 128) { LD(4, 1); }
-    else if (rank <= 256 && row <= 320) { LD(10, 2); }
-    else { LD(18, 4); }
-#undef LD
+    if (rank <= 128 && row <= 128) latent_decode_kernel<4, 1><<<grid, 512, 0, s>>>(a);
+    else if (rank <= 256 && row <= 320) latent_decode_kernel<10, 2><<<grid, 512, 0, s>>>(a);
+    else latent_decode_kernel<18, 4><<<grid, 512, 0, s>>>(a);
     return (int)hipGetLastError();
 }
