@@ -752,9 +752,13 @@ __global__ __launch_bounds__(256, four_a_cu(G, ROPE, KVM) ? 4 : 3) void attn_dec
 
 // KV page loads are nontemporal from 64 (sequence, kv head) groups up -- measured, step at 4k context:
 // B=39 x 8 kv heads 7.02-7.05 vs 7.18-7.26 ms with the default policy; B <= 10 0.7-1 % slower with nt
-// (profiles/r1_decode_nt_ab.jsonl).  So they are for one row whose splits fill the chip: in a step of 8 layers that row's keys
-// are gone from the caches by the next.  us a launch, 32 / 8 heads over 13500 keys 19.7 -> 18.2, 32000 32 -> 28.3; decode steps of one
-// row over 13500, 25278 and 32000 keys 1059 -> 1048, 1140 -> 1120 and 1012 -> 998, over 4526 the same; 3 - 7 rows lost 0.5 - 1 %
+// (profiles/r1_decode_nt_ab.jsonl).  So they are for one row whose splits fill the chip and whose pages one head group reads: in a
+// step of 8 layers they are gone from the caches by the next.  Whole decode steps, us, through the caches -> past them, two captures
+// on one state: one row over 13500, 25278 and (70B, 4 layers) 32000 keys 1041 -> 1030, 1082 -> 1068, 1012 -> 995, over 4526 1000 -> 1004;
+// 8-bit caches over 4526, 13500 and 32000 968 -> 970, 1002 -> 1005, 1073 -> 1060; one layer over 13500, which the last cache holds,
+// 304.0 -> 305.4.  Pages that three head groups read (24 / 8 heads, 8-bit) over 13500 1088 -> 1095: these stay.  Two rows 1005 -> 1007
+// over 4526, 1142 -> 1117 over 13500, 1247 -> 1212 over 25278, four over 4600 1057 -> 1043; where their splits do not fill the chip, as
+// three and four over 13500, the same: more than one row stays with the caches as yet.
 constexpr int NT_MIN_GROUPS = 64;
 
 static bool decode_packed(int G) { return G == 1 || G == 2 || G == 4 || G == 8 || G == 16; }
@@ -790,7 +794,7 @@ static int launch_mfma(const void* q, int q_stride, const void* kcache, const vo
                                                                      (bf16*)out, out_stride, Hc, gq, ep)
 #define MFMA_L(G_, R_)                                                                                        \
     do {                                                                                                      \
-        const bool nt_ = B * Hkv >= NT_MIN_GROUPS || (B == 1 && S * Hkv >= 256);                              \
+        const bool nt_ = B * Hkv >= NT_MIN_GROUPS || (B == 1 && gq == 1 && S * Hkv >= 256);                   \
         if (kv8 == 3) { if (nt_) MFMA_K(G_, R_, true, 3, false); else MFMA_K(G_, R_, false, 3, false); }                    \
         else if (kv8 == 2) { if (nt_) MFMA_K(G_, R_, true, 2, false); else MFMA_K(G_, R_, false, 2, false); }               \
         else if (!R_ && hl) { if (nt_) MFMA_K(G_, false, true, 0, true); else MFMA_K(G_, false, false, 0, true); }  \
