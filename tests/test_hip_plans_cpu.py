@@ -300,6 +300,22 @@ def test_fp32_scan_in_chunks(rows, heads, vdim, chunks):
     assert hip.ssm_chunk32_rows(rows, heads, vdim) == chunks
 
 
+@pytest.mark.parametrize("rows,heads,state,chunks", [
+    ([40], 128, 128, False),     # 15.3, 16.1
+    ([48], 128, 128, False),     # 15.2, 16.2
+    ([48], 24, 128, False),      # 14.3, 15.2
+    ([56], 128, 128, True),      # 18.7, 16.5
+    ([65], 24, 128, True),       # 21.2, 19.6
+    ([64] * 4, 24, 128, True),   # 19.3, 16.8
+    ([64] * 4, 128, 128, False), # 35.6, 37.0
+    ([48], 128, 96, False),      # 14.5, 14.5
+    ([48], 128, 64, True),       # 12.4, 11.6
+    ([48], 128, 16, True)])      # 12.2, 10.6
+def test_fp32_scan_steps_sixteen_rows_at_a_time(rows, heads, state, chunks):
+    """us on the GPU, stepped and in chunks, heads of 64."""
+    assert hip.ssm_chunk32_rows(rows, heads, 64, state) == chunks
+
+
 def test_signatures_match_the_kernels():
     """ctypes checks nothing: a signature with another number of arguments reads the rest from the stack."""
     pars = c_parameters()
