@@ -76,7 +76,9 @@ __global__ __launch_bounds__(256) void ssm_chunk32_pre_kernel(const Chunk32Args 
         const double z = (double)raw + a.dt_bias[head];
         const double dt = in ? (z > 40. ? z : log1p(exp(z))) : 0.;
         const double an = (double)a.a_neg[head] * 1.4426950408889634;
-        double c = in ? fmax(an * dt, -400.) : 0.;  // 2^-400 is zero; a total decay must not make differences of infinities
+        // 2^-400 is zero; a total decay must not make differences of infinities, and what is no number stays none
+        double c = in ? an * dt : 0.;
+        if (c < -400.) c = -400.;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
             const double v = __shfl_up(c, o, 64);

@@ -244,6 +244,31 @@ def test_state_space_chunks_of_fp32(heads, P, N, groups, total):
     assert rel(got, want) < 3e-6 and rel(got_s, want_s) < 3e-6
 
 
+@pytest.mark.parametrize("where", ["decay", "step"])
+def test_state_space_chunks_of_fp32_keep_what_is_no_number(where):
+    """A decay that is no number makes all of its head none, a step size that is none its row and those after it, as token by
+    token."""
+    from llm_map_reduce_summarizer_amd import ops
+    from llm_map_reduce_summarizer_amd.ops import hip
+    heads, P, N, groups, lens = 3, 32, 64, 1, [140, 70]
+    assert hip.ssm_chunk32_rows(lens, heads, P)
+    T, C = sum(lens), heads * P + 2 * groups * N
+    xbc, u = rnd(T, C, std=0.7), rnd(1, T, 8, seed=1)
+    vec = [rnd(heads, seed=2) - 2, -torch.exp(rnd(heads, seed=3)), rnd(heads, seed=4)]
+    if where == "decay":
+        vec[1][1] = float("nan")
+    else:
+        u[0, 77, 1] = float("nan")
+    segs, state = segments(lens, [1, 0], [0, 0]), torch.zeros(2, heads, P, N, device=DEV)
+    y = ops.ssm_scan(dev(xbc), dev(u), 0, *map(dev, vec), state, segs, heads, P, N, groups).view(T, heads, P).cpu()
+    none, gone = torch.zeros(T, heads, P, dtype=torch.bool), torch.zeros(2, heads, P, N, dtype=torch.bool)
+    if where == "decay":
+        none[:, 1], gone[:, 1] = True, True
+    else:
+        none[77:140, 1], gone[1, 1] = True, True
+    assert torch.equal(y.isnan(), none) and torch.equal(state.cpu().isnan(), gone)
+
+
 @pytest.mark.parametrize("row,value", [(100, float("inf")), (64, float("nan")), (127, -float("inf"))])
 def test_state_space_chunks_of_fp32_do_not_reach_back(row, value):
     """An input that is not finite leaves the rows before it, the other value columns and the other portions alone."""
