@@ -363,10 +363,11 @@ __device__ __forceinline__ u32x4 ld_kv(const T* p) {
 // Which forms keep ONE tile in flight in registers, so that 128 of them are enough and four workgroups fit a CU, in place of two
 // tiles and three workgroups: a workgroup's step from tile to tile is a chain (pages -> LDS -> scores -> weights -> sums, two
 // barriers), and a fourth chain beside it hides more of it than a second tile in flight (at 1024 workgroups 128 KiB of bf16
-// pages are on the way to a CU, or 66 KiB of 8-bit ones, 192 and 99 before).  8 kv heads of 4 query heads, us with their plans' splits and
-// the merge, before -> this: 8-bit cache, 92 rows of 4600 163 -> 155, 39 rows 79 -> 77, 64 of 2000 58 -> 53, 92 of 600 49 -> 43, one of
-// 13500 17.0 -> 16.2; bf16, 92 of 4600 277 -> 269, 39 rows 122 -> 119, 64 of 2000 85 -> 80, 92 of 600 60 -> 44, one of 32000 33.0 -> 31.9.
-// The others would spill at 128: a bf16 K cache beside an 8-bit V one, rotated q of eight and more heads.
+// pages are on the way to a CU, or 66 KiB of 8-bit ones, 192 and 99 before).  Whole decode steps by the same splits, 8 kv heads of 4
+// query heads in 4 layers, two captures on one state, us before -> this: bf16, 92 rows of 600 951 -> 926, 64 of 2000 1013 -> 1001, 39 of
+// 4600 1108 -> 1108, 10 of 6000 727 -> 722; 8-bit cache, 92 of 4600 1328 -> 1309, 39 920 -> 910, 10 of 6000 683 -> 677; 32 rows of merulorn-8b
+// over 4096 (8 layers, unrotated heads) 1755 -> 1727.  The others would spill at 128: a bf16 K cache beside an 8-bit V one, rotated q of
+// eight and more heads.
 constexpr bool four_a_cu(int G, bool rope, int kvm) { return kvm == 3 || (kvm == 0 && (!rope || G <= 4)); }
 
 template <int G, bool ROPE, bool NT = false, int KVM = 0, bool HL = false>

@@ -15,7 +15,9 @@
 // prompt is over twice the CUs.  Against one workgroup of eight waves that staged through registers, in us, 32 / 8 heads
 // (bits the same): paged 1 x 305 14.0 -> 10.2, 1 x 2000 61.3 -> 53.1, 2 x 4096 253.7 -> 242.5 (with two-term weights
 // 345 -> 333.5), 5 x 4000 630 -> 595, 1 x 16000 2008 -> 1966; packed 13.7 -> 10.1, 60.1 -> 52.5, 250.5 -> 243,
-// 623 -> 596, 1985 -> 1969; 32 / 32 heads 5 x 4000 703 -> 652, 32 / 4 heads 596 -> 573.
+// 623 -> 596, 1985 -> 1969; 32 / 32 heads 5 x 4000 703 -> 652, 32 / 4 heads 596 -> 573.  Over seven head counts from 4 / 2 to 64 / 8 and
+// prompts of 1 x 37 to 1 x 9000 up to 39 % faster; slower where the smaller workgroups end in an uneven round: 64 / 8 heads 1 x 2000
+// 78.9 -> 81.2, 16 / 1 heads 2 x 4096 147 -> 154, 24 / 8 heads 100 x 60 packed 57.1 -> 58.5.
 //
 // fp8 caches: one workgroup of 8 waves an item (one per CU, 2 per SIMD at ~216 VGPRs); right after barrier t every wave
 // converts and writes tile t+1 (loaded into registers one tile earlier) into the other stage and issues the global loads
@@ -99,13 +101,6 @@ struct PagedKV {
     const int* prefix;         // [nseq] tokens already cached before this slice
 };
 
-// G = query heads per kv head served by one workgroup: wave w runs query head kvh*G + w%G over query rows
-// [qblock + 32(w/G), +32), so one workgroup covers 256/G query positions of ALL G heads of its kv head and
-// every staged K/V tile feeds 8 x 32 query rows whatever the GQA ratio.
-// Other GQA ratios (e.g. Llama-3.2-3B: 24 / 8 = 3) run the G = 1 instantiation over Hg = Hq "virtual kv
-// heads", one per query head, each reading the K/V columns of its real kv head h / gq (gq = Hq / Hkv):
-// no K/V reuse across the group inside a workgroup, but any ratio works.  Hg = Hkv and gq = 1 otherwise.
-// HL: the softmax weights enter the value product as two bf16 terms (hi + lo) instead of one.
 // 1 KiB from p to LDS: lane l's 16 bytes at byte offset `off` to dst + 16 l
 __device__ __forceinline__ void dma_1k(const bf16* p, int bytes, int off, char* dst) {
     typedef __attribute__((address_space(3))) void* lds_ptr;
@@ -113,6 +108,14 @@ __device__ __forceinline__ void dma_1k(const bf16* p, int bytes, int off, char* 
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr)dst, 16, off, 0, 0, 0);
 }
 
+// G = query heads per kv head of a work item, which is 256 / G query positions of all of them.  A workgroup has WV waves and HW of the
+// heads: wave w runs head w % HW of these over query rows [qblock + 32 (w / HW), + 32), BMP positions in all.  fp8 caches: WV 8, HW G,
+// BMP 256 / G, so that a staged K/V tile feeds 8 x 32 query rows.  bf16: PARTS = 2 workgroups of WV 4 share the item, by halves of its
+// positions (HW G, BMP 128 / G), or of eight heads by four each (HW 4, BMP 32), and each stages the tiles for itself.
+// Other GQA ratios (e.g. Llama-3.2-3B: 24 / 8 = 3) run the G = 1 instantiation over Hg = Hq "virtual kv
+// heads", one per query head, each reading the K/V columns of its real kv head h / gq (gq = Hq / Hkv):
+// no K/V reuse across the group inside a workgroup, but any ratio works.  Hg = Hkv and gq = 1 otherwise.
+// HL: the softmax weights enter the value product as two bf16 terms (hi + lo) instead of one.
 template <bool PAGED, int G, int KVM = 0, bool HL = false>
 __global__ __launch_bounds__(64 * waves(KVM), waves(KVM) == 4 ? 2 : 1) void attn_prefill_kernel(const bf16* __restrict__ qkv, int row_stride,
                                                               const int* __restrict__ cu_seqlens,

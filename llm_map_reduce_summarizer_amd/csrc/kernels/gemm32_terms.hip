@@ -27,8 +27,10 @@
 //     three times as many cache accesses and as long (20608 columns, 300 rows: 181 us, 165 here).
 //   * every product has an instruction or three of other work behind it: it keeps the matrix core busy for 16 cycles and the
 //     wave for four.
-// us, fp32 instruction -> this: 903 x 28672 x 4096 1560 -> 600, 903 x 4096 x 14336 809 -> 341, 300 x 20608 x 4096 436 -> 165, 160 x
-// 28672 x 4096 302 -> 155 (where W's arrival is all).  Which rows and shapes: ops/hip.py gemm32_terms.
+//   * what is looked at in W takes a fifth of the instructions beside the products: each of the two waves that have the same columns
+//     looks at half of them.  With the smallest value of all columns looked for in both, 903 x 4096 x 14336 took 8 % longer.
+// us, fp32 instruction -> this: 903 x 28672 x 4096 1550 -> 586, 903 x 4096 x 14336 808 -> 327, 300 x 20608 x 4096 432 -> 175, 160 x
+// 28672 x 4096 290 -> 153 (where W's arrival is all).  Which rows and shapes: ops/hip.py gemm32_terms.
 #include "gemm32.h"
 
 #include <type_traits>
