@@ -350,8 +350,7 @@ class LLMEngine:
 
     def _ctx_classes(self) -> int:
         """Number of context classes this engine can reach (ops.hip.CTX_CLASSES up to max_model_len)."""
-        from ..ops.hip import ctx_class
-        return ctx_class(self.max_model_len) + 1
+        return ops.hip.ctx_class(self.max_model_len) + 1
 
     def _workspace(self, B: int):
         if self.device.type != "cuda":
@@ -359,8 +358,7 @@ class LLMEngine:
         key = (B, self._ctx_cls)
         ws = self._workspaces.get(key)
         if ws is None:
-            from ..ops.hip import CTX_CLASSES
-            ws = self.model.decode_workspace(B, min(CTX_CLASSES[self._ctx_cls], self.max_model_len),
+            ws = self.model.decode_workspace(B, min(ops.hip.CTX_CLASSES[self._ctx_cls], self.max_model_len),
                                              self.kv.kv_dtype if self.kv.fp8 else False)
             self._workspaces[key] = ws
         return ws
@@ -686,8 +684,7 @@ class LLMEngine:
             self._admit_step(entries, order, seqs, spans, wanted, pages)
             if entries:
                 if self.device.type == "cuda":
-                    from ..ops.hip import ctx_class
-                    self._ctx_cls = ctx_class(max(e for _, e in spans))
+                    self._ctx_cls = ops.hip.ctx_class(max(e for _, e in spans))
                 starts = np.cumsum([0] + [e - b for b, e in spans])
                 rows = [int(starts[j]) + w for j, ws in enumerate(wanted) for w in ws]
                 x = self._pass_inputs(seqs, spans, paged=True, tables=self.pf_tables, slots=[s.pf_slot for s in seqs],
@@ -763,8 +760,7 @@ class LLMEngine:
     def _fit_ctx_class(self, seqs: Sequence[_Seq]) -> None:
         """Decode attention split plan (graphs are keyed by it) for the longest sequence in flight."""
         if seqs and self.device.type == "cuda":
-            from ..ops.hip import ctx_class
-            self._ctx_cls = max(self._ctx_cls, ctx_class(max(len(s.prompt) + s.params.max_new_tokens for s in seqs)))
+            self._ctx_cls = max(self._ctx_cls, ops.hip.ctx_class(max(len(s.prompt) + s.params.max_new_tokens for s in seqs)))
 
     def _generate(self, prompts: Sequence[Sequence[int]], params: Sequence[SamplingParams],
                   imported: Dict[int, ImportedPrefill], on_prefill, feeder=None, on_sync=None) -> List[GenOutput]:

@@ -233,15 +233,13 @@ class Segments:
 
 def decode_workspace(B, hq, hkv, d, max_ctx, device, kv8=False):
     """Split-K buffers of the decode attention for ``B`` rows whose contexts reach ``max_ctx`` (GPU only)."""
-    from .hip import DecodeWorkspace, decode_attn_plan, decode_groups
-    ng = decode_groups(hq, hkv)  # kv heads, or query heads for odd GQA ratios
-    s, fused = decode_attn_plan(B, ng, max_ctx, kv8=kv8)
-    return DecodeWorkspace(B, hq, d, s, device, ng, fused_combine=fused)
+    ng = hip.decode_groups(hq, hkv)  # kv heads, or query heads for odd GQA ratios
+    s, fused = hip.decode_attn_plan(B, ng, max_ctx, kv8=kv8)
+    return hip.DecodeWorkspace(B, hq, d, s, device, ng, fused_combine=fused)
 
 
 def prefill_items(lens, group):
-    from .hip import prefill_items as items
-    return items(lens, group)
+    return hip.prefill_items(lens, group)
 
 
 def embed_pos(ids, positions, table, scale, pos_freq):
@@ -357,29 +355,24 @@ class PortionContext:
 
 
 def latent_prefill_ok(dim8, rot8, vp):
-    from .hip import latent_prefill_form
-    return latent_prefill_form(dim8 + rot8, vp) is not None
+    return hip.latent_prefill_form(dim8 + rot8, vp) is not None
 
 
 def latent_decode_ok(rank8, row):
-    from .hip import latent_decode_form
-    return latent_decode_form(rank8, row) is not None
+    return hip.latent_decode_form(rank8, row) is not None
 
 
 def latent_block_rows(qw, vp):
     """Query rows per workgroup of the prompt-portion kernel."""
-    from .hip import latent_prefill_form
-    return latent_prefill_form(qw, vp)[1]
+    return hip.latent_prefill_form(qw, vp)[1]
 
 
 def latent_items(lens, rows):
-    from .hip import block_items
-    return block_items(lens, rows)
+    return hip.block_items(lens, rows)
 
 
 def latent_workspace(B, heads, rank, max_ctx, device):
-    from .hip import LatentWorkspace
-    return LatentWorkspace(B, heads, rank, max_ctx, device)
+    return hip.LatentWorkspace(B, heads, rank, max_ctx, device)
 
 
 def latent_prep(u, m, dq_norm, dkv_norm, eps, cs, positions, seq_idx, block_tables, cache, page, dtype, gelu=None):
@@ -431,8 +424,7 @@ def latent_prefill(q, kv, lat, ctx, m, cu, lens, items, scale, out, col):
 
 # ---------------------------------------------------------------- gated delta rule (``m``: engine.mixers.DeltaMixer)
 def delta_ok(vdim, dim):
-    from .hip import delta_step_ok
-    return delta_step_ok(vdim, dim)
+    return hip.delta_step_ok(vdim, dim)
 
 
 def delta_mix(x, u, m, a_neg, dt_bias, norm, eps, state, segs, a):
