@@ -268,7 +268,8 @@ struct LatDecode {
 
 // KB: 32-column blocks of a cached row, VB: 128-column blocks of the latent.  Grid (S, ceil(H / 32), B).  Two barriers a
 // page: the next page's registers go to the other LDS stage between them, when every wave is past the page before.
-template <int KB, int VB>
+// ONCE: one workgroup has all heads and no later layer reads these pages, so that they go past the caches (hip.py latent_decode).
+template <int KB, int VB, bool ONCE>
 __global__ __launch_bounds__(512, 1) void latent_decode_kernel(const LatDecode a) {
     constexpr int LK = 32 * KB + 8, LP = BN + 8, IT = KB / 2;
     __shared__ __attribute__((aligned(16))) bf16 sk[2][BN * LK];
@@ -309,8 +310,10 @@ __global__ __launch_bounds__(512, 1) void latent_decode_kernel(const LatDecode a
     {                                                                                                   \
         const bf16* pg_ = a.cache + (size_t)id * BN * a.row;                                            \
         id = bt[min((p) + 1, p1 - 1)];                                                                  \
-        _Pragma("unroll") for (int i = 0; i < IT; ++i)                                                  \
-            reg[i] = *reinterpret_cast<const u32x4*>(pg_ + 8 * min(tid + 512 * i, total - 1));          \
+        _Pragma("unroll") for (int i = 0; i < IT; ++i) {                                                \
+            const u32x4* p_ = reinterpret_cast<const u32x4*>(pg_ + 8 * min(tid + 512 * i, total - 1));  \
+            reg[i] = ONCE ? __builtin_nontemporal_load(p_) : *p_;                                       \
+        }                                                                                               \
     }
     f32x4 acc[VB][2];
     float m[2] = {-INFINITY, -INFINITY}, l = 0.f;  // maxima of heads r16, 16 + r16; this lane's share of head 16 hb + r16's sum
@@ -438,17 +441,21 @@ __global__ __launch_bounds__(512, 1) void latent_decode_kernel(const LatDecode a
 }
 
 // q [B][H * row] bf16; po [B][H][S][rank] fp32, ml [B][H][S] pairs.  rank % 8 == 0, row % 8 == 0; (rank, row) up to
-// (128, 128), (256, 320) or (512, 576).
+// (128, 128), (256, 320) or (512, 576).  once: pages past the caches, if a workgroup has all heads.
 MRSUM_API int mrsum_latent_decode(const void* q, const void* cache, const int* bt, int bt_stride, const int* positions, int B,
-                                  int H, int rank, int row, int S, float scale, float* po, float* ml, hipStream_t s) {
+                                  int H, int rank, int row, int S, float scale, int once, float* po, float* ml, hipStream_t s) {
     if (B <= 0) return 0;
     if (H <= 0 || S <= 0 || S > 65535 || B > 65535 || rank % 8 || row % 8 || rank <= 0 || rank > row || rank > 512 || row > 576)
         return (int)hipErrorInvalidValue;
     const LatDecode a{(const bf16*)q, (const bf16*)cache, bt, bt_stride, positions, H, rank, row, S,
                       scale * 1.4426950408889634f, po, (float2*)ml};
     const dim3 grid(S, ceil_div(H, DH), B);
-    if (rank <= 128 && row <= 128) latent_decode_kernel<4, 1><<<grid, 512, 0, s>>>(a);
-    else if (rank <= 256 && row <= 320) latent_decode_kernel<10, 2><<<grid, 512, 0, s>>>(a);
-    else latent_decode_kernel<18, 4><<<grid, 512, 0, s>>>(a);
+#define LD(KB, VB)                                                               \
+    if (once && H <= DH) latent_decode_kernel<KB, VB, true><<<grid, 512, 0, s>>>(a);     \
+    else latent_decode_kernel<KB, VB, false><<<grid, 512, 0, s>>>(a)
+    if (rank <= 128 && row <= 128) { LD(4, 1); }
+    else if (rank <= 256 && row <= 320) { LD(10, 2); }
+    else { LD(18, 4); }
+#undef LD
     return (int)hipGetLastError();
 }

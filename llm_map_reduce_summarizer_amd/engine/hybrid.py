@@ -76,6 +76,13 @@ class HybridModel:
         self.layer_hook: Optional[Callable[[int, torch.Tensor], None]] = None  # (layer, residual) after every layer
         self.kp = up(cfg.hidden, 128)
         self.layers = [self._layout(la) for la in cfg.layers]
+        readers = {}  # of each layer's latents, the last one
+        for i, la in enumerate(self.layers):
+            if la.latent is not None:
+                src = la.latent.spec.kv_from
+                readers[i if src is None else src] = la.latent
+        for m in readers.values():
+            m.last = True
         if weights_path:
             from .weights import checkpoint_reader
             self._fill(checkpoint_reader(weights_path))

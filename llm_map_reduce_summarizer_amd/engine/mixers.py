@@ -223,6 +223,7 @@ class LatentMixer(Mixer):
         self.kv_n = up(self.kv_v + s.heads * self.vp, 16)
         self.lat_k = up(s.kv_rank, 64)                       # depth of the expansion product
         self.lat = max(self.row, self.lat_k)                 # gathered row: the cached one, zeros behind it
+        self.last = False                                    # no later layer reads the cache that this one does
 
     def columns(self, take) -> None:
         s = self.spec
@@ -288,7 +289,7 @@ class LatentMixer(Mixer):
                 n = b.n_decode
                 ws = b.workspace.get(("latent", s.heads, self.rank8))
                 parts = ops.latent_decode(qa[:n], cache, b.decode_tables, b.positions, s.heads, self.rank8, page,
-                                          s.scale, ws)
+                                          s.scale, ws, self.last)
                 ops.latent_out_parts(parts, self, w.w_uv, a[:n], self.col)
             n = b.n_decode if self.mfma else 0
             if n < nd:

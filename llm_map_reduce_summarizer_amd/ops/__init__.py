@@ -391,9 +391,9 @@ def latent_out(o, m, w_uv, a, col):
     return _impl(o).latent_out(o, m, w_uv, a, col)
 
 
-def latent_decode(q, cache, block_tables, positions, heads, rank, page, scale, workspace):
+def latent_decode(q, cache, block_tables, positions, heads, rank, page, scale, workspace, last=False):
     """Split-K attention of decoded tokens over the cached rows (GPU): unmerged partial sums, see latent_out_parts."""
-    return hip.latent_decode(q, cache, block_tables, positions, heads, rank, page, scale, workspace)
+    return hip.latent_decode(q, cache, block_tables, positions, heads, rank, page, scale, workspace, last)
 
 
 def latent_out_parts(parts, m, w_uv, a, col):

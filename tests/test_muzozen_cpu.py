@@ -48,6 +48,18 @@ def test_unequal_requests_share_batches_and_reuse_slots(tmp_path):
         M.check(got[r], M.expected("mixed", ids), F32, r)
 
 
+def test_each_cache_has_one_last_reader():
+    from dataclasses import replace
+    from llm_map_reduce_summarizer_amd.engine.config import get_model_config
+    from llm_map_reduce_summarizer_amd.engine.hybrid import HybridModel
+    cfg = get_model_config("tiny-muzozen")
+    own, delta = (next(la for la in cfg.layers if (la.latent is not None) == k) for k in (True, False))
+    own = replace(own, latent=replace(own.latent, kv_from=None))
+    reads = [replace(own, latent=replace(own.latent, kv_from=i)) for i in (0, 2)]
+    m = HybridModel(replace(cfg, layers=(own, reads[0], own, delta, reads[0], own, reads[1])), torch.device("cpu"), torch.float32)
+    assert [la.latent.last for la in m.layers if la.latent is not None] == [False, False, False, True, True, True]
+
+
 def test_request_left_out_of_steps_continues(tmp_path):
     eng = M.engine("odd", tmp_path, "cpu", F32)
     a, b = M.tokens("odd", 40, 1), M.tokens("odd", 30, 2)

@@ -1,6 +1,7 @@
 """The Muzozen design on the MI355X kernels against its float64 oracle (tests/muzozen_oracle.py): every mechanism alone,
 then whole models in bf16 and fp32 through the engine's step function, scheduler and captured decode graphs."""
 import math
+from types import SimpleNamespace
 
 import pytest
 import torch
@@ -225,6 +226,29 @@ def test_latent_kernels_of_real_sizes_are_the_fused_ones():
 
 # heads, key heads, dim, vdim
 DELTA = [(4, 2, 128, 128), (3, 3, 24, 40), (2, 1, 64, 136), (6, 2, 32, 16), (2, 2, 200, 112), (3, 1, 5, 7), (2, 1, 256, 64)]
+
+
+@pytest.mark.parametrize("B,H,rank,row", [(3, 4, 128, 128), (16, 4, 256, 320), (5, 32, 512, 576), (5, 33, 512, 576)])
+def test_latent_decode_of_the_last_reader(B, H, rank, row):
+    """Pages past the caches, by one workgroup of all heads, give the bits that pages through them do."""
+    from llm_map_reduce_summarizer_amd.ops import hip
+    g, pages = torch.Generator().manual_seed(3), 4
+    cache = torch.randn(B * pages + 1, 1, 64, row, generator=g).to(torch.bfloat16).to(DEV)
+    q = torch.randn(B, H * row, generator=g).to(torch.bfloat16).to(DEV)
+    tables = (torch.randperm(B * pages, generator=g) + 1).view(B, pages).int().to(DEV)
+    positions = torch.tensor([(64 * pages - 1) * (i + 1) // B for i in range(B)], dtype=torch.int32, device=DEV)
+    out = []
+    for rows, last in ((B, False), (B, True), (1, False)):  # (from 16 rows on past the caches either way)
+        ws = hip.LatentWorkspace(B, H, rank, 64 * pages, DEV)
+        for t in (ws.part_o, ws.part_ml):
+            t.fill_(float("nan"))
+        for b in range(0, B, rows):
+            one = SimpleNamespace(splits=ws.splits, part_o=ws.part_o[b * H * ws.splits * rank:], part_ml=ws.part_ml[2 * b * H * ws.splits:])
+            hip.latent_decode(q[b: b + rows], cache, tables[b: b + rows], positions[b: b + rows].clone(), H, rank, 64, 0.1, one, last)
+        out.append((ws.part_o.clone(), ws.part_ml.clone()))
+    # (splits behind a row's last page are left as they were)
+    assert all(0 < int((~t.isnan()).sum()) for t in out[0])
+    assert all(torch.equal(x.nan_to_num(7.0), y.nan_to_num(7.0)) for o in out[1:] for x, y in zip(out[0], o))
 
 
 @pytest.mark.parametrize("rows,H,xk,K,N", [(1, 3, 24, 32, 8), (15, 2, 96, 96, 136), (16, 2, 128, 128, 128), (17, 5, 40, 64, 24),
