@@ -179,8 +179,9 @@ class HybridModel:
             elif spec.mlp is not None:
                 put(w.w_in, la.n_mix, 0, get(p + "mlp.up", (spec.mlp.ff, H)))
                 put(w.w_o, 0, la.ff_col, get(p + "mlp.down", (H, spec.mlp.ff)))
-            ops.mark_values(*(t for ns in [w] + [m.w for m in la.mixers] for t in vars(ns).values() if t is not None and t.dim() == 2))
-        ops.mark_values(self.lm_head)
+        products = [getattr(ns, k, None) for la in self.layers for ns in [la.w] + [m.w for m in la.mixers]
+                    for k in ("w_in", "w_o", "w_gu", "w_down", "w_uq")]
+        ops.mark_values(self.lm_head, *(t for t in products if t is not None))
 
     def weight_bytes(self) -> int:
         ts = [self.embed, self.bigram, self.embed_norm, self.lm_head, self.final_norm]

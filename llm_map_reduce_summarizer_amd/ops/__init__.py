@@ -272,9 +272,9 @@ def project(x, w, role):
 
 def mark_values(*weights):
     """Notes on fp32 weights on the GPU, laid out once, what their products ask of their values (hip.gemm32)."""
-    for w in weights:
-        if w.dtype == torch.float32 and _use_hip(w):
-            w.bf16_values = hip.bf16_values(w)
+    weights = [w for w in weights if w.dtype == torch.float32 and _use_hip(w)]
+    for w, known in zip(weights, hip.bf16_values(*weights) if weights else ()):
+        w.bf16_values = known
 
 
 def project_glu(x, w_gu, limit, alpha, shift):

@@ -853,8 +853,9 @@ def test_weights_of_bf16_values(at, value, held):
     from llm_map_reduce_summarizer_amd.ops import hip
     w = torch.randn(9000, 4096, generator=torch.Generator(DEV).manual_seed(1), device=DEV).to(BF).float()
     w[at] = value
-    assert hip.bf16_values(w) == held and hip.bf16_values(w[at[0]: at[0] + 1, at[1]: at[1] + 1]) == held
-    assert hip.bf16_values(w[:, :1][:0])
+    odd = w.view(-1)[1:8191].view(1, -1)  # not on 16 bytes, no multiple of four
+    odd[0, -1] = value
+    assert hip.bf16_values(w, w[:0], odd, w[8998:8999], w[8999:, :]) == [held, True, held, True, held or at[0] != 8999]
 
 
 def entries(hip, monkeypatch):
@@ -874,7 +875,7 @@ def test_gemm32_of_weights_known_to_have_more_bits(monkeypatch):
     assert names == ["mrsum_gemm32_terms"]
     ops.mark_values(w)
     assert w.bf16_values is False and torch.equal(ops.project(x, w, "o")[0], got) and torch.equal(ops.logits32(x, w), got)
-    assert names[1:] == ["mrsum_gemm32"] * 2
+    assert names[1:] == ["mrsum_bf16_values"] + ["mrsum_gemm32"] * 2
     v = w.to(BF).float()
     ops.mark_values(v)
     assert v.bf16_values is True
