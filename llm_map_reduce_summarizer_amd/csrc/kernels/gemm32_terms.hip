@@ -11,7 +11,7 @@
 // at once, makes the whole result.  A workgroup that sees it in its first K-tile or its rows of X stops there, others when their next
 // chain of 16 K-tiles ends.  What that costs, us: 903 x 28672 x 4096 on the fp32 instruction 1550, by way of here with 24 bits in all of W
 // 1612, in half of its rows 1640 (2100 where nobody asks the others), in half of its columns 1730, in its last value alone 2100; 160 x
-// 6144 x 4096 74, 96, 113, 121, 126.  What a model has
+// 6144 x 4096 75, 97, 113, 119, 126.  What a model has
 // loaded carries the answer and does not come here (ops/hip.py gemm32).
 //
 // Relative error (2-norm, random operands, K 4096 - 22528, chains of 16 K-tiles on both): 2.4e-7, the fp32 instruction 4.1e-7, as one
@@ -322,7 +322,7 @@ __device__ __forceinline__ bool terms_loop(const Gemm32Args& a, char* lds, int u
                 }
                 asm volatile("" : "+a"(acc[b][i]), "+a"(acc[b][i + 1]), "+a"(acc[b][i + 2]), "+a"(acc[b][i + 3]));
             }
-        __builtin_amdgcn_raw_buffer_store_b32(1u, rf, any() && lane == 0 ? 0 : 4, 0, 16);  // (at 4: nowhere)
+        __builtin_amdgcn_raw_ptr_buffer_atomic_add_i32(1, rf, any() && lane == 0 ? 0 : 4, 0, 0);  // (at 4: nowhere)
         if (__builtin_amdgcn_readfirstlane(*(volatile int*)heard) && end < kt1) stop = kt;
     }
 #pragma unroll
