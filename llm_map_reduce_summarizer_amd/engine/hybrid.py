@@ -228,8 +228,10 @@ class HybridModel:
         if la.attn is not None and la.ssm is not None and gelu is None and b.segs.cu is None:  # decoded rows
             xbc = la.attn.run(i, u, a, b, kv, self.cfg.rms_eps, beside=la.ssm)
             la.ssm.run(i, u, a, b, kv, self.cfg.rms_eps, xbc=xbc)
-            return ops.project(a, la.w.w_o, "o")
-        for m in la.mixers:
+            left = la.mixers[2:]
+        else:
+            left = la.mixers
+        for m in left:
             if gelu is not None and m.takes_gelu:
                 m.run(i, u, a, b, kv, self.cfg.rms_eps, gelu)
                 gelu = None

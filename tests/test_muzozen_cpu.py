@@ -48,6 +48,30 @@ def test_unequal_requests_share_batches_and_reuse_slots(tmp_path):
         M.check(got[r], M.expected("mixed", ids), F32, r)
 
 
+def test_decoded_rows_run_all_mixers_of_a_layer():
+    """Attention, a state-space mixer and latents of an earlier layer in one layer: a decoded token gives what it gives as the
+    last row of a prompt."""
+    from dataclasses import replace
+    from llm_map_reduce_summarizer_amd.engine.config import LayerSpec, get_model_config
+    from llm_map_reduce_summarizer_amd.engine.engine import LLMEngine
+    cfg = get_model_config("tiny-muzozen")
+    beside = next(la for la in get_model_config("tiny-merulorn").layers if la.attn is not None)
+    own = next(la for la in cfg.layers if la.latent is not None and la.latent.kv_from is None)
+    three = LayerSpec(beside.attn, beside.ssm, None, latent=replace(own.latent, kv_from=0))
+    cfg = replace(cfg, layers=(own, three))
+    prompt, n = [5, 9, 200, 31, 7, 64], 3
+    eng, rows = LLMEngine(cfg, device="cpu", dtype=torch.float32, max_num_seqs=2, max_model_len=128, kv_pages=8), []
+    eng.model.layer_hook = lambda i, residual: rows.append(residual[:1].clone() if residual.shape[0] < n else residual[-1:].clone())
+    toks = eng.generate([prompt], [SamplingParams(n, 0.0, 1)], ignore_eos=True)[0].token_ids
+    decoded = rows[-2 * (n - 1):]
+    for k in range(1, n):
+        rows.clear()
+        eng.step([("r%d" % k, prompt + toks[:k], [])], ["r%d" % k])
+        for got, want in zip(decoded[2 * (k - 1): 2 * k], rows):
+            # 32-bit sums in other orders
+            assert float((got - want).norm() / want.norm()) < 1e-5
+
+
 def test_each_cache_has_one_last_reader():
     from dataclasses import replace
     from llm_map_reduce_summarizer_amd.engine.config import get_model_config
