@@ -429,6 +429,9 @@ MRSUM_API int mrsum_bf16_values(const float* w, int rows, int cols, int* odd, hi
     return (int)hipGetLastError();
 }
 
+// terms: 2 ceil(M / 32) (K / 32) pieces of 3072 bytes, 16 bytes and a byte for four pieces, to a multiple of 16; on 16 bytes.  ``tiles_m``,
+// ``whole``, ``splits``: row tiles of 2 to 5 32-row units, the rest from raster position ``whole`` on in slices of K through ``part``
+// [tiles - whole][splits][40960], which the fp32 instruction's form with ``whole32``, ``splits32`` (mrsum_gemm32) uses too.
 MRSUM_API int mrsum_gemm32_terms(const float* x, int ldx, const float* w, int ldw, float* c, int ldc, int M, int N, int K,
                                  int tiles_m, int whole, int splits, int whole32, int splits32, void* terms, float* part,
                                  hipStream_t s) {
