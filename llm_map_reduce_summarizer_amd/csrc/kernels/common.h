@@ -38,9 +38,10 @@ __device__ __forceinline__ void unpack8(const uint4 v, float* f) {
     f[6] = __uint_as_float(v.w << 16); f[7] = __uint_as_float(v.w & 0xffff0000u);
 }
 
+// As a vector: one v_cvt_pk_bf16_f32.  Two 16-bit values put together take one each, and an or.
 __device__ __forceinline__ uint32_t pack2(float a, float b) {
-    bf16 x = (bf16)a, y = (bf16)b;
-    return (uint32_t)__builtin_bit_cast(uint16_t, x) | ((uint32_t)__builtin_bit_cast(uint16_t, y) << 16);
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, bf16x2{(bf16)a, (bf16)b});
 }
 
 __device__ __forceinline__ uint4 pack8(const float* f) {
