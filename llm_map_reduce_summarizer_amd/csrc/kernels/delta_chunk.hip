@@ -319,9 +319,10 @@ __device__ __forceinline__ int tile_row(int nb, int g) { return 32 * (nb >> 1) +
         const float* vs_ = vec + ((size_t)(CK) * a.heads + head) * 256;                                     \
         _Pragma("unroll") for (int i = 0; i < VIT; ++i) vecr[i] = vs_[min(tid + NTH * i, 192)];             \
     }
+#define RAGGED(T0) ((T0) + Q > re || a.N < NN || pb + 16 * WPB > a.P)
 #define STORE_CHUNK(T0)                                                                                     \
     {                                                                                                       \
-        if ((T0) + Q > re || a.N < NN || pb + 16 * WPB > a.P) {                                             \
+        if (RAGGED(T0)) {                                                                                   \
             const u32x4 zero = {0, 0, 0, 0};                                                                \
             _Pragma("unroll") for (int i = 0; i < KIT; ++i) {                                               \
                 const int idx = tid + NTH * i;                                                              \
@@ -506,11 +507,18 @@ __global__ __launch_bounds__(64 * WPB, 1) void delta_chunk_kernel(const bf16* __
     }
 }
 
+#undef RAGGED
+#define RAGGED(T0) __builtin_expect((T0) + Q > re || a.N < NN || pb + 16 * WPB > a.P, 0)
 // The same with two waves per 16 value columns, for grids that leave SIMDs idle: one carries the state (its chain is what a
-// chunk takes), the other turns the state at the chunk's start and U into output rows beside it.  Both reach it as finished
-// operands through LDS.
+// chunk takes), the other turns the state at the chunk's start and U into output rows beside it, and brings the next chunk's
+// rows into a second set of LDS images.  The state reaches it as finished operands through LDS, U as it is: two barriers a
+// chunk.  What bounds the chain are its instructions, five cycles each in a lone wave of a SIMD: with staging, conversions of
+// one value at a time and results copied between the two halves of the register file they were 1010 a chunk of 64 x 128,
+// 3.1 us, and are 570, 1.9 us.  One prompt of 4096 tokens, 32 heads of 128 x 128, with the preparation: 199.5 -> 150.5 us; 16
+// heads of 64 x 64 123 -> 111 (with staging left to all waves 123).  The bound of 512 threads keeps the registers to 256, so
+// that products stay where the vector instructions reach them.
 template <int NB, int WPB>
-__global__ __launch_bounds__(128 * WPB, 1) void delta_chunk_pair_kernel(const bf16* __restrict__ x, DeltaArgs a,
+__global__ __launch_bounds__(512) void delta_chunk_pair_kernel(const bf16* __restrict__ x, DeltaArgs a,
                                                                         const int4* __restrict__ segs,
                                                                         const int* __restrict__ slots,
                                                                         const int* __restrict__ pos0,
@@ -518,31 +526,28 @@ __global__ __launch_bounds__(128 * WPB, 1) void delta_chunk_pair_kernel(const bf
                                                                         const float* __restrict__ vec,
                                                                         float* __restrict__ state, float* __restrict__ y,
                                                                         int y0) {
-    constexpr int NTH = 128 * WPB, NN = 32 * NB, LK = row_stride<NB>(), LV = 16 * WPB + 16, NT = 2 * NB, GN = NT < 4 ? NT : 4;
-    constexpr int KIT = (Q * 4 * NB + NTH - 1) / NTH, VR = 1;
-    constexpr int VIT = NTH < 256 ? 256 / NTH : 1;
-    __shared__ __attribute__((aligned(16))) bf16 sK[Q * LK];
-    __shared__ __attribute__((aligned(16))) bf16 sQ[Q * LK];
-    __shared__ __attribute__((aligned(16))) bf16 sV[Q * LV];
-    __shared__ __attribute__((aligned(16))) float s_vec[256];
+    constexpr int NN = 32 * NB, LK = row_stride<NB>(), LV = 16 * WPB + 16, NT = 2 * NB, GN = NT < 4 ? NT : 4;
+    // images of two chunks: the output waves fill the next one while this one is read
+    __shared__ __attribute__((aligned(16))) bf16 s_k[2][Q * LK];
+    __shared__ __attribute__((aligned(16))) bf16 s_q[2][Q * LK];
+    __shared__ __attribute__((aligned(16))) bf16 s_v[2][Q * LV];
+    __shared__ __attribute__((aligned(16))) float s_vecs[2][256];
     __shared__ bf16x8 sS[WPB][2 * NB][64];  // state operands, hi and lo
-    __shared__ bf16x8 sU[WPB][4][64];       // U operands, hi and lo
+    __shared__ f32x4 sU[WPB][4][64];        // U
     const int head = blockIdx.x, pb = 16 * WPB * blockIdx.y;
     const int4 sg = segs[blockIdx.z];
     const int rb = sg.y, re = sg.z;
-    const int tid = threadIdx.x, lane = tid & 63, r16 = lane & 15, g = lane >> 4, q4 = r16 >> 2, p4 = 4 * (r16 & 3);
-    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), w = wv % WPB;
+    const int lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4, q4 = r16 >> 2, p4 = 4 * (r16 & 3);
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), w = wv % WPB;
     const int kh = head / (a.heads / a.kv_heads), inner = a.heads * a.P;
     const bf16* qcol = x + kh * a.N;
     const bf16* kcol = qcol + a.xk;
     const bf16* vcol = x + a.xv + head * a.P + pb;
     const int p = pb + 16 * w + r16;  // this lane's value column
-    u32x4 kreg[KIT], qreg[KIT], vreg[VR];
-    float vecr[VIT];
     const uint4* fr = frags + ((size_t)sg.w * a.heads + head) * FRAGS + lane;  // this chunk's T and M
     const size_t fr_step = (size_t)a.heads * FRAGS;
     uint4 lf[2 * FR];
-    int ck = sg.w;
+    int img = 0;  // this chunk's images
     if (wv < WPB) {
         float* st_p = state + ((size_t)slots[sg.x] * a.heads + head) * a.P * a.N4 + (size_t)p * a.N4;
         f32x4 st[NT];
@@ -562,14 +567,12 @@ __global__ __launch_bounds__(128 * WPB, 1) void delta_chunk_pair_kernel(const bf
     }
 #pragma unroll
         for (int f = 0; f < 2 * FR; ++f) lf[f] = fr[64 * f];
-        LOAD_CHUNK(rb, ck)
-        STORE_CHUNK(rb)
         PUBLISH()
         __syncthreads();
         for (int t0 = rb; t0 < re; t0 += Q) {
             const bool more = t0 + Q < re;
-            LOAD_CHUNK(more ? t0 + Q : t0, more ? ck + 1 : ck)
-            __builtin_amdgcn_sched_barrier(0);  // loads stay here
+            const bf16 *sK = s_k[img], *sV = s_v[img];
+            const float* s_vec = s_vecs[img];
             f32x4 r[4], u[4];
 #pragma unroll
             for (int ib = 0; ib < 4; ++ib) r[ib] = u[ib] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -593,15 +596,8 @@ __global__ __launch_bounds__(128 * WPB, 1) void delta_chunk_pair_kernel(const bf
                     r[ib][e] = __uint_as_float((uint32_t)(uint16_t)vt[e] << 16) - ek[e] * r[ib][e];
             }
             lower(u, lf, r);
-            {
-                bf16x8 h, l;
 #pragma unroll
-                for (int jp = 0; jp < 2; ++jp) {
-                    split(u[2 * jp], u[2 * jp + 1], h, l);
-                    sU[w][jp][lane] = h;
-                    sU[w][2 + jp][lane] = l;
-                }
-            }
+            for (int ib = 0; ib < 4; ++ib) sU[w][ib][lane] = u[ib];
             __syncthreads();  // U is in LDS; the output waves have read the state
             if (more) fr += fr_step;
 #pragma unroll
@@ -632,11 +628,9 @@ __global__ __launch_bounds__(128 * WPB, 1) void delta_chunk_pair_kernel(const bf
                     for (int i = 0; i < GN; ++i) st[n4 + i] = mma(kt[i], wl[jp], st[n4 + i]);
                 }
             if (more) {
-                __syncthreads();  // every wave is done with this chunk's LDS images
-                STORE_CHUNK(t0 + Q)
                 PUBLISH()
-                __syncthreads();
-                ++ck;
+                __syncthreads();  // the state and the next images are in LDS, U and this chunk's images have been read
+                img ^= 1;
             }
         }
 #undef PUBLISH
@@ -647,16 +641,25 @@ __global__ __launch_bounds__(128 * WPB, 1) void delta_chunk_pair_kernel(const bf
         }
         return;
     }
+    constexpr int NTH = 64 * WPB, KIT = (Q * 4 * NB + NTH - 1) / NTH, VR = Q * 2 * WPB / NTH, VIT = 256 / NTH;
+    const int tid = threadIdx.x - NTH;
+    bf16 *sK = s_k[0], *sQ = s_q[0], *sV = s_v[0];  // where the next chunk goes
+    float* s_vec = s_vecs[0];
+    u32x4 kreg[KIT], qreg[KIT], vreg[VR];
+    float vecr[VIT];
+    int ck = sg.w;
     fr += 64 * 2 * FR;
 #pragma unroll
     for (int f = 0; f < 2 * FR; ++f) lf[f] = fr[64 * f];
     LOAD_CHUNK(rb, ck)
     STORE_CHUNK(rb)
+    if (rb + Q < re) ++ck;
+    LOAD_CHUNK(rb + Q < re ? rb + Q : rb, ck)
     __syncthreads();
     for (int t0 = rb; t0 < re; t0 += Q) {
         const bool more = t0 + Q < re;
-        LOAD_CHUNK(more ? t0 + Q : t0, more ? ck + 1 : ck)
-        __builtin_amdgcn_sched_barrier(0);  // loads stay here
+        const bf16* q = s_q[img];
+        const float* rq = s_vecs[img] + 64;
         f32x4 o[4];
 #pragma unroll
         for (int ib = 0; ib < 4; ++ib) o[ib] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -666,33 +669,39 @@ __global__ __launch_bounds__(128 * WPB, 1) void delta_chunk_pair_kernel(const bf
             bf16x8 qf[4];
 #pragma unroll
             for (int ib = 0; ib < 4; ++ib)
-                qf[ib] = *reinterpret_cast<const bf16x8*>(sQ + row_at<NB>(r16, 32 * kb + 8 * g) + 16 * ib * LK);
+                qf[ib] = *reinterpret_cast<const bf16x8*>(q + row_at<NB>(r16, 32 * kb + 8 * g) + 16 * ib * LK);
 #pragma unroll
             for (int ib = 0; ib < 4; ++ib) o[ib] = mma(qf[ib], sh, o[ib]);
 #pragma unroll
             for (int ib = 0; ib < 4; ++ib) o[ib] = mma(qf[ib], sl, o[ib]);
         }
 #pragma unroll
-        for (int ib = 0; ib < 4; ++ib) o[ib] *= *reinterpret_cast<const f32x4*>(s_vec + 64 + 16 * ib + 4 * g);
+        for (int ib = 0; ib < 4; ++ib) o[ib] *= *reinterpret_cast<const f32x4*>(rq + 16 * ib + 4 * g);
+        if (more) {
+            img ^= 1;
+            sK = s_k[img], sQ = s_q[img], sV = s_v[img], s_vec = s_vecs[img];
+            STORE_CHUNK(t0 + Q)
+        }
         __syncthreads();  // U is in LDS; the state has been read
+        const bool two = t0 + 2 * Q < re;
+        if (two) ++ck;
+        LOAD_CHUNK(two ? t0 + 2 * Q : t0, ck)
         {
-            const bf16x8 hi[2] = {sU[w][0][lane], sU[w][1][lane]}, lo[2] = {sU[w][2][lane], sU[w][3][lane]};
-            lower(o, lf, hi, lo);
+            f32x4 u[4];
+#pragma unroll
+            for (int ib = 0; ib < 4; ++ib) u[ib] = sU[w][ib][lane];
+            lower(o, lf, u);
         }
         if (more) fr += fr_step;
 #pragma unroll
         for (int f = 0; f < 2 * FR; ++f) lf[f] = fr[64 * f];
         STORE_ROWS(o)
-        if (more) {
-            __syncthreads();  // every wave is done with this chunk's LDS images
-            STORE_CHUNK(t0 + Q)
-            __syncthreads();
-            ++ck;
-        }
+        if (more) __syncthreads();  // the state and the next images are in LDS, U has been read
     }
 }
 #undef LOAD_CHUNK
 #undef STORE_CHUNK
+#undef RAGGED
 #undef STORE_ROWS
 
 // 16-byte pieces and floats of workspace per (chunk, head)

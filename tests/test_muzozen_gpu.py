@@ -269,6 +269,30 @@ def test_head_product_of_fp32(rows, H, xk, K, N):
     assert rel(got[:, :, :N], want) < 1e-6 and (got[:, :, N:] == 7).all()
 
 
+@pytest.mark.parametrize("H,G,N,P", [(4, 2, 128, 128), (2, 1, 104, 136), (3, 3, 64, 40), (2, 2, 24, 16)])
+def test_delta_chunks_by_any_split(H, G, N, P):
+    """Segments of one to six chunks, full and ragged ones behind one another: every split forms the same sums in the same
+    order, so outputs and states have the same bits."""
+    from llm_map_reduce_summarizer_amd.ops import hip
+    from llm_map_reduce_summarizer_amd.ops.hip import _fn, _p, _stream
+    lens = [64, 1, 65, 128, 191, 321, 5]
+    T, ldx = sum(lens), 2 * G * N + H * P
+    x, u = dev(rnd(T, ldx).to(BF)), dev(rnd(T, 2 * H, seed=1).to(BF))
+    dt_bias, a_neg = dev(rnd(H, seed=2) - 3), dev(-torch.exp(rnd(H, seed=3)))
+    first, slots, pos0 = rnd(len(lens), H, P, N, seed=4), list(range(len(lens))), [7, 0, 64, 0, 9, 1, 0]
+    segs, chunks = (torch.tensor(v, dtype=torch.int32, device=DEV) for v in hip.delta_chunks(lens, 0))
+    slots, pos0 = (torch.tensor(v, dtype=torch.int32, device=DEV) for v in (slots, pos0))
+    out = []
+    for wpb, pair in ((8, 0), (4, 0), (4, 1), (2, 0), (2, 1)):
+        frags = torch.empty(len(chunks) * H * _fn("mrsum_delta_chunk_pieces")() * 4, dtype=torch.int32, device=DEV)
+        vec, y, state = torch.empty(len(chunks) * H * 256, device=DEV), torch.full((T, H * P), 7.0, device=DEV), dev(first)
+        assert _fn("mrsum_delta_chunk")(_p(x), ldx, G * N, 2 * G * N, _p(u), 0, 2 * H, T, 0, H, _p(dt_bias), _p(a_neg), _p(state),
+                                        _p(slots), _p(pos0), _p(segs), len(lens), _p(chunks), len(chunks), _p(frags), _p(vec),
+                                        _p(y), 0, H, G, P, N, wpb, pair, _stream()) == 0
+        out.append((y, state))
+    assert all(torch.equal(a, b) for o in out[1:] for a, b in zip(out[0], o))
+
+
 @pytest.mark.parametrize("H,G,dim,vdim", DELTA)
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_delta_rule(H, G, dim, vdim, dtype, monkeypatch):
