@@ -272,6 +272,16 @@ def test_work_lists_cover_every_row():
         assert delta_waves(P, N, pairs) == want
 
 
+def test_delta_split_runs_at_once():
+    """On both sides of each line of the rule: (value columns, dim, pairs, blocks and waves)."""
+    from llm_map_reduce_summarizer_amd.ops.hip import delta_waves
+    for P, N, pairs, want in ((128, 128, 64, (2, 1)), (128, 128, 65, (4, 1)), (128, 65, 128, (4, 1)), (128, 128, 129, (8, 0)),
+                              (64, 128, 128, (2, 1)), (64, 128, 129, (4, 1)), (128, 64, 128, (2, 1)), (128, 64, 129, (8, 0)),
+                              (64, 64, 384, (2, 1)), (64, 64, 385, (4, 1)), (32, 64, 9999, (2, 1)), (256, 128, 32, (2, 1)),
+                              (256, 128, 33, (4, 1)), (256, 128, 65, (8, 0)), (64, 256, 1, (4, 0)), (32, 129, 9999, (2, 0))):
+        assert delta_waves(P, N, pairs) == want, (P, N, pairs)
+
+
 def test_portion_context_places_every_page():
     from llm_map_reduce_summarizer_amd import ops
     ctx = ops.PortionContext([10, 2, 64], [0, 127, 64], [3, 0, 1], torch.device("cpu"))
