@@ -67,7 +67,7 @@ __device__ __forceinline__ void split8(const float* v, bf16x8& hi, bf16x8& lo) {
 }  // namespace
 
 template <int PW, int NB, bool STATE_ONLY>
-__global__ __launch_bounds__(STATE_ONLY ? 256 : 512, STATE_ONLY ? 2 : (PW == 1 && NB <= 4 ? 4 : 2)) void ssm_chunk_kernel(
+__global__ __launch_bounds__(STATE_ONLY ? 320 : 512, STATE_ONLY ? 2 : (PW == 1 && NB <= 4 ? 4 : 2)) void ssm_chunk_kernel(
     const ChunkArgs a) {
     constexpr int NTH = STATE_ONLY ? 256 : 512;
     constexpr int PP = 64 * PW, NN = 32 * NB;
@@ -116,6 +116,46 @@ __global__ __launch_bounds__(STATE_ONLY ? 256 : 512, STATE_ONLY ? 2 : (PW == 1 &
             const int idx = tid + NTH * i, row = idx / (8 * PW), p = 8 * (idx % (8 * PW));              \
             *reinterpret_cast<u32x4*>(sX + row * LX + p) = xreg[i];                                     \
         }                                                                                               \
+    }
+    // The raw step sizes of a chunk become dt, the running sum and the update weights beside the chunk before, in a wave that
+    // updates the state (it has half the products of one that makes output rows) or, where all do, in one of its own: between
+    // the chunk's two barriers only their stores are left.  All of it there made every wave wait for seven exchanges of lanes
+    // one after the other.
+    const float an = a.a_neg[head] * LOG2E, db = a.dt_bias[head];
+    float dtr = 0.f, cum = 0.f;
+#define LOAD_DT(T0)                                                                                     \
+    {                                                                                                   \
+        const int ti_ = min((T0) + lane, re - 1);                                                       \
+        dtr = a.u.S ? proj_at<true>(a.u, ti_, a.dt_at + head) : proj_at<false>(a.u, ti_, a.dt_at + head); \
+    }
+#define SCAN_DT(T0)                                                                                     \
+    {                                                                                                   \
+        dtr = (T0) + lane < re ? softplus(dtr + db) : 0.f;                                              \
+        cum = an * dtr;                                                                                 \
+        _Pragma("unroll") for (int o = 1; o < 64; o <<= 1) {                                            \
+            const float v = __shfl_up(cum, o, 64);                                                      \
+            if (lane >= o) cum += v;                                                                    \
+        }                                                                                               \
+    }
+#define STORE_DT()                                                                                      \
+    {                                                                                                   \
+        s_cum[lane] = cum;                                                                              \
+        s_dt[lane] = dtr;                                                                               \
+        s_w[lane] = __builtin_amdgcn_exp2f(__shfl(cum, 63, 64) - cum) * dtr;                            \
+    }
+    if (STATE_ONLY && wv == 4) {
+        LOAD_DT(rb)
+        SCAN_DT(rb)
+        STORE_DT()
+        __syncthreads();
+        for (int t0 = rb + Q; t0 < re; t0 += Q) {
+            LOAD_DT(t0)
+            SCAN_DT(t0)
+            __syncthreads();
+            STORE_DT()
+            __syncthreads();
+        }
+        return;
     }
     LOAD_CHUNK(rb)
     if (!updates) {
@@ -213,7 +253,6 @@ __global__ __launch_bounds__(STATE_ONLY ? 256 : 512, STATE_ONLY ? 2 : (PW == 1 &
         }
         return;
     }
-    const float an = a.a_neg[head] * LOG2E, db = a.dt_bias[head];
     const size_t per_head = (size_t)a.P * a.N4;
     float* slot = a.state + ((size_t)a.slots[seg] * a.heads + head) * per_head;
     float* ws = a.ws ? a.ws + ((size_t)item * a.heads + head) * per_head : nullptr;
@@ -231,25 +270,6 @@ __global__ __launch_bounds__(STATE_ONLY ? 256 : 512, STATE_ONLY ? 2 : (PW == 1 &
                     st[pw][nb] = *reinterpret_cast<const f32x4*>(src + (size_t)p * a.N4 + n);
             }
     }
-    float dtr = 0.f;
-#define LOAD_DT(T0)                                                                                     \
-    if (w == 0) {                                                                                       \
-        const int ti_ = min((T0) + lane, re - 1);                                                       \
-        dtr = a.u.S ? proj_at<true>(a.u, ti_, a.dt_at + head) : proj_at<false>(a.u, ti_, a.dt_at + head); \
-    }
-    // the raw step sizes become dt, the running sum and the update weights
-#define STORE_DT(T0)                                                                                    \
-    if (w == 0) {                                                                                       \
-        const float dt = (T0) + lane < re ? softplus(dtr + db) : 0.f;                                   \
-        float c = an * dt;                                                                              \
-        _Pragma("unroll") for (int o = 1; o < 64; o <<= 1) {                                            \
-            const float v = __shfl_up(c, o, 64);                                                        \
-            if (lane >= o) c += v;                                                                      \
-        }                                                                                               \
-        s_cum[lane] = c;                                                                                \
-        s_dt[lane] = dt;                                                                                \
-        s_w[lane] = __builtin_amdgcn_exp2f(__shfl(c, 63, 64) - c) * dt;                                 \
-    }
 #define STORE_STATE()                                                                                   \
     if constexpr (!STATE_ONLY) {                                                                        \
         _Pragma("unroll") for (int pw = 0; pw < PW; ++pw)                                               \
@@ -263,9 +283,12 @@ __global__ __launch_bounds__(STATE_ONLY ? 256 : 512, STATE_ONLY ? 2 : (PW == 1 &
                                pack2(st[pw][nb][2] - hi[2], st[pw][nb][3] - hi[3]));                    \
             }                                                                                           \
     }
-    LOAD_DT(rb)
+    if (!STATE_ONLY && w == 0) LOAD_DT(rb)
     STORE_CHUNK()
-    STORE_DT(rb)
+    if (!STATE_ONLY && w == 0) {
+        SCAN_DT(rb)
+        STORE_DT()
+    }
     STORE_STATE()
     __syncthreads();
     float total = 0.f;  // STATE_ONLY: the run's summed log2 decay
@@ -273,7 +296,7 @@ __global__ __launch_bounds__(STATE_ONLY ? 256 : 512, STATE_ONLY ? 2 : (PW == 1 &
         const bool more = t0 + Q < re;
         if (more) {
             LOAD_CHUNK(t0 + Q)
-            LOAD_DT(t0 + Q)
+            if (!STATE_ONLY && w == 0) LOAD_DT(t0 + Q)
         }
         const float clast = s_cum[Q - 1];
         total += clast;
@@ -310,9 +333,10 @@ __global__ __launch_bounds__(STATE_ONLY ? 256 : 512, STATE_ONLY ? 2 : (PW == 1 &
             }
         }
         if (more) {
+            if (!STATE_ONLY && w == 0) SCAN_DT(t0 + Q)
             __syncthreads();  // every wave is done with this chunk's LDS images
+            if (!STATE_ONLY && w == 0) STORE_DT()
             STORE_CHUNK()
-            STORE_DT(t0 + Q)
             STORE_STATE()
             __syncthreads();
         }
@@ -320,6 +344,7 @@ __global__ __launch_bounds__(STATE_ONLY ? 256 : 512, STATE_ONLY ? 2 : (PW == 1 &
 #undef LOAD_CHUNK
 #undef STORE_CHUNK
 #undef LOAD_DT
+#undef SCAN_DT
 #undef STORE_DT
 #undef STORE_STATE
     float* dst = STATE_ONLY ? ws : (it.w ? slot : nullptr);
@@ -369,7 +394,7 @@ MRSUM_API int mrsum_ssm_chunk(const void* xbc, int ldx, const void* u, int S, in
     const ChunkArgs a{(const bf16*)xbc, ldx, ProjSrc{u, S, (size_t)T * ld, ld}, dt_at, dt_bias, a_neg, d_skip, state,
                       slots, pos0, (const int4*)items, runs ? ws : nullptr, ws_decay, y, heads, P, N, N, groups};
     const dim3 grid(heads, n_items);
-#define CHUNK(PW_, NB_, SO_) ssm_chunk_kernel<PW_, NB_, SO_><<<grid, SO_ ? 256 : 512, 0, s>>>(a)
+#define CHUNK(PW_, NB_, SO_) ssm_chunk_kernel<PW_, NB_, SO_><<<grid, SO_ ? 320 : 512, 0, s>>>(a)
 #define CHUNK_N(SO_)                                                                          \
     if (P <= 64) {                                                                            \
         if (N <= 32) CHUNK(1, 1, SO_); else if (N <= 64) CHUNK(1, 2, SO_);                    \
