@@ -57,12 +57,21 @@ __device__ __forceinline__ f32x4 mma(bf16x8 a, bf16x8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
+// two values as bf16 terms (hi, lo): a conversion of both gives either
+__device__ __forceinline__ uint2 split2(float x, float y) {
+    const uint32_t h = pack2(x, y);
+    return make_uint2(h, pack2(x - __uint_as_float(h << 16), y - __uint_as_float(h & 0xffff0000u)));
+}
 __device__ __forceinline__ void split8(const float* v, bf16x8& hi, bf16x8& lo) {
+    u32x4 h, l;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        hi[j] = (bf16)v[j];
-        lo[j] = (bf16)(v[j] - (float)hi[j]);
+    for (int j = 0; j < 4; ++j) {
+        const uint2 t = split2(v[2 * j], v[2 * j + 1]);
+        h[j] = t.x;
+        l[j] = t.y;
     }
+    hi = __builtin_bit_cast(bf16x8, h);
+    lo = __builtin_bit_cast(bf16x8, l);
 }
 }  // namespace
 
@@ -275,12 +284,10 @@ __global__ __launch_bounds__(STATE_ONLY ? 320 : 512, STATE_ONLY ? 2 : (PW == 1 &
         _Pragma("unroll") for (int pw = 0; pw < PW; ++pw)                                               \
             _Pragma("unroll") for (int nb = 0; nb < NT; ++nb) {                                         \
                 const int o = (64 * pw + 16 * w + r16) * LB + 16 * nb + 4 * g;                          \
-                float hi[4];                                                                            \
-                _Pragma("unroll") for (int j = 0; j < 4; ++j) hi[j] = (float)(bf16)st[pw][nb][j];       \
-                *reinterpret_cast<uint2*>(sSh + o) = make_uint2(pack2(hi[0], hi[1]), pack2(hi[2], hi[3])); \
-                *reinterpret_cast<uint2*>(sSl + o) =                                                    \
-                    make_uint2(pack2(st[pw][nb][0] - hi[0], st[pw][nb][1] - hi[1]),                     \
-                               pack2(st[pw][nb][2] - hi[2], st[pw][nb][3] - hi[3]));                    \
+                const uint2 s01 = split2(st[pw][nb][0], st[pw][nb][1]);                                 \
+                const uint2 s23 = split2(st[pw][nb][2], st[pw][nb][3]);                                 \
+                *reinterpret_cast<uint2*>(sSh + o) = make_uint2(s01.x, s23.x);                          \
+                *reinterpret_cast<uint2*>(sSl + o) = make_uint2(s01.y, s23.y);                          \
             }                                                                                           \
     }
     if (!STATE_ONLY && w == 0) LOAD_DT(rb)
