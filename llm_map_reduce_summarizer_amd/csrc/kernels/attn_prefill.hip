@@ -363,15 +363,18 @@ __global__ __launch_bounds__(64 * waves(KVM), waves(KVM) == 4 ? 2 : 1) void attn
             for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;
         }
         float ls = 0.f;
-        bf16x8 pf[2][2], pl[2][2];
+        u32x4 pf[2][2], pl[2][2];
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const float p = __builtin_amdgcn_exp2f(fmaf(sacc[kt][i], scale_log2, -m));
-                ls += p;
-                pf[kt][i >> 3][i & 7] = (bf16)p;
-                if constexpr (HL) pl[kt][i >> 3][i & 7] = (bf16)(p - (float)(bf16)p);
+            for (int i = 0; i < 16; i += 2) {
+                const float p0 = __builtin_amdgcn_exp2f(fmaf(sacc[kt][i], scale_log2, -m));
+                const float p1 = __builtin_amdgcn_exp2f(fmaf(sacc[kt][i + 1], scale_log2, -m));
+                ls += p0;
+                ls += p1;
+                const uint2 t = split2(p0, p1);
+                pf[kt][i >> 3][(i & 7) >> 1] = t.x;
+                if constexpr (HL) pl[kt][i >> 3][(i & 7) >> 1] = t.y;
             }
         }
         l += ls;
@@ -394,10 +397,10 @@ __global__ __launch_bounds__(64 * waves(KVM), waves(KVM) == 4 ? 2 : 1) void attn
             for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
                 for (int s = 0; s < 2; ++s) {
-                    o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, va[kt][s]), pf[kt][s],
+                    o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, va[kt][s]), __builtin_bit_cast(bf16x8, pf[kt][s]),
                                                                     o[dt], 0, 0, 0);
                     if constexpr (HL)
-                        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, va[kt][s]), pl[kt][s],
+                        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, va[kt][s]), __builtin_bit_cast(bf16x8, pl[kt][s]),
                                                                         o[dt], 0, 0, 0);
                 }
         }

@@ -44,6 +44,12 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
     return __builtin_bit_cast(uint32_t, bf16x2{(bf16)a, (bf16)b});
 }
 
+// two values as bf16 terms (hi, lo): a conversion of both gives either
+__device__ __forceinline__ uint2 split2(float x, float y) {
+    const uint32_t h = pack2(x, y);
+    return make_uint2(h, pack2(x - __uint_as_float(h << 16), y - __uint_as_float(h & 0xffff0000u)));
+}
+
 __device__ __forceinline__ uint4 pack8(const float* f) {
     return make_uint4(pack2(f[0], f[1]), pack2(f[2], f[3]), pack2(f[4], f[5]), pack2(f[6], f[7]));
 }

@@ -168,15 +168,18 @@ __global__ __launch_bounds__(NTHR, 1) void latent_prefill_kernel(const LatPrefil
             for (int dt = 0; dt < VC; ++dt) o[dt] *= alpha;
         }
         float ls = 0.f;
-        bf16x8 pf[2][2], pl[2][2];
+        u32x4 pf[2][2], pl[2][2];
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const float p = __builtin_amdgcn_exp2f(fmaf(sacc[kt][i], a.scale_log2, -m));
-                ls += p;
-                pf[kt][i >> 3][i & 7] = (bf16)p;
-                pl[kt][i >> 3][i & 7] = (bf16)(p - (float)(bf16)p);
+            for (int i = 0; i < 16; i += 2) {
+                const float p0 = __builtin_amdgcn_exp2f(fmaf(sacc[kt][i], a.scale_log2, -m));
+                const float p1 = __builtin_amdgcn_exp2f(fmaf(sacc[kt][i + 1], a.scale_log2, -m));
+                ls += p0;
+                ls += p1;
+                const uint2 t = split2(p0, p1);
+                pf[kt][i >> 3][(i & 7) >> 1] = t.x;
+                pl[kt][i >> 3][(i & 7) >> 1] = t.y;
             }
         l += ls;
 #pragma unroll
@@ -193,8 +196,8 @@ __global__ __launch_bounds__(NTHR, 1) void latent_prefill_kernel(const LatPrefil
             for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
                 for (int s = 0; s < 2; ++s) {
-                    o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[kt][s], pf[kt][s], o[dt], 0, 0, 0);
-                    o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[kt][s], pl[kt][s], o[dt], 0, 0, 0);
+                    o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[kt][s], as8(pf[kt][s]), o[dt], 0, 0, 0);
+                    o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[kt][s], as8(pl[kt][s]), o[dt], 0, 0, 0);
                 }
         }
         __builtin_amdgcn_sched_group_barrier(0x100, 8, 1);

@@ -57,11 +57,6 @@ __device__ __forceinline__ f32x4 mma(bf16x8 a, bf16x8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// two values as bf16 terms (hi, lo): a conversion of both gives either
-__device__ __forceinline__ uint2 split2(float x, float y) {
-    const uint32_t h = pack2(x, y);
-    return make_uint2(h, pack2(x - __uint_as_float(h << 16), y - __uint_as_float(h & 0xffff0000u)));
-}
 __device__ __forceinline__ void split8(const float* v, bf16x8& hi, bf16x8& lo) {
     u32x4 h, l;
 #pragma unroll
