@@ -159,7 +159,7 @@ MRSUM_API int mrsum_attn_rows(const void* q, const void* kc, const void* vc, con
 // ------------------------------------------------------------------------------------------------ prompt portions
 // The same attention for many rows of few sequences, on the fp32 matrix instruction.  The row kernel reads every key
 // from memory for every (row, head): 1088 us for 900 rows of 32 heads of 128 over 8 kv heads, 4380 over 576-wide latents.
-// Here (163 and 520 us; bound by the chain of the block with the most keys, 5.5 us a tile of which its products are 1.7) 64
+// Here (112 and 520 us; bound by the chain of the block with the most keys, 5 us a tile of which its products are 1.7) 64
 // (row, head) pairs -- RB consecutive rows of HB heads of one kv head -- share key and value tiles of 32 in LDS (two buffers,
 // the next tile on its way in registers), a wave for 16 pairs.  With the page ids read when a tile is fetched, its loads
 // behind tests of the row and two barriers a tile, 183 and 758 (16-bit caches 201 and 915, now 167 and 570).
@@ -170,20 +170,30 @@ MRSUM_API int mrsum_attn_rows(const void* q, const void* kc, const void* vc, con
 // rows are padded by 4 floats (conflict-free b128 key reads and value reads).
 // Forms (NQ, NV: 16-column steps of keys and values; SHARED: values are the keys' first columns): KT 32, but 16 where 36 + 32
 // steps leave no registers for a larger tile on its way.
-template <typename T, int NQ, int NV, bool SHARED, int KT>
-__global__ __launch_bounds__(256, NQ <= 8 ? 2 : 1) void attn_portion_kernel(
+// KS 2: two groups of four waves take the tiles in turn, with buffers and sums of their own that meet in LDS at the end, so that
+// the block with the most keys walks half of them.  They take the place of two workgroups of a CU (8 us for a tile each where one
+// alone takes 5).  900 rows, 32 / 8 heads of 128 in fp32: 158 us, by the order of the blocks 148, with two groups 112; error
+// against fp64 6.7e-7 and 5.4e-7.  When: ops/hip.py portion_groups.
+template <typename T, int NQ, int NV, bool SHARED, int KT, int KS>
+__global__ __launch_bounds__(256 * KS, NQ <= 8 ? 2 : 1) void attn_portion_kernel(
     const T* __restrict__ q, const T* __restrict__ kc, const T* __restrict__ vc, const int* __restrict__ positions,
     const int* __restrict__ seq_idx, const int* __restrict__ block_tables, int bt_stride, int rows, int H, int G, int dk,
     int dv, int ldv, int pitch, float scale, const float* __restrict__ gate, T* __restrict__ out, int out_stride, int HB,
     int RB) {
     constexpr int LK = NQ * 16 + 4, LV = SHARED ? LK : NV * 16 + 4;
     constexpr int TPR = 256 / KT, FK = (NQ * 4 + TPR - 1) / TPR, FV = SHARED ? 1 : (NV * 4 + TPR - 1) / TPR;
-    __shared__ __attribute__((aligned(16))) float s_k[2][KT][LK];
-    __shared__ __attribute__((aligned(16))) float s_v[SHARED ? 1 : 2][SHARED ? 1 : KT][LV];
-    __shared__ int s_bad[3];  // tile i (slot i % 3, of SHARED i % 2) holds a value that is not finite
-    const int tid = threadIdx.x, lane = tid & 63, j16 = lane & 15, g4 = lane >> 4;
-    const int gh = H / G, hblocks = (gh + HB - 1) / HB, g = blockIdx.y / hblocks, h0 = blockIdx.y % hblocks * HB;
-    const int t0 = (gridDim.x - 1 - blockIdx.x) * RB, tend = min(rows, t0 + RB);  // the last rows, with the most keys, first
+    __shared__ __attribute__((aligned(16))) float s_ks[KS][2][KT][LK];
+    __shared__ __attribute__((aligned(16))) float s_vs[KS][SHARED ? 1 : 2][SHARED ? 1 : KT][LV];
+    __shared__ int s_bads[KS][3];  // tile i (slot i % 3, of SHARED i % 2) holds a value that is not finite
+    const int tid = threadIdx.x & 255, part = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    const int lane = tid & 63, j16 = lane & 15, g4 = lane >> 4;
+    auto& s_k = s_ks[part];
+    auto& s_v = s_vs[part];
+    auto& s_bad = s_bads[part];
+    // The last rows, with the most keys, of all heads first.  (All rows of a head first left the later heads' longest walks to begin
+    // behind the first one's short ones.)
+    const int gh = H / G, hblocks = (gh + HB - 1) / HB, per = G * hblocks, y = blockIdx.x % per, g = y / hblocks, h0 = y % hblocks * HB;
+    const int t0 = (gridDim.x / per - 1 - blockIdx.x / per) * RB, tend = min(rows, t0 + RB);
     const int pair = 16 * (tid >> 6) + j16, trow = t0 + pair / HB, hh = h0 + pair % HB;
     const bool valid = pair < RB * HB && trow < tend && hh < gh;
     const int t = valid ? trow : t0, head = g * gh + (valid ? hh : h0), pos = positions[t];
@@ -212,11 +222,11 @@ __global__ __launch_bounds__(256, NQ <= 8 ? 2 : 1) void attn_portion_kernel(
         const bool mine = valid && t >= a && t < b;
         const int* bt = block_tables + (size_t)seq * bt_stride;
         // keys past the last one are read as that (masked), columns past the row as its end and zeroed on the way into LDS
-        int page = bt[min(lr, last) / ROW_PAGE];  // of this thread's row of the tile fetched next
+        int page = bt[min(part * KT + lr, last) / ROW_PAGE];  // of this thread's row of the tile fetched next
         auto fetch = [&](int k0) {
             const int key = min(k0 + lr, last);
             const size_t slab = ((size_t)page * G + g) * ROW_PAGE + key % ROW_PAGE;
-            page = bt[min(k0 + KT + lr, last) / ROW_PAGE];
+            page = bt[min(k0 + KS * KT + lr, last) / ROW_PAGE];
 #pragma unroll
             for (int i = 0; i < FK; ++i) fk[i] = ld4(kc + slab * dk + min(lc + 4 * TPR * i, dk - 4));
             if constexpr (!SHARED) {
@@ -243,13 +253,14 @@ __global__ __launch_bounds__(256, NQ <= 8 ? 2 : 1) void attn_portion_kernel(
             if (bad) s_bad[slot] = 1;
         };
         if (tid < 3) s_bad[tid] = 0;
-        fetch(0);
+        fetch(part * KT);
         __syncthreads();
         put(0, 0);
         __syncthreads();
-        for (int k0 = 0, buf = 0, slot = 0; k0 <= last; k0 += KT, buf ^= 1) {
-            const bool more = k0 + KT <= last;
-            if (more) fetch(k0 + KT);
+        // (a group's last tile may be behind the last key: all of it is masked then)
+        for (int k0 = part * KT, buf = 0, slot = 0; k0 - part * KT <= last; k0 += KS * KT, buf ^= 1) {
+            const bool more = k0 - part * KT + KS * KT <= last;
+            if (more) fetch(k0 + KS * KT);
             f32x4 s[KT / 16];
 #pragma unroll
             for (int kb = 0; kb < KT / 16; ++kb) s[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -342,6 +353,24 @@ __global__ __launch_bounds__(256, NQ <= 8 ? 2 : 1) void attn_portion_kernel(
     }
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
+    if constexpr (KS == 2) {  // the second group's sums: a piece of 16 bytes a thread at a time, behind the last tile's barrier
+        static_assert(NV * 4 * 256 <= 2 * KT * LK && 2 * 256 <= (SHARED ? 1 : 2) * (SHARED ? 1 : KT) * LV, "LDS");
+        f32x4* so = reinterpret_cast<f32x4*>(&s_ks[1][0][0][0]);
+        float2* sml = reinterpret_cast<float2*>(&s_vs[1][0][0][0]);
+        if (part) {
+#pragma unroll
+            for (int c = 0; c < NV; ++c) so[256 * c + tid] = o[c];
+            sml[tid] = make_float2(m, l);
+        }
+        __syncthreads();
+        if (part) return;
+        const float2 other = sml[tid];
+        const float top = fmaxf(m, other.x), ref = top == -INFINITY ? 0.f : top;
+        const float f0 = expf(m - ref), f1 = expf(other.x - ref);
+        l = l * f0 + other.y * f1;
+#pragma unroll
+        for (int c = 0; c < NV; ++c) o[c] = o[c] * f0 + so[256 * c + tid] * f1;
+    }
     if (!valid) return;
     const float f = (gate ? gate[(size_t)t * H + head] : 1.f) / l;
     T* dst = out + (size_t)t * out_stride + (size_t)head * pitch;
@@ -357,34 +386,40 @@ __global__ __launch_bounds__(256, NQ <= 8 ? 2 : 1) void attn_portion_kernel(
 template <typename T>
 static int launch_portions(const void* q, const void* kc, const void* vc, const int* positions, const int* seq_idx,
                            const int* block_tables, int bt_stride, int rows, int H, int G, int dk, int dv, int ldv, int pitch,
-                           float scale, const float* gate, void* out, int out_stride, hipStream_t s) {
+                           float scale, const float* gate, void* out, int out_stride, int ks, hipStream_t s) {
     const int gh = H / G, HB = std::min(gh, 32), RB = 64 / HB;
-    const dim3 grid(ceil_div(rows, RB), G * ceil_div(gh, HB));
-#define AP(NQ, NV, SH, KT)                                                                                               \
-    attn_portion_kernel<T, NQ, NV, SH, KT><<<grid, 256, 0, s>>>((const T*)q, (const T*)kc, (const T*)vc, positions, seq_idx,  \
+    const int grid = ceil_div(rows, RB) * G * ceil_div(gh, HB);
+#define AP(NQ, NV, SH, KT, KS)                                                                                           \
+    attn_portion_kernel<T, NQ, NV, SH, KT, KS><<<grid, 256 * KS, 0, s>>>((const T*)q, (const T*)kc, (const T*)vc, positions, seq_idx,  \
                                                             block_tables, bt_stride, rows, H, G, dk, dv, ldv, pitch,      \
                                                             scale, gate, (T*)out, out_stride, HB, RB)
-    if (dk <= 64 && dv <= 64) AP(4, 4, false, 32);
-    else if (dk <= 128 && dv <= 128) AP(8, 8, false, 32);
-    else if (dk <= 256 && dv <= 256) AP(16, 16, false, 32);
-    else if (kc == vc && ldv == dk && dk <= 576 && dv <= 512) AP(36, 32, true, 16);
+    if (dk <= 64 && dv <= 64) {
+        if (ks == 2) AP(4, 4, false, 32, 2);
+        else AP(4, 4, false, 32, 1);
+    } else if (dk <= 128 && dv <= 128) {
+        if (ks == 2) AP(8, 8, false, 32, 2);
+        else AP(8, 8, false, 32, 1);
+    } else if (dk <= 256 && dv <= 256) AP(16, 16, false, 32, 1);
+    else if (kc == vc && ldv == dk && dk <= 576 && dv <= 512) AP(36, 32, true, 16, 1);
     else return (int)hipErrorInvalidValue;
 #undef AP
     return (int)hipGetLastError();
 }
 
 // Arguments as mrsum_attn_rows; widths multiples of 4, rows 16-byte (fp32) or 8-byte (bf16) aligned, and up to 256 wide, or
-// up to 576 / 512 where the values are the first columns of the keys.
+// up to 576 / 512 where the values are the first columns of the keys.  ks: groups that share a block's keys (2: rows up to 128
+// wide; wider ones have one).
 MRSUM_API int mrsum_attn_portions(const void* q, const void* kc, const void* vc, const int* positions, const int* seq_idx,
                                   const int* block_tables, int bt_stride, int T, int H, int G, int dk, int dv, int ldv,
-                                  int pitch, float scale, const float* gate, void* out, int out_stride, int f32,
+                                  int pitch, float scale, const float* gate, void* out, int out_stride, int f32, int ks,
                                   hipStream_t s) {
     if (T <= 0) return 0;
-    if (G <= 0 || H % G || dk % 4 || dv % 4 || ldv % 4 || pitch > dv || ldv < dv || G * ceil_div(H / G, 32) > 65535)
+    if (G <= 0 || H % G || dk % 4 || dv % 4 || ldv % 4 || pitch > dv || ldv < dv || G * ceil_div(H / G, 32) > 65535 ||
+        (long long)T * H > 0x7fffffff || (ks != 1 && ks != 2))
         return (int)hipErrorInvalidValue;
     if (f32)
         return launch_portions<float>(q, kc, vc, positions, seq_idx, block_tables, bt_stride, T, H, G, dk, dv, ldv, pitch,
-                                      scale, gate, out, out_stride, s);
+                                      scale, gate, out, out_stride, ks, s);
     return launch_portions<bf16>(q, kc, vc, positions, seq_idx, block_tables, bt_stride, T, H, G, dk, dv, ldv, pitch, scale,
-                                 gate, out, out_stride, s);
+                                 gate, out, out_stride, ks, s);
 }

@@ -364,3 +364,14 @@ def test_token_ids_of_one_and_many():
     for toks in ([], [10], [-1], [3, 10], [2 ** 70], [-(2 ** 70)]):
         with pytest.raises(ValueError):
             _token_ids(toks, 10)
+
+
+def test_portion_groups_by_chain_and_load():
+    """On both sides of each line: a chain of 48 keys, all walks on 256 workgroups (512 of heads up to 64), width 128."""
+    from llm_map_reduce_summarizer_amd.ops.hip import portion_groups
+    for portions, hq, hkv, d, want in ((((48, 0),), 32, 8, 128, 1), (((49, 0),), 32, 8, 128, 2), (((45, 4),), 32, 8, 128, 2),
+                                       (((1008, 0),), 32, 8, 128, 2), (((1024, 0),), 32, 8, 128, 1), (((1024, 0),), 32, 8, 64, 2),
+                                       (((2032, 0),), 32, 8, 64, 2), (((2048, 0),), 32, 8, 64, 1), (((900, 0),), 32, 8, 132, 1),
+                                       (((16, 100),) * 64, 32, 8, 128, 1), (((40, 300),) * 12, 32, 8, 128, 2),
+                                       (((400, 0),), 64, 1, 128, 2)):
+        assert portion_groups(portions, hq, hkv, d, d) == want, (portions, hq, hkv, d)

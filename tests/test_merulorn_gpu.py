@@ -1079,3 +1079,47 @@ def test_trace_runner_on_the_gpu(tmp_path, monkeypatch, capsys):
     got = torch.cat([torch.frombuffer(bytearray((tmp_path / ("%d.f32" % k)).read_bytes()), dtype=F32).view(2, -1)
                      for k in (0, 1)])
     M.check(got, M.expected("mixed", ids)[[0, 65, 66, 19]], BF)
+
+
+@pytest.mark.parametrize("H,G,d,pitch", [(8, 2, 128, 128), (3, 3, 64, 60), (5, 1, 100, 100), (2, 1, 20, 20)])
+@pytest.mark.parametrize("dtype", [BF, F32])
+@pytest.mark.parametrize("groups", [1, 2])
+def test_portion_attention_of_key_groups(H, G, d, pitch, dtype, groups):
+    """Walks of 1 key to several tiles, odd and even, sequences that share a block, and values that are not finite behind the keys
+    of a row: the groups' sums meet to what one softmax over all keys gives."""
+    from llm_map_reduce_summarizer_amd.ops.hip import _fn, _p, _stream
+    portions = [(3, 0), (70, 0), (1, 31), (5, 60), (40, 100), (2, 0), (33, 223)]
+    T, ends = sum(n for n, _ in portions), [n + b for n, b in portions]
+    pages = [-(-e // 64) for e in ends]
+    q, kc, vc = rnd(T, H * d), rnd(sum(pages), G, 64, d, seed=1), rnd(sum(pages), G, 64, d, seed=2)
+    perm, tables, at = torch.randperm(sum(pages), generator=torch.Generator().manual_seed(3)), [], 0
+    for p in pages:
+        tables.append(perm[at: at + p].tolist())
+        at += p
+    vc[tables[1][1], :, 5] = float("inf")  # key 69: the last row of the second portion alone has it
+    vc[tables[4][1], 0, 63, 0] = float("nan")  # key 127: rows 27 .. of the fifth
+    q, kc, vc = (t.to(dtype) for t in (q, kc, vc))
+    bt = torch.zeros(len(portions), max(pages), dtype=torch.int32)
+    for i, t in enumerate(tables):
+        bt[i, :len(t)] = torch.tensor(t)
+    pos = torch.cat([torch.arange(b, b + n) for n, b in portions]).int()
+    seq = torch.cat([torch.full((n,), i) for i, (n, _) in enumerate(portions)]).int()
+    gate = rnd(T, H, seed=4)
+    args = [dev(t) for t in (q, kc, vc, pos, seq, bt, gate)]
+    out = torch.full((T, H * pitch + 8), 7.0, dtype=dtype, device=DEV)
+    assert _fn("mrsum_attn_portions")(*map(_p, args[:6]), bt.stride(0), T, H, G, d, d, d, pitch, d ** -0.5, _p(args[6]), _p(out),
+                                      out.stride(0), 1 if dtype == F32 else 0, groups, _stream()) == 0
+    got, row = out.cpu(), 0
+    assert (got[:, H * pitch:] == 7).all()
+    for (n, b), t in zip(portions, tables):
+        K, V = (c[t].double().permute(1, 0, 2, 3).reshape(G, -1, d).repeat_interleave(H // G, 0) for c in (kc, vc))
+        for r in range(n):
+            w = torch.softmax((K[:, :b + r + 1] @ q[row].double().view(H, d, 1)).squeeze(-1) * d ** -0.5, -1)
+            want = (w[:, None] @ V[:, :b + r + 1]).squeeze(1)[:, :pitch] * gate[row].double()[:, None]
+            have = got[row, :H * pitch].view(H, pitch).double()
+            good = want.isfinite()
+            assert torch.equal(good, have.isfinite()), (row, r)
+            # fp32: sums of up to 256 terms in eight chains; bf16: the output's rounding
+            if good.any():
+                assert rel(have[good], want[good]) < (4e-3 if dtype == BF else 3e-6)
+            row += 1
