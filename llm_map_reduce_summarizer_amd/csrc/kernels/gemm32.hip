@@ -25,9 +25,7 @@ constexpr int LDS_BYTES = 80 * 1024;         // two workgroups on a CU
 template <int NB>
 constexpr int RUN = NB > 4 ? LONG_RUN : 4;
 
-// PAST_CACHES: W goes past the caches (gemm32_launch).  GUARDED: launched behind the terms, and does nothing unless they have met what
-// they hold short (a form of its own: the test of a pointer that is not there cost every other call 0.2 us, 16 x 768 x 768 8.1 -> 7.9)
-enum { PLAIN, PAST_CACHES, GUARDED };
+enum { PLAIN, PAST_CACHES };  // PAST_CACHES: W goes past the caches (gemm32_launch)
 }  // namespace
 
 // K-tiles [kt0, kt1) of a tile of NB row blocks; acc[row block][column block].  ONE: there are at most LONG_RUN of them
@@ -145,10 +143,9 @@ __device__ __forceinline__ void k_loop(const Gemm32Args& a, char* lds, int m0, i
     __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));  // nothing may arrive in LDS that another workgroup has by then
 }
 
+namespace {
 template <bool ONE, int FORM>
-__global__ __launch_bounds__(256, 2) void gemm32_kernel(const Gemm32Args a) {
-    if (FORM == GUARDED && !*a.inexact) return;
-    __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
+__device__ __forceinline__ void tile_or_slice(const Gemm32Args& a, char* lds) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     // an XCD's workgroups take neighbouring tiles: they share W's panels, and each XCD has taller and lower tiles alike
@@ -211,10 +208,34 @@ __global__ __launch_bounds__(256, 2) void gemm32_kernel(const Gemm32Args a) {
                 store_c(a, m0 + 16 * b + (lane & 15), n0 + 32 * w + 16 * i + 4 * (lane >> 4), acc[b][i]);
 }
 
+}  // namespace
+
+template <bool ONE, int FORM>
+__global__ __launch_bounds__(256, 2) void gemm32_kernel(const Gemm32Args a) {
+    __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
+    tile_or_slice<ONE, FORM>(a, lds);
+}
+
+// Behind a product in terms: adds what slices that has, or makes the whole result if it has met a value that terms hold short.
+// (Forms of their own: the test of a pointer that is not there cost every other call 0.2 us, 16 x 768 x 768 8.1 -> 7.9.)  A launch that
+// only looks at the flag takes 4 us.  us, the slices added by one of their own ahead -> here: 700 x 2048 x 2048 44 -> 39, 160 x 6144 x
+// 4096 56 -> 51, 300 x 4096 x 14336 126 -> 117, 903 x 4096 x 8192 200 -> 197; of 24 bits, which no longer adds them: 86 -> 75, 96 -> 85,
+// 347 -> 324, 522 -> 503.  (Without the launch below too, the last slice of a tile to arrive adding them all, 160 x 6144 took 50 and of
+// 24 bits 142: each workgroup's slice has to leave its L2.)
+template <bool ONE>
+__global__ __launch_bounds__(256, 2) void gemm32_behind_kernel(const Gemm32Args a, const Gemm32Args terms) {
+    __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
+    if (!*terms.inexact) {
+        if ((int)blockIdx.x < (terms.tiles_m * terms.tiles_n - terms.whole) * MAX_NB) add_terms_slices(terms, blockIdx.x);
+        return;
+    }
+    if ((int)blockIdx.x < a.whole + (a.tiles_m * a.tiles_n - a.whole) * a.splits) tile_or_slice<ONE, PLAIN>(a, lds);
+}
+
 // adds the slices of the split tiles; one workgroup per (tile, 2 x 16 rows)
 template <bool GUARD>
-__global__ __launch_bounds__(256) void gemm32_tail_kernel(const Gemm32Args a) {
-    if (GUARD && !*a.inexact) return;
+__global__ __launch_bounds__(256) void gemm32_tail_kernel(const Gemm32Args a, const int* inexact) {
+    if (GUARD && !*inexact) return;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, t = blockIdx.x >> 2, b = 2 * (blockIdx.x & 3);
     int tm, tn, b0, nb;
     tile32(a, a.whole + t, tm, tn);
@@ -291,7 +312,7 @@ __global__ __launch_bounds__(256) void gemm32_small_kernel(const float* __restri
 }
 
 int gemm32_launch(const float* x, int ldx, const float* w, int ldw, float* c, int ldc, int M, int N, int K, int whole, int splits,
-                  float* part, int* inexact, hipStream_t s) {
+                  float* part, const Gemm32Args* terms, hipStream_t s) {
     if (M <= 0 || N <= 0) return 0;
     if (K % 32 || ldx % 4 || ldw % 4 || (uintptr_t)x % 16 || (uintptr_t)w % 16 || (size_t)T32 * ldx * 4 >= (1u << 31) ||
         (size_t)T32 * ldw * 4 >= (1u << 31))
@@ -302,7 +323,7 @@ int gemm32_launch(const float* x, int ldx, const float* w, int ldw, float* c, in
         gemm32_small_kernel<<<dim3(ceil_div(N, TS), ceil_div(M, TS)), 256, 0, s>>>(x, ldx, w, ldw, c, ldc, M, N, K);
         return (int)hipGetLastError();
     }
-    Gemm32Args a{x, w, c, ldx, ldw, ldc, M, N, K / 32, ceil_div(M, T32), ceil_div(N, T32), 0, 1, part, inexact};
+    Gemm32Args a{x, w, c, ldx, ldw, ldc, M, N, K / 32, ceil_div(M, T32), ceil_div(N, T32), 0, 1, part, nullptr};
     const int tiles = a.tiles_m * a.tiles_n;
     if (splits > 1 && (whole < 0 || whole >= tiles || splits > a.kb || !part)) return (int)hipErrorInvalidValue;
     a.whole = splits > 1 ? whole : tiles;
@@ -313,9 +334,10 @@ int gemm32_launch(const float* x, int ldx, const float* w, int ldw, float* c, in
     // x 14336 (224 MiB) 38.2 -> 42.9 / 53.8 -> 49.6, 4 x 16384 (256 MiB) 47.6 -> 55.7 / 60.0 -> 56.4, 4 x 18432 59.7 -> 57.6 / 65.1 ->
     // 60.2, 4 x 20608 67.3 -> 60.5 / 69.7 -> 62.8; 4 x 4096 15.8 -> 17.2 / 18.4 -> 18.0; 4 x 128256 399 -> 369 (5.7 TB/s).
     const bool once = M <= 48 && (size_t)N * K * 4 > (256u << 20);
-    const int grid = a.whole + rest * a.splits;
+    const int mine = a.whole + rest * a.splits;
+    const int grid = terms ? std::max(mine, (terms->tiles_m * terms->tiles_n - terms->whole) * MAX_NB) : mine;
 #define FORMS(ONE)                                                          \
-    if (inexact) gemm32_kernel<ONE, GUARDED><<<grid, 256, 0, s>>>(a);            \
+    if (terms) gemm32_behind_kernel<ONE><<<grid, 256, 0, s>>>(a, *terms); \
     else if (once) gemm32_kernel<ONE, PAST_CACHES><<<grid, 256, 0, s>>>(a);  \
     else gemm32_kernel<ONE, PLAIN><<<grid, 256, 0, s>>>(a)
     if (ceil_div(a.kb, a.whole ? 1 : a.splits) <= LONG_RUN) {
@@ -325,8 +347,8 @@ int gemm32_launch(const float* x, int ldx, const float* w, int ldw, float* c, in
     }
 #undef FORMS
     if (!rest) return (int)hipGetLastError();
-    if (inexact) gemm32_tail_kernel<true><<<rest * 4, 256, 0, s>>>(a);
-    else gemm32_tail_kernel<false><<<rest * 4, 256, 0, s>>>(a);
+    if (terms) gemm32_tail_kernel<true><<<rest * 4, 256, 0, s>>>(a, terms->inexact);
+    else gemm32_tail_kernel<false><<<rest * 4, 256, 0, s>>>(a, nullptr);
     return (int)hipGetLastError();
 }
 

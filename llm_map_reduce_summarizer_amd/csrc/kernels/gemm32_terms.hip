@@ -7,8 +7,8 @@
 // adds in fp32: sixteen times the fp32 instruction's rate, for three times the products.  W stays 32 bits wide in memory and is
 // looked at as it is read.  If a value has lower bits, is infinite (an infinity times a term of 0 is no number) or smaller than bf16's
 // normal numbers (whose products the instruction forms with fewer bits), or if X has a value whose lowest bits would be finer than
-// bf16's (below 2^-110), a flag is set and the fp32 instruction's form (gemm32.hip), which is launched behind and otherwise returns
-// at once, makes the whole result.  A workgroup that sees it in its first K-tile or its rows of X stops there, others when their next
+// bf16's (below 2^-110), a flag is set and the fp32 instruction's form (gemm32.hip), which is launched behind and otherwise only adds
+// slices, makes the whole result.  A workgroup that sees it in its first K-tile or its rows of X stops there, others when their next
 // chain of 16 K-tiles ends.  What that costs, us, all in turn with rotating weights: 903 x 28672 x 4096 on the fp32 instruction 1593, by way of
 // here with 24 bits in all of W 1597, in half of its rows 1614 (2100 where nobody asks the others), in half of its columns 1697, in its
 // last value alone 2099; 160 x 6144 x 4096 75, 98, 113, 119, 126.  Each timed by itself the instruction takes 1548 there, and 24 bits in
@@ -36,13 +36,10 @@
 #include <type_traits>
 
 namespace {
-constexpr int TN = 256;                 // columns of a tile
-constexpr int MAX_NB = 5;               // its 32-row units
 constexpr int BLOCK = 3072;             // bytes of a K-tile of 32 of 16 rows of X: [term][lane][16]
 constexpr int WI = TN * 128, WS = 3;    // bytes of W's K-tile, and how many are in LDS; behind them X's
 constexpr int x_slots(int nb) { return nb <= 3 ? 3 : 2; }
 constexpr int LDS_BYTES = WS * WI + 2 * 2 * MAX_NB * BLOCK;
-constexpr int SLOT = MAX_NB * 32 * TN;  // scratch floats of a slice of a tile
 constexpr int TAIL = 512 + 3 * 1024;    // and behind these what is known of values that are not the sums of their terms
 static_assert(LDS_BYTES + TAIL <= 160 * 1024 && x_slots(3) * 2 * 3 * BLOCK <= 2 * 2 * MAX_NB * BLOCK, "LDS");
 
@@ -114,12 +111,6 @@ __global__ __launch_bounds__(256) void terms32_kernel(const float* __restrict__ 
 }
 
 namespace {
-// Outputs of (row block b, column block i ^ wr) of a tile of nb 32-row units: row lane & 15, columns 4 (lane >> 4) ..
-__device__ __forceinline__ void store_terms(const Gemm32Args& a, int u0, int nb, int n0, int b, int i, const f32x4& v) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    store_c(a, 32 * u0 + 16 * (nb * (w >> 1) + b) + (lane & 15), n0 + 128 * (w & 1) + 16 * (i ^ (w >> 1)) + 4 * (lane >> 4), v);
-}
-
 // K-tiles [kt0, kt1) of 32 NB rows from 32 u0 on and columns n0 ..; wave (wr, wc) has half of the rows and 128 columns: acc[row
 // block][column block ^ wr], so that the two waves that have the same columns each look at every other block of them, by the same
 // code.  False: some value is not the sum of its terms, and the sums are not made.
@@ -373,33 +364,6 @@ __global__ __launch_bounds__(256, 1) void gemm32_terms_kernel(const Gemm32Args a
     }
 }
 
-// adds the slices of the split tiles; one workgroup per (tile, 2 x 16 rows)
-__global__ __launch_bounds__(256) void gemm32_terms_tail_kernel(const Gemm32Args a) {
-    const int tid = threadIdx.x, t = blockIdx.x / MAX_NB, b = blockIdx.x % MAX_NB;
-    int tm, tn, u0, nu;
-    tile32(a, a.whole + t, tm, tn);
-    rows_of(a, (a.M + 31) >> 5, tm, tn, u0, nu);
-    if (b >= nu) return;
-    const f32x4* in = reinterpret_cast<const f32x4*>(a.part + (size_t)t * a.splits * SLOT) + b * 8 * 256 + tid;
-    f32x4 v[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = in[i * 256];
-    for (int s = 1; s < a.splits; s += 2) {  // two slices in flight
-        f32x4 q[2][8];
-#pragma unroll
-        for (int k = 0; k < 2; ++k)
-#pragma unroll
-            for (int i = 0; i < 8; ++i) q[k][i] = in[(size_t)min(s + k, a.splits - 1) * (SLOT / 4) + i * 256];
-#pragma unroll
-        for (int k = 0; k < 2; ++k)
-            if (s + k < a.splits)
-#pragma unroll
-                for (int i = 0; i < 8; ++i) v[i] += q[k][i];
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) store_terms(a, u0, nu, tn * TN, b, i, v[i]);
-}
-
 // *odd is set if one of n values is not a finite bf16 one, or is a subnormal one.  Bound by the reads: 28672 x 4096 in 88 us (5.3 TB/s).
 __global__ __launch_bounds__(256) void bf16_values_kernel(const uint32_t* __restrict__ w, size_t n, int* odd) {
     const size_t step = (size_t)gridDim.x * 256, i0 = (size_t)blockIdx.x * 256 + threadIdx.x, n4 = (uintptr_t)w % 16 ? 0 : n / 4;
@@ -451,9 +415,7 @@ MRSUM_API int mrsum_gemm32_terms(const float* x, int ldx, const float* w, int ld
         a.whole = whole;
         a.splits = splits;
     }
-    const int rest = (int)tiles - a.whole;
     terms32_kernel<<<ceil_div(pieces, 4), 256, 0, s>>>(x, ldx, static_cast<char*>(terms), M, kb, pieces, inexact);
-    gemm32_terms_kernel<<<a.whole + rest * a.splits, 256, 0, s>>>(a);
-    if (rest) gemm32_terms_tail_kernel<<<rest * MAX_NB, 256, 0, s>>>(a);
-    return gemm32_launch(x, ldx, w, ldw, c, ldc, M, N, K, whole32, splits32, part, inexact, s);
+    gemm32_terms_kernel<<<a.whole + ((int)tiles - a.whole) * a.splits, 256, 0, s>>>(a);
+    return gemm32_launch(x, ldx, w, ldw, c, ldc, M, N, K, whole32, splits32, part, &a, s);
 }
