@@ -516,9 +516,11 @@ __global__ __launch_bounds__(64 * WPB, 1) void delta_chunk_kernel(const bf16* __
 // one value at a time and results copied between the two halves of the register file they were 1010 a chunk of 64 x 128,
 // 3.1 us, and are 570, 1.9 us.  One prompt of 4096 tokens, 32 heads of 128 x 128, with the preparation: 199.5 -> 150.5 us; 16
 // heads of 64 x 64 123 -> 111 (with staging left to all waves 123).  The bound of 512 threads keeps the registers to 256, so
-// that products stay where the vector instructions reach them.
+// that products stay where the vector instructions reach them.  Of dim up to 32 in four blocks the bound of four waves a SIMD
+// keeps them to 128, for two workgroups on a CU (one with the 148 that it would take): dim 32, value columns 128, 192 (segment, head)
+// pairs of 300 tokens 42.6 -> 39.0 us, 64 columns, 512 pairs 67.3 -> 64.7, dim 24, of 1000 tokens 201 -> 195.
 template <int NB, int WPB>
-__global__ __launch_bounds__(512) void delta_chunk_pair_kernel(const bf16* __restrict__ x, DeltaArgs a,
+__global__ __launch_bounds__(512, NB == 1 && WPB == 4 ? 4 : 1) void delta_chunk_pair_kernel(const bf16* __restrict__ x, DeltaArgs a,
                                                                         const int4* __restrict__ segs,
                                                                         const int* __restrict__ slots,
                                                                         const int* __restrict__ pos0,

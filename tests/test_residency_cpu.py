@@ -1,0 +1,44 @@
+"""Workgroups that fit a compute unit by their registers and LDS, as the compiler reports them, where launch rules count on them."""
+
+import functools
+import os
+import re
+import subprocess
+
+import pytest
+
+from llm_map_reduce_summarizer_amd import _stamp
+
+HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+pytestmark = pytest.mark.skipif(not os.path.exists(HIPCC), reason="no hipcc")
+
+
+@functools.lru_cache(maxsize=None)
+def reported(source):
+    """Mangled name -> (registers of a wave, LDS bytes of a workgroup)."""
+    r = subprocess.run([HIPCC, *_stamp.HIP_FLAGS, "-c", os.path.join(_stamp.CSRC, "kernels", source), "-o", os.devnull],
+                       stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, check=True)
+    out, name, seen = {}, None, {}
+    for line in r.stdout.splitlines():
+        m = re.search(r"Function Name: (\S+)", line)
+        if m:
+            name, seen = m[1], {}
+        m = re.search(r" (VGPRs|AGPRs|LDS Size \[bytes/block\]): (\d+)", line)
+        if m and name:
+            seen[m[1]] = int(m[2])
+            if len(seen) == 3:
+                out[name] = (-(-seen["VGPRs"] // 4) * 4 + seen["AGPRs"], seen["LDS Size [bytes/block]"])
+    return out
+
+
+def workgroups(source, kernel, threads):
+    """How many workgroups of ``threads`` a CU holds: 512 registers a lane and SIMD in pieces of 8, 160 KiB of LDS."""
+    found = [v for k, v in reported(source).items() if kernel in k]
+    assert len(found) == 1, (kernel, found)
+    regs, lds = found[0]
+    waves = 4 * min(8, 512 // (-(-regs // 8) * 8))
+    return min(waves // (threads // 64), 160 * 1024 // max(lds, 1))
+
+
+def test_delta_pairs_of_narrow_heads():
+    assert workgroups("delta_chunk.hip", "delta_chunk_pair_kernelILi1ELi4E", 512) == 2
