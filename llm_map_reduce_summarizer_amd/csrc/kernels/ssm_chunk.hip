@@ -70,9 +70,11 @@ __device__ __forceinline__ void split8(const float* v, bf16x8& hi, bf16x8& lo) {
 }
 }  // namespace
 
-template <int PW, int NB, bool STATE_ONLY>
-__global__ __launch_bounds__(STATE_ONLY ? 320 : 512, STATE_ONLY ? 2 : (PW == 1 && NB <= 4 ? 4 : 2)) void ssm_chunk_kernel(
-    const ChunkArgs a) {
+// SCAN_WAVE: a wave that only makes the step sizes; STATE_ONLY, where every other wave updates the state (launch_state).
+template <int PW, int NB, bool STATE_ONLY, bool SCAN_WAVE>
+__global__ __launch_bounds__(STATE_ONLY ? (SCAN_WAVE ? 320 : 256) : 512,
+                             STATE_ONLY ? (PW == 1 && NB == 4 && !SCAN_WAVE ? 4 : 2) : (PW == 1 && NB <= 4 ? 4 : 2)) void
+ssm_chunk_kernel(const ChunkArgs a) {
     constexpr int NTH = STATE_ONLY ? 256 : 512;
     constexpr int PP = 64 * PW, NN = 32 * NB;
     constexpr int LB = NN + 16, LX = PP + 16;  // LDS row strides: +32 bytes spreads rows over the banks
@@ -122,9 +124,9 @@ __global__ __launch_bounds__(STATE_ONLY ? 320 : 512, STATE_ONLY ? 2 : (PW == 1 &
         }                                                                                               \
     }
     // The raw step sizes of a chunk become dt, the running sum and the update weights beside the chunk before, in a wave that
-    // updates the state (it has half the products of one that makes output rows) or, where all do, in one of its own: between
-    // the chunk's two barriers only their stores are left.  All of it there made every wave wait for seven exchanges of lanes
-    // one after the other.
+    // updates the state (it has half the products of one that makes output rows) or, where all do, in one of its own if SCAN_WAVE:
+    // between the chunk's two barriers only their stores are left.  All of it there made every wave wait for seven exchanges of
+    // lanes one after the other.
     const float an = a.a_neg[head] * LOG2E, db = a.dt_bias[head];
     float dtr = 0.f, cum = 0.f;
 #define LOAD_DT(T0)                                                                                     \
@@ -147,7 +149,7 @@ __global__ __launch_bounds__(STATE_ONLY ? 320 : 512, STATE_ONLY ? 2 : (PW == 1 &
         s_dt[lane] = dtr;                                                                               \
         s_w[lane] = __builtin_amdgcn_exp2f(__shfl(cum, 63, 64) - cum) * dtr;                            \
     }
-    if (STATE_ONLY && wv == 4) {
+    if (SCAN_WAVE && wv == 4) {
         LOAD_DT(rb)
         SCAN_DT(rb)
         STORE_DT()
@@ -285,9 +287,9 @@ __global__ __launch_bounds__(STATE_ONLY ? 320 : 512, STATE_ONLY ? 2 : (PW == 1 &
                 *reinterpret_cast<uint2*>(sSl + o) = make_uint2(s01.y, s23.y);                          \
             }                                                                                           \
     }
-    if (!STATE_ONLY && w == 0) LOAD_DT(rb)
+    if (!SCAN_WAVE && w == 0) LOAD_DT(rb)
     STORE_CHUNK()
-    if (!STATE_ONLY && w == 0) {
+    if (!SCAN_WAVE && w == 0) {
         SCAN_DT(rb)
         STORE_DT()
     }
@@ -298,7 +300,7 @@ __global__ __launch_bounds__(STATE_ONLY ? 320 : 512, STATE_ONLY ? 2 : (PW == 1 &
         const bool more = t0 + Q < re;
         if (more) {
             LOAD_CHUNK(t0 + Q)
-            if (!STATE_ONLY && w == 0) LOAD_DT(t0 + Q)
+            if (!SCAN_WAVE && w == 0) LOAD_DT(t0 + Q)
         }
         const float clast = s_cum[Q - 1];
         total += clast;
@@ -335,9 +337,9 @@ __global__ __launch_bounds__(STATE_ONLY ? 320 : 512, STATE_ONLY ? 2 : (PW == 1 &
             }
         }
         if (more) {
-            if (!STATE_ONLY && w == 0) SCAN_DT(t0 + Q)
+            if (!SCAN_WAVE && w == 0) SCAN_DT(t0 + Q)
             __syncthreads();  // every wave is done with this chunk's LDS images
-            if (!STATE_ONLY && w == 0) STORE_DT()
+            if (!SCAN_WAVE && w == 0) STORE_DT()
             STORE_CHUNK()
             STORE_STATE()
             __syncthreads();
@@ -380,6 +382,21 @@ __global__ __launch_bounds__(256) void ssm_combine_kernel(const ChunkArgs a, con
     }
 }
 
+namespace {
+// The state pass with a wave that only scans has a shorter chain, all passes, us: 64 heads of 64 x 128, 512 workgroups, 134 -> 124, of 64
+// x 32, 896 workgroups, 78 -> 73.  But it needs a place for five waves: of states above 128 (185 registers) a CU holds one such workgroup
+// and two of four waves, 32 heads, 512 workgroups, 105 and 101, 992 214 and 198; of 64 x 128 three and four, 896 workgroups 135
+// and 129, 1000 102 and 97, but 768, three a CU, 111.6 and 111.1.  (Of 128 x 32 three and four too, where both take the same: 896
+// workgroups 143 and 140, 1000 98 and 96, but 512 66 and 74.  ssm_runs makes at most 1023.)
+template <int PW, int NB>
+void launch_state(dim3 grid, const ChunkArgs& a, hipStream_t s) {
+    constexpr bool SOME = PW == 1 && NB == 4;
+    if constexpr (NB < 8)
+        if (!SOME || (long long)grid.x * grid.y <= 768) return ssm_chunk_kernel<PW, NB, true, true><<<grid, 320, 0, s>>>(a);
+    if constexpr (NB == 8 || SOME) ssm_chunk_kernel<PW, NB, true, false><<<grid, 256, 0, s>>>(a);
+}
+}  // namespace
+
 // Rows of the listed runs.  items int4 [n_items], runs int4 [n_runs] with ws / ws_decay when any segment is cut
 // (else runs null and n_items = segments).  P % 8 == 0, N % 8 == 0, ldx % 8 == 0; P <= 128, N <= 256 (P <= 64 above
 // 128).
@@ -396,13 +413,17 @@ MRSUM_API int mrsum_ssm_chunk(const void* xbc, int ldx, const void* u, int S, in
     const ChunkArgs a{(const bf16*)xbc, ldx, ProjSrc{u, S, (size_t)T * ld, ld}, dt_at, dt_bias, a_neg, d_skip, state,
                       slots, pos0, (const int4*)items, runs ? ws : nullptr, ws_decay, y, heads, P, N, N, groups};
     const dim3 grid(heads, n_items);
-#define CHUNK(PW_, NB_, SO_) ssm_chunk_kernel<PW_, NB_, SO_><<<grid, SO_ ? 320 : 512, 0, s>>>(a)
+#define CHUNK(PW_, NB_, SO_)                                                              \
+    {                                                                                     \
+        if constexpr (SO_) launch_state<PW_, NB_>(grid, a, s);                            \
+        else ssm_chunk_kernel<PW_, NB_, false, false><<<grid, 512, 0, s>>>(a);            \
+    }
 #define CHUNK_N(SO_)                                                                          \
     if (P <= 64) {                                                                            \
-        if (N <= 32) CHUNK(1, 1, SO_); else if (N <= 64) CHUNK(1, 2, SO_);                    \
-        else if (N <= 128) CHUNK(1, 4, SO_); else CHUNK(1, 8, SO_);                           \
+        if (N <= 32) CHUNK(1, 1, SO_) else if (N <= 64) CHUNK(1, 2, SO_)                      \
+        else if (N <= 128) CHUNK(1, 4, SO_) else CHUNK(1, 8, SO_)                             \
     } else {                                                                                  \
-        if (N <= 32) CHUNK(2, 1, SO_); else if (N <= 64) CHUNK(2, 2, SO_); else CHUNK(2, 4, SO_); \
+        if (N <= 32) CHUNK(2, 1, SO_) else if (N <= 64) CHUNK(2, 2, SO_) else CHUNK(2, 4, SO_) \
     }
     if (runs) {
         CHUNK_N(true)

@@ -167,6 +167,32 @@ def test_state_space_scan(heads, P, N, groups, dtype):
             b += n
 
 
+@pytest.mark.parametrize("heads,P,N,lens", [(3, 40, 200, [65, 700]), (96, 8, 104, [512] * 4), (97, 8, 104, [512] * 4)])
+def test_state_space_runs_without_a_scanning_wave(heads, P, N, lens):
+    """Segments cut into runs where the state pass has four waves: states above 128, and 768 workgroups (which have five) and more."""
+    from llm_map_reduce_summarizer_amd import ops
+    from llm_map_reduce_summarizer_amd.ops import hip
+    items, runs = hip.ssm_runs(lens, 0, heads)
+    assert runs is not None and (heads == 3 or (len(items) * heads > 768) == (heads == 97))
+    T, C = sum(lens), heads * P + 2 * N
+    xbc, u = rnd(T, C, std=0.7).to(BF), rnd(T, heads + 8 - heads % 8, seed=1).to(BF)
+    dt_bias, A_log, D = rnd(heads, seed=2, std=1.5) - 2, rnd(heads, seed=3, std=1.5), rnd(heads, seed=4)
+    slots, pos0 = list(range(len(lens))), [7 * (i % 2) for i in range(len(lens))]
+    init = rnd(len(lens), heads, P, N, seed=6, std=0.5)
+    state = dev(init.clone())
+    y = ops.ssm_scan(dev(xbc), dev(u), 0, dev(dt_bias), dev(-torch.exp(A_log)), dev(D), state, segments(lens, slots, pos0), heads, P,
+                     N, 1).view(T, heads, P)
+    f, some, b = xbc.double(), [0, heads // 2, heads - 1], 0
+    for i, n in enumerate(lens):
+        x, Bm, Cm = f[b: b + n, :heads * P].view(n, heads, P)[:, some], f[b: b + n, heads * P: heads * P + N], f[b: b + n, C - N:]
+        dts = O.softplus(u[b: b + n, :heads].double() + dt_bias.double())[:, some]
+        want, S = scan_with_state(x, Bm.view(n, 1, N), Cm.view(n, 1, N), dts, A_log[some].double(), D[some].double(), 1,
+                                  init[i, some].double() if pos0[i] else None)
+        # two terms of bf16 for everything that is not one, as above
+        assert rel(y[b: b + n, some], want) < 3e-5 and rel(state[i, some], S) < 3e-5, i
+        b += n
+
+
 @pytest.mark.parametrize("copies,dtype,N,rows", [(1, F32, 24, 1), (2, F32, 24, 2), (4, F32, 7, 4), (2, F32, 128, 2), (4, F32, 128, 4),
                                                  (2, F32, 200, 2), (1, BF, 260 - 12, 4)])
 def test_state_space_portions_token_by_token(copies, dtype, N, rows):

@@ -42,3 +42,12 @@ def workgroups(source, kernel, threads):
 
 def test_delta_pairs_of_narrow_heads():
     assert workgroups("delta_chunk.hip", "delta_chunk_pair_kernelILi1ELi4E", 512) == 2
+
+
+@pytest.mark.parametrize("PW,NB,scan_wave,want", [(1, 8, 0, 2), (1, 4, 0, 4), (1, 4, 1, 3), (1, 1, 1, 4), (1, 2, 1, 4), (2, 1, 1, 3),
+                                                  (2, 2, 1, 3), (2, 4, 1, 2)])
+def test_state_passes_of_the_chunked_scan(PW, NB, scan_wave, want):
+    """Two of each run at a time, which is what segments are cut for (SSM_WGS), and all of 768 with a wave that only scans; of
+    64 x 128 states all that there can be without it."""
+    kernel = "ssm_chunk_kernelILi%dELi%dELb1ELb%dE" % (PW, NB, scan_wave)
+    assert workgroups("ssm_chunk.hip", kernel, 320 if scan_wave else 256) >= want
