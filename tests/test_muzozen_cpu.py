@@ -277,9 +277,27 @@ def test_delta_split_runs_at_once():
     from llm_map_reduce_summarizer_amd.ops.hip import delta_waves
     for P, N, pairs, want in ((128, 128, 64, (2, 1)), (128, 128, 65, (4, 1)), (128, 65, 128, (4, 1)), (128, 128, 129, (8, 0)),
                               (64, 128, 128, (2, 1)), (64, 128, 129, (4, 1)), (128, 64, 128, (2, 1)), (128, 64, 129, (8, 0)),
-                              (64, 64, 384, (2, 1)), (64, 64, 385, (4, 1)), (32, 64, 9999, (2, 1)), (256, 128, 32, (2, 1)),
-                              (256, 128, 33, (4, 1)), (256, 128, 65, (8, 0)), (64, 256, 1, (4, 0)), (32, 129, 9999, (2, 0))):
+                              (64, 64, 384, (2, 1)), (64, 64, 640, (2, 1)), (64, 32, 384, (2, 1)), (64, 32, 385, (4, 1)),
+                              (32, 64, 9999, (2, 1)), (256, 128, 32, (2, 1)), (256, 128, 33, (4, 1)),
+                              (256, 128, 65, (8, 0)), (64, 256, 1, (4, 0)), (32, 129, 9999, (2, 0)), (32, 256, 256, (4, 0)),
+                              (32, 256, 257, (2, 0))):
         assert delta_waves(P, N, pairs) == want, (P, N, pairs)
+
+
+def test_delta_split_by_the_chains_of_all_segments():
+    """Lengths that differ, in both orders, 32 heads: (value columns, dim, tokens of the segments, blocks and waves)."""
+    from llm_map_reduce_summarizer_amd.ops.hip import DELTA_FORMS, delta_waves
+    for P, N, lens, want in ((128, 128, [4096] + [64] * 4, (2, 1)), (128, 128, [64] * 4 + [4096], (2, 1)),
+                             (128, 128, [4096] * 5, (8, 0)), (128, 128, [2000, 1000, 500, 250], (2, 1)),
+                             (128, 128, [250, 500, 1000, 2000], (2, 1)), (128, 128, [2000] * 4, (4, 1)),
+                             (128, 128, [1000] * 2 + [100] * 6, (4, 1)), (64, 128, [4096] + [64] * 11, (2, 1)),
+                             (128, 64, [64] * 4 + [4096], (2, 1)), (128, 32, [4096] + [64] * 7, (2, 1)),
+                             (64, 256, [4096] + [64] * 11, (4, 0)), (128, 128, [300] * 64, (8, 0)), (128, 128, [300] * 65, (8, 0)),
+                             (128, 128, [4096] + [5] * 70, (4, 1)), (128, 128, [5], (2, 1))):
+        assert delta_waves(P, N, 32 * len(lens), tuple(-(-n // 64) for n in lens)) == want, (P, N, lens)
+    # what mrsum_delta_chunk takes
+    assert all(blocks in (2, 4) or (blocks == 8 and dim <= 128 and not pair) for dim, forms in DELTA_FORMS.items()
+               for blocks, pair in forms)
 
 
 def test_portion_context_places_every_page():
