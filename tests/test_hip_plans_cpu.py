@@ -375,3 +375,12 @@ def test_portion_groups_by_chain_and_load():
                                        (((16, 100),) * 64, 32, 8, 128, 1), (((40, 300),) * 12, 32, 8, 128, 2),
                                        (((400, 0),), 64, 1, 128, 2)):
         assert portion_groups(portions, hq, hkv, d, d) == want, (portions, hq, hkv, d)
+
+
+def test_new_portions_are_walked_once():
+    """Whether they run in tiles and in how many groups are two questions about one walk over them."""
+    portions = tuple((7 + i, 1000 + 3 * i) for i in range(20))
+    before = hip._portion_walks.cache_info().misses
+    hip.portions_in_tiles(portions, 32, 8, 128, 128)
+    hip.portion_groups(portions, 32, 8, 128, 128)
+    assert hip._portion_walks.cache_info().misses == before + 1
