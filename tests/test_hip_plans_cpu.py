@@ -367,13 +367,14 @@ def test_token_ids_of_one_and_many():
 
 
 def test_portion_groups_by_chain_and_load():
-    """On both sides of each line: a chain of 48 keys, all walks on 256 workgroups (512 of heads up to 64), width 128."""
+    """On both sides of each line: a chain of 48 keys, all walks on 333 workgroups (960 of heads up to 64), width 128."""
     from llm_map_reduce_summarizer_amd.ops.hip import portion_groups
     for portions, hq, hkv, d, want in ((((48, 0),), 32, 8, 128, 1), (((49, 0),), 32, 8, 128, 2), (((45, 4),), 32, 8, 128, 2),
-                                       (((1008, 0),), 32, 8, 128, 2), (((1024, 0),), 32, 8, 128, 1), (((1024, 0),), 32, 8, 64, 2),
-                                       (((2032, 0),), 32, 8, 64, 2), (((2048, 0),), 32, 8, 64, 1), (((900, 0),), 32, 8, 132, 1),
+                                       (((1008, 0),), 32, 8, 128, 2), (((1264, 0),), 32, 8, 128, 2), (((1265, 0),), 32, 8, 128, 1),
+                                       (((1024, 0),), 32, 8, 64, 2), (((2032, 0),), 32, 8, 64, 2), (((3760, 0),), 32, 8, 64, 2),
+                                       (((3761, 0),), 32, 8, 64, 1), (((900, 0),), 32, 8, 132, 1), (((24, 76),) * 32, 32, 8, 128, 1),
                                        (((16, 100),) * 64, 32, 8, 128, 1), (((40, 300),) * 12, 32, 8, 128, 2),
-                                       (((400, 0),), 64, 1, 128, 2)):
+                                       (((100, 0),) * 24, 32, 8, 64, 1), (((400, 0),), 64, 1, 128, 2)):
         assert portion_groups(portions, hq, hkv, d, d) == want, (portions, hq, hkv, d)
 
 
@@ -384,3 +385,13 @@ def test_new_portions_are_walked_once():
     hip.portions_in_tiles(portions, 32, 8, 128, 128)
     hip.portion_groups(portions, 32, 8, 128, 128)
     assert hip._portion_walks.cache_info().misses == before + 1
+
+
+def test_portion_groups_by_their_record():
+    """The rule takes what is 0.3 % from the better of the two on average, 13 % at most."""
+    losses = []
+    for e in recorded("row_attention_groups.jsonl"):
+        us = e["us"][hip.portion_groups(tuple(map(tuple, e["portions"])), *e["heads"]) - 1]
+        losses.append(us / min(e["us"]) - 1)
+        assert losses[-1] <= 0.13, e
+    assert len(losses) > 800 and sum(losses) / len(losses) <= 0.003
