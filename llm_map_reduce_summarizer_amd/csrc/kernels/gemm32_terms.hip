@@ -9,10 +9,10 @@
 // normal numbers (whose products the instruction forms with fewer bits), or if X has a value whose lowest bits would be finer than
 // bf16's (below 2^-110), a flag is set and the fp32 instruction's form (gemm32.hip), which is launched behind and otherwise only adds
 // slices, makes the whole result.  A workgroup that sees it in its first K-tile or its rows of X stops there, others when their next
-// chain of 16 K-tiles ends.  What that costs, us, all in turn with rotating weights: 903 x 28672 x 4096 on the fp32 instruction 1593, by way of
-// here with 24 bits in all of W 1597, in half of its rows 1614 (2100 where nobody asks the others), in half of its columns 1697, in its
-// last value alone 2099; 160 x 6144 x 4096 75, 98, 113, 119, 126.  Each timed by itself the instruction takes 1548 there, and 24 bits in
-// all of W 1611.  What a model has loaded carries the answer and does not come here (ops/hip.py gemm32).
+// chain of 16 K-tiles ends.  What that costs, us, all in turn with rotating weights: 903 x 28672 x 4096 on the fp32 instruction 1603, by way of
+// here with 24 bits in all of W 1577, in half of its rows 1598 (500 more where nobody asks the others), in half of its columns 1669, in its
+// last value alone 2078; 160 x 6144 x 4096 75, 86, 101, 109, 115.  Each timed by itself the instruction takes 1536 at the former, and 24
+// bits in all of W 1577.  What a model has loaded carries the answer and does not come here (ops/hip.py gemm32).
 //
 // Relative error (2-norm, random operands, K 4096 - 22528, chains of 16 K-tiles on both): 2.4e-7, the fp32 instruction 4.1e-7, as one
 // sum takes the products of 32 columns and not of four.
@@ -29,8 +29,8 @@
 //     wave for four.
 //   * what is looked at in W takes a fifth of the instructions beside the products: each of the two waves that have the same columns
 //     looks at half of them.  With the smallest value of all columns looked for in both, 903 x 4096 x 14336 took 8 % longer.
-// us, fp32 instruction -> this: 903 x 28672 x 4096 1550 -> 586, 903 x 4096 x 14336 808 -> 327, 300 x 20608 x 4096 432 -> 175, 160 x
-// 28672 x 4096 290 -> 153 (where W's arrival is all).  Which rows and shapes: ops/hip.py gemm32_terms.
+// us, fp32 instruction -> this: 903 x 28672 x 4096 1518 -> 564, 903 x 4096 x 14336 787 -> 315, 300 x 20608 x 4096 421 -> 165, 160 x
+// 28672 x 4096 291 -> 151 (where W's arrival is all).  Which rows and shapes: ops/hip.py gemm32_terms.
 #include "gemm32.h"
 
 #include <type_traits>

@@ -240,7 +240,8 @@ def test_fp32_gemm_of_short_k_by_its_record():
 
 def test_fp32_gemm_in_terms_by_its_record():
     """The plan is the record's and near the best of each shape; the rule takes terms only where they are no slower than the fp32
-    instruction by more than 4 %, and loses 1.5 % on average against the best plan of the two."""
+    instruction, and loses 0.7 % on average against the best plan of the two, 15 % at most.  (W of 24 bits costs up to 60 us
+    and 38 %, or 10 %.)"""
     plans, losses = [], []
     for e in recorded("gemm32_terms.jsonl"):
         plan = hip.gemm32_terms(e["M"], e["N"], e["K"] // 32)
@@ -250,14 +251,15 @@ def test_fp32_gemm_in_terms_by_its_record():
         if e["M"] > 64:
             assert "%d/%d/%d" % hip._gemm32_terms_plan(e["M"], e["N"], e["K"] // 32)[:3] == e["plan"], e
             plans.append(e["us"][e["plan"]] / best - 1)
-            assert plans[-1] <= 0.21, e
+            assert plans[-1] <= 0.14, e
         if e["rule"]:
             assert "%d/%d/%d" % plan[:3] == e["plan"]
             took = e["us"][e["plan"]]
-            assert took <= 1.04 * e["fp32"], e
+            assert took <= e["fp32"] and e["bits24"] <= e["fp32"] + max(min(60, 0.38 * e["fp32"]), 0.1 * e["fp32"]), e
         if e["M"] > 64:
             losses.append(took / min(best, e["fp32"]) - 1)
-    assert len(plans) > 300 and sum(plans) / len(plans) <= 0.015 and sum(losses) / len(losses) <= 0.016
+            assert losses[-1] <= 0.15, e
+    assert len(plans) > 500 and sum(plans) / len(plans) <= 0.007 and sum(losses) / len(losses) <= 0.007
 
 
 @pytest.mark.parametrize("M,K,tiles,whole,splits", [(32, 512, 1, 1, 1), (65, 0, 1, 1, 1), (65, 512, 2, 1, 1), (161, 512, 1, 1, 1),
