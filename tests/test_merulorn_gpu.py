@@ -670,6 +670,42 @@ def test_row_attention_portions_infinite_value_of_a_tile(key, dk, dv, monkeypatc
     assert rel(got[~hit], want[~hit]) < 2e-6
 
 
+def in_two_groups(monkeypatch):
+    """Tiles of portions with two groups of waves on a block's keys, whatever portion_groups says; a list that fills as they run."""
+    from llm_map_reduce_summarizer_amd.ops import hip
+    fn, ran = hip._fn, []
+
+    def portions(*args):
+        ran.append(args[-2])
+        return fn("mrsum_attn_portions")(*args[:-2], 2, args[-1])
+    monkeypatch.setattr(hip, "_fn", lambda name: portions if name == "mrsum_attn_portions" else fn(name))
+    return ran
+
+
+@pytest.mark.parametrize("H,G,dk,dv", [(8, 2, 48, 32), (6, 2, 128, 100), (5, 5, 64, 64), (70, 1, 16, 8), (70, 1, 100, 128)])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_row_attention_portions_in_two_groups(H, G, dk, dv, dtype, monkeypatch):
+    """More than one block of heads, keys and values of different widths."""
+    ran = in_two_groups(monkeypatch)
+    test_row_attention_portions(H, G, dk, dv, dtype, monkeypatch)
+    assert ran
+
+
+@pytest.mark.parametrize("H,G,dk,dv", [(8, 2, 128, 128), (70, 1, 64, 64)])
+def test_row_attention_portions_without_keys_in_two_groups(H, G, dk, dv, monkeypatch):
+    ran = in_two_groups(monkeypatch)
+    test_row_attention_portions_without_keys(H, G, dk, dv, monkeypatch)
+    assert ran
+
+
+@pytest.mark.parametrize("key", [31, 32, 65, 97, 130])
+@pytest.mark.parametrize("dk,dv", [(128, 128), (64, 40)])
+def test_row_attention_portions_infinite_value_of_a_tile_in_two_groups(key, dk, dv, monkeypatch):
+    ran = in_two_groups(monkeypatch)
+    test_row_attention_portions_infinite_value_of_a_tile(key, dk, dv, monkeypatch)
+    assert ran
+
+
 @pytest.mark.parametrize("M,N,K,split", [(1, 130, 1024, True), (17, 1023, 2048, True), (129, 2062, 512, True),
                                          (500, 8200, 256, True), (1100, 4096, 128, False), (3, 40000, 64, False)])
 def test_gemm32_edges(M, N, K, split, monkeypatch):
