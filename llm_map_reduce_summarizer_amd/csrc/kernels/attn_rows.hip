@@ -158,11 +158,12 @@ MRSUM_API int mrsum_attn_rows(const void* q, const void* kc, const void* vc, con
 
 // ------------------------------------------------------------------------------------------------ prompt portions
 // The same attention for many rows of few sequences, on the fp32 matrix instruction.  The row kernel reads every key
-// from memory for every (row, head): 1088 us for 900 rows of 32 heads of 128 over 8 kv heads, 4380 over 576-wide latents.
-// Here (112 and 520 us; bound by the chain of the block with the most keys, 5 us a tile of which its products are 1.7) 64
+// from memory for every (row, head): 1018 us for 900 rows of 32 heads of 128 over 8 kv heads, 4390 over 576-wide latents.
+// Here (107 and 508 us; bound by the chain of the block with the most keys: 5 us a tile of which its products are 1.7 where one
+// group of waves walks it, 8 us for two tiles at once where two do, 9 us for one of 16 latents) 64
 // (row, head) pairs -- RB consecutive rows of HB heads of one kv head -- share key and value tiles of 32 in LDS (two buffers,
 // the next tile on its way in registers), a wave for 16 pairs.  With the page ids read when a tile is fetched, its loads
-// behind tests of the row and two barriers a tile, 183 and 758 (16-bit caches 201 and 915, now 167 and 570).
+// behind tests of the row and two barriers a tile, 183 and 758 (16-bit caches 201 and 915, now 111 and 561).
 //
 // Scores are computed transposed, S^T = K Q^T: lane (pair = lane & 15, g = lane >> 4) holds the scores of keys 4 g .. 4 g
 // + 3 of a 16-key block, which is how the second product O^T = V^T P^T takes its right operand, so weights stay in
@@ -172,7 +173,7 @@ MRSUM_API int mrsum_attn_rows(const void* q, const void* kc, const void* vc, con
 // steps leave no registers for a larger tile on its way.
 // KS 2: two groups of four waves take the tiles in turn, with buffers and sums of their own that meet in LDS at the end, so that
 // the block with the most keys walks half of them.  They take the place of two workgroups of a CU (8 us for a tile each where one
-// alone takes 5).  900 rows, 32 / 8 heads of 128 in fp32: 158 us, by the order of the blocks 148, with two groups 112; error
+// alone takes 5).  900 rows, 32 / 8 heads of 128 in fp32: 158 us, by the order of the blocks 143 - 148, with two groups 107 - 112; error
 // against fp64 6.7e-7 and 5.4e-7.  When: ops/hip.py portion_groups.
 template <typename T, int NQ, int NV, bool SHARED, int KT, int KS>
 __global__ __launch_bounds__(256 * KS, NQ <= 8 ? 2 : 1) void attn_portion_kernel(

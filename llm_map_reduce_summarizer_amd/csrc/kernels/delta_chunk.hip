@@ -514,8 +514,8 @@ __global__ __launch_bounds__(64 * WPB, 1) void delta_chunk_kernel(const bf16* __
 // rows into a second set of LDS images.  The state reaches it as finished operands through LDS, U as it is: two barriers a
 // chunk.  What bounds the chain are its instructions, five cycles each in a lone wave of a SIMD: with staging, conversions of
 // one value at a time and results copied between the two halves of the register file they were 1010 a chunk of 64 x 128,
-// 3.1 us, and are 570, 1.9 us.  One prompt of 4096 tokens, 32 heads of 128 x 128, with the preparation: 199.5 -> 150.5 us; 16
-// heads of 64 x 64 123 -> 111 (with staging left to all waves 123).  The bound of 512 threads keeps the registers to 256, so
+// 2.7 us, and are 570, 1.95 us.  One prompt of 4096 tokens, 32 heads of 128 x 128 in two blocks, this launch: 177 -> 125 us, the preparation
+// 28 (four blocks 202 -> 174); 16 heads of 64 x 64 132 -> 94, the preparation 16 (with staging left to all waves 12 us longer).  The bound of 512 threads keeps the registers to 256, so
 // that products stay where the vector instructions reach them.  Of dim up to 32 in four blocks the bound of four waves a SIMD
 // keeps them to 128, for two workgroups on a CU (one with the 148 that it would take): dim 32, value columns 128, 192 (segment, head)
 // pairs of 300 tokens 42.6 -> 39.0 us, 64 columns, 512 pairs 67.3 -> 64.7, dim 24, of 1000 tokens 201 -> 195.

@@ -125,8 +125,8 @@ ssm_chunk_kernel(const ChunkArgs a) {
     }
     // The raw step sizes of a chunk become dt, the running sum and the update weights beside the chunk before, in a wave that
     // updates the state (it has half the products of one that makes output rows) or, where all do, in one of its own if SCAN_WAVE:
-    // between the chunk's two barriers only their stores are left.  All of it there made every wave wait for seven exchanges of
-    // lanes one after the other.
+    // between the chunk's two barriers only their stores are left, and the update weights' one exchange of lanes and
+    // exponential.  All of it there made every wave wait for seven exchanges one after the other.
     const float an = a.a_neg[head] * LOG2E, db = a.dt_bias[head];
     float dtr = 0.f, cum = 0.f;
 #define LOAD_DT(T0)                                                                                     \

@@ -139,12 +139,12 @@ def test_narrow_gate_up_split_rules():
 
 @pytest.mark.parametrize("portions,hkv,tiles", [
     # 32 heads of 128: row kernel and tiles, us (profiles/row_attention_portions.jsonl)
-    ([(2, 1998)] * 32, 32, False),  # 775, 9457: 32 contexts in one workgroup's chain
-    ([(2, 1998)] * 32, 8, False),   # 639, 2374
-    ([(8, 1992)] * 32, 8, True),    # 1509, 612
-    ([(16, 584)] * 8, 32, False),   # 237, 371
-    ([(32, 568)] * 8, 32, True),    # 427, 192
-    ([(900, 0)], 8, True),          # 1088, 183
+    ([(2, 1998)] * 32, 32, False),  # 769, 6117: 32 contexts in one workgroup's chain
+    ([(2, 1998)] * 32, 8, False),   # 636, 1533
+    ([(8, 1992)] * 32, 8, True),    # 1478, 404
+    ([(16, 584)] * 8, 32, False),   # 236, 255
+    ([(32, 568)] * 8, 32, True),    # 431, 134
+    ([(900, 0)], 8, True),          # 1018, 107
     ([(900, 0), (2, 30)], 8, True)])
 def test_row_attention_of_short_portions(portions, hkv, tiles, monkeypatch):
     """Prompt portions go to the tiled kernel where it leads: not where a workgroup would walk many contexts."""
