@@ -389,6 +389,16 @@ def test_new_portions_are_walked_once():
     assert hip._portion_walks.cache_info().misses == before + 1
 
 
+def test_delta_splits_by_their_record():
+    """The rule takes what is 0.2 % from the best of the forms on average, 10 % at most."""
+    losses = []
+    for e in recorded("delta_splits.jsonl"):
+        form = hip.delta_waves(e["vdim"], e["dim"], e["heads"] * len(e["lens"]), tuple(-(-n // 64) for n in e["lens"]))
+        losses.append(e["us"]["%d/%d" % form] / min(e["us"].values()) - 1)
+        assert losses[-1] <= 0.1, e
+    assert len(losses) > 1400 and sum(losses) / len(losses) <= 0.002
+
+
 def test_portion_groups_by_their_record():
     """The rule takes what is 0.3 % from the better of the two on average, 13 % at most."""
     losses = []
