@@ -240,8 +240,8 @@ def test_fp32_gemm_of_short_k_by_its_record():
 
 def test_fp32_gemm_in_terms_by_its_record():
     """The plan is the record's and near the best of each shape; the rule takes terms only where they are no slower than the fp32
-    instruction, and loses 0.7 % on average against the best plan of the two, 15 % at most.  (W of 24 bits costs up to 60 us
-    and 38 %, or 10 %.)"""
+    instruction, and loses 0.9 % on average against the best plan of the two, 16 % at most.  (W of 24 bits costs up to 60 us
+    and 33 %, or 10 %.)"""
     plans, losses = [], []
     for e in recorded("gemm32_terms.jsonl"):
         plan = hip.gemm32_terms(e["M"], e["N"], e["K"] // 32)
@@ -255,11 +255,11 @@ def test_fp32_gemm_in_terms_by_its_record():
         if e["rule"]:
             assert "%d/%d/%d" % plan[:3] == e["plan"]
             took = e["us"][e["plan"]]
-            assert took <= e["fp32"] and e["bits24"] <= e["fp32"] + max(min(60, 0.38 * e["fp32"]), 0.1 * e["fp32"]), e
+            assert took <= e["fp32"] and e["bits24"] <= e["fp32"] + max(min(60, 0.33 * e["fp32"]), 0.1 * e["fp32"]), e
         if e["M"] > 64:
             losses.append(took / min(best, e["fp32"]) - 1)
-            assert losses[-1] <= 0.15, e
-    assert len(plans) > 500 and sum(plans) / len(plans) <= 0.007 and sum(losses) / len(losses) <= 0.007
+            assert losses[-1] <= 0.16, e
+    assert len(plans) > 500 and sum(plans) / len(plans) <= 0.007 and sum(losses) / len(losses) <= 0.009
 
 
 @pytest.mark.parametrize("M,K,tiles,whole,splits", [(32, 512, 1, 1, 1), (65, 0, 1, 1, 1), (65, 512, 2, 1, 1), (161, 512, 1, 1, 1),
