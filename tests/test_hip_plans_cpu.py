@@ -410,12 +410,13 @@ def test_portion_groups_by_their_record():
 
 
 def test_portions_in_tiles_by_their_record():
-    """The rule takes what is 0.6 % from the better of the two on average, 51 % at most (16 us)."""
+    """The rule takes what is 0.9 % from the better of the two on average, 69 % at most (40 % in fp32)."""
     losses = []
     for e in recorded("row_attention_portions.jsonl"):
         p = e["portions"]
         p = tuple((n, first) for count, n, first in p for _ in range(count)) if e["form"] == "sweep" else tuple(map(tuple, p))
-        took = e["tiles_us"] if hip.portions_in_tiles(p, *e["heads"]) else e["rows_us"]
+        half = e["dtype"] == "bf16" if e["form"] == "types" else 128 < max(e["heads"][2:]) <= 256
+        took = e["tiles_us"] if hip.portions_in_tiles(p, *e["heads"], half) else e["rows_us"]
         losses.append(took / min(e["tiles_us"], e["rows_us"]) - 1)
-        assert losses[-1] <= 0.51, e
-    assert len(losses) > 700 and sum(losses) / len(losses) <= 0.006
+        assert losses[-1] <= (0.69 if half else 0.41), e
+    assert len(losses) > 1800 and sum(losses) / len(losses) <= 0.0086
